@@ -255,6 +255,9 @@ struct spk_handle {
     DBuf<int> ca, cb, ba, bb;
     DBuf<NearTask> ta, tb;
     DBuf<zd> kt, zz;
+    // the triangle kernel: sides of each triangle's corners, per-box lists
+    DBuf<int> tside, tcnt;
+    DBuf<int4> tlist;
   } nw;
   spk_stats stats{};
   ~spk_handle() {
@@ -293,6 +296,65 @@ NearArgs near_args(const spk_handle *h) {
   return a;
 }
 
+// The block's coefficients for the triangle kernel, or false where it does not
+// apply: formulations with normal components or with each medium's own K,
+// other rules than the three-point one, and surfaces of more than some
+// thousand wavelengths (side D), beyond sincos_near's arguments.
+bool make_tri_form(const NearArgs &a, double D, TriForm *q) {
+  if (a.ngp != 3) return false;
+  for (int i = 0; i < 3; ++i)
+    if (a.qa[i] != kTri3.a[i] || a.qb[i] != kTri3.b[i] || a.qw[i] != kTri3.w) return false;
+  if (a.form != SPK_PMCHWT && a.form != SPK_MCTF && a.form != SPK_PMCHWT_S && a.form != SPK_ICTF)
+    return false;
+  if (!(4.0 * D * std::max(std::fabs(a.mat.k1.re), std::fabs(a.mat.k2.re)) < 1e5)) return false;
+  // assemble_zz, accumulate_D and finish_D of these formulations in one step
+  const zd e1 = zcx(a.mat.eta1), e2 = zcx(a.mat.eta2), ea = zcx(a.mat.eta_a), one = {1.0, 0.0};
+  const zd k[2] = {zcx(a.mat.k1), zcx(a.mat.k2)};
+  for (int m = 0; m < 2; ++m) {
+    q->k4[m] = k[m] * 0.25;
+    q->ik[m] = one / k[m];
+  }
+  zd a1 = e1, a2 = e2, b = -one, c = one, d1 = one / e1, d2 = one / e2;
+  if (a.form == SPK_ICTF) {
+    a1 = e1 / ea;
+    a2 = e2 / ea;
+    b = -one / ea;
+    c = ea;
+    d1 = ea / e1;
+    d2 = ea / e2;
+  } else if (a.form == SPK_MCTF) {
+    c = e1 * e2;
+    d1 = e2;
+    d2 = e1;
+  } else if (a.form == SPK_PMCHWT_S) {
+    b = -e1;
+    c = -e1;
+    d1 = e1;
+    d2 = e1 * e1 / e2;
+  }
+  const zd cc[6] = {a1, a2, b, c, d1, d2};
+  for (int i = 0; i < 6; ++i) q->c[i] = cc[i];
+  return true;
+}
+
+// side (2 edge + s) opposite each local corner of every triangle, -1 where
+// it has none; false where a corner has two (more than two triangles meet in
+// an edge): then k_near_regular fills the blocks
+bool tri_sides(const spk_handle *h, std::vector<int> *out) {
+  int nt = 0;
+  for (const ElemRec &e : h->er) nt = std::max(nt, e.elem + 1);
+  out->assign(3 * (size_t)nt, -1);
+  for (size_t s = 0; s < h->er.size(); ++s) {
+    const int *cr = &h->corner[s & ~(size_t)1];
+    const int *nd = h->er[s].node;
+    const int p = nd[0] != cr[0] && nd[0] != cr[1] ? 0 : nd[1] != cr[0] && nd[1] != cr[1] ? 1 : 2;
+    int &o = (*out)[3 * (size_t)h->er[s].elem + p];
+    if (o >= 0) return false;
+    o = (int)s;
+  }
+  return true;
+}
+
 int near_fill(spk_handle *h) {
   const int64_t nnz = h->tree.nnz;
   HIPCHK(h->d_blocks.alloc(4 * (size_t)nnz));
@@ -325,7 +387,17 @@ int near_fill(spk_handle *h) {
   launch_near_emit(a, nnz, cls.p, ba.p, bb.p, ta.p, tb.p, h->st);
   launch_near_edge(a, nb, tb.p, kt.p, h->st);
   launch_near_singular(a, na, ta.p, cls.p, bb.p, kt.p, zz.p, h->st);
-  launch_near_regular(a, nnz, cls.p, ba.p, zz.p, h->d_blocks.p, h->st);
+  TriForm tf;
+  std::vector<int> tside;
+  if (make_tri_form(a, h->tree.D, &tf) && tri_sides(h, &tside)) {
+    HIPCHK(NW.tside.upload(tside));
+    HIPCHK(NW.tlist.alloc(2 * h->tree.e2_list.size()));
+    HIPCHK(NW.tcnt.alloc(h->tree.e2_list.size()));
+    launch_near_tri(a, tf, h->N, h->spmv_wgs, h->d_row_box.p, h->d_row_r0.p, NW.tside.p,
+                    NW.tlist.p, NW.tcnt.p, cls.p, ba.p, zz.p, h->d_blocks.p, h->st);
+  } else {
+    launch_near_regular(a, nnz, cls.p, ba.p, zz.p, h->d_blocks.p, h->st);
+  }
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->st));
   h->stats.singular_pairs = na;

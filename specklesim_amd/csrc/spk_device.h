@@ -87,6 +87,55 @@ void launch_near_singular(const NearArgs &a, int ntask, const NearTask *ta, cons
                           const int *base_b, const zd *kt, zd *zz, hipStream_t st);
 void launch_near_regular(const NearArgs &a, int64_t nnz, const uint8_t *cls, const int *base_a,
                          const zd *zz, zd *blocks, hipStream_t st);
+// The three-point rule (quadrature_tri, single-precision abscissae) in the
+// frame (corner 0, e1, e2) of a triangle, point i near corner i.  Side p (free
+// vertex: corner p) has its point i at lb + dl[p][i] and at mu[p][i] from its
+// free vertex.
+struct TriRule {
+  double lb1[3], lb2[3];        // points of side 0
+  double dl1[3][3], dl2[3][3];  // side p's points from side 0's
+  double mu1[3][3], mu2[3][3];
+  double a[3], b[3], w, w2;     // the rule itself, its weight squared
+};
+constexpr TriRule tri_rule() {
+  constexpr double lo = 0.16666666666667f, hi = 0.66666666666667f, w = 0.33333333333333f;
+  TriRule q{{}, {}, {}, {}, {}, {}, {lo, lo, hi}, {lo, hi, lo}, w, w * w};
+  for (int p = 0; p < 3; ++p)
+    for (int r = 0; r < 3; ++r) {
+      // weights of the triangle's corners: the side's (p1, p2, free) are p + 1, p + 2, p
+      double lam[3] = {};
+      lam[(p + 1) % 3] = 1 - q.a[r] - q.b[r];
+      lam[(p + 2) % 3] = q.a[r];
+      lam[p] = q.b[r];
+      const int i = (p + (r == 0 ? 1 : r == 1 ? 0 : 2)) % 3;
+      if (p == 0) {
+        q.lb1[i] = lam[1];
+        q.lb2[i] = lam[2];
+      }
+      q.dl1[p][i] = lam[1];
+      q.dl2[p][i] = lam[2];
+    }
+  for (int p = 0; p < 3; ++p)
+    for (int i = 0; i < 3; ++i) {
+      q.mu1[p][i] = q.dl1[p][i] - (p == 1 ? 1.0 : 0.0);
+      q.mu2[p][i] = q.dl2[p][i] - (p == 2 ? 1.0 : 0.0);
+      q.dl1[p][i] -= q.lb1[i];
+      q.dl2[p][i] -= q.lb2[i];
+    }
+  return q;
+}
+inline constexpr TriRule kTri3 = tri_rule();
+// The near blocks of a formulation from T of both media and K: D11 = c0 T1 +
+// c1 T2, D12 = c2 K, D21 = c3 K, D22 = c4 T1 + c5 T2
+struct TriForm {
+  zd k4[2], ik[2];  // k / 4 and 1 / k of the media
+  zd c[6];
+};
+constexpr int kTriCols = 1024;  // columns per LDS chunk
+void launch_near_tri(const NearArgs &a, const TriForm &q, int N, int tiles, const int *row_box,
+                     const int *row_r0, const int *tri_side, int4 *list, int *cnt,
+                     const uint8_t *cls, const int *base_a, const zd *zz, zd *blocks,
+                     hipStream_t st);
 hipError_t exclusive_scan_int(const int *in, int *out, int64_t n, void **tmp, size_t *tmp_bytes,
                         hipStream_t st);
 

@@ -657,6 +657,322 @@ __global__ void __launch_bounds__(256) k_near_regular(NearArgs A, int64_t nnz, c
   for (int k = 0; k < 4; ++k) blocks[4 * g + k] = D[k];
 }
 
+// ---------------------------------------------------------------------------
+// The regular pairs of the formulations whose K enters as the sum of both
+// media (PMCHWT, MCTF, PMCHWT-S, ICTF) under the three-point rule.
+//
+// k_near_regular is bound by the FP64 vector ALU: a thread per block
+// evaluates 36 pairs of quadrature points, and the nine combinations of two
+// triangles' sides evaluate the same Green's functions nine times.  Here a
+// thread takes (test edge m, source triangle S): 18 point pairs serve the
+// blocks of all three edges of S.  Two identities make that cheap.
+//  * With u = ra - c_m, v = rq - c_n (c: free vertices) and c = c_m - c_n,
+//    f_m . f_n is a multiple of u . v and f_m . (f_n x R) of u . (v x c), so
+//    a point pair adds G, (u.v) G and (v.(c x u)) G'/R per medium to three
+//    complex sums, with u.v and v.(c x u) two-term sums over S's edge vectors.
+//  * The rule's abscissae are single-precision numbers, so the points of S's
+//    three sides differ by 3e-8 of an edge.  The Green's functions are taken
+//    at side 0's points and moved to the others' by one Taylor term; the
+//    next one is of order 1e-16.
+// Each block gets two contributions (its column edge's two triangles), added
+// to a zero in LDS by FP64 atomics: a + b = b + a, so the result does not
+// depend on their order.  Singular pairs come from the task kernels.
+//
+// Measured on 28.3M blocks (10 x 10 wavelengths, 29,800 edges): 4.25 ms, where
+// a thread per block took 15.9 ms.  Bound by the FP64 ALU at two waves per
+// SIMD (256 registers: 30 of the 128 doubles are sums); three waves spilled
+// and took 11.4 ms, the rule's constants loaded from memory 5.3 ms.
+// ---------------------------------------------------------------------------
+// Triangles of a box's columns, per chunk of kTriCols columns: entry (side of
+// each local corner or -1, the three local columns in 10 bits each), made by
+// the thread of the triangle's first edge in the chunk.
+__global__ void __launch_bounds__(256) k_near_tri_list(const int *e2_off, const int *e2_list,
+                                                       const ElemRec *er, const int *tri_side,
+                                                       int4 *list, int *cnt) {
+  __shared__ int col[kTriCols];
+  __shared__ int nout;
+  const int b = blockIdx.x;
+  const int c0 = e2_off[b], cols = e2_off[b + 1] - c0;
+  for (int cc = 0; cc < cols; cc += kTriCols) {
+    const int nc = min(kTriCols, cols - cc);
+    if (threadIdx.x == 0) nout = 0;
+    for (int c = threadIdx.x; c < nc; c += blockDim.x) col[c] = e2_list[c0 + cc + c];
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * nc; i += blockDim.x) {
+      const int n = col[i >> 1];
+      const int S = er[2 * n + (i & 1)].elem;
+      int sd[3], at[3];
+      bool first = true;
+      for (int r = 0; r < 3; ++r) {
+        sd[r] = tri_side[3 * S + r];
+        at[r] = 0;
+        if (sd[r] < 0) continue;
+        const int e = sd[r] >> 1;
+        int lo = 0, hi = nc - 1, f = -1;
+        while (lo <= hi) {
+          const int md = (lo + hi) >> 1, v = col[md];
+          if (v == e) {
+            f = md;
+            break;
+          }
+          if (v < e) lo = md + 1;
+          else hi = md - 1;
+        }
+        if (f < 0) sd[r] = -1;
+        else at[r] = f;
+        if (f >= 0 && e < n) first = false;
+      }
+      if (first) {
+        const int o = atomicAdd(&nout, 1);
+        list[2 * (size_t)(c0 + cc) + o] = int4{sd[0], sd[1], sd[2], at[0] | at[1] << 10 | at[2] << 20};
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) cnt[c0 + cc] = nout;
+    __syncthreads();
+  }
+}
+
+// a * b + c with c in scalar registers: the compiler copies a constant addend
+// to vector registers for every step of a polynomial
+__device__ inline double fma_sc(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+// sin and cos of |x| < 1e5: one quarter turn subtracted in two parts, Taylor
+// series to r^17 and r^16 on |r| <= pi/4 (truncation 1e-19 and 2e-18).  The
+// library's sincos carries the reduction of any argument, whose registers
+// spill in the fill kernels.
+__device__ inline void sincos_near(double x, double *sn, double *cs) {
+  const double n = rint(x * 0.63661977236758134308);
+  double r = fma(-n, 1.5707963267948965580, x);
+  r = fma(-n, 6.123233995736766036e-17, r);
+  const double z = r * r;
+  double s = fma_sc(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
+  double c = fma_sc(z, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+  s = fma_sc(s, z, 1.0 / 6227020800.0);
+  c = fma_sc(c, z, 1.0 / 479001600.0);
+  s = fma_sc(s, z, -1.0 / 39916800.0);
+  c = fma_sc(c, z, -1.0 / 3628800.0);
+  s = fma_sc(s, z, 1.0 / 362880.0);
+  c = fma_sc(c, z, 1.0 / 40320.0);
+  s = fma_sc(s, z, -1.0 / 5040.0);
+  c = fma_sc(c, z, -1.0 / 720.0);
+  s = fma_sc(s, z, 1.0 / 120.0);
+  c = fma_sc(c, z, 1.0 / 24.0);
+  s = fma_sc(s, z, -1.0 / 6.0);
+  c = fma(c, z, -0.5);
+  s = fma(s * z, r, r);
+  c = fma(c, z, 1.0);
+  const int q = (int)n;
+  const double a = (q & 1) ? c : s, b = (q & 1) ? s : c;
+  *sn = (q & 2) ? -a : a;
+  *cs = ((q + 1) & 2) ? -b : b;
+}
+// 1 / sqrt(x): the instruction's approximation and one third-order step
+__device__ inline double rsqrt_near(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// a singular pair's zz into its block; s: the column side (PMCHWT-S
+// alternates the sign of D21 with the pairs' order).  PMCHWT's and MCTF's D21
+// follows from D12 in finish_tri.
+__device__ inline void add_zz(const NearArgs &A, zd *D, const zd *zz, int s) {
+  D[0] = D[0] + zz[0];
+  D[1] = D[1] + zz[1];
+  if (A.form == SPK_ICTF) {
+    D[2] = D[2] + zz[2];
+    D[3] = D[3] + zz[3];
+  } else {
+    if (A.form == SPK_PMCHWT_S) D[2] = s ? D[2] + zz[1] : D[2] - zz[1];
+    D[3] = D[3] + zz[2];
+  }
+}
+__device__ inline void finish_tri(const NearArgs &A, zd *D) {
+  if (A.form == SPK_PMCHWT) D[2] = -D[1];
+  if (A.form == SPK_MCTF) {
+    const zd e12 = zcx(A.mat.eta1) * zcx(A.mat.eta2);
+    D[2] = -D[1] * e12;
+    D[3] = D[3] * e12;
+  }
+  finish_D(A, D);
+}
+
+// workgroup = (box, rp rows of one of its row tiles); LDS per column: T of
+// both media and K, for PMCHWT-S also K with the column side's sign.  LOSSY: a
+// medium's wavenumber is complex.
+template <int NV, bool LOSSY>
+__global__ void __launch_bounds__(256, 2) k_near_tri(NearArgs A, TriForm Q, const int *row_box,
+                                                     const int *row_r0, int rp, const int4 *list,
+                                                     const int *cnt, const uint8_t *cls,
+                                                     const int *base_a, const zd *zz, zd *blocks) {
+  extern __shared__ double acc[];  // [column][2 * NV]
+  const int b = row_box[blockIdx.x];
+  const int rA = row_r0[blockIdx.x] + blockIdx.y * rp;
+  const int rB = min(min(rA + rp, row_r0[blockIdx.x] + kSpmvRowsPerWG), A.box_count[b]);
+  if (rA >= rB) return;
+  const int c0 = A.e2_off[b], cols = A.e2_off[b + 1] - c0;
+  const zd kk[2] = {zcx(A.mat.k1), zcx(A.mat.k2)};
+  for (int cc = 0; cc < cols; cc += kTriCols) {
+    const int nc = min(kTriCols, cols - cc), nS = cnt[c0 + cc];
+    const int4 *L = list + 2 * (size_t)(c0 + cc);
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc * 2 * NV; i += blockDim.x) acc[i] = 0.0;
+    __syncthreads();
+    for (int r = rA; r < rB; ++r) {
+      const int m = A.perm[A.box_first[b] + r];
+      const int64_t g0 = A.near_off[b] + (int64_t)r * cols + cc;
+      for (int it = threadIdx.x; it < nS; it += blockDim.x) {
+        const int4 en = L[it];
+        const int r0 = en.x >= 0 ? 0 : en.y >= 0 ? 1 : 2;
+        const int s0 = r0 == 0 ? en.x : r0 == 1 ? en.y : en.z;
+        const unsigned sing = cls[g0 + ((en.w >> (10 * r0)) & 1023)] >> (s0 & 1);
+        const FnRec &fs = A.fn[s0];
+        // side r0's corners (p1, p2, free) are the triangle's r0 + 1, r0 + 2, r0
+        const int w0 = r0 == 0 ? 2 : r0 == 1 ? 1 : 0, w1 = r0 == 0 ? 0 : r0 == 1 ? 2 : 1;
+        const int w2 = 3 - w0 - w1;
+        double q0[3], e1[3], e2[3];
+        for (int k = 0; k < 3; ++k) {
+          q0[k] = fs.c[3 * w0 + k];
+          e1[k] = fs.c[3 * w1 + k] - q0[k];
+          e2[k] = fs.c[3 * w2 + k] - q0[k];
+        }
+        zd S0[3][2], S1[3][2], SK[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          S0[p][0] = S0[p][1] = S1[p][0] = S1[p][1] = SK[p] = zd{0, 0};
+#pragma unroll 1
+        for (int t = 0; t < 2; ++t) {
+          if ((sing >> (2 * t)) & 1u) continue;
+          const FnRec &fm = A.fn[2 * m + t];
+          const double fac = kTri3.w2 * fm.area * fm.df * (1.0 / (4 * PI));
+#pragma unroll 1
+          for (int j = 0; j < 3; ++j) {
+            double ra[3];
+            simplex(A.qa[j], A.qb[j], fm.c, ra);
+            double ue1, ue2, P1[3], P2[3];
+            {
+              double u[3], x[3];
+              for (int k = 0; k < 3; ++k) u[k] = ra[k] - fm.c[6 + k];
+              ue1 = dot3(u, e1);
+              ue2 = dot3(u, e2);
+              cross3(e1, e2, x);
+              const double un = dot3(u, x);
+              const double d0[3] = {fm.c[6] - q0[0], fm.c[7] - q0[1], fm.c[8] - q0[2]};
+              cross3(d0, u, x);
+              // v.(c x u) = mu1 e1.(c x u) + mu2 e2.(c x u) for v = mu1 e1 + mu2 e2
+              P1[0] = P1[1] = dot3(e1, x);
+              P2[0] = P2[2] = dot3(e2, x);
+              P1[2] = P1[0] - un;
+              P2[1] = P2[0] + un;
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              double R[3];
+              for (int k = 0; k < 3; ++k)
+                R[k] = ra[k] - (q0[k] + kTri3.lb1[i] * e1[k] + kTri3.lb2[i] * e2[k]);
+              const double R2 = dot3(R, R), rinv = rsqrt_near(R2), Rl = R2 * rinv;
+              const double g4 = rinv * fac, rinv2 = rinv * rinv;
+              const double Re1 = dot3(R, e1), Re2 = dot3(R, e2);
+              zd G[2], D[2], Fs;
+#pragma unroll
+              for (int md = 0; md < 2; ++md) {
+                // G, D = G'/R and F = D'/R
+                const double x = kk[md].x * Rl;
+                double sn, cs;
+                sincos_near(x, &sn, &cs);
+                zd f;
+                if (LOSSY) {
+                  const double y = kk[md].y * Rl, ge = g4 * exp(y);
+                  const zd ikr = {-y, x};
+                  G[md] = zd{cs * ge, -sn * ge};
+                  const zd o = zd{1.0 - y, x} * G[md];
+                  D[md] = o * -rinv2;
+                  f = (3.0 * o + (ikr * ikr) * G[md]) * (rinv2 * rinv2);
+                } else {
+                  G[md] = zd{cs * g4, -sn * g4};
+                  const zd o = zd{fma(-x, G[md].y, G[md].x), fma(x, G[md].x, G[md].y)};
+                  D[md] = o * -rinv2;
+                  const double x2 = x * x;
+                  f = zd{fma(-x2, G[md].x, 3.0 * o.x), fma(-x2, G[md].y, 3.0 * o.y)} *
+                      (rinv2 * rinv2);
+                }
+                Fs = md == 0 ? f : Fs + f;
+              }
+              const zd Ds = D[0] + D[1];
+#pragma unroll
+              for (int p = 0; p < 3; ++p) {
+                const double a = kTri3.mu1[p][i] * ue1 + kTri3.mu2[p][i] * ue2;
+                const double bb = kTri3.mu1[p][i] * P1[p] + kTri3.mu2[p][i] * P2[p];
+                zd g[2] = {G[0], G[1]}, d = Ds;
+                if (p > 0) {
+                  const double h = -(kTri3.dl1[p][i] * Re1 + kTri3.dl2[p][i] * Re2);
+                  g[0] = g[0] + D[0] * h;
+                  g[1] = g[1] + D[1] * h;
+                  d = d + Fs * h;
+                }
+#pragma unroll
+                for (int md = 0; md < 2; ++md) {
+                  S0[p][md] = S0[p][md] + g[md];
+                  S1[p][md] = S1[p][md] + g[md] * a;
+                }
+                SK[p] = SK[p] + d * bb;
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          const int sd = p == 0 ? en.x : p == 1 ? en.y : en.z;
+          if (sd < 0) continue;
+          const double w = fs.area * A.fn[sd].df;
+          double *o = acc + (size_t)((en.w >> (10 * p)) & 1023) * (2 * NV);
+#pragma unroll
+          for (int md = 0; md < 2; ++md) {
+            const zd T = mul_i(Q.k4[md] * S1[p][md] - Q.ik[md] * S0[p][md]) * w;
+            atomicAdd(o + 2 * md, T.x);
+            atomicAdd(o + 2 * md + 1, T.y);
+          }
+          const zd K = SK[p] * (0.25 * w);
+          atomicAdd(o + 4, K.x);
+          atomicAdd(o + 5, K.y);
+          if (NV == 4) {
+            const double sg = (sd & 1) ? 1.0 : -1.0;
+            atomicAdd(o + 6, K.x * sg);
+            atomicAdd(o + 7, K.y * sg);
+          }
+        }
+      }
+      __syncthreads();
+      for (int c = threadIdx.x; c < nc; c += blockDim.x) {
+        zd *o = reinterpret_cast<zd *>(acc) + (size_t)c * NV;
+        const zd T1 = o[0], T2 = o[1], K = o[2], Ka = o[NV - 1];
+        for (int k = 0; k < NV; ++k) o[k] = zd{0, 0};
+        const int64_t g = g0 + c;
+        zd D[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+        const unsigned bits = cls[g] & 15u;
+        if (bits) {
+          int64_t idx = base_a[g];
+          for (int p = 0; p < 4; ++p)
+            if (bits & (1u << p)) {
+              add_zz(A, D, zz + 4 * idx, p & 1);
+              ++idx;
+            }
+          finish_tri(A, D);
+        }
+        blocks[4 * g] = D[0] + Q.c[0] * T1 + Q.c[1] * T2;
+        blocks[4 * g + 1] = D[1] + Q.c[2] * K;
+        blocks[4 * g + 2] = D[2] + Q.c[3] * Ka;
+        blocks[4 * g + 3] = D[3] + Q.c[4] * T1 + Q.c[5] * T2;
+      }
+      __syncthreads();
+    }
+  }
+}
+
 static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 static inline unsigned gcap(int64_t n) { unsigned b = nblk(n, 256); return b < 2048u ? (b ? b : 1u) : 2048u; }
 
@@ -733,6 +1049,28 @@ void launch_near_regular(const NearArgs &a, int64_t nnz, const uint8_t *cls, con
   else
     hipLaunchKernelGGL(k_near_regular<false>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, nnz, cls,
                        base_a, zz, blocks);
+}
+
+// The triangle kernel takes the formulations without normal components and
+// without separate K of the media under the three-point rule (make_tri_form).
+void launch_near_tri(const NearArgs &a, const TriForm &q, int N, int tiles, const int *row_box,
+                     const int *row_r0, const int *tri_side, int4 *list, int *cnt,
+                     const uint8_t *cls, const int *base_a, const zd *zz, zd *blocks,
+                     hipStream_t st) {
+  if (tiles <= 0) return;
+  hipLaunchKernelGGL(k_near_tri_list, dim3(a.nbl), dim3(256), 0, st, a.e2_off, a.e2_list, a.er,
+                     tri_side, list, cnt);
+  // rows a workgroup takes in turn: fewer on small meshes, so that the grid
+  // has about a thousand workgroups or more wherever the rows allow
+  int rp = kSpmvRowsPerWG;
+  while (rp > 1 && N / rp < 1024) rp >>= 1;
+  const dim3 grid(tiles, kSpmvRowsPerWG / rp);
+  const bool lossy = a.mat.k1.im != 0.0 || a.mat.k2.im != 0.0;
+  const bool alt = a.form == SPK_PMCHWT_S;
+  auto *f = alt ? (lossy ? k_near_tri<4, true> : k_near_tri<4, false>)
+                : (lossy ? k_near_tri<3, true> : k_near_tri<3, false>);
+  hipLaunchKernelGGL(f, grid, dim3(256), kTriCols * (alt ? 64 : 48), st, a, q, row_box, row_r0, rp,
+                     list, cnt, cls, base_a, zz, blocks);
 }
 
 hipError_t exclusive_scan_int(const int *in, int *out, int64_t n, void **tmp, size_t *tmp_bytes,
