@@ -141,6 +141,7 @@ struct spk_handle {
   BatchBufs<zd> bd;
   BatchBufs<zf> bf;
   int spmv_wgs = 0;
+  PatLay lay;  // layout of the patterns and of the leaf's W (triangle handles)
   DBuf<zd> d_rt, d_W;
   // 8-node quadrilaterals with 10 edge functions (spk_setup_quad): the mesh
   // and neighbour arrays, kernel constants, the patterns' quadrature points,
@@ -306,7 +307,7 @@ bool make_tri_form(const NearArgs &a, double D, TriForm *q) {
     if (a.qa[i] != kTri3.a[i] || a.qb[i] != kTri3.b[i] || a.qw[i] != kTri3.w) return false;
   if (a.form != SPK_PMCHWT && a.form != SPK_MCTF && a.form != SPK_PMCHWT_S && a.form != SPK_ICTF)
     return false;
-  if (!(4.0 * D * std::max(std::fabs(a.mat.k1.re), std::fabs(a.mat.k2.re)) < 1e5)) return false;
+  if (!sincos_near_holds(D, zcx(a.mat.k1), zcx(a.mat.k2))) return false;
   // assemble_zz, accumulate_D and finish_D of these formulations in one step
   const zd e1 = zcx(a.mat.eta1), e2 = zcx(a.mat.eta2), ea = zcx(a.mat.eta_a), one = {1.0, 0.0};
   const zd k[2] = {zcx(a.mat.k1), zcx(a.mat.k2)};
@@ -588,8 +589,16 @@ int setup_mlfmm(spk_handle *h, std::future<std::vector<HostLevelTables>> &pre) {
     HIPCHK(h->d_rt.alloc((size_t)N * kQuadRtRows * S));
     launch_qpatterns(N, S, h->d_khat.p, h->q_pts.p, h->qdev.k1, h->qdev.k2, h->d_rt.p, h->st);
   } else {
-    HIPCHK(h->d_rt.alloc((size_t)N * 4 * S));
-    launch_patterns(N, S, h->ngp, h->d_fn.p, h->d_perm.p, h->d_leaf_box.p, h->d_leaf_centre.p,
+    PatLay &lay = h->lay;
+    lay.S = S;
+    lay.K = h->tb.K;
+    const int half = (lay.count() + 1) & ~1;
+    lay.SW = std::max(S, 2 * half);
+    lay.half[0] = h->mat.k1.im == 0.0;
+    lay.half[1] = h->mat.k2.im == 0.0;
+    for (int k = 0; k < 2; ++k) lay.L[k] = lay.half[k] ? half : S;
+    HIPCHK(h->d_rt.alloc((size_t)N * lay.stride()));
+    launch_patterns(N, lay, h->ngp, t.D, h->d_fn.p, h->d_perm.p, h->d_leaf_box.p, h->d_leaf_centre.p,
                     h->d_khat.p, h->d_tth.p, h->d_tph.p, h->d_q.p, h->d_q.p + 20, h->d_q.p + 40,
                     zcx(h->mat.k1), zcx(h->mat.k2), h->d_rt.p, h->st);
   }
@@ -673,7 +682,7 @@ int setup_mlfmm(spk_handle *h, std::future<std::vector<HostLevelTables>> &pre) {
     h->stats.boxes_per_level[l] = D.nb;
     h->stats.i4_pairs_per_level[l] = (int64_t)L.i4_box.size();
   }
-  HIPCHK(h->d_W.alloc((size_t)LL.n.size() * (h->quad ? 12 : 8) * S));
+  HIPCHK(h->d_W.alloc((size_t)LL.n.size() * (h->quad ? 12 * (size_t)S : 8 * (size_t)h->lay.SW)));
   if (tmp_need) HIPCHK(h->lvl_tmp.alloc(tmp_need));
   h->stats.tables_ms = now_ms() - t0;
   // formulation scaling of the far field (MLFMM_tri_summation_New :478-495)
@@ -764,8 +773,7 @@ static int matvec_multik(spk_handle *h, const zd *x, zd *y, bool near_on, bool f
   zd *yfar = h->d_yfar.p;
   if (far_on) {
     LevelDev &LL = h->lev[lmax];
-    const int SL = LL.S;
-    launch_agg(LL.nb, SL, N, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, h->d_rt.p, x, LL.B.p,
+    launch_agg(LL.nb, h->lay, N, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, h->d_rt.p, x, LL.B.p,
                st, true);
     for (int l = lmax - 1; l >= lmin; --l) {
       LevelDev &P = h->lev[l], &Cl = h->lev[l + 1];
@@ -785,7 +793,6 @@ static int matvec_multik(spk_handle *h, const zd *x, zd *y, bool near_on, bool f
     const zd kd1 = I * zcx(h->mat.k1), kd2 = I * zcx(h->mat.k2);
     const zd my1 = zd{h->mat.my1, 0} * I * h->mat.omega, my2 = zd{h->mat.my2, 0} * I * h->mat.omega;
     const zd ep1 = zcx(h->mat.eps1) * I * h->mat.omega, ep2 = zcx(h->mat.eps2) * I * h->mat.omega;
-    const zd *W = nullptr;
     if (h->rr_mode == SPK_RR_REFERENCE) {
       for (int l = lmin + 1; l <= lmax; ++l) {
         LevelDev &Cl = h->lev[l], &P = h->lev[l - 1];
@@ -799,8 +806,8 @@ static int matvec_multik(spk_handle *h, const zd *x, zd *y, bool near_on, bool f
                     (const zd *)Cl.down.p, Cl.D.p, st);
         }
       }
-      launch_fold(LL.nb, SL, (const zd *)LL.D.p, kd1, kd2, my1, my2, ep1, ep2, h->d_W.p, st);
-      W = h->d_W.p;
+      launch_fold_leaf(LL.nb, h->lay, (const zd *)LL.D.p, kd1, kd2, my1, my2, ep1, ep2, h->d_W.p,
+                       st);
     } else {
       // folded coefficients of every level into its (consumed) B buffer
       for (int l = lmin; l <= lmax; ++l)
@@ -818,10 +825,10 @@ static int matvec_multik(spk_handle *h, const zd *x, zd *y, bool near_on, bool f
                            (const zd *)Cl.down.p, Cl.B.p, st);
         }
       }
-      W = LL.B.p;
+      launch_half_w(LL.nb, h->lay, LL.B.p, h->d_W.p, st);
     }
-    launch_disagg(h->disagg_tasks, N, SL, h->d_disagg_task.p, h->d_perm.p, h->d_leafbox_of_pos.p,
-                  h->d_rt.p, W, h->sc1, h->sc2, near_on ? yfar : y, st, false);
+    launch_disagg(h->disagg_tasks, N, h->lay, h->d_disagg_task.p, h->d_perm.p, h->d_leafbox_of_pos.p,
+                  h->d_rt.p, (const zd *)h->d_W.p, h->sc1, h->sc2, near_on ? yfar : y, st, false);
   }
   if (near_on)
     launch_near_spmv_rows(h->spmv_wgs, N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
@@ -927,7 +934,7 @@ int matvec_t(spk_handle *h, const T *x, T *y, bool near_on = true, bool far_on =
     DBuf<T> &xt = pXt(h, tag);
     HIPCHK(xt.alloc(2 * (size_t)N));
     launch_scale_halves(N, h->sc1, h->sc2, x, xt.p, st);
-    launch_agg(LL.nb, S, N, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, pRt(h, tag),
+    launch_agg(LL.nb, h->lay, N, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, pRt(h, tag),
                (const T *)xt.p, pB(LL, tag), st, false);
     mark(1);
     const zd I = {0, 1};
@@ -947,16 +954,16 @@ int matvec_t(spk_handle *h, const T *x, T *y, bool near_on = true, bool far_on =
       launch_rr(h->lev[l].nb, S, h->lev[l].parent.p, h->lev[l].octant.p,
                 (const T *)pB(h->lev[l - 1], tag), pUp(h->lev[l], tag), pB(h->lev[l], tag), st);
     mark(4);
-    launch_fold(LL.nb, S, (const T *)pB(LL, tag), zd{0, 0}, zd{0, 0}, zd{1, 0}, zd{1, 0},
-                zd{1, 0}, zd{1, 0}, pW(h, tag), st);
+    launch_fold_leaf(LL.nb, h->lay, (const T *)pB(LL, tag), zd{0, 0}, zd{0, 0}, zd{1, 0}, zd{1, 0},
+                     zd{1, 0}, zd{1, 0}, pW(h, tag), st);
     mark(5);
-    launch_disagg(h->disagg_tasks, N, S, h->d_disagg_task.p, h->d_perm.p, h->d_leafbox_of_pos.p,
+    launch_disagg(h->disagg_tasks, N, h->lay, h->d_disagg_task.p, h->d_perm.p, h->d_leafbox_of_pos.p,
                   pRt(h, tag), (const T *)pW(h, tag), zd{1, 0}, zd{1, 0}, near_on ? yfar : y, st,
                   true);
     mark(6);
   } else if (far_on) {
     LevelDev &LL = h->lev[lmax];
-    launch_agg(LL.nb, S, N, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, pRt(h, tag), x,
+    launch_agg(LL.nb, h->lay, N, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, pRt(h, tag), x,
                pB(LL, tag), st);
     mark(1);
     for (int l = lmax - 1; l >= lmin; --l)
@@ -975,9 +982,10 @@ int matvec_t(spk_handle *h, const T *x, T *y, bool near_on = true, bool far_on =
     const zd kd1 = I * zcx(h->mat.k1), kd2 = I * zcx(h->mat.k2);
     const zd my1 = zd{h->mat.my1, 0} * I * h->mat.omega, my2 = zd{h->mat.my2, 0} * I * h->mat.omega;
     const zd ep1 = zcx(h->mat.eps1) * I * h->mat.omega, ep2 = zcx(h->mat.eps2) * I * h->mat.omega;
-    launch_fold(LL.nb, S, (const T *)pD(LL, tag), kd1, kd2, my1, my2, ep1, ep2, pW(h, tag), st);
+    launch_fold_leaf(LL.nb, h->lay, (const T *)pD(LL, tag), kd1, kd2, my1, my2, ep1, ep2,
+                     pW(h, tag), st);
     mark(5);
-    launch_disagg(h->disagg_tasks, N, S, h->d_disagg_task.p, h->d_perm.p, h->d_leafbox_of_pos.p,
+    launch_disagg(h->disagg_tasks, N, h->lay, h->d_disagg_task.p, h->d_perm.p, h->d_leafbox_of_pos.p,
                   pRt(h, tag), (const T *)pW(h, tag), h->sc1, h->sc2, near_on ? yfar : y, st);
     mark(6);
   }
@@ -1012,7 +1020,7 @@ static int batch_ensure(spk_handle *h, int R) {
     HIPCHK(BB.B[l].alloc((size_t)h->lev[l].nb * 8 * S * R));
     HIPCHK(BB.D[l].alloc((size_t)h->lev[l].nb * 8 * S * R));
   }
-  HIPCHK(BB.W.alloc((size_t)h->lev[t.l_max].nb * 8 * S * R));
+  HIPCHK(BB.W.alloc((size_t)h->lev[t.l_max].nb * 8 * h->lay.SW * R));
   HIPCHK(BB.YF.alloc((size_t)R * 2 * h->N));
   HIPCHK(BB.YP.alloc((size_t)kBatchSplit * R * 2 * h->N));
   HIPCHK(BB.XI.alloc((size_t)kBatchMax * 2 * h->N));
@@ -1064,7 +1072,7 @@ int matvec_batch_t(spk_handle *h, int R, const T *const *xs, T *const *ys, bool 
     HIPCHK(hipGetLastError());
     return SPK_OK;
   }
-  launch_batch_agg(LL.nb, S, N, R, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, pRt(h, tag),
+  launch_batch_agg(LL.nb, h->lay, N, R, h->d_box_first.p, h->d_box_count.p, h->d_perm.p, pRt(h, tag),
                    (const T *)BB.XI.p, (const T *)BB.XP.p, BB.B[lmax].p, st);
   for (int l = lmax - 1; l >= lmin; --l)
     launch_batch_ss(h->lev[l].nb, S, R, h->lev[l].child.p, (const T *)BB.B[l + 1].p,
@@ -1079,8 +1087,8 @@ int matvec_batch_t(spk_handle *h, int R, const T *const *xs, T *const *ys, bool 
   const zd kd1 = I * zcx(h->mat.k1), kd2 = I * zcx(h->mat.k2);
   const zd my1 = zd{h->mat.my1, 0} * I * h->mat.omega, my2 = zd{h->mat.my2, 0} * I * h->mat.omega;
   const zd ep1 = zcx(h->mat.eps1) * I * h->mat.omega, ep2 = zcx(h->mat.eps2) * I * h->mat.omega;
-  launch_batch_fold(LL.nb, S, R, (const T *)BB.D[lmax].p, kd1, kd2, my1, my2, ep1, ep2, BB.W.p, st);
-  launch_batch_disagg(h->ntiles, N, S, R, h->d_tile_box.p, h->d_tile_p0.p, h->d_box_first.p,
+  launch_batch_fold(LL.nb, h->lay, R, (const T *)BB.D[lmax].p, kd1, kd2, my1, my2, ep1, ep2, BB.W.p, st);
+  launch_batch_disagg(h->ntiles, N, h->lay, R, h->d_tile_box.p, h->d_tile_p0.p, h->d_box_first.p,
                       h->d_box_count.p, h->d_perm.p, pRt(h, tag), (const T *)BB.W.p, h->sc1,
                       h->sc2, BB.YP.p, BB.YF.p, h->dx_tiles, h->d_dx_box.p, h->d_dx_p0.p, st);
   launch_batch_near(h->spmv_wgs, N, R, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
@@ -1131,7 +1139,8 @@ void stage_bytes(const spk_handle *h, double *b, double c = 16.0) {
   const Tree &t = h->tree;
   const double S = h->tb.S, N = h->N;
   const double nbl = (double)t.lev[t.l_max].n.size();
-  b[0] = N * 4 * S * c + 2 * N * c + nbl * 8 * S * c;  // patterns + x + C
+  const double pat = h->quad ? N * kQuadRtRows * S * c : N * (double)h->lay.stride() * c;
+  b[0] = pat + 2 * N * c + nbl * 8 * S * c;  // patterns + x + C
   b[1] = 0;
   b[2] = 0;
   b[3] = 0;
@@ -1142,7 +1151,7 @@ void stage_bytes(const spk_handle *h, double *b, double c = 16.0) {
     if (l > t.l_min) b[3] += (double)t.lev[l - 1].n.size() * 8 * S * c + 2.0 * nb * 8 * S * c;
   }
   b[4] = 2.0 * nbl * 8 * S * c;
-  b[5] = N * 4 * S * c + nbl * 8 * S * c + 2 * N * c;  // patterns + W + y
+  b[5] = pat + nbl * 8 * S * c + 2 * N * c;  // patterns + W + y
   b[6] = (double)t.nnz * 4 * c + 2 * N * c + 2 * N * c + 2 * N * c;  // blocks + x + yfar + y
   b[7] = b[0] + b[1] + b[2] + b[3] + b[4] + b[5] + b[6];
 }
@@ -1332,7 +1341,8 @@ static int setup_operator(spk_handle *h, double t0) {
   h->stats.l_max = t.l_max;
   h->stats.samples = h->tb.S;
   h->stats.bytes_near = (double)t.nnz * 64.0;
-  h->stats.bytes_patterns = (double)h->N * (h->quad ? kQuadRtRows : 4) * h->tb.S * 16.0;
+  h->stats.bytes_patterns =
+      (double)h->N * (h->quad ? (double)kQuadRtRows * h->tb.S : (double)h->lay.stride()) * 16.0;
   if (h->p.precision == SPK_MIXED) {
     rc = build_mixed_mirror(h);
     if (rc != SPK_OK) return rc;
@@ -3550,7 +3560,15 @@ int spk_adjoint_height_gradient(spk_handle *h, const double k_in[3], const doubl
   DBuf<zd> WI, Bt;
   HIPCHK(WI.alloc(8 * S * nleaf));
   HIPCHK(Bt.alloc(8 * S * nleaf));
-  HIPCHK(hipMemcpyAsync(WI.p, h->d_W.p, 8 * S * nleaf * sizeof(zd), hipMemcpyDeviceToDevice, st));
+  {
+    // W of I at every sample, from the leaf coefficients the product left
+    const zd i1 = {0, 1};
+    const double om = h->mat.omega;
+    launch_fold((int)nleaf, (int)S, (const zd *)h->lev[t.l_max].D.p, i1 * zcx(h->mat.k1),
+                i1 * zcx(h->mat.k2), zd{0, h->mat.my1 * om}, zd{0, h->mat.my2 * om},
+                zcx(h->mat.eps1) * i1 * om, zcx(h->mat.eps2) * i1 * om, WI.p, st);
+    HIPCHK(hipGetLastError());
+  }
   // the transposed solve and its leaf sums
   if ((rc = spk_set_transposed(h, 1))) return rc;
   rc = spk_gmres_device(h, c.p, nu.p, gp, &inf[1]);
@@ -3825,11 +3843,25 @@ int spk_get_patterns(const spk_handle *h, int first, int count, double *out) {
   if (!h->ready) return fail(SPK_ERR_STATE, "spk_setup_tri has not completed");
   if (first < 0 || count < 0 || first + count > h->N) return fail(SPK_ERR_ARG, "edge range");
   if (h->quad) return fail(SPK_ERR_STATE, "quadrilateral handles: patterns have their own layout");
-  const int S = h->tb.S;
+  const PatLay &lay = h->lay;
+  const int S = lay.S;
+  std::vector<zd> row(lay.stride());
   for (int e = 0; e < count; ++e) {
     const int p = h->tree.pos[first + e];
-    HIPCHK(hipMemcpy(out + (size_t)e * 8 * S, h->d_rt.p + (size_t)p * 4 * S, 4 * (size_t)S * sizeof(zd),
+    HIPCHK(hipMemcpy(row.data(), h->d_rt.p + (size_t)p * lay.stride(), row.size() * sizeof(zd),
                      hipMemcpyDeviceToHost));
+    for (int q = 0; q < 4; ++q) {
+      const zd *f = row.data() + lay.row(q >> 1, q & 1);
+      zd *o = reinterpret_cast<zd *>(out) + ((size_t)e * 4 + q) * S;
+      if (!lay.half[q >> 1]) {
+        std::copy(f, f + S, o);
+        continue;
+      }
+      for (int i = 0; i < lay.count(); ++i) {
+        o[lay.samp(i)] = f[i];
+        o[lay.anti(i)] = lay.flips(i, q & 1) ? -conj(f[i]) : conj(f[i]);
+      }
+    }
   }
   return SPK_OK;
 }

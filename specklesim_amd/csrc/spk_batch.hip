@@ -50,59 +50,132 @@ __global__ void kb_interleave(int N, int R, const int *perm, const T *const *xs,
 }
 
 // Aggregation: C[b][it][s][r] = sum_{edges of b} conj(RT[p][q][s]) x_r(cur),
-// it = comp*4 + cur*2 + k.  Workgroup = (256 samples, leaf box, q); the
-// box's x values are staged in LDS 64 edges at a time and read as
-// broadcasts; each thread keeps 2R accumulators.  RP = R rounded up to a
-// power of two (lanes beyond R are zero and not written).
-template <class T, int RP>
-__global__ void __launch_bounds__(256) kb_agg(int S, int N, int R, const int *box_first,
-                                              const int *box_count, const T *rt, const T *XP,
-                                              T *C) {
-  __shared__ T xl[64 * 2 * RP];
-  const int s = blockIdx.x * 256 + threadIdx.x;
+// it = comp*4 + cur*2 + k.  The box's x values are staged in LDS 64 edges at a
+// time and read as broadcasts; four edges' pattern values are in flight while
+// the four before are summed.  A medium with losses: workgroup = 256 samples,
+// a thread keeps 2R sums.  A HALF medium (PatLay): workgroup = 128 entries,
+// the two pairs of waves share the edges, a thread keeps 4R sums (of the real
+// and of the imaginary parts), which give the sample's coefficients and its
+// antipode's.  RP = R rounded up to a power of two (lanes beyond R are zero
+// and not written).
+template <class T, int RP, bool HALF>
+__device__ __forceinline__ void kb_agg_part(const PatLay &lay, int R, const int *box_first,
+                                            const int *box_count, const T *rt, const T *XP, T *C,
+                                            T *xl, T *red) {
+  constexpr int V = HALF ? 2 : 1, NT = HALF ? 128 : 256, EG = 256 / NT, UE = 4;
+  const int i = blockIdx.x * NT + threadIdx.x % NT;
+  const int eg = HALF ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
   const int b = blockIdx.y, q = blockIdx.z, k = q >> 1, comp = q & 1;
+  const int n = HALF ? lay.count() : lay.S;
+  if ((int)blockIdx.x * NT >= n) return;
   const int p0 = box_first[b], cnt = box_count[b];
-  T ae[RP], ah[RP];
+  const size_t ps = lay.stride();
+  const T *F = rt + (size_t)p0 * ps + lay.row(k, comp) + min(i, n - 1);
+  T ae[V * RP], ah[V * RP];
 #pragma unroll
-  for (int r = 0; r < RP; ++r) ae[r] = ah[r] = T{0, 0};
+  for (int r = 0; r < V * RP; ++r) ae[r] = ah[r] = T{0, 0};
   for (int e0 = 0; e0 < cnt; e0 += 64) {
     const int ne = min(64, cnt - e0);
     __syncthreads();
     // the box's edges are consecutive positions: one contiguous run of XP
-    for (int i = threadIdx.x; i < ne * 2 * RP; i += 256) xl[i] = XP[(size_t)(p0 + e0) * 2 * RP + i];
+    for (int t = threadIdx.x; t < ne * 2 * RP; t += 256)
+      xl[t] = XP[(size_t)(p0 + e0) * 2 * RP + t];
     __syncthreads();
-    if (s < S) {
-      for (int g0 = 0; g0 < ne; g0 += kSumBlock<T>) {
-        T ge[RP], gh[RP];
+    const int ea = ne * eg / EG, eb = ne * (eg + 1) / EG;
+    T cur[UE], nxt[UE];
+    auto load = [&](int e, T *w) {
 #pragma unroll
-        for (int r = 0; r < RP; ++r) ge[r] = gh[r] = T{0, 0};
-        const int g1 = min(ne, g0 + kSumBlock<T>);
-        for (int e = g0; e < g1; ++e) {
-          const T f = conj(rt[((size_t)(p0 + e0 + e) * 4 + q) * S + s]);
-          const T *xe = xl + e * 2 * RP;
+      for (int u = 0; u < UE; ++u) w[u] = F[(size_t)(e0 + min(e + u, ne - 1)) * ps];
+    };
+    load(ea, cur);
+    for (int g0 = ea; g0 < eb; g0 += kSumBlock<T>) {
+      constexpr bool BLK = kSumBlock<T> < 64;
+      T ge[V * RP], gh[V * RP];
+      T *te = BLK ? ge : ae, *th = BLK ? gh : ah;
+#pragma unroll
+      for (int r = 0; r < V * RP; ++r) ge[r] = gh[r] = T{0, 0};
+      const int g1 = min(eb, g0 + kSumBlock<T>);
+      for (int e = g0; e < g1; e += UE) {
+        load(e + UE, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UE; ++u) {
+          // an edge past the end adds nothing
+          const T f = e + u < g1 ? cur[u] : T{0, 0};
+          const T *xe = xl + min(e + u, ne - 1) * 2 * RP;
 #pragma unroll
           for (int r = 0; r < RP; ++r) {
-            ge[r] = ge[r] + f * xe[r];
-            gh[r] = gh[r] + f * xe[RP + r];
+            if constexpr (HALF) {
+              te[r] = te[r] + xe[r] * f.x;
+              th[r] = th[r] + xe[RP + r] * f.x;
+              te[RP + r] = te[RP + r] + xe[r] * f.y;
+              th[RP + r] = th[RP + r] + xe[RP + r] * f.y;
+            } else {
+              te[r] = te[r] + conj(f) * xe[r];
+              th[r] = th[r] + conj(f) * xe[RP + r];
+            }
           }
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < RP; ++r) {
+        for (int u = 0; u < UE; ++u) cur[u] = nxt[u];
+      }
+      if constexpr (BLK) {
+#pragma unroll
+        for (int r = 0; r < V * RP; ++r) {
           ae[r] = ae[r] + ge[r];
           ah[r] = ah[r] + gh[r];
         }
       }
     }
   }
-  if (s < S) {
-    T *Cb = C + (size_t)b * 8 * S * R;
+  T *Ce = C + ((size_t)b * 8 + comp * 4 + k) * lay.S * R, *Ch = Ce + 2 * (size_t)lay.S * R;
+  if constexpr (HALF) {
+    const int l = threadIdx.x % NT;
+    const bool out = i < n && eg == 0;
+    const int s = lay.samp(min(i, n - 1)), t = lay.anti(min(i, n - 1));
+    const bool neg = lay.flips(i, comp);
+#pragma unroll
+    for (int r = 0; r < RP; ++r) {
+      __syncthreads();
+      if (eg == 1) {
+        red[l] = ae[r];
+        red[NT + l] = ah[r];
+        red[2 * NT + l] = ae[RP + r];
+        red[3 * NT + l] = ah[RP + r];
+      }
+      __syncthreads();
+      if (!out || r >= R) continue;
+      const T e = ae[r] + red[l], h = ah[r] + red[NT + l];
+      const T ei = ae[RP + r] + red[2 * NT + l], hi = ah[RP + r] + red[3 * NT + l];
+      const T be = {-ei.y, ei.x}, bh = {-hi.y, hi.x};
+      Ce[(size_t)s * R + r] = e - be;
+      Ch[(size_t)s * R + r] = h - bh;
+      const T te = e + be, th = h + bh;
+      Ce[(size_t)t * R + r] = neg ? -te : te;
+      Ch[(size_t)t * R + r] = neg ? -th : th;
+    }
+  } else {
+    if (i >= n) return;
 #pragma unroll
     for (int r = 0; r < RP; ++r)
       if (r < R) {
-        Cb[((size_t)(comp * 4 + 0 + k) * S + s) * R + r] = ae[r];
-        Cb[((size_t)(comp * 4 + 2 + k) * S + s) * R + r] = ah[r];
+        Ce[(size_t)i * R + r] = ae[r];
+        Ch[(size_t)i * R + r] = ah[r];
       }
   }
+}
+// MODE: 1 both media keep half of the samples, 0 neither does, 2 one of them does
+template <class T, int RP, int MODE>
+__global__ void __launch_bounds__(256) kb_agg(PatLay lay, int R, const int *box_first,
+                                              const int *box_count, const T *rt, const T *XP,
+                                              T *C) {
+  __shared__ T xl[64 * 2 * RP];
+  __shared__ T red[MODE ? 4 * 128 : 1];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.z >> 1]))
+    kb_agg_part<T, RP, true>(lay, R, box_first, box_count, rt, XP, C, xl, red);
+  else if (MODE != 1)
+    kb_agg_part<T, RP, false>(lay, R, box_first, box_count, rt, XP, C, xl, red);
 }
 
 typedef float mxf4 __attribute__((ext_vector_type(4)));
@@ -110,42 +183,50 @@ typedef float mxf4 __attribute__((ext_vector_type(4)));
 
 // Aggregation for 9..16 right-hand sides in complex64 on the matrix cores:
 // per (leaf box, q) C[s][(cur, r)] = sum_p conj(RT[p][q][s]) x_r(p, cur) is a
-// product of the box's pattern rows (samples x edges) and its x values
-// (edges x 32).  Workgroup = (256 samples, box, q), wave = 64 samples as 4
-// tiles of 16: tile 2h + par holds the samples sw + 32 h + 2 i + par, so a
-// lane's one 16-byte load gives the A values of two tiles.  A k-step covers
-// 4 edges (lane group g = edge), B[g][n] = x_n of that edge from LDS.  With
-// a = conj(f): re += fr xr + fi xi, im += fr xi - fi xr, for cur = 0 and 1.
-// Samples and edges past the end are clamped on load (their x is zero in
-// LDS, their results are not written).
-__global__ void __launch_bounds__(256) kb_agg_mx(int S, int R, const int *box_first,
-                                                 const int *box_count, const zf *rt,
-                                                 const zf *XP, zf *C) {
-  __shared__ float4 xl[64 * 16];
+// product of the box's pattern rows (entries x edges) and its x values
+// (edges x 32).  A wave takes NL pairs of 16-entry tiles, NL = 1 in a HALF
+// medium (PatLay), 2 in one with losses (workgroup = 128 or 256 entries, box,
+// q): tile 2h + par holds the entries sw + 32 h + 2 i + par, so a lane's one
+// 16-byte load gives the A values of two.  A k-step covers 4 edges (lane group
+// g = edge), B[g][n] = x_n of that edge from LDS.  In a HALF medium the sums of
+// the real and the imaginary parts stay apart, (a xr, a xi) and (b xr, b xi)
+// for both currents, and give the sample's and the antipode's values;
+// otherwise, with a = conj(f): re += fr xr + fi xi, im += fr xi - fi xr.
+// Entries and edges past the end are clamped on load (their x is zero in LDS,
+// their results are not written).
+template <bool HALF>
+__device__ __forceinline__ void kb_agg_mx_part(const PatLay &lay, int R, const int *box_first,
+                                               const int *box_count, const zf *rt, const zf *XP,
+                                               zf *C, float4 *xl) {
+  constexpr int V = HALF ? 8 : 4, NL = HALF ? 1 : 2, NT = 2 * NL;
   const int b = blockIdx.y, q = blockIdx.z, k = q >> 1, comp = q & 1;
   const int p0 = box_first[b], cnt = box_count[b];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int sw = blockIdx.x * 256 + 64 * wv;  // first sample of this wave
-  const bool active = sw < S;                 // uniform over the wave
-  // the two sample pairs of this lane (16-byte aligned: S is even)
-  const int sa = min(sw + 2 * m, S - 2), sb = min(sw + 32 + 2 * m, S - 2);
-  mxf4 acc[4][4];
+  const int L = lay.L[k];
+  if ((int)blockIdx.x * 128 * NL >= L) return;
+  const int sw = blockIdx.x * 128 * NL + 32 * NL * wv;  // first entry of this wave
+  const bool active = sw < L;                           // uniform over the wave
+  const size_t ps = lay.stride();
+  const zf *F = rt + (size_t)p0 * ps + lay.row(k, comp);
+  int so[NL];  // the entry pairs of this lane (16-byte aligned: L is even)
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int h = 0; h < NL; ++h) so[h] = min(sw + 32 * h + 2 * m, L - 2);
+  mxf4 acc[NT][V];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) acc[t][u] = mxf4{0.f, 0.f, 0.f, 0.f};
-  float4 fa[4], fb[4];
-  auto load = [&](int e0, float4 *a, float4 *bb) {
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int u = 0; u < V; ++u) acc[t][u] = mxf4{0.f, 0.f, 0.f, 0.f};
+  float4 fa[4][NL];
+  auto load = [&](int e0, float4 (*a)[NL]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int e = min(e0 + 4 * j + g, cnt - 1);
-      const zf *f = rt + ((size_t)(p0 + e) * 4 + q) * S;
-      a[j] = *reinterpret_cast<const float4 *>(f + sa);
-      bb[j] = *reinterpret_cast<const float4 *>(f + sb);
+      const zf *f = F + (size_t)min(e0 + 4 * j + g, cnt - 1) * ps;
+#pragma unroll
+      for (int h = 0; h < NL; ++h) a[j][h] = *reinterpret_cast<const float4 *>(f + so[h]);
     }
   };
-  if (active && cnt > 0) load(0, fa, fb);
+  if (active && cnt > 0) load(0, fa);
   for (int e0 = 0; e0 < cnt; e0 += 64) {
     const int ne = min(64, cnt - e0);
     __syncthreads();
@@ -156,69 +237,100 @@ __global__ void __launch_bounds__(256) kb_agg_mx(int S, int R, const int *box_fi
         const int e = (int)(threadIdx.x + 256 * u) >> 4;
         const size_t pe = (size_t)(p0 + e0 + min(e, ne - 1)) * 2;
         const zf x0 = XP[pe * 16 + n], x1 = XP[(pe + 1) * 16 + n];
-        xl[threadIdx.x + 256 * u] = e < ne ? float4{x0.x, x0.y, x1.x, x1.y} : float4{0.f, 0.f, 0.f, 0.f};
+        xl[threadIdx.x + 256 * u] =
+            e < ne ? float4{x0.x, x0.y, x1.x, x1.y} : float4{0.f, 0.f, 0.f, 0.f};
       }
     }
     __syncthreads();
     if (!active) continue;
     for (int i = 0; i < ne; i += 16) {
-      float4 na[4], nb[4];
-      load(e0 + i + 16, na, nb);
+      float4 na[4][NL];
+      load(e0 + i + 16, na);
       __builtin_amdgcn_sched_barrier(0);
       // the group's 16 edges are summed from zero and then added to the
       // running sums, so the running sums take one rounding per group
-      mxf4 gs[4][4];
+      mxf4 gs[NT][V];
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) gs[t][u] = mxf4{0.f, 0.f, 0.f, 0.f};
+        for (int u = 0; u < V; ++u) gs[t][u] = mxf4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float4 x = xl[(i + 4 * j + g) * 16 + m];
         const float n0 = -x.x, n1 = -x.z;
-        const float ar[4] = {fa[j].x, fa[j].z, fb[j].x, fb[j].z};
-        const float ai[4] = {fa[j].y, fa[j].w, fb[j].y, fb[j].w};
+        float ar[NT], ai[NT];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int h = 0; h < NL; ++h) {
+          ar[2 * h] = fa[j][h].x;
+          ai[2 * h] = fa[j][h].y;
+          ar[2 * h + 1] = fa[j][h].z;
+          ai[2 * h + 1] = fa[j][h].w;
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
           gs[t][0] = SPK_MFMA(ar[t], x.x, gs[t][0]);
           gs[t][1] = SPK_MFMA(ar[t], x.y, gs[t][1]);
           gs[t][2] = SPK_MFMA(ar[t], x.z, gs[t][2]);
           gs[t][3] = SPK_MFMA(ar[t], x.w, gs[t][3]);
         }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          gs[t][0] = SPK_MFMA(ai[t], x.y, gs[t][0]);
-          gs[t][1] = SPK_MFMA(ai[t], n0, gs[t][1]);
-          gs[t][2] = SPK_MFMA(ai[t], x.w, gs[t][2]);
-          gs[t][3] = SPK_MFMA(ai[t], n1, gs[t][3]);
+        for (int t = 0; t < NT; ++t) {
+          if constexpr (HALF) {
+            gs[t][4] = SPK_MFMA(ai[t], x.x, gs[t][4]);
+            gs[t][5] = SPK_MFMA(ai[t], x.y, gs[t][5]);
+            gs[t][6] = SPK_MFMA(ai[t], x.z, gs[t][6]);
+            gs[t][7] = SPK_MFMA(ai[t], x.w, gs[t][7]);
+          } else {
+            gs[t][0] = SPK_MFMA(ai[t], x.y, gs[t][0]);
+            gs[t][1] = SPK_MFMA(ai[t], n0, gs[t][1]);
+            gs[t][2] = SPK_MFMA(ai[t], x.w, gs[t][2]);
+            gs[t][3] = SPK_MFMA(ai[t], n1, gs[t][3]);
+          }
         }
       }
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc[t][u] += gs[t][u];
+        for (int u = 0; u < V; ++u) acc[t][u] += gs[t][u];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        fa[j] = na[j];
-        fb[j] = nb[j];
-      }
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < NL; ++h) fa[j][h] = na[j][h];
     }
   }
-  // accumulator element v of lane (g, n) in tile 2h + par: sample sw + 32h + 2(4g + v) + par
-  const int n = m;
+  // accumulator element v of lane (g, n) in tile 2h + par: entry sw + 32h + 2(4g + v) + par
+  const int n = m, lim = HALF ? lay.count() : lay.S;
   if (!active || n >= R) return;
-  zf *Cb = C + (size_t)b * 8 * S * R;
+  zf *Ce = C + ((size_t)b * 8 + comp * 4 + k) * lay.S * R + n, *Ch = Ce + 2 * (size_t)lay.S * R;
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int s = sw + 32 * (t >> 1) + 2 * (4 * g + v) + (t & 1);
-      if (s < S) {
-        Cb[((size_t)(comp * 4 + 0 + k) * S + s) * R + n] = zf{acc[t][0][v], acc[t][1][v]};
-        Cb[((size_t)(comp * 4 + 2 + k) * S + s) * R + n] = zf{acc[t][2][v], acc[t][3][v]};
+      if (s >= lim) continue;
+      if constexpr (HALF) {
+        const float sg = lay.flips(s, comp) ? -1.f : 1.f;
+        const size_t o = (size_t)lay.samp(s) * R, oa = (size_t)lay.anti(s) * R;
+        Ce[o] = zf{acc[t][0][v] + acc[t][5][v], acc[t][1][v] - acc[t][4][v]};
+        Ch[o] = zf{acc[t][2][v] + acc[t][7][v], acc[t][3][v] - acc[t][6][v]};
+        Ce[oa] = zf{acc[t][0][v] - acc[t][5][v], acc[t][1][v] + acc[t][4][v]} * sg;
+        Ch[oa] = zf{acc[t][2][v] - acc[t][7][v], acc[t][3][v] + acc[t][6][v]} * sg;
+      } else {
+        Ce[(size_t)s * R] = zf{acc[t][0][v], acc[t][1][v]};
+        Ch[(size_t)s * R] = zf{acc[t][2][v], acc[t][3][v]};
       }
     }
+}
+template <int MODE>
+__global__ void __launch_bounds__(256) kb_agg_mx(PatLay lay, int R, const int *box_first,
+                                                 const int *box_count, const zf *rt,
+                                                 const zf *XP, zf *C) {
+  __shared__ float4 xl[64 * 16];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.z >> 1]))
+    kb_agg_mx_part<true>(lay, R, box_first, box_count, rt, XP, C, xl);
+  else if (MODE != 1)
+    kb_agg_mx_part<false>(lay, R, box_first, box_count, rt, XP, C, xl);
 }
 
 // translation_SS over u = s*R + r
@@ -298,87 +410,114 @@ __global__ void kb_rr(int S, int R, const int *parent, const int *octant, const 
     dst[(size_t)it * SR + u] = dst[(size_t)it * SR + u] + src[(size_t)it * SR + u] * ((it & 1) ? d1 : d0);
 }
 
-// the folded coefficients of the disaggregation over u
+// the folded leaf coefficients as the disaggregation reads them (PatLay), over
+// (entry, right-hand side); grid z = medium
 template <class T>
-__global__ void kb_fold(int S, int R, const T *D, T kd1, T kd2, T my1, T my2, T ep1, T ep2, T *W) {
-  const int SR = S * R;
+__global__ void kb_fold(PatLay lay, int R, const T *D, T kd1, T kd2, T my1, T my2, T ep1, T ep2,
+                        T *W) {
   const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  const int b = blockIdx.y;
-  if (u >= SR) return;
-  const T *Db = D + (size_t)b * 8 * SR;
-  T *Wb = W + (size_t)b * 8 * SR;
-  for (int k = 0; k < 2; ++k) {
-    const T kd = k ? kd2 : kd1, my = k ? my2 : my1, ep = k ? ep2 : ep1;
-    const T Dae = Db[(size_t)(0 + k) * SR + u], Dah = Db[(size_t)(2 + k) * SR + u];
-    const T Dbe = Db[(size_t)(4 + k) * SR + u], Dbh = Db[(size_t)(6 + k) * SR + u];
-    Wb[(size_t)(k * 4 + 0) * SR + u] = Dbh * kd + Dae * my;
-    Wb[(size_t)(k * 4 + 1) * SR + u] = -(Dah * kd) + Dbe * my;
-    Wb[(size_t)(k * 4 + 2) * SR + u] = -(Dbe * kd) + Dah * ep;
-    Wb[(size_t)(k * 4 + 3) * SR + u] = Dae * kd + Dbh * ep;
+  const int b = blockIdx.y, k = blockIdx.z;
+  const int i = u / R, r = u - i * R;
+  if (i >= lay.L[k]) return;
+  const size_t SR = (size_t)lay.S * R, WR = (size_t)lay.SW * R;
+  const T *Db = D + (size_t)b * 8 * SR + r;
+  T *Wb = W + (size_t)b * 8 * WR + (size_t)(k * 4) * WR + r;
+  const T kd = k ? kd2 : kd1, my = k ? my2 : my1, ep = k ? ep2 : ep1;
+  auto at = [&](int s, T *w) {
+    const size_t o = (size_t)s * R;
+    const T Dae = Db[(size_t)(0 + k) * SR + o], Dah = Db[(size_t)(2 + k) * SR + o];
+    const T Dbe = Db[(size_t)(4 + k) * SR + o], Dbh = Db[(size_t)(6 + k) * SR + o];
+    w[0] = Dbh * kd + Dae * my;
+    w[1] = -(Dah * kd) + Dbe * my;
+    w[2] = -(Dbe * kd) + Dah * ep;
+    w[3] = Dae * kd + Dbh * ep;
+  };
+  T w[4], wa[4];
+  if (!lay.half[k]) {
+    at(i, w);
+    for (int j = 0; j < 4; ++j) Wb[j * WR + (size_t)i * R] = w[j];
+    return;
+  }
+  if (i < lay.count()) {
+    at(lay.samp(i), w);
+    at(lay.anti(i), wa);
+  } else {
+    for (int j = 0; j < 4; ++j) w[j] = wa[j] = T{0, 0};
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const T o = lay.flips(i, j & 1) ? -wa[j] : wa[j];
+    const T P = w[j] + o, d = w[j] - o;
+    Wb[j * WR + (size_t)i * R] = P;
+    Wb[j * WR + (size_t)(lay.L[k] + i) * R] = T{-d.y, d.x};
   }
 }
 
 // Disaggregation as a small GEMM per box: workgroup = (leaf box, tile of up
-// to 64 consecutive edges), 16 RP threads; thread = (group of 4 edges of the
-// tile, right-hand side).  Samples are staged in LDS in chunks of kBatchSC:
-// the tile's pattern rows and the box's folded W for all R; a W value read
-// from LDS serves the thread's 4 edges.
+// to 64 consecutive edges; blockIdx.y = half of one medium's entries), 16 RP
+// threads; thread = (group of 4 edges of the tile, right-hand side).  Entries
+// are staged in LDS in chunks of kBatchSC: the tile's two pattern rows of the
+// medium and the box's folded W for all R (in a HALF medium P and M, PatLay);
+// a W value read from LDS serves the thread's 4 edges.
 // yf[r][m] = sc1 * sum_{k,s} (fa W1a + fb W1b), yf[r][m + N] = sc2 * sum (fa W2a + fb W2b).
 constexpr int kBatchSC = 16;
-template <class T, int RP>
-__global__ void __launch_bounds__(256) kb_disagg(int N, int S, int R, const int *tile_box,
-                                                 const int *tile_p0, const int *box_first,
-                                                 const int *box_count, const int *perm,
-                                                 const T *rt, const T *W, T sc1, T sc2, int sblk,
-                                                 T *yp) {
-  constexpr int NT = 16 * RP, EPT = 4;
-  __shared__ T wl[8 * kBatchSC * RP];
-  __shared__ T fl[kBatchTile * 4 * kBatchSC];
+template <class T, int RP, bool HALF>
+__device__ __forceinline__ void kb_disagg_part(int N, PatLay lay, int R, const int *tile_box,
+                                               const int *tile_p0, const int *box_first,
+                                               const int *box_count, const int *perm, const T *rt,
+                                               const T *W, T sc1, T sc2, T *yp, T *wl, T *fl) {
+  constexpr int NT = 16 * RP, EPT = 4, NW = HALF ? 8 : 4;
   const int b = tile_box[blockIdx.x], p0 = tile_p0[blockIdx.x];
   const int cnt = min(kBatchTile, box_first[b] + box_count[b] - p0);
   const int eg = threadIdx.x / RP, r = threadIdx.x % RP;  // edges eg*4 .. eg*4+3
-  const int SR = S * R;
-  const T *Wb = W + (size_t)b * 8 * SR;
+  const int k = blockIdx.y >> 1, L = lay.L[k];
+  const T *Wb = W + ((size_t)b * 8 + k * 4) * lay.SW * R;
+  const T *F = rt + (size_t)p0 * lay.stride() + lay.row(k, 0);
   T se[EPT], sh[EPT];
 #pragma unroll
   for (int e = 0; e < EPT; ++e) se[e] = sh[e] = T{0, 0};
-  // this workgroup's sample range; its partial sums go to slice blockIdx.y
-  const int s_lo = blockIdx.y * sblk, s_hi = min(S, s_lo + sblk);
-  T *yf = yp + (size_t)blockIdx.y * R * 2 * N;
+  // this workgroup's entries; its partial sums go to slice 2k + (blockIdx.y & 1)
+  const int sblk = ((L + 31) / 32) * 16;
+  const int s_lo = (blockIdx.y & 1) * sblk, s_hi = min(L, s_lo + sblk);
+  T *yf = yp + (size_t)(2 * k + (blockIdx.y & 1)) * R * 2 * N;
   for (int s0 = s_lo; s0 < s_hi; s0 += kBatchSC) {
     const int ns = min(kBatchSC, s_hi - s0);
     __syncthreads();
-    // W[j][s0 + i][r] -> wl[(j * kBatchSC + i) * RP + r]
-    for (int t = threadIdx.x; t < 8 * kBatchSC * RP; t += NT) {
+    // W[j][s0 + i][r] -> wl[(j * kBatchSC + i) * RP + r], j >= 4: M of item j - 4
+    for (int t = threadIdx.x; t < NW * kBatchSC * RP; t += NT) {
       const int j = t / (kBatchSC * RP), i = (t / RP) % kBatchSC, rr = t % RP;
-      wl[t] = (i < ns && rr < R) ? Wb[(size_t)j * SR + (size_t)(s0 + i) * R + rr] : T{0, 0};
+      wl[t] = (i < ns && rr < R)
+                  ? Wb[((size_t)(j & 3) * lay.SW + (j >> 2) * L + s0 + i) * R + rr]
+                  : T{0, 0};
     }
-    // RT[p0 + e][row][s0 + i] -> fl[(e * 4 + row) * kBatchSC + i]
-    for (int t = threadIdx.x; t < kBatchTile * 4 * kBatchSC; t += NT) {
-      const int e = t / (4 * kBatchSC), row = (t / kBatchSC) & 3, i = t % kBatchSC;
-      fl[t] = (e < cnt && i < ns) ? rt[((size_t)(p0 + e) * 4 + row) * S + s0 + i] : T{0, 0};
+    // RT[p0 + e][comp][s0 + i] -> fl[(e * 2 + comp) * kBatchSC + i]
+    for (int t = threadIdx.x; t < kBatchTile * 2 * kBatchSC; t += NT) {
+      const int e = t / (2 * kBatchSC), c = (t / kBatchSC) & 1, i = t % kBatchSC;
+      fl[t] = (e < cnt && i < ns) ? F[(size_t)e * lay.stride() + (size_t)c * L + s0 + i] : T{0, 0};
     }
     __syncthreads();
     if (eg * EPT < cnt) {
-      // complex64: the chunk's samples are summed from zero, then added
+      // complex64: the chunk's entries are summed from zero, then added
       constexpr bool blk = kSumBlock<T> <= kBatchSC;
       T ge[EPT], gh[EPT];
 #pragma unroll
       for (int e = 0; e < EPT; ++e) ge[e] = gh[e] = T{0, 0};
       T *te = blk ? ge : se, *th = blk ? gh : sh;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const T *w1a = wl + (k * 4 + 0) * kBatchSC * RP + r, *w1b = wl + (k * 4 + 1) * kBatchSC * RP + r;
-        const T *w2a = wl + (k * 4 + 2) * kBatchSC * RP + r, *w2b = wl + (k * 4 + 3) * kBatchSC * RP + r;
 #pragma unroll 4
-        for (int i = 0; i < kBatchSC; ++i) {
-          const T wa = w1a[i * RP], wb = w1b[i * RP], wc = w2a[i * RP], wd = w2b[i * RP];
+      for (int i = 0; i < kBatchSC; ++i) {
+        T w[NW];
 #pragma unroll
-          for (int e = 0; e < EPT; ++e) {
-            const T *f = fl + ((eg * EPT + e) * 4 + k * 2) * kBatchSC;
-            const T a = f[i], bb = f[kBatchSC + i];
-            te[e] = te[e] + a * wa + bb * wb;
-            th[e] = th[e] + a * wc + bb * wd;
+        for (int j = 0; j < NW; ++j) w[j] = wl[(j * kBatchSC + i) * RP + r];
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) {
+          const T *f = fl + (eg * EPT + e) * 2 * kBatchSC;
+          const T a = f[i], bb = f[kBatchSC + i];
+          if constexpr (HALF) {
+            te[e] = te[e] + (w[0] * a.x + w[4] * a.y + w[1] * bb.x + w[5] * bb.y);
+            th[e] = th[e] + (w[2] * a.x + w[6] * a.y + w[3] * bb.x + w[7] * bb.y);
+          } else {
+            te[e] = te[e] + a * w[0] + bb * w[1];
+            th[e] = th[e] + a * w[2] + bb * w[3];
           }
         }
       }
@@ -401,117 +540,143 @@ __global__ void __launch_bounds__(256) kb_disagg(int N, int S, int R, const int 
     }
   }
 }
+template <class T, int RP, int MODE>
+__global__ void __launch_bounds__(256) kb_disagg(int N, PatLay lay, int R, const int *tile_box,
+                                                 const int *tile_p0, const int *box_first,
+                                                 const int *box_count, const int *perm, const T *rt,
+                                                 const T *W, T sc1, T sc2, T *yp) {
+  __shared__ T wl[(MODE ? 8 : 4) * kBatchSC * RP];
+  __shared__ T fl[kBatchTile * 2 * kBatchSC];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.y >> 1]))
+    kb_disagg_part<T, RP, true>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W,
+                                sc1, sc2, yp, wl, fl);
+  else if (MODE != 1)
+    kb_disagg_part<T, RP, false>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W,
+                                 sc1, sc2, yp, wl, fl);
+}
 
 // Disaggregation for 9..16 right-hand sides in complex64 on the matrix
-// cores: per leaf box y_r(p, e) = sum_{k,s} fa W(k,e,a) + fb W(k,e,b) with
-// fa = RT[p][2k][s], fb = RT[p][2k+1][s] is a product of the box's pattern
-// rows (edges x (k, s)) and its folded W ((k, s) x r).  Workgroup = (tile of
-// up to 128 consecutive edges of one box, sample part blockIdx.y), wave = 16
-// edges.  A k-step covers 4 samples: lane group g takes sample s + 4g + j in
-// step j, so a lane's two 16-byte loads per pattern row serve 4 steps.  W of
-// kMxSC samples is staged in LDS as [k][sample][half][r][2]: half 0 = the e
-// pair (a, b), half 1 = the h pair.  Edges and samples past the end are
-// clamped on load (their W is zero in LDS, their results are not written).
-// yf slice blockIdx.y: [r][m] = sc1 * sum (e part), [r][m + N] = sc2 * sum (h part).
+// cores: per leaf box and medium y_r(p, e) = sum_s fa W(e,a) + fb W(e,b) with
+// fa, fb the medium's two pattern rows is a product of the box's rows (edges x
+// entries) and its folded W (entries x r).  Workgroup = (tile of up to 128
+// consecutive edges of one box; blockIdx.y = half of one medium's entries),
+// wave = 16 edges.  A k-step covers 4 entries: lane group g takes entry s + 4g
+// + j in step j, so a lane's two 16-byte loads per pattern row serve 4 steps.
+// W of kMxSC entries is staged in LDS as [P/M][entry][half][r][2]: half 0 =
+// the e pair (a, b), half 1 = the h pair; a HALF medium (PatLay) multiplies P
+// with the real and M with the imaginary parts, the other one W by the complex
+// product.  Edges and entries past the end are clamped on load (their W is
+// zero in LDS, their results are not written).
+// yf slice 2k + part: [r][m] = sc1 * sum (e part), [r][m + N] = sc2 * sum (h part).
 constexpr int kMxSC = 32;
-__global__ void __launch_bounds__(512) kb_disagg_mx(int N, int S, int R, const int *tile_box,
-                                                    const int *tile_p0, const int *box_first,
-                                                    const int *box_count, const int *perm,
-                                                    const zf *rt, const zf *W, zf sc1, zf sc2,
-                                                    int sblk, zf *yp) {
-  __shared__ float4 wl[2 * kMxSC * 2 * 16];
+template <bool HALF>
+__device__ __forceinline__ void kb_disagg_mx_part(int N, PatLay lay, int R, const int *tile_box,
+                                                  const int *tile_p0, const int *box_first,
+                                                  const int *box_count, const int *perm,
+                                                  const zf *rt, const zf *W, zf sc1, zf sc2, zf *yp,
+                                                  float4 *wl) {
+  constexpr int PM = HALF ? 2 : 1;
   const int b = tile_box[blockIdx.x], p0 = tile_p0[blockIdx.x];
   const int cnt = min(128, box_first[b] + box_count[b] - p0);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
   const int ew = 16 * wv;
   const bool active = ew < cnt;  // uniform over the wave
-  const zf *F = rt + (size_t)(p0 + min(ew + m, cnt - 1)) * 4 * S;
-  const size_t SR = (size_t)S * R;
-  const zf *Wb = W + (size_t)b * 8 * SR;
-  const int s_lo = blockIdx.y * sblk, s_hi = min(S, s_lo + sblk);
+  const int k = blockIdx.y >> 1, L = lay.L[k];
+  const zf *F = rt + (size_t)(p0 + min(ew + m, cnt - 1)) * lay.stride() + lay.row(k, 0);
+  const zf *Wb = W + ((size_t)b * 8 + k * 4) * lay.SW * R;
+  const int sblk = ((L + 63) / 64) * kMxSC;
+  const int s_lo = (blockIdx.y & 1) * sblk, s_hi = min(L, s_lo + sblk);
   mxf4 er = {0.f, 0.f, 0.f, 0.f}, ei = er, hr = er, hi = er;
-  // pattern rows 2k and 2k+1 at samples s + 4g .. s + 4g + 3 (pairs clamped, S is even)
-  auto load = [&](int s, int k, float4 *a) {
-    const int s1 = min(s + 4 * g, S - 2), s2 = min(s + 4 * g + 2, S - 2);
-    const zf *fa = F + (size_t)(2 * k) * S, *fb = fa + S;
-    a[0] = *reinterpret_cast<const float4 *>(fa + s1);
-    a[1] = *reinterpret_cast<const float4 *>(fa + s2);
-    a[2] = *reinterpret_cast<const float4 *>(fb + s1);
-    a[3] = *reinterpret_cast<const float4 *>(fb + s2);
+  // both pattern rows at entries s + 4g .. s + 4g + 3 (pairs clamped, L is even)
+  auto load = [&](int s, float4 *a) {
+    const int s1 = min(s + 4 * g, L - 2), s2 = min(s + 4 * g + 2, L - 2);
+    a[0] = *reinterpret_cast<const float4 *>(F + s1);
+    a[1] = *reinterpret_cast<const float4 *>(F + s2);
+    a[2] = *reinterpret_cast<const float4 *>(F + L + s1);
+    a[3] = *reinterpret_cast<const float4 *>(F + L + s2);
   };
   float4 cur[4];
-  if (active && s_lo < s_hi) load(s_lo, 0, cur);
+  if (active && s_lo < s_hi) load(s_lo, cur);
   for (int s0 = s_lo; s0 < s_hi; s0 += kMxSC) {
     __syncthreads();
     {
-      // W[it][s0 + i][r] -> wl as complex [((k * kMxSC + i) * 2 + half) * 16 + r][jj], it = 4k + 2half + jj
+      // W[it][s0 + i][r] -> wl as complex [((pm * kMxSC + i) * 2 + half) * 16 + r][jj], it = 2half + jj
       zf *wc = reinterpret_cast<zf *>(wl);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < 4 * PM; ++u) {
         const int t = threadIdx.x + 512 * u;
-        const int r = t & 15, i = (t >> 4) & (kMxSC - 1), it = t >> 9;
+        const int r = t & 15, i = (t >> 4) & (kMxSC - 1), it = (t >> 9) & 3, pm = t >> 11;
         const int s = s0 + i;
         const bool ok = r < R && s < s_hi;
-        const zf v = Wb[((size_t)it * S + min(s, S - 1)) * R + min(r, R - 1)];
-        const int k = it >> 2, half = (it >> 1) & 1, jj = it & 1;
-        wc[(((k * kMxSC + i) * 2 + half) * 16 + r) * 2 + jj] = ok ? v : zf{0.f, 0.f};
+        const zf v = Wb[((size_t)it * lay.SW + pm * L + min(s, L - 1)) * R + min(r, R - 1)];
+        const int half = it >> 1, jj = it & 1;
+        wc[(((pm * kMxSC + i) * 2 + half) * 16 + r) * 2 + jj] = ok ? v : zf{0.f, 0.f};
       }
     }
     __syncthreads();
     if (!active) continue;
     for (int sg = 0; sg < kMxSC && s0 + sg < s_hi; sg += 16) {
+      float4 nx[4];
+      load(s0 + sg + 16, nx);
+      __builtin_amdgcn_sched_barrier(0);
+      const float fa[8] = {cur[0].x, cur[0].y, cur[0].z, cur[0].w, cur[1].x, cur[1].y, cur[1].z, cur[1].w};
+      const float fb[8] = {cur[2].x, cur[2].y, cur[2].z, cur[2].w, cur[3].x, cur[3].y, cur[3].z, cur[3].w};
+      // the group's 16 entries are summed from zero and then added to the
+      // running sums, so the running sums take one rounding per group
+      mxf4 gr = {0.f, 0.f, 0.f, 0.f}, gi = gr, gh = gr, gj = gr;
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        float4 nx[4];
-        if (k == 0)
-          load(s0 + sg, 1, nx);
-        else
-          load(s0 + sg + 16, 0, nx);
-        __builtin_amdgcn_sched_barrier(0);
-        const float fa[8] = {cur[0].x, cur[0].y, cur[0].z, cur[0].w, cur[1].x, cur[1].y, cur[1].z, cur[1].w};
-        const float fb[8] = {cur[2].x, cur[2].y, cur[2].z, cur[2].w, cur[3].x, cur[3].y, cur[3].z, cur[3].w};
-        // the group's 16 samples are summed from zero and then added to the
-        // running sums, so the running sums take one rounding per group
-        mxf4 gr = {0.f, 0.f, 0.f, 0.f}, gi = gr, gh = gr, gj = gr;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = sg + 4 * g + j;
-          const float4 we = wl[((k * kMxSC + i) * 2 + 0) * 16 + m];  // (e,a), (e,b)
-          const float4 wh = wl[((k * kMxSC + i) * 2 + 1) * 16 + m];  // (h,a), (h,b)
-          const float ar = fa[2 * j], ai = fa[2 * j + 1], br = fb[2 * j], bi = fb[2 * j + 1];
-          const float nai = -ai, nbi = -bi;
-          gr = SPK_MFMA(ar, we.x, gr);
-          gi = SPK_MFMA(ar, we.y, gi);
-          gh = SPK_MFMA(ar, wh.x, gh);
-          gj = SPK_MFMA(ar, wh.y, gj);
-          gr = SPK_MFMA(nai, we.y, gr);
+      for (int j = 0; j < 4; ++j) {
+        const int i = sg + 4 * g + j;
+        const float4 we = wl[(i * 2 + 0) * 16 + m];  // (e,a), (e,b)
+        const float4 wh = wl[(i * 2 + 1) * 16 + m];  // (h,a), (h,b)
+        const float ar = fa[2 * j], ai = fa[2 * j + 1], br = fb[2 * j], bi = fb[2 * j + 1];
+        gr = SPK_MFMA(ar, we.x, gr);
+        gi = SPK_MFMA(ar, we.y, gi);
+        gh = SPK_MFMA(ar, wh.x, gh);
+        gj = SPK_MFMA(ar, wh.y, gj);
+        if constexpr (HALF) {
+          const float4 me = wl[((kMxSC + i) * 2 + 0) * 16 + m], mh = wl[((kMxSC + i) * 2 + 1) * 16 + m];
+          gr = SPK_MFMA(ai, me.x, gr);
+          gi = SPK_MFMA(ai, me.y, gi);
+          gh = SPK_MFMA(ai, mh.x, gh);
+          gj = SPK_MFMA(ai, mh.y, gj);
+          gr = SPK_MFMA(br, we.z, gr);
+          gi = SPK_MFMA(br, we.w, gi);
+          gh = SPK_MFMA(br, wh.z, gh);
+          gj = SPK_MFMA(br, wh.w, gj);
+          gr = SPK_MFMA(bi, me.z, gr);
+          gi = SPK_MFMA(bi, me.w, gi);
+          gh = SPK_MFMA(bi, mh.z, gh);
+          gj = SPK_MFMA(bi, mh.w, gj);
+        } else {
+          gr = SPK_MFMA(-ai, we.y, gr);
           gi = SPK_MFMA(ai, we.x, gi);
-          gh = SPK_MFMA(nai, wh.y, gh);
+          gh = SPK_MFMA(-ai, wh.y, gh);
           gj = SPK_MFMA(ai, wh.x, gj);
           gr = SPK_MFMA(br, we.z, gr);
           gi = SPK_MFMA(br, we.w, gi);
           gh = SPK_MFMA(br, wh.z, gh);
           gj = SPK_MFMA(br, wh.w, gj);
-          gr = SPK_MFMA(nbi, we.w, gr);
+          gr = SPK_MFMA(-bi, we.w, gr);
           gi = SPK_MFMA(bi, we.z, gi);
-          gh = SPK_MFMA(nbi, wh.w, gh);
+          gh = SPK_MFMA(-bi, wh.w, gh);
           gj = SPK_MFMA(bi, wh.z, gj);
         }
-        er += gr;
-        ei += gi;
-        hr += gh;
-        hi += gj;
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) cur[u] = nx[u];
       }
+      er += gr;
+      ei += gi;
+      hr += gh;
+      hi += gj;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) cur[u] = nx[u];
     }
   }
   // accumulator element v of lane (g, n): edge ew + 4g + v, right-hand side n
   const int n = m;
   if (!active || n >= R) return;
-  zf *yf = yp + (size_t)blockIdx.y * R * 2 * N;
+  zf *yf = yp + (size_t)(2 * k + (blockIdx.y & 1)) * R * 2 * N;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int e = ew + 4 * g + v;
@@ -521,6 +686,20 @@ __global__ void __launch_bounds__(512) kb_disagg_mx(int N, int S, int R, const i
       yf[(size_t)n * 2 * N + mm + N] = zf{hr[v], hi[v]} * sc2;
     }
   }
+}
+template <int MODE>
+__global__ void __launch_bounds__(512) kb_disagg_mx(int N, PatLay lay, int R, const int *tile_box,
+                                                    const int *tile_p0, const int *box_first,
+                                                    const int *box_count, const int *perm,
+                                                    const zf *rt, const zf *W, zf sc1, zf sc2,
+                                                    zf *yp) {
+  __shared__ float4 wl[(MODE ? 2 : 1) * kMxSC * 2 * 16];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.y >> 1]))
+    kb_disagg_mx_part<true>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W, sc1,
+                            sc2, yp, wl);
+  else if (MODE != 1)
+    kb_disagg_mx_part<false>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W, sc1,
+                             sc2, yp, wl);
 }
 
 // Near field for R vectors: workgroup = (leaf box, 16 rows), 4 rows per
@@ -875,35 +1054,42 @@ __global__ void __launch_bounds__(256) kb_near_mx64(int N, int R, const int *row
   }
 }
 
-// aggregation: workgroup = (128 samples, box, q), wave = 32 samples as 2
-// tiles of 16 (tile t: samples sw + 16 t + i); k-step = 4 edges
-__global__ void __launch_bounds__(256) kb_agg_mx64(int S, int R, const int *box_first,
-                                                   const int *box_count, const zd *rt,
-                                                   const zd *XP, zd *C) {
-  __shared__ double4 xl[32 * 16];
+// aggregation: a wave takes NL tiles of 16 entries (NL = 1 in a HALF medium, 2
+// in one with losses; workgroup = 64 or 128 entries, box, q); tile t: entries
+// sw + 16 t + i; k-step = 4 edges; HALF as in kb_agg_mx
+template <bool HALF>
+__device__ __forceinline__ void kb_agg_mx64_part(const PatLay &lay, int R, const int *box_first,
+                                                 const int *box_count, const zd *rt,
+                                                 const zd *XP, zd *C, double4 *xl) {
+  constexpr int V = HALF ? 8 : 4, NL = HALF ? 1 : 2;
   const int b = blockIdx.y, q = blockIdx.z, k = q >> 1, comp = q & 1;
   const int p0 = box_first[b], cnt = box_count[b];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int sw = blockIdx.x * 128 + 32 * wv;
-  const bool active = sw < S;
-  const int sa = min(sw + m, S - 1), sb = min(sw + 16 + m, S - 1);
-  mxd4 acc[2][4];
+  const int L = lay.L[k];
+  if ((int)blockIdx.x * 64 * NL >= L) return;
+  const int sw = blockIdx.x * 64 * NL + 16 * NL * wv;
+  const bool active = sw < L;
+  const size_t ps = lay.stride();
+  const double2 *F = reinterpret_cast<const double2 *>(rt + (size_t)p0 * ps + lay.row(k, comp));
+  int so[NL];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < NL; ++t) so[t] = min(sw + 16 * t + m, L - 1);
+  mxd4 acc[NL][V];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) acc[t][u] = mxd4{0.0, 0.0, 0.0, 0.0};
-  double2 fa[4], fb[4];
-  auto load = [&](int e0, double2 *a, double2 *bb) {
+  for (int t = 0; t < NL; ++t)
+#pragma unroll
+    for (int u = 0; u < V; ++u) acc[t][u] = mxd4{0.0, 0.0, 0.0, 0.0};
+  double2 fa[4][NL];
+  auto load = [&](int e0, double2 (*a)[NL]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int e = min(e0 + 4 * j + g, cnt - 1);
-      const double2 *f = reinterpret_cast<const double2 *>(rt + ((size_t)(p0 + e) * 4 + q) * S);
-      a[j] = f[sa];
-      bb[j] = f[sb];
+      const double2 *f = F + (size_t)min(e0 + 4 * j + g, cnt - 1) * ps;
+#pragma unroll
+      for (int t = 0; t < NL; ++t) a[j][t] = f[so[t]];
     }
   };
-  if (active && cnt > 0) load(0, fa, fb);
+  if (active && cnt > 0) load(0, fa);
   for (int e0 = 0; e0 < cnt; e0 += 32) {
     const int ne = min(32, cnt - e0);
     __syncthreads();
@@ -914,149 +1100,188 @@ __global__ void __launch_bounds__(256) kb_agg_mx64(int S, int R, const int *box_
         const int e = (int)(threadIdx.x + 256 * u) >> 4;
         const size_t pe = (size_t)(p0 + e0 + min(e, ne - 1)) * 2;
         const zd x0 = XP[pe * 16 + n], x1 = XP[(pe + 1) * 16 + n];
-        xl[threadIdx.x + 256 * u] = e < ne ? double4{x0.x, x0.y, x1.x, x1.y} : double4{0.0, 0.0, 0.0, 0.0};
+        xl[threadIdx.x + 256 * u] =
+            e < ne ? double4{x0.x, x0.y, x1.x, x1.y} : double4{0.0, 0.0, 0.0, 0.0};
       }
     }
     __syncthreads();
     if (!active) continue;
     for (int i = 0; i < ne; i += 16) {
-      double2 na[4], nb[4];
-      load(e0 + i + 16, na, nb);
+      double2 na[4][NL];
+      load(e0 + i + 16, na);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const double4 x = xl[(i + 4 * j + g) * 16 + m];
         const double n0 = -x.x, n1 = -x.z;
-        const double ar[2] = {fa[j].x, fb[j].x}, ai[2] = {fa[j].y, fb[j].y};
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          acc[t][0] = SPK_MFMA64(ar[t], x.x, acc[t][0]);
-          acc[t][1] = SPK_MFMA64(ar[t], x.y, acc[t][1]);
-          acc[t][2] = SPK_MFMA64(ar[t], x.z, acc[t][2]);
-          acc[t][3] = SPK_MFMA64(ar[t], x.w, acc[t][3]);
+        for (int t = 0; t < NL; ++t) {
+          const double ar = fa[j][t].x;
+          acc[t][0] = SPK_MFMA64(ar, x.x, acc[t][0]);
+          acc[t][1] = SPK_MFMA64(ar, x.y, acc[t][1]);
+          acc[t][2] = SPK_MFMA64(ar, x.z, acc[t][2]);
+          acc[t][3] = SPK_MFMA64(ar, x.w, acc[t][3]);
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          acc[t][0] = SPK_MFMA64(ai[t], x.y, acc[t][0]);
-          acc[t][1] = SPK_MFMA64(ai[t], n0, acc[t][1]);
-          acc[t][2] = SPK_MFMA64(ai[t], x.w, acc[t][2]);
-          acc[t][3] = SPK_MFMA64(ai[t], n1, acc[t][3]);
+        for (int t = 0; t < NL; ++t) {
+          const double ai = fa[j][t].y;
+          if constexpr (HALF) {
+            acc[t][4] = SPK_MFMA64(ai, x.x, acc[t][4]);
+            acc[t][5] = SPK_MFMA64(ai, x.y, acc[t][5]);
+            acc[t][6] = SPK_MFMA64(ai, x.z, acc[t][6]);
+            acc[t][7] = SPK_MFMA64(ai, x.w, acc[t][7]);
+          } else {
+            acc[t][0] = SPK_MFMA64(ai, x.y, acc[t][0]);
+            acc[t][1] = SPK_MFMA64(ai, n0, acc[t][1]);
+            acc[t][2] = SPK_MFMA64(ai, x.w, acc[t][2]);
+            acc[t][3] = SPK_MFMA64(ai, n1, acc[t][3]);
+          }
         }
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        fa[j] = na[j];
-        fb[j] = nb[j];
-      }
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < NL; ++t) fa[j][t] = na[j][t];
     }
   }
-  const int n = m;
+  const int n = m, lim = HALF ? lay.count() : lay.S;
   if (!active || n >= R) return;
-  zd *Cb = C + (size_t)b * 8 * S * R;
+  zd *Ce = C + ((size_t)b * 8 + comp * 4 + k) * lay.S * R + n, *Ch = Ce + 2 * (size_t)lay.S * R;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < NL; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int s = sw + 16 * t + 4 * v + g;
-      if (s < S) {
-        Cb[((size_t)(comp * 4 + 0 + k) * S + s) * R + n] = zd{acc[t][0][v], acc[t][1][v]};
-        Cb[((size_t)(comp * 4 + 2 + k) * S + s) * R + n] = zd{acc[t][2][v], acc[t][3][v]};
+      if (s >= lim) continue;
+      if constexpr (HALF) {
+        const double sg = lay.flips(s, comp) ? -1.0 : 1.0;
+        const size_t o = (size_t)lay.samp(s) * R, oa = (size_t)lay.anti(s) * R;
+        Ce[o] = zd{acc[t][0][v] + acc[t][5][v], acc[t][1][v] - acc[t][4][v]};
+        Ch[o] = zd{acc[t][2][v] + acc[t][7][v], acc[t][3][v] - acc[t][6][v]};
+        Ce[oa] = zd{acc[t][0][v] - acc[t][5][v], acc[t][1][v] + acc[t][4][v]} * sg;
+        Ch[oa] = zd{acc[t][2][v] - acc[t][7][v], acc[t][3][v] + acc[t][6][v]} * sg;
+      } else {
+        Ce[(size_t)s * R] = zd{acc[t][0][v], acc[t][1][v]};
+        Ch[(size_t)s * R] = zd{acc[t][2][v], acc[t][3][v]};
       }
     }
 }
+template <int MODE>
+__global__ void __launch_bounds__(256) kb_agg_mx64(PatLay lay, int R, const int *box_first,
+                                                   const int *box_count, const zd *rt,
+                                                   const zd *XP, zd *C) {
+  __shared__ double4 xl[32 * 16];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.z >> 1]))
+    kb_agg_mx64_part<true>(lay, R, box_first, box_count, rt, XP, C, xl);
+  else if (MODE != 1)
+    kb_agg_mx64_part<false>(lay, R, box_first, box_count, rt, XP, C, xl);
+}
 
-// disaggregation: workgroup = (up to 128 edges of a box, sample part),
-// wave = 16 edges; k-step = 4 samples (lane group g takes sample s + 4g + j
-// in step j); W staged in LDS 16 samples at a time as [k][sample][e/h][r]
+// disaggregation: workgroup = (up to 128 edges of a box; blockIdx.y = half of
+// one medium's entries), wave = 16 edges; k-step = 4 entries (lane group g
+// takes entry s + 4g + j in step j); W staged in LDS 16 entries at a time as
+// [P/M][entry][e/h][r]; HALF as in kb_disagg_mx
 constexpr int kMx64SC = 16;
-__global__ void __launch_bounds__(512) kb_disagg_mx64(int N, int S, int R, const int *tile_box,
-                                                      const int *tile_p0, const int *box_first,
-                                                      const int *box_count, const int *perm,
-                                                      const zd *rt, const zd *W, zd sc1, zd sc2,
-                                                      int sblk, zd *yp) {
-  __shared__ double4 wl[2 * kMx64SC * 2 * 16];
+template <bool HALF>
+__device__ __forceinline__ void kb_disagg_mx64_part(int N, PatLay lay, int R, const int *tile_box,
+                                                    const int *tile_p0, const int *box_first,
+                                                    const int *box_count, const int *perm,
+                                                    const zd *rt, const zd *W, zd sc1, zd sc2,
+                                                    zd *yp, double4 *wl) {
+  constexpr int PM = HALF ? 2 : 1;
   const int b = tile_box[blockIdx.x], p0 = tile_p0[blockIdx.x];
   const int cnt = min(128, box_first[b] + box_count[b] - p0);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
   const int ew = 16 * wv;
   const bool active = ew < cnt;
-  const double2 *F = reinterpret_cast<const double2 *>(rt + (size_t)(p0 + min(ew + m, cnt - 1)) * 4 * S);
-  const size_t SR = (size_t)S * R;
-  const zd *Wb = W + (size_t)b * 8 * SR;
-  const int s_lo = blockIdx.y * sblk, s_hi = min(S, s_lo + sblk);
+  const int k = blockIdx.y >> 1, L = lay.L[k];
+  const double2 *F = reinterpret_cast<const double2 *>(
+      rt + (size_t)(p0 + min(ew + m, cnt - 1)) * lay.stride() + lay.row(k, 0));
+  const zd *Wb = W + ((size_t)b * 8 + k * 4) * lay.SW * R;
+  const int sblk = ((L + 31) / 32) * kMx64SC;
+  const int s_lo = (blockIdx.y & 1) * sblk, s_hi = min(L, s_lo + sblk);
   mxd4 er = {0.0, 0.0, 0.0, 0.0}, ei = er, hr = er, hi = er;
-  // pattern rows 2k and 2k+1 at samples s + 4g .. s + 4g + 3 (clamped)
-  auto load = [&](int s, int k, double2 *a) {
-    const double2 *fa = F + (size_t)(2 * k) * S, *fb = fa + S;
+  // both pattern rows at entries s + 4g .. s + 4g + 3 (clamped)
+  auto load = [&](int s, double2 *a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int sj = min(s + 4 * g + j, S - 1);
-      a[j] = fa[sj];
-      a[4 + j] = fb[sj];
+      const int sj = min(s + 4 * g + j, L - 1);
+      a[j] = F[sj];
+      a[4 + j] = F[L + sj];
     }
   };
   double2 cur[8];
-  if (active && s_lo < s_hi) load(s_lo, 0, cur);
+  if (active && s_lo < s_hi) load(s_lo, cur);
   for (int s0 = s_lo; s0 < s_hi; s0 += kMx64SC) {
     __syncthreads();
     {
-      // W[it][s0 + i][r] -> wl as complex [((k * SC + i) * 2 + half) * 16 + r][jj], it = 4k + 2half + jj
+      // W[it][s0 + i][r] -> wl as complex [((pm * SC + i) * 2 + half) * 16 + r][jj], it = 2half + jj
       zd *wc = reinterpret_cast<zd *>(wl);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < 2 * PM; ++u) {
         const int t = threadIdx.x + 512 * u;
-        const int r = t & 15, i = (t >> 4) & (kMx64SC - 1), it = t >> 8;
+        const int r = t & 15, i = (t >> 4) & (kMx64SC - 1), it = (t >> 8) & 3, pm = t >> 10;
         const int s = s0 + i;
         const bool ok = r < R && s < s_hi;
-        const zd v = Wb[((size_t)it * S + min(s, S - 1)) * R + min(r, R - 1)];
-        const int k = it >> 2, half = (it >> 1) & 1, jj = it & 1;
-        wc[(((k * kMx64SC + i) * 2 + half) * 16 + r) * 2 + jj] = ok ? v : zd{0.0, 0.0};
+        const zd v = Wb[((size_t)it * lay.SW + pm * L + min(s, L - 1)) * R + min(r, R - 1)];
+        const int half = it >> 1, jj = it & 1;
+        wc[(((pm * kMx64SC + i) * 2 + half) * 16 + r) * 2 + jj] = ok ? v : zd{0.0, 0.0};
       }
     }
     __syncthreads();
     if (!active) continue;
+    double2 nx[8];
+    load(s0 + kMx64SC, nx);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      double2 nx[8];
-      if (k == 0)
-        load(s0, 1, nx);
-      else
-        load(s0 + kMx64SC, 0, nx);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i = 4 * g + j;
-        const double4 we = wl[((k * kMx64SC + i) * 2 + 0) * 16 + m];  // (e,a), (e,b)
-        const double4 wh = wl[((k * kMx64SC + i) * 2 + 1) * 16 + m];  // (h,a), (h,b)
-        const double ar = cur[j].x, ai = cur[j].y, br = cur[4 + j].x, bi = cur[4 + j].y;
-        const double nai = -ai, nbi = -bi;
-        er = SPK_MFMA64(ar, we.x, er);
-        ei = SPK_MFMA64(ar, we.y, ei);
-        hr = SPK_MFMA64(ar, wh.x, hr);
-        hi = SPK_MFMA64(ar, wh.y, hi);
-        er = SPK_MFMA64(nai, we.y, er);
+    for (int j = 0; j < 4; ++j) {
+      const int i = 4 * g + j;
+      const double4 we = wl[(i * 2 + 0) * 16 + m];  // (e,a), (e,b)
+      const double4 wh = wl[(i * 2 + 1) * 16 + m];  // (h,a), (h,b)
+      const double ar = cur[j].x, ai = cur[j].y, br = cur[4 + j].x, bi = cur[4 + j].y;
+      er = SPK_MFMA64(ar, we.x, er);
+      ei = SPK_MFMA64(ar, we.y, ei);
+      hr = SPK_MFMA64(ar, wh.x, hr);
+      hi = SPK_MFMA64(ar, wh.y, hi);
+      if constexpr (HALF) {
+        const double4 me = wl[((kMx64SC + i) * 2 + 0) * 16 + m];
+        const double4 mh = wl[((kMx64SC + i) * 2 + 1) * 16 + m];
+        er = SPK_MFMA64(ai, me.x, er);
+        ei = SPK_MFMA64(ai, me.y, ei);
+        hr = SPK_MFMA64(ai, mh.x, hr);
+        hi = SPK_MFMA64(ai, mh.y, hi);
+        er = SPK_MFMA64(br, we.z, er);
+        ei = SPK_MFMA64(br, we.w, ei);
+        hr = SPK_MFMA64(br, wh.z, hr);
+        hi = SPK_MFMA64(br, wh.w, hi);
+        er = SPK_MFMA64(bi, me.z, er);
+        ei = SPK_MFMA64(bi, me.w, ei);
+        hr = SPK_MFMA64(bi, mh.z, hr);
+        hi = SPK_MFMA64(bi, mh.w, hi);
+      } else {
+        er = SPK_MFMA64(-ai, we.y, er);
         ei = SPK_MFMA64(ai, we.x, ei);
-        hr = SPK_MFMA64(nai, wh.y, hr);
+        hr = SPK_MFMA64(-ai, wh.y, hr);
         hi = SPK_MFMA64(ai, wh.x, hi);
         er = SPK_MFMA64(br, we.z, er);
         ei = SPK_MFMA64(br, we.w, ei);
         hr = SPK_MFMA64(br, wh.z, hr);
         hi = SPK_MFMA64(br, wh.w, hi);
-        er = SPK_MFMA64(nbi, we.w, er);
+        er = SPK_MFMA64(-bi, we.w, er);
         ei = SPK_MFMA64(bi, we.z, ei);
-        hr = SPK_MFMA64(nbi, wh.w, hr);
+        hr = SPK_MFMA64(-bi, wh.w, hr);
         hi = SPK_MFMA64(bi, wh.z, hi);
       }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) cur[u] = nx[u];
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) cur[u] = nx[u];
   }
   const int n = m;
   if (!active || n >= R) return;
-  zd *yf = yp + (size_t)blockIdx.y * R * 2 * N;
+  zd *yf = yp + (size_t)(2 * k + (blockIdx.y & 1)) * R * 2 * N;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int e = ew + 4 * v + g;
@@ -1066,6 +1291,20 @@ __global__ void __launch_bounds__(512) kb_disagg_mx64(int N, int S, int R, const
       yf[(size_t)n * 2 * N + mm + N] = zd{hr[v], hi[v]} * sc2;
     }
   }
+}
+template <int MODE>
+__global__ void __launch_bounds__(512) kb_disagg_mx64(int N, PatLay lay, int R, const int *tile_box,
+                                                      const int *tile_p0, const int *box_first,
+                                                      const int *box_count, const int *perm,
+                                                      const zd *rt, const zd *W, zd sc1, zd sc2,
+                                                      zd *yp) {
+  __shared__ double4 wl[(MODE ? 2 : 1) * kMx64SC * 2 * 16];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.y >> 1]))
+    kb_disagg_mx64_part<true>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W, sc1,
+                              sc2, yp, wl);
+  else if (MODE != 1)
+    kb_disagg_mx64_part<false>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W, sc1,
+                               sc2, yp, wl);
 }
 
 // ---------------------------------------------------------------------------
@@ -1818,33 +2057,46 @@ void launch_batch_interleave(int N, int R, const int *perm, const T *const *xs, 
 #undef SPK_IL_CASE
   }
 }
+// kernels on pattern rows take a MODE: 1 both media keep half of the samples,
+// 0 neither does, 2 one of them does.  Both media go in one launch: at 8
+// vectors and 64 boxes either medium's blocks alone leave most of the chip
+// idle (0.16 and 0.19 ms one after the other, 0.20 ms together).
+static int half_mode(const PatLay &lay) {
+  return lay.half[0] && lay.half[1] ? 1 : lay.half[0] || lay.half[1] ? 2 : 0;
+}
 template <class T>
-void launch_batch_agg(int nbl, int S, int N, int R, const int *box_first, const int *box_count,
-                      const int *perm, const T *rt, const T *XI, const T *XP, T *C,
-                      hipStream_t st) {
+void launch_batch_agg(int nbl, const PatLay &lay, int N, int R, const int *box_first,
+                      const int *box_count, const int *perm, const T *rt, const T *XI, const T *XP,
+                      T *C, hipStream_t st) {
   if (nbl <= 0) return;
   (void)XI;
   (void)perm;
-  const dim3 g(bnblk(S, 256), nbl, 4);
-  if constexpr (std::is_same<T, zf>::value) {
-    if (batch_pad(R) == 16) {
-      hipLaunchKernelGGL(kb_agg_mx, g, dim3(256), 0, st, S, R, box_first, box_count, rt, XP, C);
-      return;
-    }
-  } else {
-    if (batch_pad(R) == 16) {
-      hipLaunchKernelGGL(kb_agg_mx64, dim3(bnblk(S, 128), nbl, 4), dim3(256), 0, st, S, R, box_first,
-                         box_count, rt, XP, C);
-      return;
-    }
+  (void)N;
+  const int mode = half_mode(lay);
+  // tiles of e entries in a half medium's rows, 2e in a whole medium's
+  auto grid = [&](int e) {
+    unsigned t = 0;
+    for (int k = 0; k < 2; ++k) t = std::max(t, bnblk(lay.L[k], lay.half[k] ? e : 2 * e));
+    return dim3(t, nbl, 4);
+  };
+  if (batch_pad(R) == 16) {
+    if constexpr (std::is_same<T, zf>::value)
+      hipLaunchKernelGGL((mode == 1 ? kb_agg_mx<1> : mode == 2 ? kb_agg_mx<2> : kb_agg_mx<0>),
+                         grid(128), dim3(256), 0, st, lay, R, box_first, box_count, rt, XP, C);
+    else
+      hipLaunchKernelGGL((mode == 1 ? kb_agg_mx64<1> : mode == 2 ? kb_agg_mx64<2> : kb_agg_mx64<0>),
+                         grid(64), dim3(256), 0, st, lay, R, box_first, box_count, rt, XP, C);
+    return;
   }
   switch (batch_pad(R)) {
-#define SPK_AGG_CASE(RP)                                                                       \
-  case RP:                                                                                     \
-    hipLaunchKernelGGL((kb_agg<T, RP>), g, dim3(256), 0, st, S, N, R, box_first, box_count,     \
-                       rt, XP, C);                                                             \
+#define SPK_AGG_CASE(RP)                                                                           \
+  case RP:                                                                                         \
+    hipLaunchKernelGGL((mode == 1   ? kb_agg<T, RP, 1>                                             \
+                        : mode == 2 ? kb_agg<T, RP, 2>                                             \
+                                    : kb_agg<T, RP, 0>),                                           \
+                       grid(128), dim3(256), 0, st, lay, R, box_first, box_count, rt, XP, C);      \
     break;
-    SPK_AGG_CASE(1) SPK_AGG_CASE(2) SPK_AGG_CASE(4) SPK_AGG_CASE(8) SPK_AGG_CASE(16)
+    SPK_AGG_CASE(1) SPK_AGG_CASE(2) SPK_AGG_CASE(4) SPK_AGG_CASE(8)
 #undef SPK_AGG_CASE
   }
 }
@@ -1872,10 +2124,11 @@ void launch_batch_rr(int nb, int S, int R, const int *parent, const int *octant,
                      parent, octant, Dp, down, Dc);
 }
 template <class T>
-void launch_batch_fold(int nbl, int S, int R, const T *D, zd kd1, zd kd2, zd my1, zd my2, zd ep1,
-                       zd ep2, T *W, hipStream_t st) {
+void launch_batch_fold(int nbl, const PatLay &lay, int R, const T *D, zd kd1, zd kd2, zd my1,
+                       zd my2, zd ep1, zd ep2, T *W, hipStream_t st) {
   if (nbl <= 0) return;
-  hipLaunchKernelGGL(kb_fold<T>, dim3(bnblk((int64_t)S * R, 256), nbl), dim3(256), 0, st, S, R, D,
+  const int64_t n = (int64_t)std::max(lay.L[0], lay.L[1]) * R;
+  hipLaunchKernelGGL(kb_fold<T>, dim3(bnblk(n, 256), nbl, 2), dim3(256), 0, st, lay, R, D,
                      cvt<T>(kd1), cvt<T>(kd2), cvt<T>(my1), cvt<T>(my2), cvt<T>(ep1), cvt<T>(ep2),
                      W);
 }
@@ -1890,33 +2143,38 @@ __global__ void kb_sum_split(int64_t len, const T *yp, T *yf) {
 }
 
 template <class T>
-void launch_batch_disagg(int ntiles, int N, int S, int R, const int *tile_box, const int *tile_p0,
-                         const int *box_first, const int *box_count, const int *perm, const T *rt,
-                         const T *W, zd sc1, zd sc2, T *yp, T *yf, int mx_tiles,
-                         const int *mx_box, const int *mx_p0, hipStream_t st) {
+void launch_batch_disagg(int ntiles, int N, const PatLay &lay, int R, const int *tile_box,
+                         const int *tile_p0, const int *box_first, const int *box_count,
+                         const int *perm, const T *rt, const T *W, zd sc1, zd sc2, T *yp, T *yf,
+                         int mx_tiles, const int *mx_box, const int *mx_p0, hipStream_t st) {
   if (ntiles <= 0) return;
-  // samples split over kBatchSplit workgroups per tile (multiples of 16 samples)
-  const int sblk = (int)bnblk(bnblk(S, 16), kBatchSplit) * 16;
-  const dim3 g(ntiles, kBatchSplit);
-  bool done = false;
-  if (batch_pad(R) == 16 && mx_tiles > 0) {
+  // two workgroups per tile and medium, each half of the medium's entries
+  const int mode = half_mode(lay);
+  if (batch_pad(R) == 16) {
+    const dim3 g(mx_tiles, 4);
     if constexpr (std::is_same<T, zf>::value)
-      hipLaunchKernelGGL(kb_disagg_mx, dim3(mx_tiles, kBatchSplit), dim3(512), 0, st, N, S, R,
-                         mx_box, mx_p0, box_first, box_count, perm, rt, W, cvt<T>(sc1),
-                         cvt<T>(sc2), sblk, yp);
+      hipLaunchKernelGGL(
+          (mode == 1 ? kb_disagg_mx<1> : mode == 2 ? kb_disagg_mx<2> : kb_disagg_mx<0>), g,
+          dim3(512), 0, st, N, lay, R, mx_box, mx_p0, box_first, box_count, perm, rt, W,
+          cvt<T>(sc1), cvt<T>(sc2), yp);
     else
-      hipLaunchKernelGGL(kb_disagg_mx64, dim3(mx_tiles, kBatchSplit), dim3(512), 0, st, N, S, R,
-                         mx_box, mx_p0, box_first, box_count, perm, rt, W, sc1, sc2, sblk, yp);
-    done = true;
-  }
-  if (!done) switch (batch_pad(R)) {
-#define SPK_DIS_CASE(RP)                                                                        \
-  case RP:                                                                                      \
-    hipLaunchKernelGGL((kb_disagg<T, RP>), g, dim3(16 * RP), 0, st, N, S, R, tile_box, tile_p0, \
-                       box_first, box_count, perm, rt, W, cvt<T>(sc1), cvt<T>(sc2), sblk, yp);  \
+      hipLaunchKernelGGL(
+          (mode == 1 ? kb_disagg_mx64<1> : mode == 2 ? kb_disagg_mx64<2> : kb_disagg_mx64<0>), g,
+          dim3(512), 0, st, N, lay, R, mx_box, mx_p0, box_first, box_count, perm, rt, W, sc1, sc2,
+          yp);
+  } else {
+    switch (batch_pad(R)) {
+#define SPK_DIS_CASE(RP)                                                                          \
+  case RP:                                                                                        \
+    hipLaunchKernelGGL((mode == 1   ? kb_disagg<T, RP, 1>                                         \
+                        : mode == 2 ? kb_disagg<T, RP, 2>                                         \
+                                    : kb_disagg<T, RP, 0>),                                       \
+                       dim3(ntiles, 4), dim3(16 * RP), 0, st, N, lay, R, tile_box, tile_p0,       \
+                       box_first, box_count, perm, rt, W, cvt<T>(sc1), cvt<T>(sc2), yp);          \
     break;
-    SPK_DIS_CASE(1) SPK_DIS_CASE(2) SPK_DIS_CASE(4) SPK_DIS_CASE(8) SPK_DIS_CASE(16)
+      SPK_DIS_CASE(1) SPK_DIS_CASE(2) SPK_DIS_CASE(4) SPK_DIS_CASE(8)
 #undef SPK_DIS_CASE
+    }
   }
   const int64_t len = (int64_t)R * 2 * N;
   hipLaunchKernelGGL(kb_sum_split<T>, dim3(bnblk(len, 256)), dim3(256), 0, st, len, (const T *)yp,
@@ -1968,7 +2226,7 @@ void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row
 #define SPK_BATCH_INSTANTIATE(T)                                                                  \
   template void launch_batch_interleave<T>(int, int, const int *, const T *const *, T *, T *,     \
                                            hipStream_t);                                          \
-  template void launch_batch_agg<T>(int, int, int, int, const int *, const int *, const int *,     \
+  template void launch_batch_agg<T>(int, const PatLay &, int, int, const int *, const int *, const int *,     \
                                     const T *, const T *, const T *, T *, hipStream_t);            \
   template void launch_batch_ss<T>(int, int, int, const int *, const T *, const T *, T *,          \
                                    hipStream_t);                                                   \
@@ -1976,9 +2234,9 @@ void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row
                                     const T *, const T *, T *, hipStream_t);                       \
   template void launch_batch_rr<T>(int, int, int, const int *, const int *, const T *, const T *,  \
                                    T *, hipStream_t);                                              \
-  template void launch_batch_fold<T>(int, int, int, const T *, zd, zd, zd, zd, zd, zd, T *,        \
+  template void launch_batch_fold<T>(int, const PatLay &, int, const T *, zd, zd, zd, zd, zd, zd, T *,        \
                                      hipStream_t);                                                 \
-  template void launch_batch_disagg<T>(int, int, int, int, const int *, const int *, const int *,  \
+  template void launch_batch_disagg<T>(int, int, const PatLay &, int, const int *, const int *, const int *,  \
                                        const int *, const int *, const T *, const T *, zd, zd,     \
                                        T *, T *, int, const int *, const int *, hipStream_t);      \
   template void launch_batch_near<T>(int, int, int, const int *, const int *, const int *,         \

@@ -139,19 +139,52 @@ void launch_near_tri(const NearArgs &a, const TriForm &q, int N, int tiles, cons
 hipError_t exclusive_scan_int(const int *in, int *out, int64_t n, void **tmp, size_t *tmp_bytes,
                         hipStream_t st);
 
-// MLFMM (FP64)
-struct MlfmmArgs {
-  int N, S, nbl;
-  const int *perm;        // position -> edge
-  const int *box_first, *box_count;
+// Layout of the radiation patterns and of the folded leaf coefficients.
+//
+// In a medium of real wavenumber the pattern at -k is known from that at k:
+// e^{-ik(-k).r} is the conjugate, theta^ is the same at both and phi^ changes
+// sign (not at the poles, whose two unit vectors are fixed).  The sample grid
+// holds the antipode of every direction, so such a medium's rows keep half of
+// the samples: the first K^2 and the north pole, S/2 in all (padded to an
+// even length L with zeros).  With f = a + ib and sg = 1 for theta and the
+// poles, -1 for phi:
+//   up    sum conj(f) x at k = Sa - iSb, at -k = sg (Sa + iSb), Sa = sum a x, Sb = sum b x
+//   down  sum f W + sg conj(f) W' = sum a P + b M,  P = W + sg W', M = i(W - sg W')
+// which also halves the arithmetic.  A medium with losses keeps all S samples.
+//
+// patterns [position][medium][component][L], folded W [box][medium * 4 +
+// {1a, 1b, 2a, 2b}][SW]: P in [0, L) and M in [L, 2L) in a half medium, the S
+// values themselves in a full one.
+struct PatLay {
+  int S = 0, K = 0, SW = 0;
+  int L[2] = {0, 0};
+  bool half[2] = {false, false};
+  __host__ __device__ size_t stride() const { return 2 * (size_t)(L[0] + L[1]); }
+  __host__ __device__ size_t row(int k, int c) const {
+    return k ? 2 * (size_t)L[0] + (size_t)c * L[1] : (size_t)c * L[0];
+  }
+  // samples of half-row entry h, and how many there are
+  __host__ __device__ int count() const { return K * K + 1; }
+  __host__ __device__ int samp(int h) const { return h < K * K ? h : S - 2; }
+  __host__ __device__ int anti(int h) const {
+    if (h >= K * K) return S - 1;
+    const int j = h / (2 * K), c = h - j * 2 * K;
+    return (K - 1 - j) * 2 * K + (c < K ? c + K : c - K);
+  }
+  // the sign of the component's conjugate at the antipode
+  __host__ __device__ bool flips(int h, int comp) const { return comp == 1 && h < K * K; }
 };
-void launch_patterns(int N, int S, int ngp, const FnRec *fn, const int *perm, const int *leaf_box,
+// whether every k R of a surface of side D is below sincos_near's 1e5
+inline bool sincos_near_holds(double D, zd k1, zd k2) {
+  return 4.0 * D * (fabs(k1.x) > fabs(k2.x) ? fabs(k1.x) : fabs(k2.x)) < 1e5;
+}
+void launch_patterns(int N, const PatLay &lay, int ngp, double D, const FnRec *fn, const int *perm, const int *leaf_box,
                      const double *leaf_centre, const double *khat, const double *tth,
                      const double *tph, const double *qa, const double *qb, const double *qw,
                      zd k1, zd k2, zd *rt, hipStream_t st);
 // conj_rt = false: the transposed operator's aggregation (patterns not conjugated)
 template <class T>
-void launch_agg(int nbl, int S, int N, const int *box_first, const int *box_count,
+void launch_agg(int nbl, const PatLay &lay, int N, const int *box_first, const int *box_count,
                 const int *perm, const T *rt, const T *x, T *C, hipStream_t st,
                 bool conj_rt = true);
 template <class T>
@@ -172,12 +205,19 @@ void launch_m2l(int nb, int S, const int *i4_off, const int *i4_box, const int *
 template <class T>
 void launch_rr(int nb, int S, const int *parent, const int *octant, const T *Dp, const T *down,
                T *Dc, hipStream_t st);
+// folded coefficients of a level, all S samples of every item (stride S)
 template <class T>
 void launch_fold(int nbl, int S, const T *D, zd kd1, zd kd2, zd my1, zd my2, zd ep1, zd ep2,
                  T *W, hipStream_t st);
+// the leaf's folded coefficients as the disaggregation reads them (PatLay)
+template <class T>
+void launch_fold_leaf(int nbl, const PatLay &lay, const T *D, zd kd1, zd kd2, zd my1, zd my2,
+                      zd ep1, zd ep2, T *W, hipStream_t st);
+// the same from coefficients folded before (launch_fold's layout)
+void launch_half_w(int nbl, const PatLay &lay, const zd *Wf, zd *W, hipStream_t st);
 // conj_rt: the transposed operator's disaggregation (conjugated patterns)
 template <class T>
-void launch_disagg(int ntask, int N, int S, const int *task, const int *perm,
+void launch_disagg(int ntask, int N, const PatLay &lay, const int *task, const int *perm,
                    const int *leaf_box_of_pos, const T *rt, const T *W, zd sc1, zd sc2, T *y,
                    hipStream_t st, bool conj_rt = false);
 template <class T>
@@ -206,7 +246,7 @@ constexpr int kDisaggEdges = 4;
 // disaggregation tile
 constexpr int kBatchMax = 16;
 constexpr int kBatchTile = 64;
-// workgroups per disaggregation tile, each summing a share of the samples
+// workgroups per disaggregation tile: two shares of each medium's samples
 constexpr int kBatchSplit = 4;
 // arbitrary (m, n) pairs, one thread per pair (parity probe)
 void launch_near_pairs(const NearArgs &a, int npairs, const int *m, const int *n, zd *out,
@@ -317,9 +357,9 @@ template <class T>
 void launch_batch_interleave(int N, int R, const int *perm, const T *const *xs, T *XI, T *XP,
                              hipStream_t st);
 template <class T>
-void launch_batch_agg(int nbl, int S, int N, int R, const int *box_first, const int *box_count,
-                      const int *perm, const T *rt, const T *XI, const T *XP, T *C,
-                      hipStream_t st);
+void launch_batch_agg(int nbl, const PatLay &lay, int N, int R, const int *box_first,
+                      const int *box_count, const int *perm, const T *rt, const T *XI, const T *XP,
+                      T *C, hipStream_t st);
 template <class T>
 void launch_batch_ss(int nb, int S, int R, const int *child, const T *Cc, const T *up, T *P,
                      hipStream_t st);
@@ -330,13 +370,13 @@ template <class T>
 void launch_batch_rr(int nb, int S, int R, const int *parent, const int *octant, const T *Dp,
                      const T *down, T *Dc, hipStream_t st);
 template <class T>
-void launch_batch_fold(int nbl, int S, int R, const T *D, zd kd1, zd kd2, zd my1, zd my2, zd ep1,
+void launch_batch_fold(int nbl, const PatLay &lay, int R, const T *D, zd kd1, zd kd2, zd my1, zd my2, zd ep1,
                        zd ep2, T *W, hipStream_t st);
 // tiles of up to kBatchTile consecutive edges of one leaf box (mx tiles: up
 // to 128, for complex64 with 9..16 right-hand sides on the matrix cores)
 // yp: kBatchSplit partial slices of R x 2N, summed into yf
 template <class T>
-void launch_batch_disagg(int ntiles, int N, int S, int R, const int *tile_box, const int *tile_p0,
+void launch_batch_disagg(int ntiles, int N, const PatLay &lay, int R, const int *tile_box, const int *tile_p0,
                          const int *box_first, const int *box_count, const int *perm, const T *rt,
                          const T *W, zd sc1, zd sc2, T *yp, T *yf, int mx_tiles,
                          const int *mx_box, const int *mx_p0, hipStream_t st);

@@ -1182,56 +1182,90 @@ void launch_blu_scatter(int ngroups, int nmax, int N, const int *p0, const int *
 // ---------------------------------------------------------------------------
 // MLFMM kernels
 // ---------------------------------------------------------------------------
-// PreCalculate_RT / RT_function_SCSArr_New (src/lib_sie_tri_mlfmm.f90:503-583):
-// one thread per (position, sample).
-__global__ void k_patterns(int N, int S, int ngp, const FnRec *fn, const int *perm,
-                           const int *leaf_box, const double *leaf_centre, const double *khat,
-                           const double *tth, const double *tph, const double *qa,
-                           const double *qb, const double *qw, zd k1, zd k2, zd *rt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int p = blockIdx.y;
-  if (i >= S || p >= N) return;
-  const int m = perm[p];
-  const double *Rc = &leaf_centre[3 * leaf_box[m]];
-  const double kh[3] = {khat[3 * i], khat[3 * i + 1], khat[3 * i + 2]};
-  zd o[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-  for (int ll = 0; ll < 2; ++ll) {
-    const FnRec &f = fn[2 * m + ll];
-    const double dfm = f.sign * f.length;
-    zd sa[3] = {{0, 0}, {0, 0}, {0, 0}}, sb[3] = {{0, 0}, {0, 0}, {0, 0}};
-    for (int j = 0; j < ngp; ++j) {
-      double Ro[3], fm[3], Roc[3];
-      simplex(qa[j], qb[j], f.c, Ro);
-      for (int k = 0; k < 3; ++k) {
-        fm[k] = 0.5 * (Ro[k] - f.c[6 + k]) * dfm;
-        Roc[k] = Ro[k] - Rc[k];
-      }
-      const double tmp = dot3(kh, Roc);
-      const zd ff1 = expmikr(k1, tmp) * qw[j];
-      const zd ff2 = expmikr(k2, tmp) * qw[j];
-      for (int k = 0; k < 3; ++k) {
-        sa[k] = sa[k] + fm[k] * ff1;
-        sb[k] = sb[k] + fm[k] * ff2;
-      }
-    }
-    const double tt3[3] = {tth[3 * i], tth[3 * i + 1], tth[3 * i + 2]};
-    const double tp3[3] = {tph[3 * i], tph[3 * i + 1], tph[3 * i + 2]};
-    o[0] = o[0] + dot_rc(tt3, sa);
-    o[1] = o[1] + dot_rc(tp3, sa);
-    o[2] = o[2] + dot_rc(tt3, sb);
-    o[3] = o[3] + dot_rc(tp3, sb);
+// PreCalculate_RT / RT_function_SCSArr_New (src/lib_sie_tri_mlfmm.f90:503-583).
+// One workgroup per position: the quadrature points of the edge's two
+// triangles (offset from the leaf centre, weighted function value) go to LDS
+// once, then each thread takes every 128th sample: where both media keep half
+// of the samples (PatLay) those, else all S.  NEAR: sincos_near (arguments
+// below 1e5).  Bound by the FP64 ALU (12 exponentials a sample): 0.28 ms at
+// 29,800 edges and 362 samples; with a thread per sample that repeated the
+// geometry and the library's sincos 0.90 ms.
+template <bool NEAR>
+__device__ inline zd exp_mikr(zd k, double R) {
+  if constexpr (!NEAR) {
+    return expmikr(k, R);
+  } else {
+    double s, c;
+    sincos_near(k.x * R, &s, &c);
+    const double e = k.y != 0.0 ? exp(k.y * R) : 1.0;
+    return zd{e * c, -e * s};
   }
-  zd *out = rt + (size_t)p * 4 * S;
-  for (int q = 0; q < 4; ++q) out[(size_t)q * S + i] = o[q];
+}
+constexpr int kPatT = 128;
+template <bool NEAR>
+__global__ void __launch_bounds__(kPatT) k_patterns(PatLay lay, int n, int ngp, const FnRec *fn,
+                                                    const int *perm, const int *leaf_box,
+                                                    const double *leaf_centre, const double *khat,
+                                                    const double *tth, const double *tph,
+                                                    const double *qa, const double *qb,
+                                                    const double *qw, zd k1, zd k2, zd *rt) {
+  __shared__ double pt[40 * 6];  // 2 x 20 points at most
+  const int p = blockIdx.x;
+  const bool both = lay.half[0] && lay.half[1];
+  zd *out = rt + (size_t)p * lay.stride();
+  const int H = lay.count(), m = perm[p];
+  if (threadIdx.x < 2 * ngp) {
+    const FnRec &f = fn[2 * m + (int)threadIdx.x / ngp];
+    const int j = threadIdx.x % ngp;
+    const double *Rc = &leaf_centre[3 * leaf_box[m]];
+    double Ro[3];
+    simplex(qa[j], qb[j], f.c, Ro);
+    for (int k = 0; k < 3; ++k) {
+      pt[6 * threadIdx.x + k] = Ro[k] - Rc[k];
+      pt[6 * threadIdx.x + 3 + k] = 0.5 * (Ro[k] - f.c[6 + k]) * (f.sign * f.length) * qw[j];
+    }
+  }
+  if (threadIdx.x < 4 && lay.half[threadIdx.x >> 1]) {
+    const int k = threadIdx.x >> 1;
+    for (int h = H; h < lay.L[k]; ++h) out[lay.row(k, threadIdx.x & 1) + h] = zd{0, 0};
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += kPatT) {
+    // the sample, and its entry in a half row (-1: the antipode's)
+    const int s = both ? lay.samp(i) : i;
+    const int h = both ? i : s < H - 1 ? s : s == lay.S - 2 ? H - 1 : -1;
+    double kh[3], th[3], ph[3];
+    for (int k = 0; k < 3; ++k) {
+      kh[k] = khat[3 * s + k];
+      th[k] = tth[3 * s + k];
+      ph[k] = tph[3 * s + k];
+    }
+    zd o[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    for (int j = 0; j < 2 * ngp; ++j) {
+      const double *q = pt + 6 * j;
+      const double x = dot3(kh, q), ft = dot3(th, q + 3), fp = dot3(ph, q + 3);
+      const zd e1 = exp_mikr<NEAR>(k1, x), e2 = exp_mikr<NEAR>(k2, x);
+      o[0] = o[0] + e1 * ft;
+      o[1] = o[1] + e1 * fp;
+      o[2] = o[2] + e2 * ft;
+      o[3] = o[3] + e2 * fp;
+    }
+    for (int q = 0; q < 4; ++q) {
+      const int e = lay.half[q >> 1] ? h : s;
+      if (e >= 0) out[lay.row(q >> 1, q & 1) + e] = o[q];
+    }
+  }
 }
 
-void launch_patterns(int N, int S, int ngp, const FnRec *fn, const int *perm, const int *leaf_box,
-                     const double *leaf_centre, const double *khat, const double *tth,
-                     const double *tph, const double *qa, const double *qb, const double *qw,
-                     zd k1, zd k2, zd *rt, hipStream_t st) {
+void launch_patterns(int N, const PatLay &lay, int ngp, double D, const FnRec *fn, const int *perm,
+                     const int *leaf_box, const double *leaf_centre, const double *khat,
+                     const double *tth, const double *tph, const double *qa, const double *qb,
+                     const double *qw, zd k1, zd k2, zd *rt, hipStream_t st) {
   if (N <= 0) return;
-  hipLaunchKernelGGL(k_patterns, dim3(nblk(S, 256), N), dim3(256), 0, st, N, S, ngp, fn, perm,
-                     leaf_box, leaf_centre, khat, tth, tph, qa, qb, qw, k1, k2, rt);
+  const int n = lay.half[0] && lay.half[1] ? lay.count() : lay.S;
+  hipLaunchKernelGGL(sincos_near_holds(D, k1, k2) ? k_patterns<true> : k_patterns<false>, dim3(N),
+                     dim3(kPatT), 0, st, lay, n, ngp, fn, perm, leaf_box, leaf_centre, khat, tth,
+                     tph, qa, qb, qw, k1, k2, rt);
 }
 
 // The matvec kernels below are templates on the complex type T: zd
@@ -1251,48 +1285,180 @@ __device__ inline zf2 ld2(const zf *p) {
   return zf2{zf{v.x, v.y}, zf{v.z, v.w}};
 }
 
-// CONJ = false: the patterns themselves (the transposed operator's
-// disaggregation, aggregated)
-template <class T, bool CONJ>
-__global__ void k_agg(int S, int N, const int *box_first, const int *box_count, const int *perm,
-                      const T *rt, const T *x, T *C) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  const int b = blockIdx.y, q = blockIdx.z;  // q = k*2 + comp
-  if (s >= S) return;
-  const int k = q >> 1, comp = q & 1;
-  T ae = {0, 0}, ah = {0, 0};
+// Workgroup = EW waves, (64 16-byte pattern words, leaf box, medium k): the
+// waves share the box's edges, each with both components' rows; the box's x
+// goes to LDS once and the waves' sums are added in order.  HALF: the medium
+// keeps half of the samples (PatLay) and an entry gives the coefficients of
+// its sample and of the antipode.  CONJ = false: the patterns themselves (the
+// transposed operator's disaggregation, aggregated).
+//
+// Bound by HBM: 0.69 GB at 29,800 edges, 145 us in FP64 and 77 us in complex64,
+// where rows of all S samples took 270 and 139 us.
+constexpr int kAggXE = 128;  // edges staged at a time
+template <class T, bool HALF, bool CONJ, int EW>
+__device__ __forceinline__ void agg_part(const PatLay &lay, int N, const int *box_first,
+                                         const int *box_count, const int *perm, const T *rt,
+                                         const T *x, T *C, T *xl, T *red) {
+  constexpr int PK = kPack<T>;         // entries per lane
+  constexpr int V = HALF ? 4 : 2;      // sums per entry and component
+  constexpr int NV = 2 * PK * V;
+  constexpr int XE = kAggXE;
+  constexpr int UE = 4;
+  constexpr bool BLK = kSumBlock<T> < XE;
+  using Word = float4;
+  const int lane = threadIdx.x & 63;
+  const int wv = EW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int b = blockIdx.y, k = blockIdx.z;
+  const int L = lay.L[k];
+  if ((int)blockIdx.x * 64 * PK >= L) return;
+  const int i = (blockIdx.x * 64 + lane) * PK;
   const int p0 = box_first[b], cnt = box_count[b];
-  for (int e0 = 0; e0 < cnt; e0 += kSumBlock<T>) {
-    T ge = {0, 0}, gh = {0, 0};
-    const int e1 = min(cnt, e0 + kSumBlock<T>);
-#pragma unroll 4
-    for (int e = e0; e < e1; ++e) {
-      const int p = p0 + e;
-      const int m = perm[p];
-      const T r = rt[((size_t)p * 4 + q) * S + s];
-      const T f = CONJ ? conj(r) : r;
-      const T xe = x[m], xh = x[m + N];
-      ge = ge + f * xe;
-      gh = gh + f * xh;
+  const size_t ps = lay.stride();
+  const T *F = rt + (size_t)p0 * ps + lay.row(k, 0) + min(i, L - PK);
+  T v[NV];
+#pragma unroll
+  for (int u = 0; u < NV; ++u) v[u] = T{0, 0};
+  auto term = [&](T *g, T f, T xe, T xh) {
+    if constexpr (HALF) {
+      g[0] = g[0] + xe * f.x;
+      g[1] = g[1] + xh * f.x;
+      g[2] = g[2] + xe * f.y;
+      g[3] = g[3] + xh * f.y;
+    } else {
+      const T c = CONJ ? conj(f) : f;
+      g[0] = g[0] + c * xe;
+      g[1] = g[1] + c * xh;
     }
-    ae = ae + ge;
-    ah = ah + gh;
+  };
+  for (int e0 = 0; e0 < cnt; e0 += XE) {
+    const int ne = min(XE, cnt - e0);
+    __syncthreads();
+    for (int t = threadIdx.x; t < 2 * ne; t += 64 * EW)
+      xl[t] = x[perm[p0 + e0 + (t >> 1)] + (int64_t)(t & 1) * N];
+    __syncthreads();
+    // four edges' words are in flight while the four before are summed; an
+    // edge past the end is clamped on load and gets x = 0
+    const int ea = ne * wv / EW, eb = ne * (wv + 1) / EW;
+    if (ea >= eb) continue;
+    Word cur[UE][2], nxt[UE][2];
+    auto load = [&](int e, Word (*w)[2]) {
+#pragma unroll
+      for (int u = 0; u < UE; ++u) {
+        const T *f = F + (size_t)(e0 + min(e + u, eb - 1)) * ps;
+        w[u][0] = *reinterpret_cast<const Word *>(f);
+        w[u][1] = *reinterpret_cast<const Word *>(f + L);
+      }
+    };
+    load(ea, cur);
+    for (int g0 = ea; g0 < eb; g0 += kSumBlock<T>) {
+      T g[NV];
+      T *acc = BLK ? g : v;
+#pragma unroll
+      for (int u = 0; u < NV; ++u) g[u] = T{0, 0};
+      const int g1 = min(eb, g0 + kSumBlock<T>);
+      for (int e = g0; e < g1; e += UE) {
+        load(e + UE, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UE; ++u) {
+          const bool in = e + u < g1;
+          const int eu = in ? e + u : e;
+          const T xe = in ? xl[2 * eu] : T{0, 0}, xh = in ? xl[2 * eu + 1] : T{0, 0};
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const T *f = reinterpret_cast<const T *>(&cur[u][c]);
+#pragma unroll
+            for (int d = 0; d < PK; ++d) term(acc + (c * PK + d) * V, f[d], xe, xh);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UE; ++u) {
+          cur[u][0] = nxt[u][0];
+          cur[u][1] = nxt[u][1];
+        }
+      }
+      if constexpr (BLK) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) v[u] = v[u] + g[u];
+      }
+    }
   }
-  T *Cb = C + (size_t)b * 8 * S;
-  Cb[(size_t)(comp * 4 + 0 * 2 + k) * S + s] = ae;
-  Cb[(size_t)(comp * 4 + 1 * 2 + k) * S + s] = ah;
+  if constexpr (EW > 1) {
+    if (wv > 0)
+#pragma unroll
+      for (int u = 0; u < NV; ++u) red[((wv - 1) * NV + u) * 64 + lane] = v[u];
+    __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int w = 0; w < EW - 1; ++w)
+#pragma unroll
+      for (int u = 0; u < NV; ++u) v[u] = v[u] + red[(w * NV + u) * 64 + lane];
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int d = 0; d < PK; ++d) {
+      const int e = i + d;
+      if (e >= (HALF ? lay.count() : lay.S)) continue;
+      const T *g = v + (c * PK + d) * V;
+      T *Ce = C + ((size_t)b * 8 + c * 4 + k) * lay.S, *Ch = Ce + 2 * (size_t)lay.S;
+      if constexpr (HALF) {
+        // Sa -+ i Sb (conjugated patterns: - at the sample, + at the antipode)
+        const int s = lay.samp(e), t = lay.anti(e);
+        const bool neg = lay.flips(e, c);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const T ib = {-g[2 + u].y, g[2 + u].x};
+          const T lo = CONJ ? g[u] - ib : g[u] + ib, hi = CONJ ? g[u] + ib : g[u] - ib;
+          T *o = u ? Ch : Ce;
+          o[s] = lo;
+          o[t] = neg ? -hi : hi;
+        }
+      } else {
+        Ce[e] = g[0];
+        Ch[e] = g[1];
+      }
+    }
 }
 
+// MODE: 1 both media keep half of the samples, 0 neither does, 2 one of them does
+template <class T, int MODE, bool CONJ, int EW>
+__global__ void __launch_bounds__(64 * EW) k_agg(PatLay lay, int N, const int *box_first,
+                                                 const int *box_count, const int *perm,
+                                                 const T *rt, const T *x, T *C) {
+  __shared__ T xl[kAggXE * 2];
+  __shared__ T red[EW > 1 ? (EW - 1) * 2 * kPack<T> * (MODE ? 4 : 2) * 64 : 1];
+  if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.z]))
+    agg_part<T, true, CONJ, EW>(lay, N, box_first, box_count, perm, rt, x, C, xl, red);
+  else if (MODE != 1)
+    agg_part<T, false, CONJ, EW>(lay, N, box_first, box_count, perm, rt, x, C, xl, red);
+}
+
+template <class T, int EW>
+static void agg_waves(int nbl, const PatLay &lay, int N, const int *box_first,
+                      const int *box_count, const int *perm, const T *rt, const T *x, T *C,
+                      hipStream_t st, bool conj_rt) {
+  const int L = lay.L[0] > lay.L[1] ? lay.L[0] : lay.L[1];
+  auto *f = lay.half[0] && lay.half[1]
+                ? (conj_rt ? k_agg<T, 1, true, EW> : k_agg<T, 1, false, EW>)
+            : lay.half[0] || lay.half[1]
+                ? (conj_rt ? k_agg<T, 2, true, EW> : k_agg<T, 2, false, EW>)
+                : (conj_rt ? k_agg<T, 0, true, EW> : k_agg<T, 0, false, EW>);
+  hipLaunchKernelGGL(f, dim3(nblk(L, 64 * kPack<T>), nbl, 2), dim3(64 * EW), 0, st, lay, N,
+                     box_first, box_count, perm, rt, x, C);
+}
 template <class T>
-void launch_agg(int nbl, int S, int N, const int *box_first, const int *box_count,
+void launch_agg(int nbl, const PatLay &lay, int N, const int *box_first, const int *box_count,
                 const int *perm, const T *rt, const T *x, T *C, hipStream_t st, bool conj_rt) {
   if (nbl <= 0) return;
-  if (conj_rt)
-    hipLaunchKernelGGL((k_agg<T, true>), dim3(nblk(S, 256), nbl, 4), dim3(256), 0, st, S, N,
-                       box_first, box_count, perm, rt, x, C);
-  else
-    hipLaunchKernelGGL((k_agg<T, false>), dim3(nblk(S, 256), nbl, 4), dim3(256), 0, st, S, N,
-                       box_first, box_count, perm, rt, x, C);
+  // one wave a workgroup where those fill the chip (768 tiles: three a CU),
+  // else the box's edges are shared by more: 64 boxes of 167 edges in
+  // complex64, 384 tiles, 50 us by one wave and 33 by four; 4 boxes of 184
+  // edges in FP64, 48 tiles, 30 us by one wave, 23 by four, 14 by eight
+  const int tiles = (nblk(lay.L[0], 64 * kPack<T>) + nblk(lay.L[1], 64 * kPack<T>)) * nbl;
+  auto *f = tiles >= 768 ? agg_waves<T, 1> : tiles >= 192 ? agg_waves<T, 4> : agg_waves<T, 8>;
+  f(nbl, lay, N, box_first, box_count, perm, rt, x, C, st, conj_rt);
 }
 
 // translation_SS (:466-528): P[it][s] = sum_o C_child[it][s] * up[o][k][s]
@@ -1412,6 +1578,78 @@ void launch_fold(int nbl, int S, const T *D, zd kd1, zd kd2, zd my1, zd my2, zd 
                      cvt<T>(kd2), cvt<T>(my1), cvt<T>(my2), cvt<T>(ep1), cvt<T>(ep2), W);
 }
 
+// four folded values of a medium at one sample
+template <class T>
+__device__ inline void fold4(const T *Db, int S, int k, int s, T kd, T my, T ep, T *w) {
+  const T Dae = Db[(size_t)(0 + k) * S + s], Dah = Db[(size_t)(2 + k) * S + s];
+  const T Dbe = Db[(size_t)(4 + k) * S + s], Dbh = Db[(size_t)(6 + k) * S + s];
+  w[0] = Dbh * kd + Dae * my;
+  w[1] = -(Dah * kd) + Dbe * my;
+  w[2] = -(Dbe * kd) + Dah * ep;
+  w[3] = Dae * kd + Dbh * ep;
+}
+// one medium's part of entry i of the leaf's W from the values w at a sample
+// and wa at its antipode
+template <class T>
+__device__ inline void put_half(const PatLay &lay, int k, int h, const T *w, const T *wa, T *Wb) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const T o = lay.flips(h, j & 1) ? -wa[j] : wa[j];
+    const T P = w[j] + o, d = w[j] - o;
+    T *W = Wb + (size_t)(k * 4 + j) * lay.SW;
+    W[h] = P;
+    W[lay.L[k] + h] = T{-d.y, d.x};
+  }
+}
+// FOLDED: D holds folded values already ([medium * 4 + j][S])
+template <class T, bool FOLDED>
+__global__ void k_fold_leaf(PatLay lay, const T *D, T kd1, T kd2, T my1, T my2, T ep1, T ep2,
+                            T *W) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int b = blockIdx.y, k = blockIdx.z, S = lay.S;
+  const T *Db = D + (size_t)b * 8 * S;
+  T *Wb = W + (size_t)b * 8 * lay.SW;
+  const T kd = k ? kd2 : kd1, my = k ? my2 : my1, ep = k ? ep2 : ep1;
+  auto at = [&](int s, T *w) {
+    if constexpr (FOLDED) {
+      for (int j = 0; j < 4; ++j) w[j] = Db[(size_t)(k * 4 + j) * S + s];
+    } else {
+      fold4(Db, S, k, s, kd, my, ep, w);
+    }
+  };
+  T w[4], wa[4];
+  if (lay.half[k]) {
+    if (i >= lay.L[k]) return;
+    if (i < lay.count()) {
+      at(lay.samp(i), w);
+      at(lay.anti(i), wa);
+    } else {
+      for (int j = 0; j < 4; ++j) w[j] = wa[j] = T{0, 0};
+    }
+    put_half(lay, k, i, w, wa, Wb);
+  } else {
+    if (i >= S) return;
+    at(i, w);
+    for (int j = 0; j < 4; ++j) Wb[(size_t)(k * 4 + j) * lay.SW + i] = w[j];
+  }
+}
+template <class T>
+void launch_fold_leaf(int nbl, const PatLay &lay, const T *D, zd kd1, zd kd2, zd my1, zd my2,
+                      zd ep1, zd ep2, T *W, hipStream_t st) {
+  if (nbl <= 0) return;
+  const int n = lay.L[0] > lay.L[1] ? lay.L[0] : lay.L[1];
+  hipLaunchKernelGGL((k_fold_leaf<T, false>), dim3(nblk(n, 128), nbl, 2), dim3(128), 0, st, lay, D,
+                     cvt<T>(kd1), cvt<T>(kd2), cvt<T>(my1), cvt<T>(my2), cvt<T>(ep1), cvt<T>(ep2),
+                     W);
+}
+void launch_half_w(int nbl, const PatLay &lay, const zd *Wf, zd *W, hipStream_t st) {
+  if (nbl <= 0) return;
+  const int n = lay.L[0] > lay.L[1] ? lay.L[0] : lay.L[1];
+  const zd z = {0, 0};
+  hipLaunchKernelGGL((k_fold_leaf<zd, true>), dim3(nblk(n, 128), nbl, 2), dim3(128), 0, st, lay, Wf,
+                     z, z, z, z, z, z, W);
+}
+
 // The transpose of k_fold per box and sample: from the aggregated adjoint
 // sums C (layout [comp*4 + cur*2 + k], comp = theta/phi, cur = e/h) to the
 // adjoint of D (the same layout):
@@ -1520,96 +1758,171 @@ __device__ inline zf wave_sum(zf v) {
   return v;
 }
 
-// one wavefront per position: y[m] = sc1*y_e, y[m+N] = sc2*y_h (far part)
-// One wavefront per task of up to kDisaggEdges consecutive edges of one leaf
-// box: each W sample is loaded once for the group (W is the box's folded
-// coefficient array), the patterns of the group's edges stream from HBM.
-// task[t] = p0 * 8 + count.  Per edge the sums run in the same order as one
-// wavefront per edge would (media, then lane-strided samples).
+// y[m] = sc1*y_e, y[m+N] = sc2*y_h (far part).  A task is up to kDisaggEdges
+// consecutive edges of one leaf box, task[t] = p0 * 8 + count: each W entry (W
+// is the box's folded coefficient array) is loaded once for the group, the
+// patterns of the group's edges stream from HBM.  In FP64 a wave takes one
+// medium of a task and the two sums are added (workgroup: two tasks), in
+// complex64, whose rows are half as long, a wave takes both (four tasks).
 // CONJ: the conjugated patterns (the transposed operator's aggregation,
-// disaggregated)
+// disaggregated).
+//
+// Bound by HBM and the L2 reads of W: at 29,800 edges 154 us in FP64 (273 us
+// on rows of all S samples; 158 us with both media in a wave) and 77 us in
+// complex64 (139 us; 89 us with a wave per medium).
+template <class T>
+constexpr int kDisaggKW = sizeof(T) == 16 ? 2 : 1;
 template <class T, bool CONJ>
-__global__ void __launch_bounds__(256) k_disagg(int ntask, int N, int S, const int *task,
+__global__ void __launch_bounds__(256) k_disagg(int ntask, int N, PatLay lay, const int *task,
                                                 const int *perm, const int *leaf_box_of_pos,
                                                 const T *rt, const T *W, T sc1, T sc2, T *y) {
   constexpr int E = kDisaggEdges;
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= ntask) return;
+  constexpr int KW = kDisaggKW<T>, TW = 4 / KW;  // waves a task, tasks a workgroup
+  __shared__ T part[TW][2 * E];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tw = wv % TW;
+  const int t = min((int)blockIdx.x * TW + tw, ntask - 1);
   const int code = task[t], p0 = code >> 3, cnt = code & 7;
   const int b = leaf_box_of_pos[p0];
-  const T *Wb = W + (size_t)b * 8 * S;
+  const T *Wb = W + (size_t)b * 8 * lay.SW;
   T s1[E], s2[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) s1[e] = s2[e] = T{0, 0};
-  for (int k = 0; k < 2; ++k) {
-    const T *w1a = Wb + (size_t)(k * 4 + 0) * S, *w1b = Wb + (size_t)(k * 4 + 1) * S;
-    const T *w2a = Wb + (size_t)(k * 4 + 2) * S, *w2b = Wb + (size_t)(k * 4 + 3) * S;
+  auto medium = [&](int k) {
+    const int L = lay.L[k];
+    const T *w = Wb + (size_t)(k * 4) * lay.SW;
+    const size_t ws = lay.SW;
     // the group's pattern rows (a short group repeats its last edge, whose
     // products are then dropped), so that all loads of a step issue together
     const T *f[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) f[e] = rt + ((size_t)(p0 + min(e, cnt - 1)) * 4 + k * 2) * S;
-    if constexpr (kPack<T> == 2) {
+    for (int e = 0; e < E; ++e)
+      f[e] = rt + (size_t)(p0 + min(e, cnt - 1)) * lay.stride() + lay.row(k, 0);
+    if (lay.half[k]) {
+      // a P + b M (conjugated patterns: a P - b M) of four items
+      auto step = [&](const T *fa, const T *fb, const T *P, const T *M) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const auto ay = CONJ ? -fa[e].y : fa[e].y, by = CONJ ? -fb[e].y : fb[e].y;
+          s1[e] = s1[e] + (P[0] * fa[e].x + M[0] * ay + P[1] * fb[e].x + M[1] * by);
+          s2[e] = s2[e] + (P[2] * fa[e].x + M[2] * ay + P[3] * fb[e].x + M[3] * by);
+        }
+      };
+      if constexpr (kPack<T> == 2) {
+        // complex64: two consecutive entries per 16-byte load (L is even)
+        for (int h = 2 * lane; h < L; h += 128) {
+          T P[2][4], M[2][4], fa[2][E], fb[2][E];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const zf2 a = ld2(w + j * ws + h), c = ld2(w + j * ws + L + h);
+            P[0][j] = a.a;
+            P[1][j] = a.b;
+            M[0][j] = c.a;
+            M[1][j] = c.b;
+          }
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const zf2 a = ld2(f[e] + h), c = ld2(f[e] + L + h);
+            fa[0][e] = a.a;
+            fa[1][e] = a.b;
+            fb[0][e] = c.a;
+            fb[1][e] = c.b;
+          }
+          step(fa[0], fb[0], P[0], M[0]);
+          step(fa[1], fb[1], P[1], M[1]);
+        }
+      } else {
+        for (int h = lane; h < L; h += 64) {
+          T P[4], M[4], fa[E], fb[E];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            P[j] = w[j * ws + h];
+            M[j] = w[j * ws + L + h];
+          }
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            fa[e] = f[e][h];
+            fb[e] = f[e][L + h];
+          }
+          step(fa, fb, P, M);
+        }
+      }
+    } else if constexpr (kPack<T> == 2) {
       // complex64: each lane takes two consecutive samples per 16-byte load
-      for (int s = 2 * lane; s < S; s += 128) {
-        const zf2 wa = ld2(w1a + s), wb = ld2(w1b + s), wc = ld2(w2a + s), wd = ld2(w2b + s);
+      for (int s = 2 * lane; s < L; s += 128) {
+        const zf2 wa = ld2(w + s), wb = ld2(w + ws + s), wc = ld2(w + 2 * ws + s),
+                  wd = ld2(w + 3 * ws + s);
         zf2 a[E], bb[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
           a[e] = ld2(f[e] + s);
-          bb[e] = ld2(f[e] + S + s);
+          bb[e] = ld2(f[e] + L + s);
           if (CONJ) {
             a[e] = zf2{conj(a[e].a), conj(a[e].b)};
             bb[e] = zf2{conj(bb[e].a), conj(bb[e].b)};
           }
         }
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-          if (e < cnt) {
-            s1[e] = s1[e] + a[e].a * wa.a + bb[e].a * wb.a + a[e].b * wa.b + bb[e].b * wb.b;
-            s2[e] = s2[e] + a[e].a * wc.a + bb[e].a * wd.a + a[e].b * wc.b + bb[e].b * wd.b;
-          }
+        for (int e = 0; e < E; ++e) {
+          s1[e] = s1[e] + a[e].a * wa.a + bb[e].a * wb.a + a[e].b * wa.b + bb[e].b * wb.b;
+          s2[e] = s2[e] + a[e].a * wc.a + bb[e].a * wd.a + a[e].b * wc.b + bb[e].b * wd.b;
+        }
       }
     } else {
-      for (int s = lane; s < S; s += 64) {
-        const T wa = w1a[s], wb = w1b[s], wc = w2a[s], wd = w2b[s];
+      for (int s = lane; s < L; s += 64) {
+        const T wa = w[s], wb = w[ws + s], wc = w[2 * ws + s], wd = w[3 * ws + s];
         T a[E], bb[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
           a[e] = CONJ ? conj(f[e][s]) : f[e][s];
-          bb[e] = CONJ ? conj(f[e][S + s]) : f[e][S + s];
+          bb[e] = CONJ ? conj(f[e][L + s]) : f[e][L + s];
         }
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-          if (e < cnt) {
-            s1[e] = s1[e] + a[e] * wa + bb[e] * wb;
-            s2[e] = s2[e] + a[e] * wc + bb[e] * wd;
-          }
+        for (int e = 0; e < E; ++e) {
+          s1[e] = s1[e] + a[e] * wa + bb[e] * wb;
+          s2[e] = s2[e] + a[e] * wc + bb[e] * wd;
+        }
       }
     }
+  };
+  if constexpr (KW == 2) {
+    medium(wv / TW);
+  } else {
+    medium(0);
+    medium(1);
   }
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const T r1 = wave_sum(s1[e]), r2 = wave_sum(s2[e]);
-    if (lane == 0 && e < cnt) {
+    s1[e] = wave_sum(s1[e]);
+    s2[e] = wave_sum(s2[e]);
+    if (KW == 2 && lane == 0 && wv >= TW) {
+      part[tw][2 * e] = s1[e];
+      part[tw][2 * e + 1] = s2[e];
+    }
+  }
+  if constexpr (KW == 2) __syncthreads();
+  if (lane > 0 || wv >= TW || (int)blockIdx.x * TW + tw >= ntask) return;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (e < cnt) {
       const int m = perm[p0 + e];
+      const T r1 = KW == 2 ? s1[e] + part[tw][2 * e] : s1[e];
+      const T r2 = KW == 2 ? s2[e] + part[tw][2 * e + 1] : s2[e];
       y[m] = r1 * sc1;
       y[m + N] = r2 * sc2;
     }
-  }
 }
 
 template <class T>
-void launch_disagg(int ntask, int N, int S, const int *task, const int *perm,
+void launch_disagg(int ntask, int N, const PatLay &lay, const int *task, const int *perm,
                    const int *leaf_box_of_pos, const T *rt, const T *W, zd sc1, zd sc2, T *y,
                    hipStream_t st, bool conj_rt) {
   if (ntask <= 0) return;
   if (conj_rt)
-    hipLaunchKernelGGL((k_disagg<T, true>), dim3(nblk(ntask, 4)), dim3(256), 0, st, ntask, N, S,
+    hipLaunchKernelGGL((k_disagg<T, true>), dim3(nblk(ntask, 4 / kDisaggKW<T>)), dim3(256), 0, st, ntask, N, lay,
                        task, perm, leaf_box_of_pos, rt, W, cvt<T>(sc1), cvt<T>(sc2), y);
   else
-    hipLaunchKernelGGL((k_disagg<T, false>), dim3(nblk(ntask, 4)), dim3(256), 0, st, ntask, N, S,
+    hipLaunchKernelGGL((k_disagg<T, false>), dim3(nblk(ntask, 4 / kDisaggKW<T>)), dim3(256), 0, st, ntask, N, lay,
                        task, perm, leaf_box_of_pos, rt, W, cvt<T>(sc1), cvt<T>(sc2), y);
 }
 
@@ -1771,7 +2084,7 @@ void launch_rr_folded(int nb, int S, const int *parent, const int *octant, const
 }
 
 #define SPK_MATVEC_INSTANTIATE(T)                                                               \
-  template void launch_agg<T>(int, int, int, const int *, const int *, const int *, const T *,   \
+  template void launch_agg<T>(int, const PatLay &, int, const int *, const int *, const int *, const T *,   \
                               const T *, T *, hipStream_t, bool);                                \
   template void launch_fold_t<T>(int, int, const T *, zd, zd, zd, zd, zd, zd, T *, hipStream_t); \
   template void launch_scale_halves<T>(int, zd, zd, const T *, T *, hipStream_t);                \
@@ -1784,7 +2097,8 @@ void launch_rr_folded(int nb, int S, const int *parent, const int *octant, const
   template void launch_rr<T>(int, int, const int *, const int *, const T *, const T *, T *,      \
                              hipStream_t);                                                       \
   template void launch_fold<T>(int, int, const T *, zd, zd, zd, zd, zd, zd, T *, hipStream_t);   \
-  template void launch_disagg<T>(int, int, int, const int *, const int *, const int *, const T *, \
+  template void launch_fold_leaf<T>(int, const PatLay &, const T *, zd, zd, zd, zd, zd, zd, T *, hipStream_t);   \
+  template void launch_disagg<T>(int, int, const PatLay &, const int *, const int *, const int *, const T *, \
                                  const T *, zd, zd, T *, hipStream_t, bool);                     \
   template void launch_near_spmv_rows<T>(int, int, const int *, const int *, const int *,        \
                                          const int *, const int *, const int *, const int64_t *, \

@@ -1,0 +1,57 @@
+"""Pattern rows that keep half of the sample directions (media of real
+wavenumber) and whole rows (media with losses), in every kernel that reads
+them: patterns, products of one and several vectors in both precisions and the
+transposed product, for odd and even truncation numbers (an even K leaves an
+odd half, padded), against the oracle's operator on all samples.
+
+Tolerances: the products are held to 1e-9, the bound of the translation sums'
+cancellation on these leaf boxes (0.58 wavelengths, K <= 19: 4e-11 measured);
+complex64 has 2^29 times FP64's rounding, held to 1e-2.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from specklesim_amd import SieTriMlfmm, meshes
+
+pytestmark = pytest.mark.gpu
+LAM = 633e-9
+
+
+@pytest.fixture(scope="module")
+def mesh():
+    return meshes.rough_surface(24, 24, 2.4, 2.4, 0.1, 0.5, 9, LAM)
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("K,eps1,eps2", [
+    (19, 1.0, 2.25), (12, 1.0, 2.25), (13, 1.0, 2.25 - 0.2j), (12, 1.2 - 0.1j, 2.25),
+    (8, 1.2 - 0.1j, 2.25 - 0.2j), (3, 1.0, 2.25),
+])
+def test_products_on_half_and_whole_rows(mesh, K, eps1, eps2):
+    pp, tt = mesh
+    kw = dict(eps_r1=eps1, formulation="ICTF", normal_convention=2)
+    o = O.Oracle(pp, tt, LAM, eps2, K=K, **kw)
+    o.tree()
+    o.near_csr(fill=True)
+    o.mlfmm_setup()
+    g = SieTriMlfmm(LAM, eps2, truncation_number=K, precision="mixed", **kw).precalculation_tri(pp, tt)
+    pat = g.patterns(0, 40)
+    for m in (0, 7, 39):
+        ref = o.pattern(m)
+        assert np.abs(pat[m] - ref).max() < 1e-12 * np.abs(ref).max()
+    rng = np.random.default_rng(3)
+    X = rng.standard_normal((16, 2 * g.N)) + 1j * rng.standard_normal((16, 2 * g.N))
+    Y = np.stack([o.matvec(x) for x in X])
+    assert _rel(g.calculate_vector_b_tri(X[0]), Y[0]) < 1e-9
+    assert _rel(g.calculate_vector_b_tri_c64(X[0]), Y[0]) < 1e-2
+    for R in (1, 2, 3, 7, 9, 16):
+        assert _rel(g.calculate_vector_b_tri_batch(X[:R]), Y[:R]) < 1e-9, R
+        assert _rel(g.calculate_vector_b_tri_batch(X[:R], c64=True), Y[:R]) < 1e-2, R
+    # u.(Z^T v) = v.(Z u)
+    g.set_transposed(True)
+    t = X[1] @ g.calculate_vector_b_tri(X[2])
+    assert abs(t - X[2] @ Y[1]) < 1e-9 * np.linalg.norm(X[2]) * np.linalg.norm(Y[1])
