@@ -176,6 +176,7 @@ struct spk_handle {
   DBuf<double> d_khat, d_tth, d_tph, d_q, d_leaf_centre, d_trf;
   std::vector<LevelDev> lev;
   DBuf<zd> d_x, d_y, d_yfar, d_tmp;
+  DBuf<zd> d_scpart;  // the scattered field's partial sums (allocated by the setup)
   // the transposed operator (spk_set_transposed): flag, edge -> position map,
   // scaled input of the transposed far field
   bool transposed = false;
@@ -1375,6 +1376,7 @@ int spk_setup_tri(spk_handle *h, int np, const double *pp, int nt, const int *tt
   HIPCHK(h->d_er.upload(h->er));
   HIPCHK(h->d_rref.upload(h->rref));
   h->pp_host.assign(pp, pp + 3 * (size_t)np);
+  HIPCHK(h->d_scpart.alloc(6 * (size_t)kScatPartials));
   return setup_operator(h, t0);
 }
 
@@ -1765,6 +1767,14 @@ static ScatArgs scat_args(const spk_handle *h, int npts) {
   return a;
 }
 
+// a bound of the distances from npts points to the surface
+static double scat_reach(const spk_handle *h, int npts, const double *r) {
+  double m = 0.0;
+  for (int i = 0; i < 3 * npts; ++i) m = std::max(m, std::fabs(r[i]));
+  for (double v : h->pp_host) m = std::max(m, std::fabs(v));
+  return 4.0 * m;  // 2 sqrt(3) largest coordinate
+}
+
 // One field evaluation through device staging: the points dr[3*npts] are
 // copied in, one workgroup per point writes every component of dE, dH
 // [3*npts], which are copied out.
@@ -1778,7 +1788,7 @@ static int scattered_staged(spk_handle *h, int npts, const double *r, const zd *
     launch_quad_local(h->qtopo(), d_x, h->q_seh.p, h->st);
     launch_quad_field(h->qdev, h->qtopo(), npts, dr, h->q_seh.p, (double *)dE, (double *)dH, h->st);
   } else {
-    launch_scattered(a, h->d_fn.p, d_x, dr, dE, dH, h->st);
+    launch_scattered(a, scat_reach(h, npts, r), h->d_fn.p, d_x, dr, h->d_scpart.p, dE, dH, h->st);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(E, dE, 3 * (size_t)npts * sizeof(zd), hipMemcpyDeviceToHost, h->st));
@@ -3541,7 +3551,7 @@ int spk_adjoint_height_gradient(spk_handle *h, const double k_in[3], const doubl
   if ((rc = rhs_plane_dev(h, k_in, e_in, b.p))) return rc;
   if ((rc = spk_gmres_device(h, b.p, I.p, gp, &inf[0]))) return rc;
   const ScatArgs sa = scat_args(h, npts);
-  launch_scattered(sa, h->d_fn.p, I.p, dr.p, E.p, H.p, st);
+  launch_scattered(sa, scat_reach(h, npts, r), h->d_fn.p, I.p, dr.p, h->d_scpart.p, E.p, H.p, st);
   HIPCHK(hipGetLastError());
   std::vector<zd> Eh(3 * (size_t)npts);
   HIPCHK(hipMemcpyAsync(Eh.data(), E.p, Eh.size() * sizeof(zd), hipMemcpyDeviceToHost, st));

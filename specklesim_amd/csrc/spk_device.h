@@ -32,6 +32,10 @@ __host__ __device__ inline zd operator/(zd a, zd b) {
 __host__ __device__ inline zd operator/(zd a, double s) { return zd{a.x / s, a.y / s}; }
 __host__ __device__ inline zd operator/(double s, zd b) { return zd{s, 0.0} / b; }
 __host__ __device__ inline zd zcx(const cplx &c) { return zd{c.re, c.im}; }
+// a b + c in four fused operations (a * b + c as written takes six)
+__device__ inline zd cfma(zd a, zd b, zd c) {
+  return zd{fma(-a.y, b.y, fma(a.x, b.x, c.x)), fma(a.y, b.x, fma(a.x, b.y, c.y))};
+}
 // i*a
 __host__ __device__ inline zd mul_i(zd a) { return zd{-a.y, a.x}; }
 
@@ -174,9 +178,9 @@ struct PatLay {
   // the sign of the component's conjugate at the antipode
   __host__ __device__ bool flips(int h, int comp) const { return comp == 1 && h < K * K; }
 };
-// whether every k R of a surface of side D is below sincos_near's 1e5
+// whether every k R of a surface of side D is below sincos_near's 1e8
 inline bool sincos_near_holds(double D, zd k1, zd k2) {
-  return 4.0 * D * (fabs(k1.x) > fabs(k2.x) ? fabs(k1.x) : fabs(k2.x)) < 1e5;
+  return 4.0 * D * (fabs(k1.x) > fabs(k2.x) ? fabs(k1.x) : fabs(k2.x)) < 1e8;
 }
 void launch_patterns(int N, const PatLay &lay, int ngp, double D, const FnRec *fn, const int *perm, const int *leaf_box,
                      const double *leaf_centre, const double *khat, const double *tth,
@@ -271,8 +275,11 @@ struct ScatArgs {
   double qa[3], qb[3], qw[3];
   zd k1, iwmy, iweps, inv_iwmy;
 };
-void launch_scattered(const ScatArgs &a, const FnRec *fn, const zd *x, const double *r, zd *E,
-                      zd *H, hipStream_t st);
+// reach: a bound of the distances between points and surface; part: workspace
+// of 6 * kScatPartials values
+constexpr int kScatPartials = 1 << 17;
+void launch_scattered(const ScatArgs &a, double reach, const FnRec *fn, const zd *x,
+                      const double *r, zd *part, zd *E, zd *H, hipStream_t st);
 
 // adjoint gradient with respect to node heights (central differences of
 // the local quantities, node moved by +-dz along z)
