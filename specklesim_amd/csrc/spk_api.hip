@@ -3690,13 +3690,63 @@ int spk_adjoint_height_gradient(spk_handle *h, const double k_in[3], const doubl
   DBuf<int> d_aedge_t;
   HIPCHK(d_aedge_t.upload(aedge_t));
   const NearArgs A = near_args(h);
-  constexpr int kGroups = 64;
+  TriForm tf;
+  std::vector<int> tside;
+  const bool by_tri = make_tri_form(A, t.D, &tf) && tri_sides(h, &tside);
+  // workgroups a node: a triangle pair's task is about fifty times an entry's
+  const int kGroups = by_tri ? 8 : 64, nparts = by_tri ? kGroups + 1 : kGroups;
   DBuf<zd> near_part, far_out, rhs_out, fld_out;
-  HIPCHK(near_part.alloc((size_t)n_nodes * kGroups));
+  HIPCHK(near_part.alloc((size_t)n_nodes * nparts));
   HIPCHK(far_out.alloc(std::max(nslot, 1)));
   HIPCHK(rhs_out.alloc(std::max(nslot, 1)));
   HIPCHK(fld_out.alloc(std::max(nslot, 1)));
-  {
+  DBuf<int> d_tri[8];
+  DBuf<int4> d_bcoord;
+  if (by_tri) {
+    const int nt = (int)tside.size() / 3, nbl = (int)t.box_first.size();
+    std::vector<int> tnode(3 * (size_t)nt, 0), nto(n_nodes + 1, 0), ntl, nbo(n_nodes + 1, 0), nb;
+    for (const ElemRec &e : h->er)
+      for (int c = 0; c < 3; ++c) tnode[3 * (size_t)e.elem + c] = e.node[c] - 1;
+    for (int k = 0; k < n_nodes; ++k) {
+      for (int q = aoff[k]; q < aoff[k + 1]; ++q) {
+        for (int u = 0; u < 2; ++u) {
+          const ElemRec &e = h->er[2 * (size_t)aedge[q] + u];
+          const bool holds = e.node[0] - 1 == nodes[k] || e.node[1] - 1 == nodes[k] ||
+                             e.node[2] - 1 == nodes[k];
+          if (holds && std::find(ntl.begin() + nto[k], ntl.end(), e.elem) == ntl.end())
+            ntl.push_back(e.elem);
+        }
+        const int bx = t.leaf_box[aedge[q]];
+        if (std::find(nb.begin() + nbo[k], nb.end(), bx) == nb.end()) nb.push_back(bx);
+      }
+      nto[k + 1] = (int)ntl.size();
+      nbo[k + 1] = (int)nb.size();
+    }
+    std::vector<int> bto(nbl + 1, 0), btl, mark(nt, -1);
+    std::vector<int4> bc(nbl);
+    for (int b = 0; b < nbl; ++b) {
+      for (int ci = t.e2_off[b]; ci < t.e2_off[b + 1]; ++ci)
+        for (int u = 0; u < 2; ++u) {
+          const int el = h->er[2 * (size_t)t.e2_list[ci] + u].elem;
+          if (mark[el] == b) continue;
+          mark[el] = b;
+          btl.push_back(el);
+        }
+      bto[b + 1] = (int)btl.size();
+      // Morton index: x in bits 3i + 2, y in 3i + 1, z in 3i
+      const int64_t u = t.lev[t.l_max].n[b];
+      int c[3] = {0, 0, 0};
+      for (int i = 0; i < t.l_max; ++i)
+        for (int d = 0; d < 3; ++d) c[d] |= (int)((u >> (3 * i + 2 - d)) & 1) << i;
+      bc[b] = int4{c[0], c[1], c[2], 0};
+    }
+    const std::vector<int> *src[8] = {&tside, &tnode, &nto, &ntl, &nbo, &nb, &bto, &btl};
+    for (int i = 0; i < 8; ++i) HIPCHK(d_tri[i].upload(*src[i]));
+    HIPCHK(d_bcoord.upload(bc));
+    const AdjTri R{d_tri[0].p, d_tri[1].p, d_tri[2].p, d_tri[3].p, d_tri[4].p,
+                   d_tri[5].p, d_tri[6].p, d_tri[7].p, d_bcoord.p};
+    launch_adj_near_tri(A, G, R, tf, kGroups, nu.p, I.p, near_part.p, st);
+  } else {
     AdjArgs Gn = G;
     Gn.aff_edge = d_aedge_t.p;
     launch_adj_near(A, Gn, kGroups, nu.p, I.p, near_part.p, st);
@@ -3722,7 +3772,7 @@ int spk_adjoint_height_gradient(spk_handle *h, const double k_in[3], const doubl
   launch_adj_rhs(G, rhs_args(h, k_in, e_in), nu.p, rhs_out.p, st);
   launch_adj_field(G, sa, dr.p, dw.p, E.p, I.p, fld_out.p, st);
   HIPCHK(hipGetLastError());
-  std::vector<zd> hn((size_t)n_nodes * kGroups), hf(std::max(nslot, 1)), hr(std::max(nslot, 1)),
+  std::vector<zd> hn((size_t)n_nodes * nparts), hf(std::max(nslot, 1)), hr(std::max(nslot, 1)),
       hq(std::max(nslot, 1));
   HIPCHK(hipMemcpyAsync(hn.data(), near_part.p, hn.size() * sizeof(zd), hipMemcpyDeviceToHost, st));
   HIPCHK(hipMemcpyAsync(hf.data(), far_out.p, hf.size() * sizeof(zd), hipMemcpyDeviceToHost, st));
@@ -3731,7 +3781,7 @@ int spk_adjoint_height_gradient(spk_handle *h, const double k_in[3], const doubl
   HIPCHK(hipStreamSynchronize(st));
   for (int k = 0; k < n_nodes; ++k) {
     zc tz(0.0, 0.0), tf(0.0, 0.0);
-    for (int g = 0; g < kGroups; ++g) tz += zc(hn[(size_t)k * kGroups + g].x, hn[(size_t)k * kGroups + g].y);
+    for (int g = 0; g < nparts; ++g) tz += zc(hn[(size_t)k * nparts + g].x, hn[(size_t)k * nparts + g].y);
     for (int q = aoff[k]; q < aoff[k + 1]; ++q) {
       tz += zc(hf[q].x, hf[q].y);
       tf += zc(hq[q].x, hq[q].y) + zc(hr[q].x, hr[q].y);
@@ -3739,7 +3789,7 @@ int spk_adjoint_height_gradient(spk_handle *h, const double k_in[3], const doubl
     grad[k] = 2.0 * (tf - tz).real() / (2.0 * dz);
     if (terms) {
       zc tn(0.0, 0.0), tfar(0.0, 0.0), tfld(0.0, 0.0), trhs(0.0, 0.0);
-      for (int g = 0; g < kGroups; ++g) tn += zc(hn[(size_t)k * kGroups + g].x, hn[(size_t)k * kGroups + g].y);
+      for (int g = 0; g < nparts; ++g) tn += zc(hn[(size_t)k * nparts + g].x, hn[(size_t)k * nparts + g].y);
       for (int q = aoff[k]; q < aoff[k + 1]; ++q) {
         tfar += zc(hf[q].x, hf[q].y);
         tfld += zc(hq[q].x, hq[q].y);

@@ -306,6 +306,19 @@ struct AdjFar {
 };
 void launch_adj_near(const NearArgs &A, const AdjArgs &G, int groups, const zd *nu, const zd *I,
                      zd *partial, hipStream_t st);
+// the near share by triangle pairs: sides and 0-based nodes of every triangle's
+// corners, each requested node's triangles and the leaf boxes of its edges, the
+// triangles of every box's columns, the boxes' integer coordinates
+struct AdjTri {
+  const int *tside, *tnode;
+  const int *ntri_off, *ntri;
+  const int *nbox_off, *nbox;
+  const int *btri_off, *btri;
+  const int4 *bcoord;
+};
+// partial: [node][groups + 1]
+void launch_adj_near_tri(const NearArgs &A, const AdjArgs &G, const AdjTri &R, const TriForm &Q,
+                         int groups, const zd *nu, const zd *I, zd *partial, hipStream_t st);
 void launch_adj_far(const AdjArgs &G, const AdjFar &F, const zd *nu, const zd *I, const zd *W,
                     const zd *Bt, zd *out, hipStream_t st);
 void launch_adj_rhs(const AdjArgs &G, const RhsArgs &a, const zd *nu, zd *out, hipStream_t st);

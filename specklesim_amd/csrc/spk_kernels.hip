@@ -804,6 +804,90 @@ __device__ inline void finish_tri(const NearArgs &A, zd *D) {
   finish_D(A, D);
 }
 
+// S0 += G, S1 += (u.v) G (both media) and SK += (v.(c x u)) G'/R (their sum),
+// each times fac, over the nine point pairs of a test side with corners cm
+// (p1, p2, free) and the triangle (q0, q0 + e1, q0 + e2), for the triangle's
+// three sides
+template <bool LOSSY>
+__device__ __forceinline__ void tri_sums(const zd *kk, const double *cm, const double *q0,
+                                         const double *e1, const double *e2, double fac,
+                                         zd (*S0)[2], zd (*S1)[2], zd *SK) {
+#pragma unroll 1
+  for (int j = 0; j < 3; ++j) {
+    double ra[3];
+    simplex(kTri3.a[j], kTri3.b[j], cm, ra);
+    double ue1, ue2, P1[3], P2[3];
+    {
+      double u[3], x[3];
+      for (int k = 0; k < 3; ++k) u[k] = ra[k] - cm[6 + k];
+      ue1 = dot3(u, e1);
+      ue2 = dot3(u, e2);
+      cross3(e1, e2, x);
+      const double un = dot3(u, x);
+      const double d0[3] = {cm[6] - q0[0], cm[7] - q0[1], cm[8] - q0[2]};
+      cross3(d0, u, x);
+      // v.(c x u) = mu1 e1.(c x u) + mu2 e2.(c x u) for v = mu1 e1 + mu2 e2
+      P1[0] = P1[1] = dot3(e1, x);
+      P2[0] = P2[2] = dot3(e2, x);
+      P1[2] = P1[0] - un;
+      P2[1] = P2[0] + un;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double R[3];
+      for (int k = 0; k < 3; ++k)
+        R[k] = ra[k] - (q0[k] + kTri3.lb1[i] * e1[k] + kTri3.lb2[i] * e2[k]);
+      const double R2 = dot3(R, R), rinv = rsqrt_near(R2), Rl = R2 * rinv;
+      const double g4 = rinv * fac, rinv2 = rinv * rinv;
+      const double Re1 = dot3(R, e1), Re2 = dot3(R, e2);
+      zd G[2], D[2], Fs;
+#pragma unroll
+      for (int md = 0; md < 2; ++md) {
+        // G, D = G'/R and F = D'/R
+        const double x = kk[md].x * Rl;
+        double sn, cs;
+        sincos_near(x, &sn, &cs);
+        zd f;
+        if (LOSSY) {
+          const double y = kk[md].y * Rl, ge = g4 * exp(y);
+          const zd ikr = {-y, x};
+          G[md] = zd{cs * ge, -sn * ge};
+          const zd o = zd{1.0 - y, x} * G[md];
+          D[md] = o * -rinv2;
+          f = (3.0 * o + (ikr * ikr) * G[md]) * (rinv2 * rinv2);
+        } else {
+          G[md] = zd{cs * g4, -sn * g4};
+          const zd o = zd{fma(-x, G[md].y, G[md].x), fma(x, G[md].x, G[md].y)};
+          D[md] = o * -rinv2;
+          const double x2 = x * x;
+          f = zd{fma(-x2, G[md].x, 3.0 * o.x), fma(-x2, G[md].y, 3.0 * o.y)} *
+              (rinv2 * rinv2);
+        }
+        Fs = md == 0 ? f : Fs + f;
+      }
+      const zd Ds = D[0] + D[1];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const double a = kTri3.mu1[p][i] * ue1 + kTri3.mu2[p][i] * ue2;
+        const double bb = kTri3.mu1[p][i] * P1[p] + kTri3.mu2[p][i] * P2[p];
+        zd g[2] = {G[0], G[1]}, d = Ds;
+        if (p > 0) {
+          const double h = -(kTri3.dl1[p][i] * Re1 + kTri3.dl2[p][i] * Re2);
+          g[0] = g[0] + D[0] * h;
+          g[1] = g[1] + D[1] * h;
+          d = d + Fs * h;
+        }
+#pragma unroll
+        for (int md = 0; md < 2; ++md) {
+          S0[p][md] = S0[p][md] + g[md];
+          S1[p][md] = S1[p][md] + g[md] * a;
+        }
+        SK[p] = SK[p] + d * bb;
+      }
+    }
+  }
+}
+
 // workgroup = (box, rp rows of one of its row tiles); LDS per column: T of
 // both media and K, for PMCHWT-S also K with the column side's sign.  LOSSY: a
 // medium's wavenumber is complex.
@@ -852,80 +936,7 @@ __global__ void __launch_bounds__(256, 2) k_near_tri(NearArgs A, TriForm Q, cons
           if ((sing >> (2 * t)) & 1u) continue;
           const FnRec &fm = A.fn[2 * m + t];
           const double fac = kTri3.w2 * fm.area * fm.df * (1.0 / (4 * PI));
-#pragma unroll 1
-          for (int j = 0; j < 3; ++j) {
-            double ra[3];
-            simplex(A.qa[j], A.qb[j], fm.c, ra);
-            double ue1, ue2, P1[3], P2[3];
-            {
-              double u[3], x[3];
-              for (int k = 0; k < 3; ++k) u[k] = ra[k] - fm.c[6 + k];
-              ue1 = dot3(u, e1);
-              ue2 = dot3(u, e2);
-              cross3(e1, e2, x);
-              const double un = dot3(u, x);
-              const double d0[3] = {fm.c[6] - q0[0], fm.c[7] - q0[1], fm.c[8] - q0[2]};
-              cross3(d0, u, x);
-              // v.(c x u) = mu1 e1.(c x u) + mu2 e2.(c x u) for v = mu1 e1 + mu2 e2
-              P1[0] = P1[1] = dot3(e1, x);
-              P2[0] = P2[2] = dot3(e2, x);
-              P1[2] = P1[0] - un;
-              P2[1] = P2[0] + un;
-            }
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              double R[3];
-              for (int k = 0; k < 3; ++k)
-                R[k] = ra[k] - (q0[k] + kTri3.lb1[i] * e1[k] + kTri3.lb2[i] * e2[k]);
-              const double R2 = dot3(R, R), rinv = rsqrt_near(R2), Rl = R2 * rinv;
-              const double g4 = rinv * fac, rinv2 = rinv * rinv;
-              const double Re1 = dot3(R, e1), Re2 = dot3(R, e2);
-              zd G[2], D[2], Fs;
-#pragma unroll
-              for (int md = 0; md < 2; ++md) {
-                // G, D = G'/R and F = D'/R
-                const double x = kk[md].x * Rl;
-                double sn, cs;
-                sincos_near(x, &sn, &cs);
-                zd f;
-                if (LOSSY) {
-                  const double y = kk[md].y * Rl, ge = g4 * exp(y);
-                  const zd ikr = {-y, x};
-                  G[md] = zd{cs * ge, -sn * ge};
-                  const zd o = zd{1.0 - y, x} * G[md];
-                  D[md] = o * -rinv2;
-                  f = (3.0 * o + (ikr * ikr) * G[md]) * (rinv2 * rinv2);
-                } else {
-                  G[md] = zd{cs * g4, -sn * g4};
-                  const zd o = zd{fma(-x, G[md].y, G[md].x), fma(x, G[md].x, G[md].y)};
-                  D[md] = o * -rinv2;
-                  const double x2 = x * x;
-                  f = zd{fma(-x2, G[md].x, 3.0 * o.x), fma(-x2, G[md].y, 3.0 * o.y)} *
-                      (rinv2 * rinv2);
-                }
-                Fs = md == 0 ? f : Fs + f;
-              }
-              const zd Ds = D[0] + D[1];
-#pragma unroll
-              for (int p = 0; p < 3; ++p) {
-                const double a = kTri3.mu1[p][i] * ue1 + kTri3.mu2[p][i] * ue2;
-                const double bb = kTri3.mu1[p][i] * P1[p] + kTri3.mu2[p][i] * P2[p];
-                zd g[2] = {G[0], G[1]}, d = Ds;
-                if (p > 0) {
-                  const double h = -(kTri3.dl1[p][i] * Re1 + kTri3.dl2[p][i] * Re2);
-                  g[0] = g[0] + D[0] * h;
-                  g[1] = g[1] + D[1] * h;
-                  d = d + Fs * h;
-                }
-#pragma unroll
-                for (int md = 0; md < 2; ++md) {
-                  S0[p][md] = S0[p][md] + g[md];
-                  S1[p][md] = S1[p][md] + g[md] * a;
-                }
-                SK[p] = SK[p] + d * bb;
-              }
-            }
-          }
+          tri_sums<LOSSY>(kk, fm.c, q0, e1, e2, fac, S0, S1, SK);
         }
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
@@ -3269,6 +3280,240 @@ __global__ void __launch_bounds__(256) k_adj_near(NearArgs A, AdjArgs G, const z
   if (threadIdx.x == 0) partial[(size_t)k * gridDim.x + blockIdx.x] = acc;
 }
 
+// ---------------------------------------------------------------------------
+// The same share by pairs of triangles, where the triangle kernel of the near
+// fill applies (make_tri_form).  k_adj_near is bound by the FP64 ALU: it
+// evaluates every side combination of a triangle pair by itself, with regular
+// and singular pairs in one wave.  Here a task is (moved triangle T, triangle
+// S near one of T's edges).  Under the symmetric rule a regular pair's T and K
+// are the same with test and source exchanged, so S's rows against T's
+// columns come from the same sums; each of T's sides takes tri_sums over S at
+// +dz and -dz (54 point pairs serve 18 entries at either height).  Singular
+// pairs go to k_adj_near_sing.  961 nodes of a 2640-edge patch: 3.0 + 1.8 ms, where
+// k_adj_near takes 73 ms.
+// ---------------------------------------------------------------------------
+// whether test edge m takes the singular branch for triangles a distance apart;
+// written out so that both kernels round alike
+__device__ inline bool adj_singular(const NearArgs &A, int m, const double *a, const double *b) {
+  const double x = a[0] - b[0], y = a[1] - b[1], z = a[2] - b[2];
+  return !(sqrt(fma(z, z, fma(y, y, x * x))) > 1.5 * A.rref[m]);
+}
+__device__ inline bool adj_near(const int4 *bc, int a, int b) {
+  const int4 p = bc[a], q = bc[b];
+  return abs(p.x - q.x) <= 1 && abs(p.y - q.y) <= 1 && abs(p.z - q.z) <= 1;
+}
+struct AdjPair {
+  int T, S;
+  bool smoved;
+};
+// task t of node k; false where S was met in an earlier box's list
+__device__ inline bool adj_task(const AdjArgs &G, const AdjTri &R, int k, int64_t t, int64_t total,
+                                AdjPair &o) {
+  o.T = R.ntri[R.ntri_off[k] + (int)(t / total)];
+  int64_t l = t % total;
+  const int b0 = R.nbox_off[k];
+  int bi = b0;
+  while (l >= R.btri_off[R.nbox[bi] + 1] - R.btri_off[R.nbox[bi]]) {
+    l -= R.btri_off[R.nbox[bi] + 1] - R.btri_off[R.nbox[bi]];
+    ++bi;
+  }
+  o.S = R.btri[R.btri_off[R.nbox[bi]] + (int)l];
+  for (int bj = b0; bj < bi; ++bj)
+    for (int q = 0; q < 3; ++q) {
+      const int sd = R.tside[3 * o.S + q];
+      if (sd >= 0 && adj_near(R.bcoord, G.leaf_box[sd >> 1], R.nbox[bj])) return false;
+    }
+  const int pn = G.node[k], *nd = R.tnode + 3 * o.S;
+  o.smoved = nd[0] == pn || nd[1] == pn || nd[2] == pn;
+  return true;
+}
+__device__ inline int64_t adj_total(const AdjTri &R, int k) {
+  int64_t n = 0;
+  for (int b = R.nbox_off[k]; b < R.nbox_off[k + 1]; ++b)
+    n += R.btri_off[R.nbox[b] + 1] - R.btri_off[R.nbox[b]];
+  return n;
+}
+__device__ inline const double *adj_mid(const NearArgs &A, const AdjTri &R, int T) {
+  const int *sd = R.tside + 3 * T;
+  return A.fn[sd[0] >= 0 ? sd[0] : sd[1] >= 0 ? sd[1] : sd[2]].mid;
+}
+
+template <bool LOSSY>
+__global__ void __launch_bounds__(256, 2) k_adj_near_tri(NearArgs A, AdjArgs G, AdjTri R, TriForm Q,
+                                                         const zd *nu, const zd *I, zd *partial) {
+  const int k = blockIdx.y, pn = G.node[k];
+  const int64_t total = adj_total(R, k);
+  const int64_t ntask = total * (R.ntri_off[k + 1] - R.ntri_off[k]);
+  const zd kk[2] = {zcx(A.mat.k1), zcx(A.mat.k2)};
+  zd acc = {0, 0};
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < ntask;
+       t += (int64_t)gridDim.x * blockDim.x) {
+    AdjPair tp;
+    if (!adj_task(G, R, k, t, total, tp) || tp.T == tp.S) continue;
+    const double *mT = adj_mid(A, R, tp.T), *mS = adj_mid(A, R, tp.S);
+#pragma unroll 1
+    for (int p = 0; p < 3; ++p) {
+      const int sm = R.tside[3 * tp.T + p];
+      if (sm < 0) continue;
+      const int m = sm >> 1;
+      // entries (m, n) [bit n] and (n, m) [bit 4 + n] that are near and regular
+      unsigned use = 0;
+      const bool rm = !adj_singular(A, m, mT, mS);
+      for (int q = 0; q < 3; ++q) {
+        const int sn = R.tside[3 * tp.S + q];
+        if (sn < 0 || !adj_near(R.bcoord, G.leaf_box[m], G.leaf_box[sn >> 1])) continue;
+        if (rm) use |= 1u << q;
+        if (!tp.smoved && !adj_singular(A, sn >> 1, mT, mS)) use |= 16u << q;
+      }
+      if (!use) continue;
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+        const double dz = h ? -G.dz : G.dz;
+        auto corner = [&](int T, int c, double *o) {
+          const int v = R.tnode[3 * T + c];
+          for (int d = 0; d < 3; ++d) o[d] = G.pp[3 * v + d];
+          if (v == pn) o[2] += dz;
+        };
+        double cm[9], q0[3], e1[3], e2[3];
+        corner(tp.T, p == 2 ? 0 : p + 1, cm);
+        corner(tp.T, p == 0 ? 2 : p - 1, cm + 3);
+        corner(tp.T, p, cm + 6);
+        const double l[3] = {cm[0] - cm[3], cm[1] - cm[4], cm[2] - cm[5]};
+        // area * df = sign * length of the edge
+        const double fac = kTri3.w2 * ((sm & 1) ? -1.0 : 1.0) * len3(l) * (1.0 / (4 * PI));
+        corner(tp.S, 0, q0);
+        corner(tp.S, 1, e1);
+        corner(tp.S, 2, e2);
+        for (int d = 0; d < 3; ++d) {
+          e1[d] -= q0[d];
+          e2[d] -= q0[d];
+        }
+        zd S0[3][2], S1[3][2], SK[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          S0[q][0] = S0[q][1] = S1[q][0] = S1[q][1] = SK[q] = zd{0, 0};
+        tri_sums<LOSSY>(kk, cm, q0, e1, e2, fac, S0, S1, SK);
+        const zd nm = nu[m], nmh = nu[m + G.N], im = I[m], imh = I[m + G.N];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const int sn = R.tside[3 * tp.S + q];
+          if (!((use >> q) & 17u)) continue;
+          const int n = sn >> 1;
+          const zd nn = nu[n], nnh = nu[n + G.N], in = I[n], inh = I[n + G.N];
+          zd w11 = {0, 0}, w22 = {0, 0}, w12 = {0, 0}, w21 = {0, 0};
+          if ((use >> q) & 1u) {
+            w11 = nm * in;
+            w22 = nmh * inh;
+            w12 = nm * inh;
+            w21 = nmh * in;
+            if (A.form == SPK_PMCHWT_S && !(sn & 1)) w21 = -w21;
+          }
+          if ((use >> q) & 16u) {
+            w11 = w11 + nn * im;
+            w22 = w22 + nnh * imh;
+            w12 = w12 + nn * imh;
+            w21 = (A.form == SPK_PMCHWT_S && !(sm & 1)) ? w21 - nnh * im : w21 + nnh * im;
+          }
+          // side q's edge of S as the corners lie now
+          double a[3], len;
+          for (int d = 0; d < 3; ++d)
+            a[d] = q == 0 ? e2[d] - e1[d] : q == 1 ? e2[d] : e1[d];
+          len = ((sn & 1) ? -1.0 : 1.0) * len3(a);
+          zd v = (Q.c[2] * w12 + Q.c[3] * w21) * (SK[q] * 0.25);
+          for (int md = 0; md < 2; ++md)
+            v = v + (Q.c[md] * w11 + Q.c[4 + md] * w22) *
+                        mul_i(Q.k4[md] * S1[q][md] - Q.ik[md] * S0[q][md]);
+          acc = acc + v * (h ? -len : len);
+        }
+      }
+    }
+  }
+  acc = block_sum(acc);
+  if (threadIdx.x == 0) partial[(size_t)k * (gridDim.x + 1) + blockIdx.x] = acc;
+}
+
+// the singular pairs of a node: candidates in order into an LDS list, then a
+// thread per (pair, sides, direction)
+__global__ void __launch_bounds__(256) k_adj_near_sing(NearArgs A, AdjArgs G, AdjTri R, int groups,
+                                                       const zd *nu, const zd *I, zd *partial) {
+  constexpr int CAP = 512;
+  __shared__ int lT[CAP], lS[CAP];
+  __shared__ int wcount[4];
+  const int k = blockIdx.x, pn = G.node[k];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t total = adj_total(R, k);
+  const int64_t ntask = total * (R.ntri_off[k + 1] - R.ntri_off[k]);
+  zd acc = {0, 0};
+  int cnt = 0;
+  for (int64_t t0 = 0; t0 < ntask; t0 += 256) {
+    const int64_t t = t0 + threadIdx.x;
+    bool take = false;
+    AdjPair tp{0, 0, false};
+    if (t < ntask && adj_task(G, R, k, t, total, tp)) {
+      const double *mT = adj_mid(A, R, tp.T), *mS = adj_mid(A, R, tp.S);
+      for (int q = 0; q < 3; ++q) {
+        const int sm = R.tside[3 * tp.T + q], sn = R.tside[3 * tp.S + q];
+        if (sm >= 0 && adj_singular(A, sm >> 1, mT, mS)) take = true;
+        if (sn >= 0 && !tp.smoved && adj_singular(A, sn >> 1, mT, mS)) take = true;
+      }
+    }
+    const unsigned long long bal = __ballot(take);
+    if (lane == 0) wcount[wv] = __popcll(bal);
+    __syncthreads();
+    int at = cnt + __popcll(bal & ((1ull << lane) - 1ull));
+    for (int w = 0; w < wv; ++w) at += wcount[w];
+    cnt += wcount[0] + wcount[1] + wcount[2] + wcount[3];
+    if (take) {
+      lT[at] = tp.T;
+      lS[at] = tp.smoved ? -1 - tp.S : tp.S;
+    }
+    __syncthreads();
+    if (cnt <= CAP - 256 && t0 + 256 < ntask) continue;
+    for (int i = threadIdx.x; i < cnt * 18; i += 256) {
+      const int pr = i / 18, c = i - 18 * pr, dir = c / 9, p = (c % 9) / 3, q = c % 3;
+      const int T = lT[pr], S = lS[pr] < 0 ? -1 - lS[pr] : lS[pr];
+      const bool smoved = lS[pr] < 0;
+      const int sT = R.tside[3 * T + p], sS = R.tside[3 * S + q];
+      if (sT < 0 || sS < 0 || (dir && smoved)) continue;
+      const int sm = dir ? sS : sT, sn = dir ? sT : sS, m = sm >> 1, n = sn >> 1;
+      if (!adj_singular(A, m, adj_mid(A, R, T), adj_mid(A, R, S))) continue;
+      if (!adj_near(R.bcoord, G.leaf_box[m], G.leaf_box[n])) continue;
+      const ElemRec ea = A.er[sm], eb = A.er[sn];
+      const bool iqs = ea.elem == eb.elem, swap = A.edge_swap && !iqs && edge_adj(ea, eb);
+      zd d[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+        const double dz = h ? -G.dz : G.dz;
+        const int *snm = G.side_nodes + 6 * sm, *snn = G.side_nodes + 6 * sn;
+        const FnRec fa = side_holds(snm, pn) ? fn_rebuild(G.pp, snm, sm & 1, G.normal_convention, pn, dz)
+                                             : A.fn[sm];
+        const FnRec fb = side_holds(snn, pn) ? fn_rebuild(G.pp, snn, sn & 1, G.normal_convention, pn, dz)
+                                             : A.fn[sn];
+        Rel rv[2];
+        singular_pair(fa, fb, iqs, A, rv);
+        if (swap) {
+          zd kt[2];
+          edge_adjacent_kt(fa, fb, A, kt);
+          rv[0].Kt = kt[0];
+          rv[1].Kt = kt[1];
+        }
+        zd z[4];
+        assemble_zz(A, rv, z);
+        for (int j = 0; j < 4; ++j) d[j] = h ? d[j] - z[j] : z[j];
+      }
+      zd Db[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+      add_zz(A, Db, d, sn & 1);
+      finish_tri(A, Db);
+      const zd ie = I[n], ih = I[n + G.N];
+      acc = acc + nu[m] * (Db[0] * ie + Db[1] * ih) + nu[m + G.N] * (Db[2] * ie + Db[3] * ih);
+    }
+    cnt = 0;
+    __syncthreads();
+  }
+  acc = block_sum(acc);
+  if (threadIdx.x == 0) partial[(size_t)k * (groups + 1) + groups] = acc;
+}
+
 // the four pattern components of edge m (sides fs[2]) at sample s: theta
 // and phi projections for media 1 and 2 (k_patterns' integrand)
 __device__ void pattern_sample(const FnRec *fs, const double *Rc, const double *kh,
@@ -3481,6 +3726,15 @@ void launch_adj_near(const NearArgs &A, const AdjArgs &G, int groups, const zd *
                      zd *partial, hipStream_t st) {
   if (G.nnode <= 0) return;
   hipLaunchKernelGGL(k_adj_near, dim3(groups, G.nnode), dim3(256), 0, st, A, G, nu, I, partial);
+}
+void launch_adj_near_tri(const NearArgs &A, const AdjArgs &G, const AdjTri &R, const TriForm &Q,
+                         int groups, const zd *nu, const zd *I, zd *partial, hipStream_t st) {
+  if (G.nnode <= 0) return;
+  const bool lossy = A.mat.k1.im != 0.0 || A.mat.k2.im != 0.0;
+  hipLaunchKernelGGL(lossy ? k_adj_near_tri<true> : k_adj_near_tri<false>, dim3(groups, G.nnode),
+                     dim3(256), 0, st, A, G, R, Q, nu, I, partial);
+  hipLaunchKernelGGL(k_adj_near_sing, dim3(G.nnode), dim3(256), 0, st, A, G, R, groups, nu, I,
+                     partial);
 }
 void launch_adj_far(const AdjArgs &G, const AdjFar &F, const zd *nu, const zd *I, const zd *W,
                     const zd *Bt, zd *out, hipStream_t st) {
