@@ -109,6 +109,7 @@ struct spk_handle {
   DBuf<int> d_perm, d_box_first, d_box_count, d_e2_off, d_e2_list, d_leaf_box, d_leafbox_of_pos;
   DBuf<int64_t> d_near_off;
   DBuf<zd> d_blocks;
+  NearRel rel;  // what a near block keeps
   DBuf<int> d_row_box, d_row_r0, d_disagg_task;
   DBuf<int> d_mx_box, d_mx_r0;  // groups of row tiles of a box (batched fp8 product)
   int mx_groups = 0;
@@ -339,6 +340,31 @@ bool make_tri_form(const NearArgs &a, double D, TriForm *q) {
   return true;
 }
 
+// What the near blocks of a formulation keep.  PMCHWT, MCTF and ICTF take K of
+// both media into D12 and D21 with constant factors (assemble_zz), at most one
+// of which is far from 1; PMCHWT-S alternates D21's sign and the others have
+// further terms there.  Three components are a quarter fewer bytes wherever
+// the blocks are read, four and three on the 10 x 10 wavelength patch (28.3M
+// blocks): FP64 334 and 248 us (5.5 TB/s), complex64 186 and 137, fp8 49 and
+// 42; 16 vectors FP64 545 and 474, complex64 240 and 207, fp8 82 and 66.
+NearRel near_rel(int form, const Material &mat) {
+  NearRel r;
+  if (form == SPK_PMCHWT)
+    r.c = zd{-1.0, 0.0};
+  else if (form == SPK_MCTF)
+    r.c = -(zcx(mat.eta1) * zcx(mat.eta2));
+  else if (form == SPK_ICTF)
+    r.c = -(zcx(mat.eta_a) * zcx(mat.eta_a));
+  else
+    return r;
+  // a factor that complex64 holds (any impedance of a medium does)
+  const double a = std::hypot(r.c.x, r.c.y);
+  if (!(a > 1e-15 && a < 1e15)) return NearRel{};
+  r.nc = 3;
+  r.ic = zd{1.0, 0.0} / r.c;
+  return r;
+}
+
 // side (2 edge + s) opposite each local corner of every triangle, -1 where
 // it has none; false where a corner has two (more than two triangles meet in
 // an edge): then k_near_regular fills the blocks
@@ -359,7 +385,8 @@ bool tri_sides(const spk_handle *h, std::vector<int> *out) {
 
 int near_fill(spk_handle *h) {
   const int64_t nnz = h->tree.nnz;
-  HIPCHK(h->d_blocks.alloc(4 * (size_t)nnz));
+  h->rel = near_rel(h->p.formulation, h->mat);
+  HIPCHK(h->d_blocks.alloc(h->rel.nc * (size_t)nnz));
   if (nnz == 0) return SPK_OK;
   NearArgs a = near_args(h);
   auto &NW = h->nw;
@@ -395,10 +422,10 @@ int near_fill(spk_handle *h) {
     HIPCHK(NW.tside.upload(tside));
     HIPCHK(NW.tlist.alloc(2 * h->tree.e2_list.size()));
     HIPCHK(NW.tcnt.alloc(h->tree.e2_list.size()));
-    launch_near_tri(a, tf, h->N, h->spmv_wgs, h->d_row_box.p, h->d_row_r0.p, NW.tside.p,
+    launch_near_tri(a, tf, h->rel, h->N, h->spmv_wgs, h->d_row_box.p, h->d_row_r0.p, NW.tside.p,
                     NW.tlist.p, NW.tcnt.p, cls.p, ba.p, zz.p, h->d_blocks.p, h->st);
   } else {
-    launch_near_regular(a, nnz, cls.p, ba.p, zz.p, h->d_blocks.p, h->st);
+    launch_near_regular(a, h->rel, nnz, cls.p, ba.p, zz.p, h->d_blocks.p, h->st);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->st));
@@ -419,6 +446,7 @@ int near_fill_quad(spk_handle *h) {
   const QuadMesh &m = h->qmesh;
   const int nbl = (int)t.box_first.size();
   const int64_t nnz = t.nnz;
+  h->rel = NearRel{};
   HIPCHK(h->d_blocks.alloc(4 * (size_t)nnz));
   if (nnz == 0) return SPK_OK;
   std::vector<int> tb_off(nbl + 1, 0), tb_list, colA(t.e2_list.size()), colB(t.e2_list.size(), -1);
@@ -834,7 +862,7 @@ static int matvec_multik(spk_handle *h, const zd *x, zd *y, bool near_on, bool f
   if (near_on)
     launch_near_spmv_rows(h->spmv_wgs, N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                           h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                          h->d_perm.p, (const zd *)h->d_blocks.p, x, far_on ? (const zd *)yfar : nullptr, y,
+                          h->d_perm.p, h->rel, (const zd *)h->d_blocks.p, x, far_on ? (const zd *)yfar : nullptr, y,
                           st);
   HIPCHK(hipGetLastError());
   return SPK_OK;
@@ -888,7 +916,7 @@ static int matvec_quad_t(spk_handle *h, const T *x, T *y, bool near_on, bool far
   if (near_on)
     launch_near_spmv_rows(h->spmv_wgs, N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                           h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                          h->d_perm.p, pBlk(h, tag), x, far_on ? (const T *)yfar : nullptr, y,
+                          h->d_perm.p, h->rel, pBlk(h, tag), x, far_on ? (const T *)yfar : nullptr, y,
                           st);
   mark(7);
   HIPCHK(hipGetLastError());
@@ -993,7 +1021,7 @@ int matvec_t(spk_handle *h, const T *x, T *y, bool near_on = true, bool far_on =
   if (near_on)
     launch_near_spmv_rows(h->spmv_wgs, N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                           h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                          h->d_perm.p, pBlk(h, tag), x, far_on ? (const T *)yfar : nullptr, y,
+                          h->d_perm.p, h->rel, pBlk(h, tag), x, far_on ? (const T *)yfar : nullptr, y,
                           st);
   mark(7);
   HIPCHK(hipGetLastError());
@@ -1053,14 +1081,14 @@ int matvec_batch_t(spk_handle *h, int R, const T *const *xs, T *const *ys, bool 
   const int S = h->tb.S, N = h->N, lmax = t.l_max, lmin = t.l_min;
   hipStream_t st = h->st;
   LevelDev &LL = h->lev[lmax];
-  launch_batch_interleave(N, R, h->d_perm.p, xs, BB.XI.p, BB.XP.p, st);
+  launch_batch_interleave(N, R, h->rel, h->d_perm.p, xs, BB.XI.p, BB.XP.p, st);
   if (!far_on) {
     if constexpr (std::is_same<T, zf>::value) {
       if (f8_scale && R > 8) {
         launch_batch_near_f8(h->spmv_wgs, N, R, h->d_row_box.p, h->d_row_r0.p, h->mx_groups,
                              h->d_mx_box.p, h->d_mx_r0.p, h->d_box_first.p,
                              h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                             h->d_perm.p, blocks_bf, f8_scale, (const zf *)BB.XI.p, BB.XB.p, ys,
+                             h->d_perm.p, h->rel, blocks_bf, f8_scale, (const zf *)BB.XI.p, BB.XB.p, ys,
                              h->mx_tpw, st);
         HIPCHK(hipGetLastError());
         return SPK_OK;
@@ -1068,7 +1096,7 @@ int matvec_batch_t(spk_handle *h, int R, const T *const *xs, T *const *ys, bool 
     }
     launch_batch_near(h->spmv_wgs, N, R, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                       h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p, h->d_perm.p,
-                      pBlk(h, tag), (const T *)BB.XI.p, (const T *)nullptr, ys, st,
+                      h->rel, pBlk(h, tag), (const T *)BB.XI.p, (const T *)nullptr, ys, st,
                       f8_scale ? nullptr : blocks_bf);
     HIPCHK(hipGetLastError());
     return SPK_OK;
@@ -1094,7 +1122,7 @@ int matvec_batch_t(spk_handle *h, int R, const T *const *xs, T *const *ys, bool 
                       h->sc2, BB.YP.p, BB.YF.p, h->dx_tiles, h->d_dx_box.p, h->d_dx_p0.p, st);
   launch_batch_near(h->spmv_wgs, N, R, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                     h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p, h->d_perm.p,
-                    pBlk(h, tag), (const T *)BB.XI.p, (const T *)BB.YF.p, ys, st);
+                    h->rel, pBlk(h, tag), (const T *)BB.XI.p, (const T *)BB.YF.p, ys, st);
   HIPCHK(hipGetLastError());
   return SPK_OK;
 }
@@ -1153,7 +1181,7 @@ void stage_bytes(const spk_handle *h, double *b, double c = 16.0) {
   }
   b[4] = 2.0 * nbl * 8 * S * c;
   b[5] = pat + nbl * 8 * S * c + 2 * N * c;  // patterns + W + y
-  b[6] = (double)t.nnz * 4 * c + 2 * N * c + 2 * N * c + 2 * N * c;  // blocks + x + yfar + y
+  b[6] = (double)t.nnz * h->rel.nc * c + 2 * N * c + 2 * N * c + 2 * N * c;  // blocks + x + yfar + y
   b[7] = b[0] + b[1] + b[2] + b[3] + b[4] + b[5] + b[6];
 }
 
@@ -1341,7 +1369,7 @@ static int setup_operator(spk_handle *h, double t0) {
   h->stats.l_min = t.l_min;
   h->stats.l_max = t.l_max;
   h->stats.samples = h->tb.S;
-  h->stats.bytes_near = (double)t.nnz * 64.0;
+  h->stats.bytes_near = (double)t.nnz * h->rel.nc * 16.0;
   h->stats.bytes_patterns =
       (double)h->N * (h->quad ? (double)kQuadRtRows * h->tb.S : (double)h->lay.stride()) * 16.0;
   if (h->p.precision == SPK_MIXED) {
@@ -1531,7 +1559,7 @@ int spk_set_transposed(spk_handle *h, int transposed) {
     HIPCHK(tmp.alloc(h->d_blocks.n));
     launch_near_transpose(nbl, max_rows, h->d_box_first.p, h->d_box_count.p, h->d_e2_off.p,
                           h->d_e2_list.p, h->d_near_off.p, h->d_perm.p, h->d_pos.p,
-                          h->d_leaf_box.p, (const zd *)h->d_blocks.p, tmp.p, h->st);
+                          h->d_leaf_box.p, h->rel.nc, (const zd *)h->d_blocks.p, tmp.p, h->st);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(h->st));
     std::swap(h->d_blocks, tmp);
@@ -1541,7 +1569,7 @@ int spk_set_transposed(spk_handle *h, int transposed) {
     HIPCHK(tmp.alloc(h->f_blocks.n));
     launch_near_transpose(nbl, max_rows, h->d_box_first.p, h->d_box_count.p, h->d_e2_off.p,
                           h->d_e2_list.p, h->d_near_off.p, h->d_perm.p, h->d_pos.p,
-                          h->d_leaf_box.p, (const zf *)h->f_blocks.p, tmp.p, h->st);
+                          h->d_leaf_box.p, h->rel.nc, (const zf *)h->f_blocks.p, tmp.p, h->st);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(h->st));
     std::swap(h->f_blocks, tmp);
@@ -1549,6 +1577,7 @@ int spk_set_transposed(spk_handle *h, int transposed) {
   h->near_bf_ok = h->near_f8_ok = false;
   h->ig.reset();
   h->transposed = want;
+  h->rel.tr = want ? 1 : 0;
   return SPK_OK;
 }
 
@@ -2392,10 +2421,10 @@ static int ensure_near_bf(spk_handle *h) {
 // the fp8 copy of the complex64 near blocks (built once per setup)
 static int ensure_near_f8(spk_handle *h) {
   if (!h->near_f8_ok) {
-    HIPCHK(h->d_blk_f8.alloc(h->f_blocks.n / 2));
+    HIPCHK(h->d_blk_f8.alloc((size_t)h->rel.nc * f8_pairs(h->tree.nnz, h->N)));
     HIPCHK(h->d_f8_scale.alloc(4 * (size_t)h->N));
     launch_near_to_f8(h->N, h->d_leafbox_of_pos.p, h->d_box_first.p, h->d_e2_off.p,
-                      h->d_near_off.p, h->f_blocks.p, h->d_blk_f8.p, h->d_f8_scale.p, h->st);
+                      h->d_near_off.p, h->rel, h->f_blocks.p, h->d_blk_f8.p, h->d_f8_scale.p, h->st);
     HIPCHK(hipGetLastError());
     h->near_f8_ok = true;
   }
@@ -2460,7 +2489,7 @@ static int ensure_block_lu(spk_handle *h) {
   HIPCHK(hipMemsetAsync(B.A.p, 0, B.A.n * sizeof(zd), h->st));
   launch_blu_extract(B.ngroups, B.nmax, B.p0.p, B.cnt.p, h->d_perm.p, h->d_pos.p,
                      h->d_leafbox_of_pos.p, h->d_box_first.p, h->d_e2_off.p, h->d_e2_list.p,
-                     h->d_near_off.p, h->d_blocks.p, B.A.p, h->st);
+                     h->d_near_off.p, h->rel, h->d_blocks.p, B.A.p, h->st);
   HIPCHK(hipGetLastError());
   if (!B.rb && rocblas_create_handle(&B.rb) != rocblas_status_success)
     return fail(SPK_ERR_HIP, "rocblas_create_handle failed");
@@ -2763,13 +2792,13 @@ static int fgmres_near(spk_handle *h, int R, const zd *const *b, zd *const *x,
               if (f8) {
                 launch_near_spmv_f8(h->spmv_wgs, h->N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                                     h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                                    h->d_perm.p, f8, h->d_f8_scale.p, ui, wo, h->st);
+                                    h->d_perm.p, h->rel, f8, h->d_f8_scale.p, ui, wo, h->st);
                 continue;
               }
               if (bf) {
                 launch_near_spmv_bf(h->spmv_wgs, h->N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                                     h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                                    h->d_perm.p, bf, ui, wo, h->st);
+                                    h->d_perm.p, h->rel, bf, ui, wo, h->st);
                 continue;
               }
             }
@@ -3001,11 +3030,11 @@ int spk_near_product_lowp(spk_handle *h, int format, int batched, int R, const v
       if (f8)
         launch_near_spmv_f8(h->spmv_wgs, h->N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                             h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                            h->d_perm.p, f8, h->d_f8_scale.p, x, y, h->st);
+                            h->d_perm.p, h->rel, f8, h->d_f8_scale.p, x, y, h->st);
       else if (bf)
         launch_near_spmv_bf(h->spmv_wgs, h->N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                             h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                            h->d_perm.p, bf, x, y, h->st);
+                            h->d_perm.p, h->rel, bf, x, y, h->st);
       else if ((rc = matvec_t<zf>(h, x, y, true, false)))
         return rc;
     }
@@ -3272,7 +3301,7 @@ int spk_gmres_device(spk_handle *h, const void *d_b, void *d_x, const spk_gmres_
   if (prec && !h->diag_ready) {
     HIPCHK(h->d_diag.alloc(n));
     launch_jacobi_diag(h->N, h->d_perm.p, h->d_leafbox_of_pos.p, h->d_box_first.p, h->d_e2_off.p,
-                       h->d_e2_list.p, h->d_near_off.p, h->d_blocks.p, h->d_diag.p, h->st);
+                       h->d_e2_list.p, h->d_near_off.p, h->rel, h->d_blocks.p, h->d_diag.p, h->st);
     HIPCHK(hipGetLastError());
     h->diag_ready = true;
   }
@@ -3858,7 +3887,7 @@ int spk_get_near_csr(const spk_handle *h, int64_t *ia, int32_t *ja, double *abcd
   const Tree &t = h->tree;
   std::vector<zd> blocks;
   if (abcd) {
-    blocks.resize(4 * (size_t)t.nnz);
+    blocks.resize(h->d_blocks.n);
     HIPCHK(hipMemcpy(blocks.data(), h->d_blocks.p, blocks.size() * sizeof(zd), hipMemcpyDeviceToHost));
   }
   int64_t off = 0;
@@ -3869,8 +3898,9 @@ int spk_get_near_csr(const spk_handle *h, int64_t *ia, int32_t *ja, double *abcd
     if (ia) ia[m] = off;
     if (ja) std::memcpy(ja + off, &t.e2_list[t.e2_off[b]], cols * sizeof(int));
     if (abcd) {
-      const zd *src = &blocks[4 * (size_t)(t.near_off[b] + (int64_t)r * cols)];
-      std::memcpy(abcd + 8 * off, src, 4 * (size_t)cols * sizeof(zd));
+      const zd *src = &blocks[h->rel.nc * (size_t)(t.near_off[b] + (int64_t)r * cols)];
+      zd *dst = reinterpret_cast<zd *>(abcd + 8 * off);
+      for (int c = 0; c < cols; ++c) get_block(h->rel, src + h->rel.nc * (size_t)c, dst + 4 * (size_t)c);
     }
     off += cols;
   }
@@ -4024,11 +4054,11 @@ static int profile_near_lp(spk_handle *h, int reps, double *ms, double *bytes, b
     if (f8)
       launch_near_spmv_f8(h->spmv_wgs, h->N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                           h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                          h->d_perm.p, h->d_blk_f8.p, h->d_f8_scale.p, x.p, y.p, h->st);
+                          h->d_perm.p, h->rel, h->d_blk_f8.p, h->d_f8_scale.p, x.p, y.p, h->st);
     else
       launch_near_spmv_bf(h->spmv_wgs, h->N, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                           h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                          h->d_perm.p, h->d_blk_bf.p, x.p, y.p, h->st);
+                          h->d_perm.p, h->rel, h->d_blk_bf.p, x.p, y.p, h->st);
   };
   run();
   HIPCHK(hipEventRecord(e0, h->st));
@@ -4040,9 +4070,9 @@ static int profile_near_lp(spk_handle *h, int reps, double *ms, double *bytes, b
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   *ms = (double)t / reps;
-  const double nblocks = (double)(h->f_blocks.n / 4);
-  *bytes = f8 ? nblocks * 8.0 + 16.0 * (double)h->N + 3.0 * (double)n * 8.0
-              : nblocks * 16.0 + 3.0 * (double)n * 8.0;
+  const double nval = (double)h->f_blocks.n;  // kept components
+  *bytes = f8 ? nval * 2.0 + 16.0 * (double)h->N + 3.0 * (double)n * 8.0
+              : nval * 4.0 + 3.0 * (double)n * 8.0;
   return SPK_OK;
 }
 extern "C" {

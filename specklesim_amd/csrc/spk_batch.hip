@@ -38,14 +38,17 @@ __device__ inline T bshfl_down(T v, int off) {
 // The R input vectors interleaved: XI[(m * 2 + cur) * RP + r] = x_r[m + cur N]
 // (zero for r >= R), so that a column's 2 RP values are one contiguous run.
 // XP: the same in edge-position order, XP[(p * 2 + cur) * RP + r] = x_r[perm[p] + cur N].
+// With transposed near blocks of three components XI carries NearRel's factor.
 template <class T, int RP>
-__global__ void kb_interleave(int N, int R, const int *perm, const T *const *xs, T *XI, T *XP) {
+__global__ void kb_interleave(int N, int R, NearRel rel, const int *perm, const T *const *xs, T *XI,
+                              T *XP) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)2 * N * RP) return;
   const int r = (int)(t % RP);
   const int64_t mc = t / RP;
   const int m = (int)(mc >> 1), cur = (int)(mc & 1);
-  XI[t] = r < R ? xs[r][m + (int64_t)cur * N] : T{0, 0};
+  const T v = r < R ? xs[r][m + (int64_t)cur * N] : T{0, 0};
+  XI[t] = cur && rel.nc == 3 && rel.tr ? rel_scale(v, rel.c) : v;
   XP[t] = r < R ? xs[r][perm[m] + (int64_t)cur * N] : T{0, 0};
 }
 
@@ -708,13 +711,13 @@ __global__ void __launch_bounds__(512) kb_disagg_mx(int N, PatLay lay, int R, co
 // 2x2 blocks of its columns (lanes of the same column share one address) and
 // applies them to its RPL vectors, read from the LDS copy of the box's E2
 // columns.  Rows are reduced over the column lanes at the end.
-template <class T, int RP>
+template <class T, int RP, int NC>
 __global__ void __launch_bounds__(256) kb_near(int N, int R, const int *row_box, const int *row_r0,
                                                const int *box_first, const int *box_count,
                                                const int *e2_off, const int *e2_list,
                                                const int64_t *near_off, const int *perm,
-                                               const T *blocks, const T *XI, const T *yf,
-                                               T *const *ys) {
+                                               NearRel rel, const T *blocks, const T *XI,
+                                               const T *yf, T *const *ys) {
   constexpr int RG = RP >= 8 ? RP / 4 : 1, RPL = RP / RG, CL = 64 / RG;
   constexpr int KC = 32768 / (2 * RP * (int)sizeof(T));  // columns per LDS chunk (32 KB)
   constexpr int NQ = kSpmvRowsPerWG / 4;
@@ -741,9 +744,11 @@ __global__ void __launch_bounds__(256) kb_near(int N, int R, const int *row_box,
     for (int q = 0; q < NQ; ++q) {
       const int row = r0 + wv + 4 * q;
       if (row < r0 + rows) {
-        const T *Z = blocks + 4 * (near_off[b] + (int64_t)row * cols + cc);
+        const T *Z = blocks + NC * (near_off[b] + (int64_t)row * cols + cc);
         for (int c = cl; c < nc; c += CL) {
-          const T z0 = Z[4 * c], z1 = Z[4 * c + 1], z2 = Z[4 * c + 2], z3 = Z[4 * c + 3];
+          const T z0 = Z[NC * c], z1 = Z[NC * c + 1], z3 = Z[NC * c + NC - 1];
+          T z2 = z1;
+          if constexpr (NC == 4) z2 = Z[NC * c + 2];
           const T *xe = xsl + (c * 2 + 0) * RP + rg * RPL, *xh = xsl + (c * 2 + 1) * RP + rg * RPL;
 #pragma unroll
           for (int v = 0; v < RPL; ++v) {
@@ -768,6 +773,7 @@ __global__ void __launch_bounds__(256) kb_near(int N, int R, const int *row_box,
       const int r = rg * RPL + v;
       if (cl == 0 && r < R && row < r0 + rows) {
         const int m = perm[box_first[b] + row];
+        if (NC == 3) sh = rel_scale(sh, rel.out());
         if (yf) {
           se = se + yf[(size_t)r * 2 * N + m];
           sh = sh + yf[(size_t)r * 2 * N + m + N];
@@ -797,13 +803,14 @@ __global__ void __launch_bounds__(256) kb_near(int N, int R, const int *row_box,
 // BF: the blocks are the bf16 copy (one 16-byte load per block, widened to
 // fp32 in registers).
 constexpr int kMxCols = 128;
-template <bool BF>
+template <bool BF, int NC>
 __global__ void __launch_bounds__(256) kb_near_mx(int N, int R, const int *row_box,
                                                   const int *row_r0, const int *box_first,
                                                   const int *box_count, const int *e2_off,
                                                   const int *e2_list, const int64_t *near_off,
-                                                  const int *perm, const void *blocks, const zf *XI,
-                                                  const zf *yf, zf *const *ys) {
+                                                  const int *perm, NearRel rel,
+                                                  const void *blocks, const zf *XI, const zf *yf,
+                                                  zf *const *ys) {
   constexpr int PER = kMxCols * 16 / 256;
   __shared__ float4 xsl[kMxCols * 16];
   const int b = row_box[blockIdx.x];
@@ -814,8 +821,8 @@ __global__ void __launch_bounds__(256) kb_near_mx(int N, int R, const int *row_b
   const int rw = row_r0[blockIdx.x];  // first row of the tile (rw < nrow)
   const int row = min(rw + m, nrow - 1);
   const int64_t roff = near_off[b] + (int64_t)row * cols;  // first block of the row
-  const float4 *Zr = reinterpret_cast<const float4 *>(blocks) + 2 * roff;
-  const uint4 *Zb = reinterpret_cast<const uint4 *>(blocks) + roff;
+  const float2 *Zr = reinterpret_cast<const float2 *>(blocks) + NC * roff;
+  const Words<NC> *Zb = reinterpret_cast<const Words<NC> *>(blocks) + roff;
   mxf4 er = {0.f, 0.f, 0.f, 0.f}, ei = er, hr = er, hi = er;
   float4 za[4], zb[4];
   auto load = [&](int cg, float4 *a, float4 *bb) {
@@ -823,14 +830,21 @@ __global__ void __launch_bounds__(256) kb_near_mx(int N, int R, const int *row_b
     for (int j = 0; j < 4; ++j) {
       const int c = min(cg + 4 * j + g, cols - 1);
       if constexpr (BF) {
-        const uint4 v = Zb[c];
+        const Words<NC> v = Zb[c];
+        uint32_t w2 = v.y;
+        if constexpr (NC == 4) w2 = v.z;
+        const uint32_t w3 = last_word(v);
         a[j] = float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u),
                       __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u)};
-        bb[j] = float4{__uint_as_float(v.z << 16), __uint_as_float(v.z & 0xFFFF0000u),
-                       __uint_as_float(v.w << 16), __uint_as_float(v.w & 0xFFFF0000u)};
+        bb[j] = float4{__uint_as_float(w2 << 16), __uint_as_float(w2 & 0xFFFF0000u),
+                       __uint_as_float(w3 << 16), __uint_as_float(w3 & 0xFFFF0000u)};
+      } else if constexpr (NC == 4) {
+        a[j] = reinterpret_cast<const float4 *>(Zr)[2 * c];
+        bb[j] = reinterpret_cast<const float4 *>(Zr)[2 * c + 1];
       } else {
-        a[j] = Zr[2 * c];
-        bb[j] = Zr[2 * c + 1];
+        const float2 z0 = Zr[3 * c], z1 = Zr[3 * c + 1], z2 = Zr[3 * c + 2];
+        a[j] = float4{z0.x, z0.y, z1.x, z1.y};
+        bb[j] = float4{z1.x, z1.y, z2.x, z2.y};
       }
     }
   };
@@ -917,6 +931,7 @@ __global__ void __launch_bounds__(256) kb_near_mx(int N, int R, const int *row_b
     if (r < nrow) {
       const int mm = perm[pf + r];
       zf se = {er[i], ei[i]}, sh = {hr[i], hi[i]};
+      if (NC == 3) sh = rel_scale(sh, rel.out());
       if (yf) {
         se = se + yf[(size_t)n * 2 * N + mm];
         sh = sh + yf[(size_t)n * 2 * N + mm + N];
@@ -940,12 +955,13 @@ typedef double mxd4 __attribute__((ext_vector_type(4)));
 // near field: workgroup = (box, 16 rows), 4 waves take every fourth group of
 // 16 columns, x staged in LDS 64 columns at a time as (xe, xh) per (column, r)
 constexpr int kMx64Cols = 64;
+template <int NC>
 __global__ void __launch_bounds__(256) kb_near_mx64(int N, int R, const int *row_box,
                                                     const int *row_r0, const int *box_first,
                                                     const int *box_count, const int *e2_off,
                                                     const int *e2_list, const int64_t *near_off,
-                                                    const int *perm, const zd *blocks, const zd *XI,
-                                                    const zd *yf, zd *const *ys) {
+                                                    const int *perm, NearRel rel, const zd *blocks,
+                                                    const zd *XI, const zd *yf, zd *const *ys) {
   constexpr int PER = kMx64Cols * 16 / 256;
   __shared__ double4 xsl[kMx64Cols * 16];
   const int b = row_box[blockIdx.x];
@@ -955,15 +971,15 @@ __global__ void __launch_bounds__(256) kb_near_mx64(int N, int R, const int *row
   const int m = lane & 15, g = lane >> 4;
   const int rw = row_r0[blockIdx.x];
   const int row = min(rw + m, nrow - 1);
-  const double2 *Zr = reinterpret_cast<const double2 *>(blocks) + 4 * (near_off[b] + (int64_t)row * cols);
+  const double2 *Zr = reinterpret_cast<const double2 *>(blocks) + NC * (near_off[b] + (int64_t)row * cols);
   mxd4 er = {0.0, 0.0, 0.0, 0.0}, ei = er, hr = er, hi = er;
-  double2 cur[4][4];
-  auto load = [&](int cg, double2 (*z)[4]) {
+  double2 cur[4][NC];
+  auto load = [&](int cg, double2 (*z)[NC]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int c = min(cg + 4 * j + g, cols - 1);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) z[j][e] = Zr[4 * c + e];
+      for (int e = 0; e < NC; ++e) z[j][e] = Zr[NC * c + e];
     }
   };
   if (cols > 0) load(16 * wv, cur);
@@ -985,13 +1001,13 @@ __global__ void __launch_bounds__(256) kb_near_mx64(int N, int R, const int *row
     }
     __syncthreads();
     for (int off = 16 * wv; off < nc; off += 64) {
-      double2 nx[4][4];
+      double2 nx[4][NC];
       load(cc + off + 64, nx);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const double4 x = xsl[(off + 4 * j + g) * 16 + m];
-        const double2 z0 = cur[j][0], z1 = cur[j][1], z2 = cur[j][2], z3 = cur[j][3];
+        const double2 z0 = cur[j][0], z1 = cur[j][1], z2 = cur[j][NC - 2], z3 = cur[j][NC - 1];
         const double nxi = -x.y, nhi = -x.w;
         er = SPK_MFMA64(z0.x, x.x, er);
         ei = SPK_MFMA64(z0.x, x.y, ei);
@@ -1014,7 +1030,7 @@ __global__ void __launch_bounds__(256) kb_near_mx64(int N, int R, const int *row
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) cur[j][e] = nx[j][e];
+        for (int e = 0; e < NC; ++e) cur[j][e] = nx[j][e];
     }
   }
   __syncthreads();
@@ -1044,6 +1060,7 @@ __global__ void __launch_bounds__(256) kb_near_mx64(int N, int R, const int *row
     if (r < nrow) {
       const int mm = perm[pf + r];
       zd se = {er[i], ei[i]}, sh = {hr[i], hi[i]};
+      if (NC == 3) sh = sh * rel.out();
       if (yf) {
         se = se + yf[(size_t)n * 2 * N + mm];
         sh = sh + yf[(size_t)n * 2 * N + mm + N];
@@ -1334,11 +1351,13 @@ __device__ inline mxs4 as_s4(uint32_t a, uint32_t b) {
   v[3] = (short)(b >> 16);
   return v;
 }
+template <int NC>
 __global__ void __launch_bounds__(256) kb_near_mxb(int N, int R, const int *row_box,
                                                    const int *row_r0, const int *box_first,
                                                    const int *box_count, const int *e2_off,
                                                    const int *e2_list, const int64_t *near_off,
-                                                   const int *perm, const uint4 *blocks, const zf *XI,
+                                                   const int *perm, NearRel rel,
+                                                   const Words<NC> *blocks, const zf *XI,
                                                    zf *const *ys) {
   constexpr int PER = kMxCols * 16 / 256;
   __shared__ uint4 xsl[kMxCols * 16];
@@ -1349,10 +1368,10 @@ __global__ void __launch_bounds__(256) kb_near_mxb(int N, int R, const int *row_
   const int m = lane & 15, g = lane >> 4;
   const int rw = row_r0[blockIdx.x];
   const int row = min(rw + m, nrow - 1);
-  const uint4 *Zr = blocks + near_off[b] + (int64_t)row * cols;
+  const Words<NC> *Zr = blocks + near_off[b] + (int64_t)row * cols;
   mxf4 er = {0.f, 0.f, 0.f, 0.f}, ei = er, hr = er, hi = er;
-  uint4 cur[4];
-  auto load = [&](int cg, uint4 *z) {
+  Words<NC> cur[4];
+  auto load = [&](int cg, Words<NC> *z) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) z[j] = Zr[min(cg + 4 * j + g, cols - 1)];
   };
@@ -1377,14 +1396,19 @@ __global__ void __launch_bounds__(256) kb_near_mxb(int N, int R, const int *row_
     }
     __syncthreads();
     for (int off = 16 * wv; off < nc; off += 64) {
-      uint4 nx[4];
+      Words<NC> nx[4];
       load(cc + off + 64, nx);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint4 x = xsl[(off + 4 * j + g) * 16 + m];
         const mxs4 be = as_s4(x.x, x.y), bi = as_s4(x.z, x.w);
-        const mxs4 ae = as_s4(cur[j].x, cur[j].y), ah = as_s4(cur[j].z, cur[j].w);
+        const mxs4 ae = as_s4(cur[j].x, cur[j].y);
+        mxs4 ah;
+        if constexpr (NC == 3)
+          ah = as_s4(cur[j].y, cur[j].z);
+        else
+          ah = as_s4(cur[j].z, cur[j].w);
         er = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ae, be, er, 0, 0, 0);
         ei = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ae, bi, ei, 0, 0, 0);
         hr = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, be, hr, 0, 0, 0);
@@ -1423,35 +1447,36 @@ __global__ void __launch_bounds__(256) kb_near_mxb(int N, int R, const int *row_
     if (r < nrow) {
       const int mm = perm[pf + r];
       ys[n][mm] = zf{er[i], ei[i]};
-      ys[n][mm + N] = zf{hr[i], hi[i]};
+      const zf sh = {hr[i], hi[i]};
+      ys[n][mm + N] = NC == 3 ? rel_scale(sh, rel.out()) : sh;
     }
   }
 }
 
-// The same product on the fp8 copy of the blocks (E4M3FN, 8 bytes per 2x2
-// block, per-row component scales).  The scales differ per component, so each
-// component gets its own accumulators: one product covers 8 columns of one
-// component, k = 2 * column + (re, im); lane g * 16 + m holds A = (Zc_r, Zc_i)
-// of row m at columns 2g and 2g + 1 of the 8 (decoded by v_cvt_pk_f32_fp8;
+// The same product on the fp8 copy of the blocks (E4M3FN, 2 bytes per kept
+// component, pairs of columns, per-row component scales).  The scales differ
+// per component, so each product with a component gets its own accumulators:
+// one product covers 8 columns of one component, k = 2 * column + (re, im);
+// lane g * 16 + m holds A = (Zc_r, Zc_i) of row m at columns 2g and 2g + 1 of
+// the 8, one dword of the copy (decoded by v_cvt_pk_f32_fp8;
 // an fp8 value has 3 mantissa bits, so its fp32 form is exactly bf16 and the
 // high halves are the operand) and B = the staged x words of those columns.
 // The row's scales multiply the component sums before the waves' sums are
 // added.  A workgroup covers RT row tiles of 16 rows (one x staging for all).
-template <bool HI>
-__device__ inline mxs4 fp8_comp_pair(uint32_t w0, uint32_t w1) {
-  const auto a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w0, HI);
-  const auto b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w1, HI);
+__device__ inline mxs4 fp8_pair(uint32_t w) {
+  const auto a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
+  const auto b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
   return as_s4((__float_as_uint(a[0]) >> 16) | (__float_as_uint(a[1]) & 0xFFFF0000u),
                (__float_as_uint(b[0]) >> 16) | (__float_as_uint(b[1]) & 0xFFFF0000u));
 }
-template <int RT>
+template <int RT, int NC>
 __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row_box,
                                                     const int *row_r0, const int *box_first,
                                                     const int *box_count, const int *e2_off,
                                                     const int *e2_list, const int64_t *near_off,
-                                                    const int *perm, const uint2 *blocks,
-                                                    const float4 *scale, const uint32_t *XB,
-                                                    zf *const *ys) {
+                                                    const int *perm, NearRel rel,
+                                                    const Words<NC> *blocks, const float4 *scale,
+                                                    const uint32_t *XB, zf *const *ys) {
   constexpr int PER = kMxCols * 16 / 256;
   __shared__ uint4 xsl[kMxCols * 16];
   const int b = row_box[blockIdx.x];
@@ -1460,22 +1485,24 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
   const int rw = row_r0[blockIdx.x];
-  const uint2 *Zr[RT];
+  const int pairs = (cols + 1) / 2;
+  const Words<NC> *Zr[RT];
 #pragma unroll
-  for (int t = 0; t < RT; ++t) Zr[t] = blocks + near_off[b] + (int64_t)min(rw + 16 * t + m, nrow - 1) * cols;
+  for (int t = 0; t < RT; ++t)
+    Zr[t] = blocks + f8_pairs(near_off[b], pf) + (int64_t)min(rw + 16 * t + m, nrow - 1) * pairs;
   // acc[t][c][0] real, acc[t][c][1] imaginary part of component c's sum, row tile t
   mxf4 acc[RT][4][2];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[t][c][0] = acc[t][c][1] = mxf4{0.f, 0.f, 0.f, 0.f};
-  // a lane's blocks of one 16-column step: columns cg + 8 jj + 2g + u
-  uint2 cur[RT][4];
-  auto load = [&](int cg, uint2 (*z)[4]) {
+  // a lane's pairs of one 16-column step: columns cg + 8 jj + 2g, + 1
+  Words<NC> cur[RT][2];
+  auto load = [&](int cg, Words<NC> (*z)[2]) {
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) z[t][j] = Zr[t][min(cg + 8 * (j >> 1) + 2 * g + (j & 1), cols - 1)];
+      for (int j = 0; j < 2; ++j) z[t][j] = Zr[t][min(cg / 2 + 4 * j + g, pairs - 1)];
   };
   if (cols > 0) load(16 * wv, cur);
   for (int cc = 0; cc < cols; cc += kMxCols) {
@@ -1500,7 +1527,7 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
     }
     __syncthreads();
     for (int off = 16 * wv; off < nc; off += 64) {
-      uint2 nx[RT][4];
+      Words<NC> nx[RT][2];
       load(cc + off + 64, nx);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1511,9 +1538,10 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
         const mxs4 bei = as_s4(x0.z, x1.z), bhi = as_s4(x0.w, x1.w);
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
-          const uint2 z0 = cur[t][2 * jj], z1 = cur[t][2 * jj + 1];
-          const mxs4 a0 = fp8_comp_pair<false>(z0.x, z1.x), a1 = fp8_comp_pair<true>(z0.x, z1.x);
-          const mxs4 a2 = fp8_comp_pair<false>(z0.y, z1.y), a3 = fp8_comp_pair<true>(z0.y, z1.y);
+          const Words<NC> z = cur[t][jj];
+          const mxs4 a0 = fp8_pair(z.x), a1 = fp8_pair(z.y), a3 = fp8_pair(last_word(z));
+          mxs4 a2 = a1;
+          if constexpr (NC == 4) a2 = fp8_pair(z.z);
           mxf4(&A)[4][2] = acc[t];
           A[0][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, ber, A[0][0], 0, 0, 0);
           A[0][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, bei, A[0][1], 0, 0, 0);
@@ -1529,7 +1557,7 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
 #pragma unroll
       for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) cur[t][j] = nx[t][j];
+        for (int j = 0; j < 2; ++j) cur[t][j] = nx[t][j];
     }
   }
   // element i of this lane in tile t is output row rw + 16t + 4g + i: scale,
@@ -1544,8 +1572,9 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
       const float4 sc = scale[pf + r];
       er[i] = sc.x * acc[t][0][0][i] + sc.y * acc[t][1][0][i];
       ei[i] = sc.x * acc[t][0][1][i] + sc.y * acc[t][1][1][i];
-      hr[i] = sc.z * acc[t][2][0][i] + sc.w * acc[t][3][0][i];
-      hi[i] = sc.z * acc[t][2][1][i] + sc.w * acc[t][3][1][i];
+      const float s2 = NC == 3 ? sc.y : sc.z, s3 = NC == 3 ? sc.z : sc.w;
+      hr[i] = s2 * acc[t][2][0][i] + s3 * acc[t][3][0][i];
+      hi[i] = s2 * acc[t][2][1][i] + s3 * acc[t][3][1][i];
     }
     __syncthreads();
     if (wv > 0) {
@@ -1573,7 +1602,8 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
           if (r < nrow) {
             const int mm = perm[pf + r];
             ys[n][mm] = zf{er[i], ei[i]};
-            ys[n][mm + N] = zf{hr[i], hi[i]};
+            const zf sh = {hr[i], hi[i]};
+            ys[n][mm + N] = NC == 3 ? rel_scale(sh, rel.out()) : sh;
           }
         }
       }
@@ -1588,14 +1618,14 @@ __global__ void __launch_bounds__(256) kb_near_mxf8(int N, int R, const int *row
 // per workgroup; TPW = 4 stages x once for 64 rows but leaves a quarter of
 // the workgroups.  Waves without rows (a box's last group) take part in the
 // staging only.
-template <int TPW>
+template <int TPW, int NC>
 __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *grp_box,
                                                      const int *grp_r0, const int *box_first,
                                                      const int *box_count, const int *e2_off,
                                                      const int *e2_list, const int64_t *near_off,
-                                                     const int *perm, const uint2 *blocks,
-                                                     const float4 *scale, const uint32_t *XB,
-                                                     zf *const *ys) {
+                                                     const int *perm, NearRel rel,
+                                                     const Words<NC> *blocks, const float4 *scale,
+                                                     const uint32_t *XB, zf *const *ys) {
   constexpr int CS = 4 / TPW;
   constexpr int PER = kMxCols * 16 / 256;
   __shared__ uint4 xsl[kMxCols * 16];
@@ -1607,16 +1637,17 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
   const int m = lane & 15, g = lane >> 4;
   const int rw = grp_r0[blockIdx.x] + 16 * tile;
   const bool active = rw < nrow;
-  const uint2 *Zr = blocks + near_off[b] + (int64_t)min(rw + m, nrow - 1) * cols;
+  const int pairs = (cols + 1) / 2;
+  const Words<NC> *Zr = blocks + f8_pairs(near_off[b], pf) + (int64_t)min(rw + m, nrow - 1) * pairs;
   // acc[c][0] real, acc[c][1] imaginary part of component c's sum
   mxf4 acc[4][2];
 #pragma unroll
   for (int c = 0; c < 4; ++c) acc[c][0] = acc[c][1] = mxf4{0.f, 0.f, 0.f, 0.f};
-  // a lane's blocks of one 16-column step: columns cg + 8 jj + 2g + u
-  uint2 cur[4];
-  auto load = [&](int cg, uint2 *z) {
+  // a lane's pairs of one 16-column step: columns cg + 8 jj + 2g, + 1
+  Words<NC> cur[2];
+  auto load = [&](int cg, Words<NC> *z) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) z[j] = Zr[min(cg + 8 * (j >> 1) + 2 * g + (j & 1), cols - 1)];
+    for (int j = 0; j < 2; ++j) z[j] = Zr[min(cg / 2 + 4 * j + g, pairs - 1)];
   };
   if (active && cols > 0) load(16 * split, cur);
   for (int cc = 0; cc < cols; cc += kMxCols) {
@@ -1640,7 +1671,7 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
     __syncthreads();
     if (active) {
       for (int off = 16 * split; off < nc; off += 16 * CS) {
-        uint2 nx[4];
+        Words<NC> nx[2];
         load(cc + off + 16 * CS, nx);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1649,9 +1680,10 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
           const uint4 x0 = xsl[col * 16 + m], x1 = xsl[(col + 1) * 16 + m];
           const mxs4 ber = as_s4(x0.x, x1.x), bhr = as_s4(x0.y, x1.y);
           const mxs4 bei = as_s4(x0.z, x1.z), bhi = as_s4(x0.w, x1.w);
-          const uint2 z0 = cur[2 * jj], z1 = cur[2 * jj + 1];
-          const mxs4 a0 = fp8_comp_pair<false>(z0.x, z1.x), a1 = fp8_comp_pair<true>(z0.x, z1.x);
-          const mxs4 a2 = fp8_comp_pair<false>(z0.y, z1.y), a3 = fp8_comp_pair<true>(z0.y, z1.y);
+          const Words<NC> z = cur[jj];
+          const mxs4 a0 = fp8_pair(z.x), a1 = fp8_pair(z.y), a3 = fp8_pair(last_word(z));
+          mxs4 a2 = a1;
+          if constexpr (NC == 4) a2 = fp8_pair(z.z);
           acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, ber, acc[0][0], 0, 0, 0);
           acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, bei, acc[0][1], 0, 0, 0);
           acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, bhr, acc[1][0], 0, 0, 0);
@@ -1663,7 +1695,7 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) cur[j] = nx[j];
+        for (int j = 0; j < 2; ++j) cur[j] = nx[j];
       }
     }
   }
@@ -1676,8 +1708,9 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
     const float4 sc = scale[pf + r];
     er[i] = sc.x * acc[0][0][i] + sc.y * acc[1][0][i];
     ei[i] = sc.x * acc[0][1][i] + sc.y * acc[1][1][i];
-    hr[i] = sc.z * acc[2][0][i] + sc.w * acc[3][0][i];
-    hi[i] = sc.z * acc[2][1][i] + sc.w * acc[3][1][i];
+    const float s2 = NC == 3 ? sc.y : sc.z, s3 = NC == 3 ? sc.z : sc.w;
+    hr[i] = s2 * acc[2][0][i] + s3 * acc[3][0][i];
+    hi[i] = s2 * acc[2][1][i] + s3 * acc[3][1][i];
   }
   if constexpr (CS > 1) {
     mxf4 *red = reinterpret_cast<mxf4 *>(xsl);
@@ -1709,7 +1742,8 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
     if (r < nrow) {
       const int mm = perm[pf + r];
       ys[n][mm] = zf{er[i], ei[i]};
-      ys[n][mm + N] = zf{hr[i], hi[i]};
+      const zf sh = {hr[i], hi[i]};
+      ys[n][mm + N] = NC == 3 ? rel_scale(sh, rel.out()) : sh;
     }
   }
 }
@@ -1724,29 +1758,41 @@ __global__ void __launch_bounds__(256) kb_x_to_bf(int64_t len, const zf *XI, uin
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < len) XB[i] = bf16_pair(XI[i].x, XI[i].y);
 }
+template <int NC>
+static void batch_near_f8(int nwg, int N, int R, const int *row_box, const int *row_r0, int ngrp,
+                          const int *grp_box, const int *grp_r0, const int *box_first,
+                          const int *box_count, const int *e2_off, const int *e2_list,
+                          const int64_t *near_off, const int *perm, const NearRel &rel,
+                          const uint32_t *blocks, const float *scale, const uint32_t *XB,
+                          zf *const *ys, int tpw, hipStream_t st) {
+  const auto *Z = (const Words<NC> *)blocks;
+  // tpw row tiles per workgroup (grp_box / grp_r0 are the map of groups of
+  // tpw 16-row tiles); 1 runs the original kernel on the 16-row tile map
+  if (tpw == 1 || ngrp <= 0)
+    hipLaunchKernelGGL((kb_near_mxf8<1, NC>), dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel, Z,
+                       (const float4 *)scale, XB, ys);
+  else if (tpw == 2)
+    hipLaunchKernelGGL((kb_near_mxf8g<2, NC>), dim3(ngrp), dim3(256), 0, st, N, R, grp_box, grp_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel, Z,
+                       (const float4 *)scale, XB, ys);
+  else
+    hipLaunchKernelGGL((kb_near_mxf8g<4, NC>), dim3(ngrp), dim3(256), 0, st, N, R, grp_box, grp_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel, Z,
+                       (const float4 *)scale, XB, ys);
+}
 void launch_batch_near_f8(int nwg, int N, int R, const int *row_box, const int *row_r0,
                           int ngrp, const int *grp_box, const int *grp_r0,
                           const int *box_first, const int *box_count, const int *e2_off,
                           const int *e2_list, const int64_t *near_off, const int *perm,
-                          const uint32_t *blocks, const float *scale, const zf *XI,
-                          uint32_t *XB, zf *const *ys, int tpw, hipStream_t st) {
+                          const NearRel &rel, const uint32_t *blocks, const float *scale,
+                          const zf *XI, uint32_t *XB, zf *const *ys, int tpw, hipStream_t st) {
   if (nwg <= 0) return;
   const int64_t len = (int64_t)N * 2 * 16;
   hipLaunchKernelGGL(kb_x_to_bf, dim3(bnblk(len, 256)), dim3(256), 0, st, len, XI, XB);
-  // tpw row tiles per workgroup (grp_box / grp_r0 are the map of groups of
-  // tpw 16-row tiles); 1 runs the original kernel on the 16-row tile map
-  if (tpw == 1 || ngrp <= 0)
-    hipLaunchKernelGGL(kb_near_mxf8<1>, dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,
-                       box_first, box_count, e2_off, e2_list, near_off, perm, (const uint2 *)blocks,
-                       (const float4 *)scale, (const uint32_t *)XB, ys);
-  else if (tpw == 2)
-    hipLaunchKernelGGL(kb_near_mxf8g<2>, dim3(ngrp), dim3(256), 0, st, N, R, grp_box, grp_r0,
-                       box_first, box_count, e2_off, e2_list, near_off, perm, (const uint2 *)blocks,
-                       (const float4 *)scale, (const uint32_t *)XB, ys);
-  else
-    hipLaunchKernelGGL(kb_near_mxf8g<4>, dim3(ngrp), dim3(256), 0, st, N, R, grp_box, grp_r0,
-                       box_first, box_count, e2_off, e2_list, near_off, perm, (const uint2 *)blocks,
-                       (const float4 *)scale, (const uint32_t *)XB, ys);
+  auto *f = rel.nc == 3 ? batch_near_f8<3> : batch_near_f8<4>;
+  f(nwg, N, R, row_box, row_r0, ngrp, grp_box, grp_r0, box_first, box_count, e2_off, e2_list,
+    near_off, perm, rel, blocks, scale, XB, ys, tpw, st);
 }
 
 // Row tiles per workgroup of the batched fp8 near product: 1 by default,
@@ -2044,14 +2090,15 @@ void launch_arnoldi_cgs(int64_t n, int P, int j, int kin, T *U, size_t ldu, T *W
 }
 
 template <class T>
-void launch_batch_interleave(int N, int R, const int *perm, const T *const *xs, T *XI, T *XP,
-                             hipStream_t st) {
+void launch_batch_interleave(int N, int R, const NearRel &rel, const int *perm,
+                             const T *const *xs, T *XI, T *XP, hipStream_t st) {
   const int RP = batch_pad(R);
   const unsigned g = bnblk((int64_t)2 * N * RP, 256);
   switch (RP) {
 #define SPK_IL_CASE(P)                                                                          \
   case P:                                                                                       \
-    hipLaunchKernelGGL((kb_interleave<T, P>), dim3(g), dim3(256), 0, st, N, R, perm, xs, XI, XP); \
+    hipLaunchKernelGGL((kb_interleave<T, P>), dim3(g), dim3(256), 0, st, N, R, rel, perm, xs, XI, \
+                       XP);                                                                     \
     break;
     SPK_IL_CASE(1) SPK_IL_CASE(2) SPK_IL_CASE(4) SPK_IL_CASE(8) SPK_IL_CASE(16)
 #undef SPK_IL_CASE
@@ -2180,33 +2227,33 @@ void launch_batch_disagg(int ntiles, int N, const PatLay &lay, int R, const int 
   hipLaunchKernelGGL(kb_sum_split<T>, dim3(bnblk(len, 256)), dim3(256), 0, st, len, (const T *)yp,
                      yf);
 }
-template <class T>
-void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row_r0,
+template <class T, int NC>
+static void batch_near(int nwg, int N, int R, const int *row_box, const int *row_r0,
                        const int *box_first, const int *box_count, const int *e2_off,
                        const int *e2_list, const int64_t *near_off, const int *perm,
-                       const T *blocks, const T *XI, const T *yf, T *const *ys,
+                       const NearRel &rel, const T *blocks, const T *XI, const T *yf, T *const *ys,
                        hipStream_t st, const uint32_t *blocks_bf) {
-  if (nwg <= 0) return;
+  const dim3 grid(nwg), wg(256);
   if constexpr (std::is_same<T, zd>::value) {
     if (batch_pad(R) == 16) {
-      hipLaunchKernelGGL(kb_near_mx64, dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,
-                         box_first, box_count, e2_off, e2_list, near_off, perm, blocks, XI, yf, ys);
+      hipLaunchKernelGGL(kb_near_mx64<NC>, grid, wg, 0, st, N, R, row_box, row_r0, box_first,
+                         box_count, e2_off, e2_list, near_off, perm, rel, blocks, XI, yf, ys);
       return;
     }
   }
   if constexpr (std::is_same<T, zf>::value) {
     if (batch_pad(R) == 16) {
       if (blocks_bf && !yf)  // the preconditioner's product: bf16 operands throughout
-        hipLaunchKernelGGL(kb_near_mxb, dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,
-                           box_first, box_count, e2_off, e2_list, near_off, perm,
-                           (const uint4 *)blocks_bf, XI, ys);
+        hipLaunchKernelGGL(kb_near_mxb<NC>, grid, wg, 0, st, N, R, row_box, row_r0, box_first,
+                           box_count, e2_off, e2_list, near_off, perm, rel,
+                           (const Words<NC> *)blocks_bf, XI, ys);
       else if (blocks_bf)
-        hipLaunchKernelGGL(kb_near_mx<true>, dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,
-                           box_first, box_count, e2_off, e2_list, near_off, perm,
+        hipLaunchKernelGGL((kb_near_mx<true, NC>), grid, wg, 0, st, N, R, row_box, row_r0,
+                           box_first, box_count, e2_off, e2_list, near_off, perm, rel,
                            (const void *)blocks_bf, XI, yf, ys);
       else
-        hipLaunchKernelGGL(kb_near_mx<false>, dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,
-                           box_first, box_count, e2_off, e2_list, near_off, perm,
+        hipLaunchKernelGGL((kb_near_mx<false, NC>), grid, wg, 0, st, N, R, row_box, row_r0,
+                           box_first, box_count, e2_off, e2_list, near_off, perm, rel,
                            (const void *)blocks, XI, yf, ys);
       return;
     }
@@ -2214,18 +2261,28 @@ void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row
   switch (batch_pad(R)) {
 #define SPK_NEAR_CASE(RP)                                                                       \
   case RP:                                                                                      \
-    hipLaunchKernelGGL((kb_near<T, RP>), dim3(nwg), dim3(256), 0, st, N, R, row_box, row_r0,    \
-                       box_first, box_count, e2_off, e2_list, near_off, perm, blocks, XI, yf,    \
-                       ys);                                                                     \
+    hipLaunchKernelGGL((kb_near<T, RP, NC>), grid, wg, 0, st, N, R, row_box, row_r0, box_first, \
+                       box_count, e2_off, e2_list, near_off, perm, rel, blocks, XI, yf, ys);    \
     break;
-    SPK_NEAR_CASE(1) SPK_NEAR_CASE(2) SPK_NEAR_CASE(4) SPK_NEAR_CASE(8) SPK_NEAR_CASE(16)
+    SPK_NEAR_CASE(1) SPK_NEAR_CASE(2) SPK_NEAR_CASE(4) SPK_NEAR_CASE(8)
 #undef SPK_NEAR_CASE
   }
 }
+template <class T>
+void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row_r0,
+                       const int *box_first, const int *box_count, const int *e2_off,
+                       const int *e2_list, const int64_t *near_off, const int *perm,
+                       const NearRel &rel, const T *blocks, const T *XI, const T *yf, T *const *ys,
+                       hipStream_t st, const uint32_t *blocks_bf) {
+  if (nwg <= 0) return;
+  auto *f = rel.nc == 3 ? batch_near<T, 3> : batch_near<T, 4>;
+  f(nwg, N, R, row_box, row_r0, box_first, box_count, e2_off, e2_list, near_off, perm, rel, blocks,
+    XI, yf, ys, st, blocks_bf);
+}
 
 #define SPK_BATCH_INSTANTIATE(T)                                                                  \
-  template void launch_batch_interleave<T>(int, int, const int *, const T *const *, T *, T *,     \
-                                           hipStream_t);                                          \
+  template void launch_batch_interleave<T>(int, int, const NearRel &, const int *,                \
+                                           const T *const *, T *, T *, hipStream_t);              \
   template void launch_batch_agg<T>(int, const PatLay &, int, int, const int *, const int *, const int *,     \
                                     const T *, const T *, const T *, T *, hipStream_t);            \
   template void launch_batch_ss<T>(int, int, int, const int *, const T *, const T *, T *,          \
@@ -2241,8 +2298,8 @@ void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row
                                        T *, T *, int, const int *, const int *, hipStream_t);      \
   template void launch_batch_near<T>(int, int, int, const int *, const int *, const int *,         \
                                      const int *, const int *, const int *, const int64_t *,       \
-                                     const int *, const T *, const T *, const T *, T *const *,     \
-                                     hipStream_t, const uint32_t *);
+                                     const int *, const NearRel &, const T *, const T *,           \
+                                     const T *, T *const *, hipStream_t, const uint32_t *);
 SPK_BATCH_INSTANTIATE(zd)
 SPK_BATCH_INSTANTIATE(zf)
 template void launch_batch_orth<zf>(int64_t, int, int, const int *, const zf *const *, zf *const *,

@@ -75,6 +75,53 @@ struct NearArgs {
   double qa12[12], qb12[12], qw12[12];
 };
 
+// The components a near block keeps.  Where K enters as the sum of both media,
+// D21 = c D12 with one constant c for the whole matrix: such blocks keep
+// (D11, D12, D22 / c), nc = 3, and the near operator is
+//   diag(1, c) B,  B = [D11 D12; D12 D22 / c]
+// so the product scales its second half by c once per row.  Transposing
+// permutes B and leaves it in the same form; the factor moves to the input:
+// B^T diag(1, c).  Other formulations keep all four components.
+struct NearRel {
+  int nc = 4;
+  zd c = {1.0, 0.0}, ic = {1.0, 0.0};  // c and 1 / c
+  int tr = 0;                          // the transposed blocks
+  __host__ __device__ zd out() const { return tr ? zd{1.0, 0.0} : c; }
+};
+// the four components of a stored block
+__host__ __device__ inline void get_block(const NearRel &rel, const zd *z, zd *D) {
+  D[0] = z[0];
+  D[1] = z[1];
+  if (rel.nc == 3) {
+    D[2] = z[1] * rel.c;
+    D[3] = z[2] * rel.c;
+    if (rel.tr) {  // B^T diag(1, c): the factor is the second column's
+      D[1] = D[2];
+      D[2] = z[1];
+    }
+  } else {
+    D[2] = z[2];
+    D[3] = z[3];
+  }
+}
+// the second half's factor, in FP64
+template <class T>
+__host__ __device__ inline T rel_scale(T v, zd c) {
+  const zd r = zd{(double)v.x, (double)v.y} * c;
+  using F = decltype(v.x);
+  return T{(F)r.x, (F)r.y};
+}
+// NC dwords: a bf16 block or a pair of columns in fp8
+template <int NC>
+using Words = std::conditional_t<NC == 3, uint3, uint4>;
+__device__ inline uint32_t last_word(uint3 v) { return v.z; }
+__device__ inline uint32_t last_word(uint4 v) { return v.w; }
+// first pair of columns of a leaf box in the fp8 copy: its rows are padded to
+// an even number of columns, which at most adds one column per row
+__host__ __device__ inline int64_t f8_pairs(int64_t near_off, int64_t box_first) {
+  return (near_off + box_first + 1) / 2;
+}
+
 struct NearTask {
   int64_t g;  // block index
   int p;      // triangle pair (t-1)*2+(s-1)
@@ -89,8 +136,8 @@ void launch_near_emit(const NearArgs &a, int64_t nnz, const uint8_t *cls, const 
 void launch_near_edge(const NearArgs &a, int ntask, const NearTask *tb, zd *kt, hipStream_t st);
 void launch_near_singular(const NearArgs &a, int ntask, const NearTask *ta, const uint8_t *cls,
                           const int *base_b, const zd *kt, zd *zz, hipStream_t st);
-void launch_near_regular(const NearArgs &a, int64_t nnz, const uint8_t *cls, const int *base_a,
-                         const zd *zz, zd *blocks, hipStream_t st);
+void launch_near_regular(const NearArgs &a, const NearRel &rel, int64_t nnz, const uint8_t *cls,
+                         const int *base_a, const zd *zz, zd *blocks, hipStream_t st);
 // The three-point rule (quadrature_tri, single-precision abscissae) in the
 // frame (corner 0, e1, e2) of a triangle, point i near corner i.  Side p (free
 // vertex: corner p) has its point i at lb + dl[p][i] and at mu[p][i] from its
@@ -136,7 +183,7 @@ struct TriForm {
   zd c[6];
 };
 constexpr int kTriCols = 1024;  // columns per LDS chunk
-void launch_near_tri(const NearArgs &a, const TriForm &q, int N, int tiles, const int *row_box,
+void launch_near_tri(const NearArgs &a, const TriForm &q, const NearRel &rel, int N, int tiles, const int *row_box,
                      const int *row_r0, const int *tri_side, int4 *list, int *cnt,
                      const uint8_t *cls, const int *base_a, const zd *zz, zd *blocks,
                      hipStream_t st);
@@ -199,8 +246,8 @@ void launch_scale_halves(int N, zd sc1, zd sc2, const T *x, T *out, hipStream_t 
 template <class T>
 void launch_near_transpose(int nbl, int max_rows, const int *box_first, const int *box_count,
                            const int *e2_off, const int *e2_list, const int64_t *near_off,
-                           const int *perm, const int *pos, const int *leaf_box, const T *in,
-                           T *out, hipStream_t st);
+                           const int *perm, const int *pos, const int *leaf_box, int nc,
+                           const T *in, T *out, hipStream_t st);
 template <class T>
 void launch_ss(int nb, int S, const int *child, const T *Cc, const T *up, T *P, hipStream_t st);
 template <class T>
@@ -228,7 +275,8 @@ template <class T>
 void launch_near_spmv_rows(int nwg, int N, const int *row_box, const int *row_r0,
                            const int *box_first, const int *box_count, const int *e2_off,
                            const int *e2_list, const int64_t *near_off, const int *perm,
-                           const T *blocks, const T *x, const T *yadd, T *y, hipStream_t st);
+                           const NearRel &rel, const T *blocks, const T *x, const T *yadd, T *y,
+                           hipStream_t st);
 void launch_to_zf(int64_t n, const zd *a, zf *b, hipStream_t st);
 // TL table of one level from the host's per-slot series factors
 void launch_tl_level(int S, int K, const double *khat, const double *trf, const double *rhat,
@@ -330,7 +378,7 @@ void launch_adj_field(const AdjArgs &G, const ScatArgs &a, const double *r, cons
 // Jacobi preconditioner: diag = [Z_mm(1,1); Z_mm(2,2)] (reference order), y = x / diag
 void launch_jacobi_diag(int N, const int *perm, const int *leaf_box_of_pos, const int *box_first,
                         const int *e2_off, const int *e2_list, const int64_t *near_off,
-                        const zd *blocks, zd *diag, hipStream_t st);
+                        const NearRel &rel, const zd *blocks, zd *diag, hipStream_t st);
 void launch_div_diag(int64_t n, const zd *diag, const zd *x, zd *y, hipStream_t st);
 
 // BLAS-1 (deterministic reductions)
@@ -374,8 +422,8 @@ size_t gemv_n_partial_elems(int64_t n, int kmax);
 // XI[(m * 2 + cur) * RP + r] = xs[r][m + cur N], RP = R rounded up to a power of two
 // and XP[(p * 2 + cur) * RP + r] = xs[r][perm[p] + cur N] (edge-position order)
 template <class T>
-void launch_batch_interleave(int N, int R, const int *perm, const T *const *xs, T *XI, T *XP,
-                             hipStream_t st);
+void launch_batch_interleave(int N, int R, const NearRel &rel, const int *perm,
+                             const T *const *xs, T *XI, T *XP, hipStream_t st);
 template <class T>
 void launch_batch_agg(int nbl, const PatLay &lay, int N, int R, const int *box_first,
                       const int *box_count, const int *perm, const T *rt, const T *XI, const T *XP,
@@ -407,8 +455,8 @@ template <class T>
 void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row_r0,
                        const int *box_first, const int *box_count, const int *e2_off,
                        const int *e2_list, const int64_t *near_off, const int *perm,
-                       const T *blocks, const T *XI, const T *yf, T *const *ys,
-                       hipStream_t st, const uint32_t *blocks_bf = nullptr);
+                       const NearRel &rel, const T *blocks, const T *XI, const T *yf,
+                       T *const *ys, hipStream_t st, const uint32_t *blocks_bf = nullptr);
 // the near-field preconditioner's product for 9..16 right-hand sides (XI as
 // launch_batch_interleave writes it; XB: scratch of N * 32 words for x in
 // bf16) on the fp8 copy of the blocks, on the matrix cores; workgroups = the
@@ -427,8 +475,8 @@ void launch_batch_near_f8(int nwg, int N, int R, const int *row_box, const int *
                           int ngrp, const int *grp_box, const int *grp_r0,
                           const int *box_first, const int *box_count, const int *e2_off,
                           const int *e2_list, const int64_t *near_off, const int *perm,
-                          const uint32_t *blocks, const float *scale, const zf *XI,
-                          uint32_t *XB, zf *const *ys, int tpw, hipStream_t st);
+                          const NearRel &rel, const uint32_t *blocks, const float *scale,
+                          const zf *XI, uint32_t *XB, zf *const *ys, int tpw, hipStream_t st);
 
 // one ICGS pass over P bases (coefficients into hs[r][0..ks[r]), |w_r|^2
 // into hs[r][ks[r]]); partial: batch_orth_partial_elems(n, P, maxk)
@@ -443,19 +491,20 @@ void launch_to_bf(int64_t n, const zf *a, uint32_t *b, hipStream_t st);
 void launch_near_spmv_bf(int nwg, int N, const int *row_box, const int *row_r0,
                          const int *box_first, const int *box_count, const int *e2_off,
                          const int *e2_list, const int64_t *near_off, const int *perm,
-                         const uint32_t *blocks, const zf *x, zf *y, hipStream_t st);
-// the near field in fp8 (OCP E4M3FN) for the single-vector preconditioner:
-// 8 bytes per 2x2 block (Z0r, Z0i, Z1r, Z1i, Z2r, Z2i, Z3r, Z3i), scale[4 p + k]
-// = the scale of component k of the row at position p (its largest |re|,
-// |im| maps to 448); one workgroup per row position
+                         const NearRel &rel, const uint32_t *blocks, const zf *x, zf *y,
+                         hipStream_t st);
+// the near field in fp8 (OCP E4M3FN) for the preconditioner: 2 bytes per kept
+// component (NearRel), columns in pairs from pair f8_pairs of a box on,
+// scale[4 p + k] = the scale of component k of the row at position p (its
+// largest |re|, |im| maps to 448); one workgroup per row position
 void launch_near_to_f8(int N, const int *leaf_box_of_pos, const int *box_first, const int *e2_off,
-                       const int64_t *near_off, const zf *blocks, uint32_t *out, float *scale,
-                       hipStream_t st);
+                       const int64_t *near_off, const NearRel &rel, const zf *blocks, uint32_t *out,
+                       float *scale, hipStream_t st);
 void launch_near_spmv_f8(int nwg, int N, const int *row_box, const int *row_r0,
                          const int *box_first, const int *box_count, const int *e2_off,
                          const int *e2_list, const int64_t *near_off, const int *perm,
-                         const uint32_t *blocks, const float *scale, const zf *x, zf *y,
-                         hipStream_t st);
+                         const NearRel &rel, const uint32_t *blocks, const float *scale, const zf *x,
+                         zf *y, hipStream_t st);
 // one Arnoldi step (one classical Gram-Schmidt pass, three launches) of P
 // near-field inner solves after w_s = A U_s[:, j]: h_s = U_s[:, 0..j]^H w_s
 // (also in hb + s * ldh), w_s -= U_s h_s, H_s[:, j] = (h_s, |w_s|),
@@ -481,7 +530,7 @@ void launch_zadd(int64_t n, const zd *a, zd *y, hipStream_t st);  // y += a
 void launch_blu_extract(int ngroups, int nmax, const int *p0, const int *cnt, const int *perm,
                         const int *pos, const int *leafbox_of_pos, const int *box_first,
                         const int *e2_off, const int *e2_list, const int64_t *near_off,
-                        const zd *blocks, zd *A, hipStream_t st);
+                        const NearRel &rel, const zd *blocks, zd *A, hipStream_t st);
 // x_g = v gathered into the group layout (zero padded), z = y_g scattered back
 void launch_blu_gather(int ngroups, int nmax, int N, const int *p0, const int *cnt,
                        const int *perm, const zd *v, zd *X, hipStream_t st);

@@ -8,11 +8,13 @@
 //     the reference edge number.
 //   * Near field: every leaf box b owns a dense block matrix
 //     Z_b[rows = edges of b][cols = E2(b) sorted ascending] of 2x2 complex
-//     blocks (D11,D12,D21,D22), row-major, 64 B per block in FP64.  The
+//     blocks (D11,D12,D21,D22), row-major, 64 B per block in FP64, or, where
+//     D21 is a constant c times D12, (D11,D12,D22/c) in 48 B (NearRel).  The
 //     reference CSR row of edge m is row (pos(m)-first_b) of Z_b with
 //     ja = E2(b), so the CSR is recovered exactly (ia, ja, values).
-//   * Radiation patterns: RT[p][q][S], q = k*2+comp (k medium, comp
-//     theta/phi), S = 2K^2+2 samples, sample index fastest.
+//   * Radiation patterns: RT[p][q][L], q = k*2+comp (k medium, comp
+//     theta/phi), sample index fastest: L = S = 2K^2+2 samples, or S/2 where
+//     the medium's wavenumber is real (PatLay).
 //   * MLFMM box coefficients per level: [box][8][S] with item
 //     it = comp*4 + cur*2 + k (cur = xe/xh), identical to the reference's
 //     a_nm/b_nm item(1..4) lists.

@@ -529,6 +529,17 @@ __device__ inline void finish_D(const NearArgs &A, zd *D) {
   }
 }
 
+// block g in the layout of NearRel
+__device__ inline void put_block(const NearRel &rel, int64_t g, const zd *D, zd *blocks) {
+  if (rel.nc == 3) {
+    blocks[3 * g] = D[0];
+    blocks[3 * g + 1] = D[1];
+    blocks[3 * g + 2] = D[3] * rel.ic;
+  } else {
+    for (int k = 0; k < 4; ++k) blocks[4 * g + k] = D[k];
+  }
+}
+
 // block index -> (row edge m, column edge n)
 __device__ inline void decode_block(const NearArgs &A, int64_t g, int &m, int &n) {
   int lo = 0, hi = A.nbl - 1;
@@ -632,8 +643,9 @@ __global__ void __launch_bounds__(128) k_near_singular(NearArgs A, int ntask, co
 }
 
 template <bool NEED_N>
-__global__ void __launch_bounds__(256) k_near_regular(NearArgs A, int64_t nnz, const uint8_t *cls,
-                                                      const int *base_a, const zd *zz, zd *blocks) {
+__global__ void __launch_bounds__(256) k_near_regular(NearArgs A, NearRel rel, int64_t nnz,
+                                                      const uint8_t *cls, const int *base_a,
+                                                      const zd *zz, zd *blocks) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= nnz) return;
   int m, n;
@@ -656,7 +668,7 @@ __global__ void __launch_bounds__(256) k_near_regular(NearArgs A, int64_t nnz, c
     accumulate_D(A, D, z);
   }
   finish_D(A, D);
-  for (int k = 0; k < 4; ++k) blocks[4 * g + k] = D[k];
+  put_block(rel, g, D, blocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -892,7 +904,8 @@ __device__ __forceinline__ void tri_sums(const zd *kk, const double *cm, const d
 // both media and K, for PMCHWT-S also K with the column side's sign.  LOSSY: a
 // medium's wavenumber is complex.
 template <int NV, bool LOSSY>
-__global__ void __launch_bounds__(256, 2) k_near_tri(NearArgs A, TriForm Q, const int *row_box,
+__global__ void __launch_bounds__(256, 2) k_near_tri(NearArgs A, TriForm Q, NearRel rel,
+                                                     const int *row_box,
                                                      const int *row_r0, int rp, const int4 *list,
                                                      const int *cnt, const uint8_t *cls,
                                                      const int *base_a, const zd *zz, zd *blocks) {
@@ -977,10 +990,11 @@ __global__ void __launch_bounds__(256, 2) k_near_tri(NearArgs A, TriForm Q, cons
             }
           finish_tri(A, D);
         }
-        blocks[4 * g] = D[0] + Q.c[0] * T1 + Q.c[1] * T2;
-        blocks[4 * g + 1] = D[1] + Q.c[2] * K;
-        blocks[4 * g + 2] = D[2] + Q.c[3] * Ka;
-        blocks[4 * g + 3] = D[3] + Q.c[4] * T1 + Q.c[5] * T2;
+        D[0] = D[0] + Q.c[0] * T1 + Q.c[1] * T2;
+        D[1] = D[1] + Q.c[2] * K;
+        D[2] = D[2] + Q.c[3] * Ka;
+        D[3] = D[3] + Q.c[4] * T1 + Q.c[5] * T2;
+        put_block(rel, g, D, blocks);
       }
       __syncthreads();
     }
@@ -1053,21 +1067,21 @@ void launch_near_singular(const NearArgs &a, int ntask, const NearTask *ta, cons
   hipLaunchKernelGGL(k_near_singular, dim3(nblk(ntask, 128)), dim3(128), 0, st, a, ntask, ta, cls,
                      base_b, kt, zz);
 }
-void launch_near_regular(const NearArgs &a, int64_t nnz, const uint8_t *cls, const int *base_a,
-                         const zd *zz, zd *blocks, hipStream_t st) {
+void launch_near_regular(const NearArgs &a, const NearRel &rel, int64_t nnz, const uint8_t *cls,
+                         const int *base_a, const zd *zz, zd *blocks, hipStream_t st) {
   if (nnz <= 0) return;
   const bool need_n = (a.form == SPK_JMCFIE || a.form == SPK_CNF || a.form == SPK_MNMF);
   if (need_n)
-    hipLaunchKernelGGL(k_near_regular<true>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, nnz, cls,
-                       base_a, zz, blocks);
+    hipLaunchKernelGGL(k_near_regular<true>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, rel, nnz,
+                       cls, base_a, zz, blocks);
   else
-    hipLaunchKernelGGL(k_near_regular<false>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, nnz, cls,
-                       base_a, zz, blocks);
+    hipLaunchKernelGGL(k_near_regular<false>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, rel, nnz,
+                       cls, base_a, zz, blocks);
 }
 
 // The triangle kernel takes the formulations without normal components and
 // without separate K of the media under the three-point rule (make_tri_form).
-void launch_near_tri(const NearArgs &a, const TriForm &q, int N, int tiles, const int *row_box,
+void launch_near_tri(const NearArgs &a, const TriForm &q, const NearRel &rel, int N, int tiles, const int *row_box,
                      const int *row_r0, const int *tri_side, int4 *list, int *cnt,
                      const uint8_t *cls, const int *base_a, const zd *zz, zd *blocks,
                      hipStream_t st) {
@@ -1083,7 +1097,7 @@ void launch_near_tri(const NearArgs &a, const TriForm &q, int N, int tiles, cons
   const bool alt = a.form == SPK_PMCHWT_S;
   auto *f = alt ? (lossy ? k_near_tri<4, true> : k_near_tri<4, false>)
                 : (lossy ? k_near_tri<3, true> : k_near_tri<3, false>);
-  hipLaunchKernelGGL(f, grid, dim3(256), kTriCols * (alt ? 64 : 48), st, a, q, row_box, row_r0, rp,
+  hipLaunchKernelGGL(f, grid, dim3(256), kTriCols * (alt ? 64 : 48), st, a, q, rel, row_box, row_r0, rp,
                      list, cnt, cls, base_a, zz, blocks);
 }
 
@@ -1117,7 +1131,7 @@ __global__ void __launch_bounds__(256) k_blu_extract(int nmax, const int *p0, co
                                                      const int *leafbox_of_pos,
                                                      const int *box_first, const int *e2_off,
                                                      const int *e2_list, const int64_t *near_off,
-                                                     const zd *blocks, zd *A) {
+                                                     NearRel rel, const zd *blocks, zd *A) {
   const int g = blockIdx.y, r = blockIdx.x;
   const int c0 = cnt[g], q0 = p0[g];
   zd *Ag = A + (size_t)g * nmax * nmax;
@@ -1134,11 +1148,12 @@ __global__ void __launch_bounds__(256) k_blu_extract(int nmax, const int *p0, co
   const int b = leafbox_of_pos[p];
   const int cols = e2_off[b + 1] - e2_off[b];
   const int rr = p - box_first[b];
-  const zd *row = blocks + 4 * (size_t)(near_off[b] + (int64_t)rr * cols);
+  const zd *row = blocks + rel.nc * (size_t)(near_off[b] + (int64_t)rr * cols);
   for (int c = threadIdx.x; c < cols; c += blockDim.x) {
     const int q = pos[e2_list[e2_off[b] + c]] - q0;
     if (q < 0 || q >= c0) continue;
-    const zd *bl = row + 4 * (size_t)c;
+    zd bl[4];
+    get_block(rel, row + rel.nc * (size_t)c, bl);
     Ag[(size_t)q * nmax + r] = bl[0];
     Ag[(size_t)(c0 + q) * nmax + r] = bl[1];
     Ag[(size_t)q * nmax + c0 + r] = bl[2];
@@ -1174,11 +1189,11 @@ __global__ void k_blu_scatter(int nmax, int N, const int *p0, const int *cnt, co
 void launch_blu_extract(int ngroups, int nmax, const int *p0, const int *cnt, const int *perm,
                         const int *pos, const int *leafbox_of_pos, const int *box_first,
                         const int *e2_off, const int *e2_list, const int64_t *near_off,
-                        const zd *blocks, zd *A, hipStream_t st) {
+                        const NearRel &rel, const zd *blocks, zd *A, hipStream_t st) {
   if (ngroups <= 0) return;
   // rows 0 .. nmax/2: real rows below cnt, padding pairs above
   hipLaunchKernelGGL(k_blu_extract, dim3((nmax + 1) / 2, ngroups), dim3(256), 0, st, nmax, p0, cnt,
-                     perm, pos, leafbox_of_pos, box_first, e2_off, e2_list, near_off, blocks, A);
+                     perm, pos, leafbox_of_pos, box_first, e2_off, e2_list, near_off, rel, blocks, A);
 }
 void launch_blu_gather(int ngroups, int nmax, int N, const int *p0, const int *cnt,
                        const int *perm, const zd *v, zd *X, hipStream_t st) {
@@ -1719,7 +1734,7 @@ template <class T>
 __global__ void k_near_transpose(int nbl, const int *box_first, const int *box_count,
                                  const int *e2_off, const int *e2_list, const int64_t *near_off,
                                  const int *perm, const int *pos, const int *leaf_box,
-                                 const T *in, T *out) {
+                                 int nc, const T *in, T *out) {
   const int b = blockIdx.y;
   const int r = blockIdx.x;
   if (b >= nbl || r >= box_count[b]) return;
@@ -1738,23 +1753,23 @@ __global__ void k_near_transpose(int nbl, const int *box_first, const int *box_c
       else
         hi = mid;
     }
-    const T *src = in + 4 * (near_off[bq] + (int64_t)rq * qc + lo);
-    T *dst = out + 4 * (near_off[b] + (int64_t)r * cols + c);
+    const T *src = in + nc * (near_off[bq] + (int64_t)rq * qc + lo);
+    T *dst = out + nc * (near_off[b] + (int64_t)r * cols + c);
     dst[0] = src[0];
-    dst[1] = src[2];
-    dst[2] = src[1];
-    dst[3] = src[3];
+    dst[1] = src[nc - 2];  // three components (NearRel): D12 stays D12
+    if (nc == 4) dst[2] = src[1];
+    dst[nc - 1] = src[nc - 1];
   }
 }
 
 template <class T>
 void launch_near_transpose(int nbl, int max_rows, const int *box_first, const int *box_count,
                            const int *e2_off, const int *e2_list, const int64_t *near_off,
-                           const int *perm, const int *pos, const int *leaf_box, const T *in,
-                           T *out, hipStream_t st) {
+                           const int *perm, const int *pos, const int *leaf_box, int nc,
+                           const T *in, T *out, hipStream_t st) {
   if (nbl <= 0 || max_rows <= 0) return;
   hipLaunchKernelGGL(k_near_transpose<T>, dim3(max_rows, nbl), dim3(256), 0, st, nbl, box_first,
-                     box_count, e2_off, e2_list, near_off, perm, pos, leaf_box, in, out);
+                     box_count, e2_off, e2_list, near_off, perm, pos, leaf_box, nc, in, out);
 }
 
 __device__ inline zd wave_sum(zd v) {
@@ -1946,13 +1961,14 @@ void launch_disagg(int ntask, int N, const PatLay &lay, const int *task, const i
 constexpr int kRowsPerWG = kSpmvRowsPerWG;
 constexpr int kColChunk = 1024;
 
-template <class T>
+// NC components per block (NearRel): with three the middle one serves both rows
+template <class T, int NC>
 __global__ void __launch_bounds__(256) k_near_spmv(int N, const int *row_box, const int *row_r0,
                                                    const int *box_first, const int *box_count,
                                                    const int *e2_off, const int *e2_list,
                                                    const int64_t *near_off, const int *perm,
-                                                   const T *blocks, const T *x, const T *yadd,
-                                                   T *y) {
+                                                   NearRel rel, const T *blocks, const T *x,
+                                                   const T *yadd, T *y) {
   __shared__ T xs[2 * kColChunk];
   const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x];
   const int rows = min(kRowsPerWG, box_count[b] - r0);
@@ -1966,30 +1982,28 @@ __global__ void __launch_bounds__(256) k_near_spmv(int N, const int *row_box, co
     for (int c = threadIdx.x; c < nc; c += blockDim.x) {
       const int n = e2_list[c0 + cc + c];
       xs[2 * c] = x[n];
-      xs[2 * c + 1] = x[n + N];
+      xs[2 * c + 1] = NC == 3 && rel.tr ? rel_scale(x[n + N], rel.c) : x[n + N];
     }
     __syncthreads();
     for (int q = 0; q < kRowsPerWG / 4; ++q) {
       const int r = r0 + wv + 4 * q;
       if (r >= r0 + rows) break;
-      const T *Z = blocks + 4 * (near_off[b] + (int64_t)(r - 0) * cols + cc);
+      const T *Z = blocks + NC * (near_off[b] + (int64_t)r * cols + cc);
       for (int c = lane; c < nc; c += 64) {
-        T z0, z1, z2, z3;
-        if constexpr (kPack<T> == 2) {
+        T z[NC];
+        if constexpr (NC == 4 && kPack<T> == 2) {
           const zf2 u = ld2(Z + 4 * c), v = ld2(Z + 4 * c + 2);
-          z0 = u.a;
-          z1 = u.b;
-          z2 = v.a;
-          z3 = v.b;
+          z[0] = u.a;
+          z[1] = u.b;
+          z[2] = v.a;
+          z[3] = v.b;
         } else {
-          z0 = Z[4 * c];
-          z1 = Z[4 * c + 1];
-          z2 = Z[4 * c + 2];
-          z3 = Z[4 * c + 3];
+#pragma unroll
+          for (int k = 0; k < NC; ++k) z[k] = Z[NC * c + k];
         }
         const T xe = xs[2 * c], xh = xs[2 * c + 1];
-        ae[q] = ae[q] + z0 * xe + z1 * xh;
-        ah[q] = ah[q] + z2 * xe + z3 * xh;
+        ae[q] = ae[q] + z[0] * xe + z[1] * xh;
+        ah[q] = ah[q] + z[NC - 2] * xe + z[NC - 1] * xh;
       }
     }
   }
@@ -1998,7 +2012,7 @@ __global__ void __launch_bounds__(256) k_near_spmv(int N, const int *row_box, co
     const T se = wave_sum(ae[q]), sh = wave_sum(ah[q]);
     if (r < r0 + rows && lane == 0) {
       const int m = perm[box_first[b] + r];
-      T oe = se, oh = sh;
+      T oe = se, oh = NC == 3 ? rel_scale(sh, rel.out()) : sh;
       if (yadd) {
         oe = oe + yadd[m];
         oh = oh + yadd[m + N];
@@ -2013,10 +2027,12 @@ template <class T>
 void launch_near_spmv_rows(int nwg, int N, const int *row_box, const int *row_r0,
                            const int *box_first, const int *box_count, const int *e2_off,
                            const int *e2_list, const int64_t *near_off, const int *perm,
-                           const T *blocks, const T *x, const T *yadd, T *y, hipStream_t st) {
+                           const NearRel &rel, const T *blocks, const T *x, const T *yadd, T *y,
+                           hipStream_t st) {
   if (nwg <= 0) return;
-  hipLaunchKernelGGL(k_near_spmv<T>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0, box_first,
-                     box_count, e2_off, e2_list, near_off, perm, blocks, x, yadd, y);
+  auto *f = rel.nc == 3 ? k_near_spmv<T, 3> : k_near_spmv<T, 4>;
+  hipLaunchKernelGGL(f, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0, box_first, box_count,
+                     e2_off, e2_list, near_off, perm, rel, blocks, x, yadd, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -2104,7 +2120,7 @@ void launch_rr_folded(int nb, int S, const int *parent, const int *octant, const
   template void launch_scale_halves<T>(int, zd, zd, const T *, T *, hipStream_t);                \
   template void launch_near_transpose<T>(int, int, const int *, const int *, const int *,        \
                                          const int *, const int64_t *, const int *, const int *, \
-                                         const int *, const T *, T *, hipStream_t);              \
+                                         const int *, int, const T *, T *, hipStream_t);         \
   template void launch_ss<T>(int, int, const int *, const T *, const T *, T *, hipStream_t);     \
   template void launch_m2l<T>(int, int, const int *, const int *, const int *, const T *,        \
                               const T *, T *, hipStream_t);                                      \
@@ -2116,13 +2132,13 @@ void launch_rr_folded(int nb, int S, const int *parent, const int *octant, const
                                  const T *, zd, zd, T *, hipStream_t, bool);                     \
   template void launch_near_spmv_rows<T>(int, int, const int *, const int *, const int *,        \
                                          const int *, const int *, const int *, const int64_t *, \
-                                         const int *, const T *, const T *, const T *, T *,      \
-                                         hipStream_t);
+                                         const int *, const NearRel &, const T *, const T *,     \
+                                         const T *, T *, hipStream_t);
 SPK_MATVEC_INSTANTIATE(zd)
 SPK_MATVEC_INSTANTIATE(zf)
 
 // Near field in bf16 (the preconditioner's copy): a complex value is one
-// 32-bit word, real part in the low half; a 2x2 block is 16 bytes.
+// 32-bit word, real part in the low half; a block is 4 bytes per kept component (NearRel).
 __device__ inline uint32_t f32_to_bf16(float f) {
   uint32_t u = __float_as_uint(f);
   u += 0x7FFFu + ((u >> 16) & 1u);  // round to nearest even (finite values)
@@ -2137,11 +2153,13 @@ void launch_to_bf(int64_t n, const zf *a, uint32_t *b, hipStream_t st) {
   hipLaunchKernelGGL(k_to_bf, dim3(2048), dim3(256), 0, st, n, a, b);
 }
 // the near SpMV of k_near_spmv (complex64 x and y) on bf16 blocks
+template <int NC>
 __global__ void __launch_bounds__(256) k_near_spmv_bf(int N, const int *row_box, const int *row_r0,
                                                       const int *box_first, const int *box_count,
                                                       const int *e2_off, const int *e2_list,
                                                       const int64_t *near_off, const int *perm,
-                                                      const uint4 *blocks, const zf *x, zf *y) {
+                                                      NearRel rel, const Words<NC> *blocks,
+                                                      const zf *x, zf *y) {
   __shared__ zf xs[2 * kColChunk];
   const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x];
   const int rows = min(kRowsPerWG, box_count[b] - r0);
@@ -2157,17 +2175,19 @@ __global__ void __launch_bounds__(256) k_near_spmv_bf(int N, const int *row_box,
     for (int c = threadIdx.x; c < nc; c += blockDim.x) {
       const int n = e2_list[c0 + cc + c];
       xs[2 * c] = x[n];
-      xs[2 * c + 1] = x[n + N];
+      xs[2 * c + 1] = NC == 3 && rel.tr ? rel_scale(x[n + N], rel.c) : x[n + N];
     }
     __syncthreads();
     for (int q = 0; q < kRowsPerWG / 4; ++q) {
       const int r = r0 + wv + 4 * q;
       if (r >= r0 + rows) break;
-      const uint4 *Z = blocks + (near_off[b] + (int64_t)r * cols + cc);
+      const Words<NC> *Z = blocks + (near_off[b] + (int64_t)r * cols + cc);
       for (int c = lane; c < nc; c += 64) {
-        const uint4 v = Z[c];
+        const Words<NC> v = Z[c];
         const zf z0 = {lo(v.x), hi(v.x)}, z1 = {lo(v.y), hi(v.y)};
-        const zf z2 = {lo(v.z), hi(v.z)}, z3 = {lo(v.w), hi(v.w)};
+        const zf z3 = {lo(last_word(v)), hi(last_word(v))};
+        zf z2 = z1;
+        if constexpr (NC == 4) z2 = zf{lo(v.z), hi(v.z)};
         const zf xe = xs[2 * c], xh = xs[2 * c + 1];
         ae[q] = ae[q] + z0 * xe + z1 * xh;
         ah[q] = ah[q] + z2 * xe + z3 * xh;
@@ -2180,48 +2200,61 @@ __global__ void __launch_bounds__(256) k_near_spmv_bf(int N, const int *row_box,
     if (r < r0 + rows && lane == 0) {
       const int m = perm[box_first[b] + r];
       y[m] = se;
-      y[m + N] = sh;
+      y[m + N] = NC == 3 ? rel_scale(sh, rel.out()) : sh;
     }
   }
 }
 void launch_near_spmv_bf(int nwg, int N, const int *row_box, const int *row_r0,
                          const int *box_first, const int *box_count, const int *e2_off,
                          const int *e2_list, const int64_t *near_off, const int *perm,
-                         const uint32_t *blocks, const zf *x, zf *y, hipStream_t st) {
+                         const NearRel &rel, const uint32_t *blocks, const zf *x, zf *y,
+                         hipStream_t st) {
   if (nwg <= 0) return;
-  hipLaunchKernelGGL(k_near_spmv_bf, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0, box_first,
-                     box_count, e2_off, e2_list, near_off, perm, (const uint4 *)blocks, x, y);
+  if (rel.nc == 3)
+    hipLaunchKernelGGL(k_near_spmv_bf<3>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
+                       (const uint3 *)blocks, x, y);
+  else
+    hipLaunchKernelGGL(k_near_spmv_bf<4>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
+                       (const uint4 *)blocks, x, y);
 }
 
-// Near field in fp8 (OCP E4M3FN, the single-vector preconditioner's copy):
-// a 2x2 block is 8 bytes (Z0r, Z0i, Z1r, Z1i, Z2r, Z2i, Z3r, Z3i); every
-// scalar row and component has its own scale (the row's largest |re|, |im|
-// of that component maps to 448), scale[p] = (s0, s1, s2, s3) for position p;
+// Near field in fp8 (OCP E4M3FN, the preconditioner's copy): two columns of a
+// row are NC dwords, dword k = kept component k (NearRel) of both columns (re,
+// im, re, im from the low byte up), so that a lane's load is NC consecutive
+// dwords and one dword is one matrix-core operand pair.  A row is
+// ceil(cols / 2) pairs (an odd last column is followed by zeros), box b's
+// rows begin at pair f8_pairs(near_off[b], box_first[b]).  Every scalar row
+// and component has its own scale (the row's largest |re|, |im| of that
+// component maps to 448), scale[p] for position p with NC of its four used;
 // f32_to_e4m3 (spk_fp8.h) encodes.
 // one workgroup per row position: the row's component maxima, then its blocks encoded
+template <int NC>
 __global__ void __launch_bounds__(256) k_near_to_f8(int N, const int *leaf_box_of_pos,
                                                     const int *box_first, const int *e2_off,
                                                     const int64_t *near_off, const zf *blocks,
-                                                    uint2 *out, float4 *scale) {
+                                                    uint32_t *out, float4 *scale) {
   __shared__ float red[4][4];
   __shared__ float inv[4];
   const int p = blockIdx.x;
   const int b = leaf_box_of_pos[p], r = p - box_first[b];
-  const int cols = e2_off[b + 1] - e2_off[b];
-  const int64_t g0 = near_off[b] + (int64_t)r * cols;
-  float mx[4] = {0.f, 0.f, 0.f, 0.f};
+  const int cols = e2_off[b + 1] - e2_off[b], pairs = (cols + 1) / 2;
+  const zf *Z = blocks + NC * (near_off[b] + (int64_t)r * cols);
+  float mx[NC];
+  for (int k = 0; k < NC; ++k) mx[k] = 0.f;
   for (int c = threadIdx.x; c < cols; c += 256)
-    for (int k = 0; k < 4; ++k) {
-      const zf z = blocks[4 * (g0 + c) + k];
+    for (int k = 0; k < NC; ++k) {
+      const zf z = Z[NC * c + k];
       mx[k] = fmaxf(mx[k], fmaxf(fabsf(z.x), fabsf(z.y)));
     }
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < NC; ++k) {
     float v = mx[k];
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_down(v, off, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = v;
   }
   __syncthreads();
-  if (threadIdx.x < 4) {
+  if (threadIdx.x < NC) {
     const int k = threadIdx.x;
     const float m = fmaxf(fmaxf(red[0][k], red[1][k]), fmaxf(red[2][k], red[3][k]));
     const float sc = m > 0.f ? m / 448.f : 1.f;
@@ -2229,81 +2262,101 @@ __global__ void __launch_bounds__(256) k_near_to_f8(int N, const int *leaf_box_o
     reinterpret_cast<float *>(scale + p)[k] = sc;
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < cols; c += 256) {
-    uint32_t w[2] = {0u, 0u};
-    for (int k = 0; k < 4; ++k) {
-      const zf z = blocks[4 * (g0 + c) + k];
-      const uint32_t lo = f32_to_e4m3(z.x * inv[k]), hi = f32_to_e4m3(z.y * inv[k]);
-      w[k >> 1] |= (lo | (hi << 8)) << (16 * (k & 1));
+  uint32_t *o = out + NC * (f8_pairs(near_off[b], box_first[b]) + (int64_t)r * pairs);
+  for (int c = threadIdx.x; c < pairs; c += 256)
+    for (int k = 0; k < NC; ++k) {
+      uint32_t w = 0u;
+      for (int u = 0; u < 2; ++u) {
+        if (2 * c + u >= cols) break;
+        const zf z = Z[NC * (2 * c + u) + k];
+        const uint32_t lo = f32_to_e4m3(z.x * inv[k]), hi = f32_to_e4m3(z.y * inv[k]);
+        w |= (lo | (hi << 8)) << (16 * u);
+      }
+      o[NC * c + k] = w;
     }
-    out[g0 + c] = uint2{w[0], w[1]};
-  }
 }
 void launch_near_to_f8(int N, const int *leaf_box_of_pos, const int *box_first, const int *e2_off,
-                       const int64_t *near_off, const zf *blocks, uint32_t *out, float *scale,
-                       hipStream_t st) {
+                       const int64_t *near_off, const NearRel &rel, const zf *blocks, uint32_t *out,
+                       float *scale, hipStream_t st) {
   if (N <= 0) return;
-  hipLaunchKernelGGL(k_near_to_f8, dim3(N), dim3(256), 0, st, N, leaf_box_of_pos, box_first, e2_off,
-                     near_off, blocks, (uint2 *)out, (float4 *)scale);
+  auto *f = rel.nc == 3 ? k_near_to_f8<3> : k_near_to_f8<4>;
+  hipLaunchKernelGGL(f, dim3(N), dim3(256), 0, st, N, leaf_box_of_pos, box_first, e2_off, near_off,
+                     blocks, out, (float4 *)scale);
 }
 // the near SpMV of k_near_spmv (complex64 x and y) on the fp8 blocks: the
-// four components are summed apart and scaled once per row.  A wave owns rows
-// r0 + wv + 4q (q < 4) and walks their columns together, two 64-column groups
-// per step, so eight 8-byte loads are in flight per lane and each x value read
-// from LDS serves four rows (rows past the box end read row r0 and are not
-// written; a column past the chunk end reads the last column with x = 0).
+// products with each component are summed apart and scaled once per row.  A
+// wave owns rows r0 + wv + 4q (q < 4) and walks their columns together, a pair
+// of columns per lane and step; a step's pairs are loaded before the last
+// step's are used, and the x values read from LDS serve four rows (rows past
+// the box end read row r0 and are not written; pairs past the chunk end read
+// the chunk's last pair with x = 0).
+template <int NC>
 __global__ void __launch_bounds__(256) k_near_spmv_f8(int N, const int *row_box, const int *row_r0,
                                                       const int *box_first, const int *box_count,
                                                       const int *e2_off, const int *e2_list,
                                                       const int64_t *near_off, const int *perm,
-                                                      const uint2 *blocks, const float4 *scale,
-                                                      const zf *x, zf *y) {
-  __shared__ zf xs[2 * kColChunk];
+                                                      NearRel rel, const Words<NC> *blocks,
+                                                      const float4 *scale, const zf *x, zf *y) {
+  // x of a chunk: column 2i at [0][i], 2i + 1 at [1][i], (xe, xh) each
+  __shared__ float4 xs[2][kColChunk / 2];
   const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x];
   const int rows = min(kRowsPerWG, box_count[b] - r0);
-  const int c0 = e2_off[b], cols = e2_off[b + 1] - c0;
+  const int c0 = e2_off[b], cols = e2_off[b + 1] - c0, pairs = (cols + 1) / 2;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   constexpr int NQ = kRowsPerWG / 4;
-  const uint2 *Zq[NQ];
+  const Words<NC> *Zq[NQ];
+  const int64_t z0 = f8_pairs(near_off[b], box_first[b]);
   for (int q = 0; q < NQ; ++q) {
     const int r = r0 + wv + 4 * q;
-    Zq[q] = blocks + (near_off[b] + (int64_t)(r < r0 + rows ? r : r0) * cols);
+    Zq[q] = blocks + (z0 + (int64_t)(r < r0 + rows ? r : r0) * pairs);
   }
+  // sums of D11 xe, D12 xh, D21 xe (of D12 xe) and D22 xh
   zf a0[NQ], a1[NQ], a2[NQ], a3[NQ];
   for (int q = 0; q < NQ; ++q) a0[q] = a1[q] = a2[q] = a3[q] = zf{0, 0};
-  auto acc = [&](int q, uint2 v, zf xe, zf xh) {
-    const auto q0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v.x, false);
-    const auto q1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v.x, true);
-    const auto q2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v.y, false);
-    const auto q3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)v.y, true);
-    a0[q] = a0[q] + zf{q0[0], q0[1]} * xe;
-    a1[q] = a1[q] + zf{q1[0], q1[1]} * xh;
-    a2[q] = a2[q] + zf{q2[0], q2[1]} * xe;
-    a3[q] = a3[q] + zf{q3[0], q3[1]} * xh;
+  auto dec = [](uint32_t w, zf &u, zf &v) {
+    const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
+    const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
+    u = zf{lo[0], lo[1]};
+    v = zf{hi[0], hi[1]};
   };
+  auto acc = [&](int q, const Words<NC> &w, const float4 &xa, const float4 &xb) {
+    const zf ea = {xa.x, xa.y}, ha = {xa.z, xa.w}, eb = {xb.x, xb.y}, hb = {xb.z, xb.w};
+    zf u, v;
+    dec(w.x, u, v);
+    a0[q] = a0[q] + u * ea + v * eb;
+    dec(w.y, u, v);
+    a1[q] = a1[q] + u * ha + v * hb;
+    if constexpr (NC == 4) dec(w.z, u, v);
+    a2[q] = a2[q] + u * ea + v * eb;
+    dec(last_word(w), u, v);
+    a3[q] = a3[q] + u * ha + v * hb;
+  };
+  Words<NC> cur[NQ];
+  if (pairs > 0)
+    for (int q = 0; q < NQ; ++q) cur[q] = Zq[q][min(lane, pairs - 1)];
   for (int cc = 0; cc < cols; cc += kColChunk) {
-    const int nc = min(kColChunk, cols - cc);
+    const int nc = min(kColChunk, cols - cc), np = (nc + 1) / 2;
     __syncthreads();
-    for (int c = threadIdx.x; c < nc; c += blockDim.x) {
-      const int n = e2_list[c0 + cc + c];
-      xs[2 * c] = x[n];
-      xs[2 * c + 1] = x[n + N];
+    for (int c = threadIdx.x; c < 2 * np; c += 256) {
+      float4 v = {0.f, 0.f, 0.f, 0.f};
+      if (c < nc) {
+        const int n = e2_list[c0 + cc + c];
+        const zf xe = x[n];
+        const zf xh = NC == 3 && rel.tr ? rel_scale(x[n + N], rel.c) : x[n + N];
+        v = float4{xe.x, xe.y, xh.x, xh.y};
+      }
+      xs[c & 1][c >> 1] = v;
     }
     __syncthreads();
-    for (int c = lane; c < nc; c += 128) {
-      const int c1 = min(c + 64, nc - 1);
-      uint2 v0[NQ], v1[NQ];
-      for (int q = 0; q < NQ; ++q) {
-        v0[q] = Zq[q][cc + c];
-        v1[q] = Zq[q][cc + c1];
-      }
-      const zf xe0 = xs[2 * c], xh0 = xs[2 * c + 1];
-      zf xe1 = xs[2 * c1], xh1 = xs[2 * c1 + 1];
-      if (c + 64 >= nc) xe1 = xh1 = zf{0, 0};
-      for (int q = 0; q < NQ; ++q) {
-        acc(q, v0[q], xe0, xh0);
-        acc(q, v1[q], xe1, xh1);
-      }
+    for (int i = lane; i < np; i += 64) {
+      // the next step's pairs, of the next chunk after this chunk's last
+      const int nx = i + 64 < np ? cc / 2 + i + 64 : (cc + kColChunk) / 2 + lane;
+      Words<NC> nxt[NQ];
+      for (int q = 0; q < NQ; ++q) nxt[q] = Zq[q][min(nx, pairs - 1)];
+      __builtin_amdgcn_sched_barrier(0);
+      const float4 xa = xs[0][i], xb = xs[1][i];
+      for (int q = 0; q < NQ; ++q) acc(q, cur[q], xa, xb);
+      for (int q = 0; q < NQ; ++q) cur[q] = nxt[q];
     }
   }
   for (int q = 0; q < NQ; ++q) {
@@ -2314,19 +2367,24 @@ __global__ void __launch_bounds__(256) k_near_spmv_f8(int N, const int *row_box,
       const float4 sc = scale[p];
       const int m = perm[p];
       y[m] = s0 * sc.x + s1 * sc.y;
-      y[m + N] = s2 * sc.z + s3 * sc.w;
+      y[m + N] = NC == 3 ? rel_scale(s2 * sc.y + s3 * sc.z, rel.out()) : s2 * sc.z + s3 * sc.w;
     }
   }
 }
 void launch_near_spmv_f8(int nwg, int N, const int *row_box, const int *row_r0,
                          const int *box_first, const int *box_count, const int *e2_off,
                          const int *e2_list, const int64_t *near_off, const int *perm,
-                         const uint32_t *blocks, const float *scale, const zf *x, zf *y,
-                         hipStream_t st) {
+                         const NearRel &rel, const uint32_t *blocks, const float *scale, const zf *x,
+                         zf *y, hipStream_t st) {
   if (nwg <= 0) return;
-  hipLaunchKernelGGL(k_near_spmv_f8, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0, box_first,
-                     box_count, e2_off, e2_list, near_off, perm, (const uint2 *)blocks,
-                     (const float4 *)scale, x, y);
+  if (rel.nc == 3)
+    hipLaunchKernelGGL(k_near_spmv_f8<3>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
+                       (const uint3 *)blocks, (const float4 *)scale, x, y);
+  else
+    hipLaunchKernelGGL(k_near_spmv_f8<4>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
+                       (const uint4 *)blocks, (const float4 *)scale, x, y);
 }
 
 // complex128 -> complex64 copy (the mixed-precision operator's tables)
@@ -2348,7 +2406,7 @@ void launch_to_zf(int64_t n, const zd *a, zf *b, hipStream_t st) {
 // ---------------------------------------------------------------------------
 __global__ void k_jacobi_diag(int N, const int *perm, const int *leaf_box_of_pos,
                               const int *box_first, const int *e2_off, const int *e2_list,
-                              const int64_t *near_off, const zd *blocks, zd *diag) {
+                              const int64_t *near_off, NearRel rel, const zd *blocks, zd *diag) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= N) return;
   const int m = perm[p], b = leaf_box_of_pos[p];
@@ -2366,19 +2424,20 @@ __global__ void k_jacobi_diag(int N, const int *perm, const int *leaf_box_of_pos
   }
   zd d11 = {0, 0}, d22 = {0, 0};
   if (c >= 0) {
-    const zd *Z = blocks + 4 * (near_off[b] + (int64_t)r * cols + c);
-    d11 = Z[0];
-    d22 = Z[3];
+    zd D[4];
+    get_block(rel, blocks + rel.nc * (near_off[b] + (int64_t)r * cols + c), D);
+    d11 = D[0];
+    d22 = D[3];
   }
   diag[m] = d11;
   diag[m + N] = d22;
 }
 void launch_jacobi_diag(int N, const int *perm, const int *leaf_box_of_pos, const int *box_first,
                         const int *e2_off, const int *e2_list, const int64_t *near_off,
-                        const zd *blocks, zd *diag, hipStream_t st) {
+                        const NearRel &rel, const zd *blocks, zd *diag, hipStream_t st) {
   if (N <= 0) return;
   hipLaunchKernelGGL(k_jacobi_diag, dim3(nblk(N, 256)), dim3(256), 0, st, N, perm,
-                     leaf_box_of_pos, box_first, e2_off, e2_list, near_off, blocks, diag);
+                     leaf_box_of_pos, box_first, e2_off, e2_list, near_off, rel, blocks, diag);
 }
 __global__ void k_div_diag(int64_t n, const zd *diag, const zd *x, zd *y) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;

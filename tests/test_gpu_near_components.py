@@ -1,0 +1,72 @@
+"""Near blocks that keep three components (D21 a constant times D12: PMCHWT,
+MCTF, ICTF) against the products of the four-component blocks (near_csr, which
+test_gpu_near_tri pins to single evaluations) on the host, beside formulations
+that keep four: forward and transposed, every format of the blocks, every
+batched kernel; leaf boxes of a few columns, odd column counts and several
+column chunks; a lossy medium (a complex factor).
+
+Tolerances, of each half of the product: FP64 sums of some thousand terms,
+1e-12; complex64 blocks and x, 2e-6; bf16 and fp8 round a component to 2^-9 and
+2^-4 of at most its row's largest, so the halves differ by less than 5e-3 and
+6e-2 (averaged over a row's terms).
+"""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from specklesim_amd import SieTriMlfmm, meshes
+
+pytestmark = pytest.mark.gpu
+LAM = 633e-9
+
+
+def half_err(a, b, n):
+    return max(np.linalg.norm(a[:n] - b[:n]) / np.linalg.norm(b[:n]),
+               np.linalg.norm(a[n:] - b[n:]) / np.linalg.norm(b[n:]))
+
+
+@pytest.mark.parametrize("form,s_opt,eps", [
+    ("ICTF", 20, 2.25), ("ICTF", 250, 2.25 - 0.3j), ("ICTF", 4000, 2.25), ("PMCHWT", 50, 2.25 - 0.3j),
+    ("MCTF", 100, 4.0), ("PMCHWT-S", 50, 2.25), ("MCTF2", 100, 2.25 - 0.3j)])
+def test_products_of_the_kept_components(form, s_opt, eps):
+    pp, tt = meshes.rough_surface(21, 19, 2.1, 1.9, 0.1, 0.5, 6, LAM)
+    s = SieTriMlfmm(LAM, eps, formulation=form, precision="mixed",
+                    tree_s_opt=s_opt).precalculation_tri(pp, tt)
+    n = s.N
+    ia, ja, v = s.near_csr()
+    v = v.reshape(-1, 4)
+    A = sp.bmat([[sp.csr_matrix((v[:, 2 * i + j], ja, ia), shape=(n, n)) for j in range(2)]
+                 for i in range(2)], format="csr")
+    rng = np.random.default_rng(3)
+    X = (rng.standard_normal((16, 2 * n)) + 1j * rng.standard_normal((16, 2 * n))).astype(np.complex64)
+    # a half of each row's terms at most cancels: scale x so that both count
+    X[:, n:] *= np.linalg.norm(v[:, 0]) / np.linalg.norm(v[:, 1])
+    for tr in (False, True):
+        s.set_transposed(tr)
+        Z = A.T if tr else A
+        Y = np.stack([Z @ x.astype(np.complex128) for x in X])
+        assert half_err(s.matvec_parts(X[0].astype(np.complex128))[0], Y[0], n) < 1e-12, tr
+        for fmt, tol in (("c64", 2e-6), ("bf16", 5e-3), ("fp8", 6e-2)):
+            got = s.near_product_lowp(X[:2], fmt, batched=False)
+            for r in range(2):
+                assert half_err(got[r].astype(np.complex128), Y[r], n) < tol, (fmt, tr)
+            for R in (1, 2, 3, 6, 16):
+                got = s.near_product_lowp(X[:R], fmt, batched=True)
+                for r in range(R):
+                    e = half_err(got[r].astype(np.complex128), Y[r], n)
+                    assert e < max(tol, 5e-3 if fmt != "c64" else 0), (fmt, tr, R, r, e)
+    s.set_transposed(False)
+
+
+@pytest.mark.parametrize("R", [1, 2, 3, 6, 16])
+def test_batched_fp64_products(R):
+    """The FP64 batches' near part: whole products against single ones, to
+    1e-10: the far part's translation sums cancel some 1e5 times their result
+    on leaf boxes of 0.3 wavelengths, and the batches add in another order."""
+    pp, tt = meshes.rough_surface(21, 19, 2.1, 1.9, 0.1, 0.5, 6, LAM)
+    s = SieTriMlfmm(LAM, 2.25 - 0.3j, formulation="MCTF").precalculation_tri(pp, tt)
+    rng = np.random.default_rng(4)
+    X = rng.standard_normal((R, 2 * s.N)) + 1j * rng.standard_normal((R, 2 * s.N))
+    Y = s.calculate_vector_b_tri_batch(X)
+    for r in range(R):
+        assert half_err(Y[r], s.calculate_vector_b_tri(X[r]), s.N) < 1e-10
