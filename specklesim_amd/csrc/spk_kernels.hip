@@ -1955,14 +1955,29 @@ void launch_disagg(int ntask, int N, const PatLay &lay, const int *task, const i
                        task, perm, leaf_box_of_pos, rt, W, cvt<T>(sc1), cvt<T>(sc2), y);
 }
 
-// Near SpMV over the box-dense block matrices.  Workgroup = (leaf box,
-// chunk of kRowsPerWG rows); x of the box's E2 columns staged in LDS in
-// chunks of kColChunk; one wavefront per row, lanes over columns.
+// Near SpMV over the box-dense block matrices.  Workgroup = (leaf box, rows of
+// a tile of kRowsPerWG); x of the box's E2 columns staged in LDS in chunks of
+// kColChunk; a wavefront per row in turn, lanes over columns.
 constexpr int kRowsPerWG = kSpmvRowsPerWG;
 constexpr int kColChunk = 1024;
+// Rows a wave takes: one row with four columns' blocks per lane in flight
+// hides the latency of the loads on small meshes, where 16 rows per workgroup
+// leave most of the chip idle; more rows share the staging of x, which the
+// low bytes of the fp8 copy need sooner.  us with 1, 2, 4 rows per wave (16
+// rows per workgroup with 4) at N edges:
+//   N        FP64                 complex64             fp8
+//   1,160    12.0   14.1   25.2   10.4   13.5   23.9     5.8    6.0    9.4
+//   4,720    28.0   28.1   35.9   16.6   17.9   26.4     9.0    8.7   11.3
+//   10,680  129.1  138.5  132.6   69.6   75.3   83.8    26.5   26.5   26.7
+//   29,800  246.7  243.8  249.0  137.1  136.3  138.8    54.2   41.8   41.8
+//   58,520  908.0  894.6  913.7  464.2  463.9  471.2   180.1  142.9  136.0
+static int near_rows_per_wave(int N) { return N < 24576 ? 1 : 2; }
+static int near_rows_per_wave_f8(int N) { return N < 4096 ? 1 : N < 32768 ? 2 : 4; }
 
-// NC components per block (NearRel): with three the middle one serves both rows
-template <class T, int NC>
+// NC components per block (NearRel): with three the middle one serves both
+// rows.  A workgroup takes 4 NQ rows of the tile, NQ per wave in turn (grid.y
+// covers the tile); a lane has U columns' blocks in flight.
+template <class T, int NC, int NQ>
 __global__ void __launch_bounds__(256) k_near_spmv(int N, const int *row_box, const int *row_r0,
                                                    const int *box_first, const int *box_count,
                                                    const int *e2_off, const int *e2_list,
@@ -1970,12 +1985,14 @@ __global__ void __launch_bounds__(256) k_near_spmv(int N, const int *row_box, co
                                                    NearRel rel, const T *blocks, const T *x,
                                                    const T *yadd, T *y) {
   __shared__ T xs[2 * kColChunk];
-  const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x];
-  const int rows = min(kRowsPerWG, box_count[b] - r0);
+  constexpr int U = 4 / NQ;
+  const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x] + 4 * NQ * blockIdx.y;
+  const int rows = min(4 * NQ, box_count[b] - r0);
+  if (rows <= 0) return;
   const int c0 = e2_off[b], cols = e2_off[b + 1] - c0;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  T ae[kRowsPerWG / 4], ah[kRowsPerWG / 4];
-  for (int q = 0; q < kRowsPerWG / 4; ++q) ae[q] = ah[q] = T{0, 0};
+  T ae[NQ], ah[NQ];
+  for (int q = 0; q < NQ; ++q) ae[q] = ah[q] = T{0, 0};
   for (int cc = 0; cc < cols; cc += kColChunk) {
     const int nc = min(kColChunk, cols - cc);
     __syncthreads();
@@ -1985,29 +2002,41 @@ __global__ void __launch_bounds__(256) k_near_spmv(int N, const int *row_box, co
       xs[2 * c + 1] = NC == 3 && rel.tr ? rel_scale(x[n + N], rel.c) : x[n + N];
     }
     __syncthreads();
-    for (int q = 0; q < kRowsPerWG / 4; ++q) {
+    for (int q = 0; q < NQ; ++q) {
       const int r = r0 + wv + 4 * q;
       if (r >= r0 + rows) break;
       const T *Z = blocks + NC * (near_off[b] + (int64_t)r * cols + cc);
-      for (int c = lane; c < nc; c += 64) {
-        T z[NC];
-        if constexpr (NC == 4 && kPack<T> == 2) {
-          const zf2 u = ld2(Z + 4 * c), v = ld2(Z + 4 * c + 2);
-          z[0] = u.a;
-          z[1] = u.b;
-          z[2] = v.a;
-          z[3] = v.b;
-        } else {
+      for (int c = lane; c < nc; c += 64 * U) {
+        T z[U][NC];
 #pragma unroll
-          for (int k = 0; k < NC; ++k) z[k] = Z[NC * c + k];
+        for (int u = 0; u < U; ++u) {
+          const int cu = u ? min(c + 64 * u, nc - 1) : c;
+          if constexpr (NC == 4 && kPack<T> == 2) {
+            const zf2 v = ld2(Z + 4 * cu), w = ld2(Z + 4 * cu + 2);
+            z[u][0] = v.a;
+            z[u][1] = v.b;
+            z[u][2] = w.a;
+            z[u][3] = w.b;
+          } else {
+#pragma unroll
+            for (int k = 0; k < NC; ++k) z[u][k] = Z[NC * cu + k];
+          }
         }
-        const T xe = xs[2 * c], xh = xs[2 * c + 1];
-        ae[q] = ae[q] + z[0] * xe + z[1] * xh;
-        ah[q] = ah[q] + z[NC - 2] * xe + z[NC - 1] * xh;
+        if constexpr (U > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          T xe = {0, 0}, xh = {0, 0};
+          if (u == 0 || c + 64 * u < nc) {
+            xe = xs[2 * (c + 64 * u)];
+            xh = xs[2 * (c + 64 * u) + 1];
+          }
+          ae[q] = ae[q] + z[u][0] * xe + z[u][1] * xh;
+          ah[q] = ah[q] + z[u][NC - 2] * xe + z[u][NC - 1] * xh;
+        }
       }
     }
   }
-  for (int q = 0; q < kRowsPerWG / 4; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int r = r0 + wv + 4 * q;
     const T se = wave_sum(ae[q]), sh = wave_sum(ah[q]);
     if (r < r0 + rows && lane == 0) {
@@ -2030,9 +2059,14 @@ void launch_near_spmv_rows(int nwg, int N, const int *row_box, const int *row_r0
                            const NearRel &rel, const T *blocks, const T *x, const T *yadd, T *y,
                            hipStream_t st) {
   if (nwg <= 0) return;
-  auto *f = rel.nc == 3 ? k_near_spmv<T, 3> : k_near_spmv<T, 4>;
-  hipLaunchKernelGGL(f, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0, box_first, box_count,
-                     e2_off, e2_list, near_off, perm, rel, blocks, x, yadd, y);
+  const int nq = near_rows_per_wave(N);
+  auto pick = [&](auto nc) {
+    constexpr int NC = decltype(nc)::value;
+    return nq == 1 ? k_near_spmv<T, NC, 1> : k_near_spmv<T, NC, 2>;
+  };
+  auto *f = rel.nc == 3 ? pick(std::integral_constant<int, 3>{}) : pick(std::integral_constant<int, 4>{});
+  hipLaunchKernelGGL(f, dim3(nwg, kRowsPerWG / 4 / nq), dim3(256), 0, st, N, row_box, row_r0,
+                     box_first, box_count, e2_off, e2_list, near_off, perm, rel, blocks, x, yadd, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -2285,12 +2319,11 @@ void launch_near_to_f8(int N, const int *leaf_box_of_pos, const int *box_first, 
 }
 // the near SpMV of k_near_spmv (complex64 x and y) on the fp8 blocks: the
 // products with each component are summed apart and scaled once per row.  A
-// wave owns rows r0 + wv + 4q (q < 4) and walks their columns together, a pair
+// wave owns rows r0 + wv + 4q (q < NQ) and walks their columns together, U pairs
 // of columns per lane and step; a step's pairs are loaded before the last
-// step's are used, and the x values read from LDS serve four rows (rows past
-// the box end read row r0 and are not written; pairs past the chunk end read
-// the chunk's last pair with x = 0).
-template <int NC>
+// step's are used, and the x values read from LDS serve NQ rows (rows past the
+// box end read row r0 and are not written; pairs past the chunk end have x = 0).
+template <int NC, int NQ>
 __global__ void __launch_bounds__(256) k_near_spmv_f8(int N, const int *row_box, const int *row_r0,
                                                       const int *box_first, const int *box_count,
                                                       const int *e2_off, const int *e2_list,
@@ -2299,11 +2332,12 @@ __global__ void __launch_bounds__(256) k_near_spmv_f8(int N, const int *row_box,
                                                       const float4 *scale, const zf *x, zf *y) {
   // x of a chunk: column 2i at [0][i], 2i + 1 at [1][i], (xe, xh) each
   __shared__ float4 xs[2][kColChunk / 2];
-  const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x];
-  const int rows = min(kRowsPerWG, box_count[b] - r0);
+  constexpr int U = 4 / NQ;
+  const int b = row_box[blockIdx.x], r0 = row_r0[blockIdx.x] + 4 * NQ * blockIdx.y;
+  const int rows = min(4 * NQ, box_count[b] - r0);
+  if (rows <= 0) return;
   const int c0 = e2_off[b], cols = e2_off[b + 1] - c0, pairs = (cols + 1) / 2;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr int NQ = kRowsPerWG / 4;
   const Words<NC> *Zq[NQ];
   const int64_t z0 = f8_pairs(near_off[b], box_first[b]);
   for (int q = 0; q < NQ; ++q) {
@@ -2331,9 +2365,14 @@ __global__ void __launch_bounds__(256) k_near_spmv_f8(int N, const int *row_box,
     dec(last_word(w), u, v);
     a3[q] = a3[q] + u * ha + v * hb;
   };
-  Words<NC> cur[NQ];
-  if (pairs > 0)
-    for (int q = 0; q < NQ; ++q) cur[q] = Zq[q][min(lane, pairs - 1)];
+  Words<NC> cur[NQ][U];
+  auto load = [&](int i, Words<NC> (*w)[U]) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[q][u] = Zq[q][min(i + 64 * u, pairs - 1)];
+  };
+  if (pairs > 0) load(lane, cur);
   for (int cc = 0; cc < cols; cc += kColChunk) {
     const int nc = min(kColChunk, cols - cc), np = (nc + 1) / 2;
     __syncthreads();
@@ -2348,15 +2387,25 @@ __global__ void __launch_bounds__(256) k_near_spmv_f8(int N, const int *row_box,
       xs[c & 1][c >> 1] = v;
     }
     __syncthreads();
-    for (int i = lane; i < np; i += 64) {
+    for (int i = lane; i < np; i += 64 * U) {
       // the next step's pairs, of the next chunk after this chunk's last
-      const int nx = i + 64 < np ? cc / 2 + i + 64 : (cc + kColChunk) / 2 + lane;
-      Words<NC> nxt[NQ];
-      for (int q = 0; q < NQ; ++q) nxt[q] = Zq[q][min(nx, pairs - 1)];
+      Words<NC> nxt[NQ][U];
+      load(i + 64 * U < np ? cc / 2 + i + 64 * U : (cc + kColChunk) / 2 + lane, nxt);
       __builtin_amdgcn_sched_barrier(0);
-      const float4 xa = xs[0][i], xb = xs[1][i];
-      for (int q = 0; q < NQ; ++q) acc(q, cur[q], xa, xb);
-      for (int q = 0; q < NQ; ++q) cur[q] = nxt[q];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float4 xa = {0.f, 0.f, 0.f, 0.f}, xb = xa;
+        if (u == 0 || i + 64 * u < np) {
+          xa = xs[0][i + 64 * u];
+          xb = xs[1][i + 64 * u];
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) acc(q, cur[q][u], xa, xb);
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int u = 0; u < U; ++u) cur[q][u] = nxt[q][u];
     }
   }
   for (int q = 0; q < NQ; ++q) {
@@ -2377,14 +2426,20 @@ void launch_near_spmv_f8(int nwg, int N, const int *row_box, const int *row_r0,
                          const NearRel &rel, const uint32_t *blocks, const float *scale, const zf *x,
                          zf *y, hipStream_t st) {
   if (nwg <= 0) return;
+  const int nq = near_rows_per_wave_f8(N);
+  auto launch = [&](auto nc) {
+    constexpr int NC = decltype(nc)::value;
+    auto *f = nq == 1   ? k_near_spmv_f8<NC, 1>
+              : nq == 2 ? k_near_spmv_f8<NC, 2>
+                        : k_near_spmv_f8<NC, 4>;
+    hipLaunchKernelGGL(f, dim3(nwg, kRowsPerWG / 4 / nq), dim3(256), 0, st, N, row_box, row_r0,
+                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
+                       (const Words<NC> *)blocks, (const float4 *)scale, x, y);
+  };
   if (rel.nc == 3)
-    hipLaunchKernelGGL(k_near_spmv_f8<3>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0,
-                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
-                       (const uint3 *)blocks, (const float4 *)scale, x, y);
+    launch(std::integral_constant<int, 3>{});
   else
-    hipLaunchKernelGGL(k_near_spmv_f8<4>, dim3(nwg), dim3(256), 0, st, N, row_box, row_r0,
-                       box_first, box_count, e2_off, e2_list, near_off, perm, rel,
-                       (const uint4 *)blocks, (const float4 *)scale, x, y);
+    launch(std::integral_constant<int, 4>{});
 }
 
 // complex128 -> complex64 copy (the mixed-precision operator's tables)

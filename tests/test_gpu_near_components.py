@@ -70,3 +70,19 @@ def test_batched_fp64_products(R):
     Y = s.calculate_vector_b_tri_batch(X)
     for r in range(R):
         assert half_err(Y[r], s.calculate_vector_b_tri(X[r]), s.N) < 1e-10
+
+
+@pytest.mark.parametrize("cells", [10, 46, 88, 106])
+def test_rows_per_wave(cells):
+    """One, two and four rows per wave (280 to 33,496 edges): each format's
+    single product against the batched kernels and the FP64 product."""
+    pp, tt = meshes.rough_surface(cells, cells, cells / 10, cells / 10, 0.1, 0.5, 6, LAM)
+    s = SieTriMlfmm(LAM, 2.25, formulation="ICTF", precision="mixed").precalculation_tri(pp, tt)
+    rng = np.random.default_rng(5)
+    X = (rng.standard_normal((16, 2 * s.N)) + 1j * rng.standard_normal((16, 2 * s.N))).astype(np.complex64)
+    ref = s.matvec_parts(X[0].astype(np.complex128))[0]
+    for fmt, tol in (("c64", 2e-6), ("fp8", 6e-2)):
+        y = s.near_product_lowp(X[:1], fmt, batched=False)[0].astype(np.complex128)
+        yb = s.near_product_lowp(X, fmt, batched=True)[0].astype(np.complex128)
+        assert half_err(y, ref, s.N) < tol, fmt
+        assert half_err(yb, y, s.N) < max(2e-6, 5e-3 * (fmt == "fp8")), fmt
