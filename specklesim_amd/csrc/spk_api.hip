@@ -1081,19 +1081,21 @@ int matvec_batch_t(spk_handle *h, int R, const T *const *xs, T *const *ys, bool 
   const int S = h->tb.S, N = h->N, lmax = t.l_max, lmin = t.l_min;
   hipStream_t st = h->st;
   LevelDev &LL = h->lev[lmax];
-  launch_batch_interleave(N, R, h->rel, h->d_perm.p, xs, BB.XI.p, BB.XP.p, st);
   if (!far_on) {
     if constexpr (std::is_same<T, zf>::value) {
       if (f8_scale && R > 8) {
         launch_batch_near_f8(h->spmv_wgs, N, R, h->d_row_box.p, h->d_row_r0.p, h->mx_groups,
                              h->d_mx_box.p, h->d_mx_r0.p, h->d_box_first.p,
                              h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p,
-                             h->d_perm.p, h->rel, blocks_bf, f8_scale, (const zf *)BB.XI.p, BB.XB.p, ys,
+                             h->d_perm.p, h->rel, blocks_bf, f8_scale, xs, BB.XB.p, ys,
                              h->mx_tpw, st);
         HIPCHK(hipGetLastError());
         return SPK_OK;
       }
     }
+  }
+  launch_batch_interleave(N, R, h->rel, h->d_perm.p, xs, BB.XI.p, BB.XP.p, st);
+  if (!far_on) {
     launch_batch_near(h->spmv_wgs, N, R, h->d_row_box.p, h->d_row_r0.p, h->d_box_first.p,
                       h->d_box_count.p, h->d_e2_off.p, h->d_e2_list.p, h->d_near_off.p, h->d_perm.p,
                       h->rel, pBlk(h, tag), (const T *)BB.XI.p, (const T *)nullptr, ys, st,
@@ -2443,8 +2445,8 @@ static DBuf<zd> &fgWi(spk_handle::FgWork &F, zd *) { return F.Wid; }
 // solve with it replaces most outer steps, each of which costs a full FP64
 // product (near field plus the MLFMM far field).
 //  - Inner: the active right-hand sides' inner steps share one (batched)
-//    near-field product; their Arnoldi runs on the device (two classical
-//    Gram-Schmidt passes, coefficients and norms stay in HBM) and the host
+//    near-field product; their Arnoldi runs on the device (one classical
+//    Gram-Schmidt pass, coefficients and norms stay in HBM) and the host
 //    solves the small least-squares problems once per outer step.
 //  - Outer: z_r = U_r y_r is kept, w = Z z_r in FP64, ICGS with the CERFACS
 //    reorthogonalisation test, Givens rotations on the host; the Arnoldi
@@ -2875,7 +2877,11 @@ static int fgmres_near(spk_handle *h, int R, const zd *const *b, zd *const *x,
           for (int i = c + 1; i < kk; ++i) sum -= HC(c, i) * yy[i];
           yy[c] = sum / HC(c, c);
         }
-        for (int c = 0; c < kk; ++c) yall[(size_t)s * kin + c] = zd{yy[c].real(), yy[c].imag()};
+        // the stored columns are m_c times the basis vectors
+        for (int c = 0; c < kk; ++c) {
+          const double im = c ? 1.0 / Hs[(size_t)(c - 1) * (kin + 1) + kin].x : 1.0;
+          yall[(size_t)s * kin + c] = zd{yy[c].real() * im, yy[c].imag() * im};
+        }
         klen[s] = kk;
       }
       // from pinned memory, which is next written by a later copy on this stream

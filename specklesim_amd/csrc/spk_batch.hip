@@ -1752,11 +1752,33 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
 // (blocks, scale as k_near_spmv_f8 reads them); workgroups = row tiles of
 // 16 rows.  Two tiles per workgroup (x staged once for 32 rows, 156 VGPRs)
 // measured the same, 105 us at 16 vectors on the 10 x 10 lambda patch.
-// XB[i] = XI[i] in bf16 (re in the low half, im in the high half), rounded
-// to nearest even as bf16_pair rounds
-__global__ void __launch_bounds__(256) kb_x_to_bf(int64_t len, const zf *XI, uint32_t *XB) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < len) XB[i] = bf16_pair(XI[i].x, XI[i].y);
+// XB[(m * 2 + cur) * 16 + r] = x_r[m + cur N] in bf16 (re in the low half, im
+// in the high half), rounded to nearest even as bf16_pair rounds, zero for r >=
+// R; the second half scaled where NearRel asks for it.  Workgroup = 64
+// positions, turned over in LDS so that the vectors are read and XB is written
+// along the lanes: 5.5 us at 16 vectors of 59,600 values, where interleaving in
+// complex64 and rounding that took 14.
+__global__ void __launch_bounds__(256) kb_x_to_bf(int N, int R, NearRel rel, const zf *const *xs,
+                                                  uint32_t *XB) {
+  __shared__ uint32_t tl[2 * 64 * 17];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m0 = blockIdx.x * 64, m = min(m0 + lane, N - 1);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int r = wv + 4 * k;
+    zf e = {0, 0}, h = {0, 0};
+    if (r < R) {
+      e = xs[r][m];
+      h = xs[r][m + (int64_t)N];
+      if (rel.nc == 3 && rel.tr) h = rel_scale(h, rel.c);
+    }
+    tl[(2 * lane) * 17 + r] = bf16_pair(e.x, e.y);
+    tl[(2 * lane + 1) * 17 + r] = bf16_pair(h.x, h.y);
+  }
+  __syncthreads();
+  const int words = min(64, N - m0) * 32;
+  for (int w = threadIdx.x; w < words; w += 256)
+    XB[(size_t)m0 * 32 + w] = tl[(w >> 4) * 17 + (w & 15)];
 }
 template <int NC>
 static void batch_near_f8(int nwg, int N, int R, const int *row_box, const int *row_r0, int ngrp,
@@ -1786,10 +1808,10 @@ void launch_batch_near_f8(int nwg, int N, int R, const int *row_box, const int *
                           const int *box_first, const int *box_count, const int *e2_off,
                           const int *e2_list, const int64_t *near_off, const int *perm,
                           const NearRel &rel, const uint32_t *blocks, const float *scale,
-                          const zf *XI, uint32_t *XB, zf *const *ys, int tpw, hipStream_t st) {
+                          const zf *const *xs, uint32_t *XB, zf *const *ys, int tpw,
+                          hipStream_t st) {
   if (nwg <= 0) return;
-  const int64_t len = (int64_t)N * 2 * 16;
-  hipLaunchKernelGGL(kb_x_to_bf, dim3(bnblk(len, 256)), dim3(256), 0, st, len, XI, XB);
+  hipLaunchKernelGGL(kb_x_to_bf, dim3(bnblk(N, 64)), dim3(256), 0, st, N, R, rel, xs, XB);
   auto *f = rel.nc == 3 ? batch_near_f8<3> : batch_near_f8<4>;
   f(nwg, N, R, row_box, row_r0, ngrp, grp_box, grp_r0, box_first, box_count, e2_off, e2_list,
     near_off, perm, rel, blocks, scale, XB, ys, tpw, st);
@@ -1960,19 +1982,29 @@ void launch_batch_orth(int64_t n, int P, int maxk, const int *ks, const T *const
 
 // ---------------------------------------------------------------------------
 // Device-side Arnoldi step of P near-field inner solves (the FGMRES
-// preconditioner), one classical Gram-Schmidt pass in three launches:
-//   dot:  partial[s][c][g] = sum over the rows of chunk g of conj(U_s[:, c]) w_s
-//         (one workgroup per 1024-row chunk, column and slot)
-//   upd:  h_s = sum_g partial (fixed order, in every workgroup), w_s -= U_s h_s,
-//         pnrm[s][g] = |w_s|^2 over chunk g
-//   fin:  |w_s| = sqrt(sum_g pnrm); H_s[:, j] = (h_s, |w_s|); U_s[:, j + 1] = w_s / |w_s|
-// Slot s: U + s * ldu (column c at c * n), w: W + s * n, h: hb + s * ldh,
+// preconditioner), one classical Gram-Schmidt pass in two launches after
+// w_s = A V_s[:, j].  The stored columns V_c = m_c u_c are not normalised (m_0 =
+// 1): the norm m_j of the last one is summed, from its writer's partial sums,
+// by the launch that needs it, so no launch only scales a vector.
+//   dot:  partial[s][c][g] = sum over the rows of chunk g of conj(V_s[:, c]) w_s
+//   upd:  h_c = sum_g partial / (m_c m_j), V_s[:, j + 1] = (w / m_j - sum h_c u_c) / q_j
+//         with q_j = |h|, which keeps the column near 1 whatever the operator's
+//         scale, pn[s][g] = |V_s[:, j + 1]|^2 over chunk g;
+//         H[:, j] = h, H[j, j - 1] = q_(j-1) m_j, and m_j at H[kin, j - 1]
+//   tail: H[kin, kin - 1] after the last step
+// All sums in a fixed order, in complex128.  Slot s: V = U + s * ldu (column c
+// at c * n), w: W + s * n, hb + s * ldh: (m_c, q_(c-1)) of column c,
 // H + s * (kin + 1) * kin (column-major, leading dimension kin + 1).
-// Products accumulate in complex128.
+// Both are bound by latency for one vector: the update's workgroups sum the
+// partials with eight lanes per column and keep eight columns' values in
+// flight.  us per step before (three launches, one column at a time, the third
+// for the normalisation) and now: one vector of 5,280 values 6.4 + 3.1 -> 5.2
+// after the dots' 4.0, of 59,600 values 7.3 + 4.6 -> 7.4 after 4.7; 16 vectors
+// of 59,600 25.5 + 5.6 -> 29.1 after 26 (4.5 TB/s over the columns).
 // ---------------------------------------------------------------------------
 constexpr int kArnRows = 1024;  // rows per workgroup of the dot kernel
-// partial[s][c][g] = sum over rows [g * kArnRows, (g + 1) * kArnRows) of
-// conj(U_s[:, c]) w_s: one workgroup per (row chunk, column, slot)
+// one workgroup per (row chunk, column, slot); four columns per workgroup, to
+// share the reads of w, took 33 us for 26 at 16 vectors
 template <class T>
 __global__ void __launch_bounds__(256) k_arn_dot(int64_t n, int k, int G, const T *U, size_t ldu,
                                                  const T *W, zd *partial) {
@@ -1993,83 +2025,113 @@ __global__ void __launch_bounds__(256) k_arn_dot(int64_t n, int k, int G, const 
   if (threadIdx.x == 0) partial[((size_t)s * k + c) * G + g] = red[0] + red[1] + red[2] + red[3];
 }
 template <class T>
-__global__ void __launch_bounds__(256) k_arn_upd(int64_t n, int64_t rows, int k, int G, int Gd,
-                                                 const T *U, size_t ldu, T *W, const zd *partial,
-                                                 zd *hb, int ldh, double *pnrm) {
-  __shared__ zd hs[64];
-  __shared__ double red[4];
-  const int s = blockIdx.y, g = blockIdx.x;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  // h_c = sum over the G partials: wave wv takes columns wv, wv + 4, ...;
-  // lanes stride the partials, then a shuffle tree (a fixed order)
-  for (int c = wv; c < k; c += 4) {
-    const zd *p = partial + ((size_t)s * k + c) * Gd;
-    zd acc = {0, 0};
-    for (int q = lane; q < Gd; q += 64) acc = acc + p[q];
-    acc = bwave_sum(acc);
-    if (lane == 0) {
-      hs[c] = acc;
-      if (g == 0) hb[(size_t)s * ldh + c] = acc;
+__global__ void __launch_bounds__(256) k_arn_upd(int64_t n, int64_t rows, int j, int kin, int G,
+                                                 int Gd, T *U, size_t ldu, const T *W,
+                                                 const zd *partial, zd *hb, int ldh, zd *H,
+                                                 const double *pn_in, double *pn_out) {
+  constexpr int CB = 8;  // columns in flight
+  __shared__ zd hs[64 + CB];
+  __shared__ double red[4], wsc;
+  const int s = blockIdx.y, g = blockIdx.x, k = j + 1;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  zd *hbs = hb + (size_t)s * ldh, *Hs = H + (size_t)s * (kin + 1) * kin;
+  const T *Us = U + (size_t)s * ldu, *w = W + (size_t)s * n;
+  T *out = U + (size_t)s * ldu + (size_t)(j + 1) * n;
+  const int64_t r0 = (int64_t)g * rows, r1 = min(n, r0 + rows);
+  double mc = 0.0, qj = 0.0;
+  if (wv == 0 && lane < j) mc = hbs[lane].x;
+  if (t == 0 && j > 0) qj = hbs[j].y;
+  {  // |V_j|^2 and the coefficients' sums
+    double a = j > 0 && t < G ? pn_in[(size_t)s * G + t] : 0.0;
+    for (int c = t >> 3; c < k; c += 32) {
+      const zd *p = partial + ((size_t)s * k + c) * Gd;
+      zd acc = {0, 0};
+#pragma unroll 8
+      for (int q = t & 7; q < Gd; q += 8) acc = acc + p[q];
+      for (int off = 4; off > 0; off >>= 1) {
+        acc.x += __shfl_xor(acc.x, off, 64);
+        acc.y += __shfl_xor(acc.y, off, 64);
+      }
+      if ((t & 7) == 0) hs[c] = acc;
+    }
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
+    if (lane == 0) red[wv] = a;
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const double mj = j > 0 ? sqrt(red[0] + red[1] + red[2] + red[3]) : 1.0;
+    const double ij = mj > 0.0 ? 1.0 / mj : 0.0;
+    double ic = 0.0;
+    zd h = {0, 0};
+    if (lane < k) {
+      if (lane == j) mc = mj;
+      ic = mc > 0.0 ? 1.0 / mc : 0.0;
+      h = hs[lane] * (ic * ij);
+    }
+    double q = h.x * h.x + h.y * h.y;
+    for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
+    q = q > 0.0 ? sqrt(q) : 1.0;
+    hs[lane] = h * (ic / q);  // zero from column k on
+    if (lane < CB) hs[64 + lane] = zd{0, 0};
+    if (lane == 0) wsc = ij / q;
+    if (g == 0) {
+      if (lane < k) Hs[(size_t)j * (kin + 1) + lane] = h;
+      if (lane == 0) {
+        if (j > 0) {
+          Hs[(size_t)(j - 1) * (kin + 1) + j] = zd{qj * mj, 0.0};
+          Hs[(size_t)(j - 1) * (kin + 1) + kin] = zd{mj, 0.0};
+        }
+        hbs[j].x = mj;
+        hbs[j + 1].y = q;
+      }
     }
   }
   __syncthreads();
-  const T *Us = U + (size_t)s * ldu;
-  T *w = W + (size_t)s * n;
-  const int64_t r0 = (int64_t)g * rows, r1 = min(n, r0 + rows);
+  const double ws = wsc;
   double nrm = 0.0;
-  for (int64_t i = r0 + threadIdx.x; i < r1; i += 256) {
-    zd wi = bwiden(w[i]);
-    for (int c = 0; c < k; ++c) {
-      const zd u = bwiden(Us[(size_t)c * n + i]), hc = hs[c];
-      wi.x -= u.x * hc.x - u.y * hc.y;
-      wi.y -= u.x * hc.y + u.y * hc.x;
+  for (int64_t i = r0 + t; i < r1; i += 256) {
+    zd wi = bwiden(w[i]) * ws;
+    for (int c = 0; c < k; c += CB) {
+      T u[CB];
+#pragma unroll
+      for (int b = 0; b < CB; ++b) u[b] = Us[(size_t)min(c + b, j) * n + i];
+#pragma unroll
+      for (int b = 0; b < CB; ++b) {
+        const zd uc = bwiden(u[b]), hc = hs[c + b];
+        wi.x -= uc.x * hc.x - uc.y * hc.y;
+        wi.y -= uc.x * hc.y + uc.y * hc.x;
+      }
     }
     using F = decltype(w[i].x);
     const T wt = T{(F)wi.x, (F)wi.y};
-    w[i] = wt;
-    const zd ws = bwiden(wt);
-    nrm += ws.x * ws.x + ws.y * ws.y;
+    out[i] = wt;
+    const zd wd = bwiden(wt);
+    nrm += wd.x * wd.x + wd.y * wd.y;
   }
   for (int off = 32; off > 0; off >>= 1) nrm += __shfl_down(nrm, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = nrm;
+  if (lane == 0) red[wv] = nrm;
   __syncthreads();
-  if (threadIdx.x == 0) pnrm[(size_t)s * G + g] = red[0] + red[1] + red[2] + red[3];
+  if (t == 0) pn_out[(size_t)s * G + g] = red[0] + red[1] + red[2] + red[3];
 }
-template <class T>
-__global__ void __launch_bounds__(256) k_arn_fin(int64_t n, int64_t rows, int j, int kin, int G,
-                                                 const double *pnrm, const zd *hb, int ldh,
-                                                 const T *W, size_t ldu, T *U, zd *H) {
-  __shared__ double nrm;
-  const int s = blockIdx.y, g = blockIdx.x;
-  if (threadIdx.x < 64) {
-    double a = 0.0;
-    for (int q = threadIdx.x; q < G; q += 64) a += pnrm[(size_t)s * G + q];
-    for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
-    if (threadIdx.x == 0) nrm = sqrt(fmax(a, 0.0));
-  }
-  __syncthreads();
-  const double nv = nrm, inv = nv > 0.0 ? 1.0 / nv : 0.0;
-  if (g == 0 && threadIdx.x <= j + 1) {
-    const int i = threadIdx.x;
-    H[(size_t)s * (kin + 1) * kin + (size_t)j * (kin + 1) + i] =
-        i <= j ? hb[(size_t)s * ldh + i] : zd{nv, 0.0};
-  }
-  const T *w = W + (size_t)s * n;
-  T *u = U + (size_t)s * ldu + (size_t)(j + 1) * n;
-  const int64_t r0 = (int64_t)g * rows, r1 = min(n, r0 + rows);
-  using F = decltype(w[0].x);
-  for (int64_t i = r0 + threadIdx.x; i < r1; i += 256) {
-    const T v = w[i];
-    u[i] = T{(F)(v.x * inv), (F)(v.y * inv)};
-  }
+__global__ void __launch_bounds__(64) k_arn_tail(int kin, int G, const double *pn, const zd *hb,
+                                                 int ldh, zd *H) {
+  const int s = blockIdx.x;
+  double a = 0.0;
+  for (int q = threadIdx.x; q < G; q += 64) a += pn[(size_t)s * G + q];
+  for (int off = 32; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
+  if (threadIdx.x == 0)
+    H[(size_t)s * (kin + 1) * kin + (size_t)(kin - 1) * (kin + 1) + kin] =
+        zd{hb[(size_t)s * ldh + kin].y * sqrt(a), 0.0};
 }
-// row chunks of the update and normalisation (at most 256): 256 rows for
+// row chunks of the update (at most 256, one norm partial each): 256 rows for
 // fewer than 4 slots (more workgroups for a short grid), 512 otherwise
 static int arnoldi_chunks(int64_t n, int P) {
   const int64_t rows = P < 4 ? 256 : 512;
   return (int)std::max<int64_t>(1, std::min<int64_t>(256, (n + rows - 1) / rows));
 }
 static int arnoldi_dot_chunks(int64_t n) { return (int)((n + kArnRows - 1) / kArnRows); }
+// the dots' partials, then two sets of norm partials (a step reads the set
+// that the step before it wrote)
 size_t arnoldi_partial_elems(int64_t n, int P, int kin) {
   return (size_t)P * (kin + 1) * (size_t)std::max(256, arnoldi_dot_chunks(n)) + (size_t)P * 256;
 }
@@ -2081,12 +2143,14 @@ void launch_arnoldi_cgs(int64_t n, int P, int j, int kin, T *U, size_t ldu, T *W
   const int64_t rows = (n + G - 1) / G;
   const int k = j + 1;
   double *pn = reinterpret_cast<double *>(partial + (size_t)P * (kin + 1) * std::max(256, Gd));
+  double *pj = pn + (size_t)(j & 1) * P * 256, *pi = pn + (size_t)(~j & 1) * P * 256;
   hipLaunchKernelGGL(k_arn_dot<T>, dim3(Gd, k, P), dim3(256), 0, st, n, k, Gd, (const T *)U, ldu,
                      (const T *)W, partial);
-  hipLaunchKernelGGL(k_arn_upd<T>, dim3(G, P), dim3(256), 0, st, n, rows, k, G, Gd, (const T *)U,
-                     ldu, W, (const zd *)partial, hb, ldh, pn);
-  hipLaunchKernelGGL(k_arn_fin<T>, dim3(G, P), dim3(256), 0, st, n, rows, j, kin, G,
-                     (const double *)pn, (const zd *)hb, ldh, (const T *)W, ldu, U, H);
+  hipLaunchKernelGGL(k_arn_upd<T>, dim3(G, P), dim3(256), 0, st, n, rows, j, kin, G, Gd, U, ldu,
+                     (const T *)W, (const zd *)partial, hb, ldh, H, (const double *)pi, pj);
+  if (k == kin)
+    hipLaunchKernelGGL(k_arn_tail, dim3(P), dim3(64), 0, st, kin, G, (const double *)pj,
+                       (const zd *)hb, ldh, H);
 }
 
 template <class T>

@@ -457,9 +457,8 @@ void launch_batch_near(int nwg, int N, int R, const int *row_box, const int *row
                        const int *e2_list, const int64_t *near_off, const int *perm,
                        const NearRel &rel, const T *blocks, const T *XI, const T *yf,
                        T *const *ys, hipStream_t st, const uint32_t *blocks_bf = nullptr);
-// the near-field preconditioner's product for 9..16 right-hand sides (XI as
-// launch_batch_interleave writes it; XB: scratch of N * 32 words for x in
-// bf16) on the fp8 copy of the blocks, on the matrix cores; workgroups = the
+// the near-field preconditioner's product for 9..16 right-hand sides (XB:
+// scratch of N * 32 words for x in bf16) on the fp8 copy of the blocks, on the matrix cores; workgroups = the
 // row tiles (box, first row) of kSpmvRowsPerWG rows
 int near_mx_tiles_per_group();
 // levels of different truncation numbers (spk_kernels.hip)
@@ -476,7 +475,8 @@ void launch_batch_near_f8(int nwg, int N, int R, const int *row_box, const int *
                           const int *box_first, const int *box_count, const int *e2_off,
                           const int *e2_list, const int64_t *near_off, const int *perm,
                           const NearRel &rel, const uint32_t *blocks, const float *scale,
-                          const zf *XI, uint32_t *XB, zf *const *ys, int tpw, hipStream_t st);
+                          const zf *const *xs, uint32_t *XB, zf *const *ys, int tpw,
+                          hipStream_t st);
 
 // one ICGS pass over P bases (coefficients into hs[r][0..ks[r]), |w_r|^2
 // into hs[r][ks[r]]); partial: batch_orth_partial_elems(n, P, maxk)
@@ -505,12 +505,13 @@ void launch_near_spmv_f8(int nwg, int N, const int *row_box, const int *row_r0,
                          const int *e2_list, const int64_t *near_off, const int *perm,
                          const NearRel &rel, const uint32_t *blocks, const float *scale, const zf *x,
                          zf *y, hipStream_t st);
-// one Arnoldi step (one classical Gram-Schmidt pass, three launches) of P
-// near-field inner solves after w_s = A U_s[:, j]: h_s = U_s[:, 0..j]^H w_s
-// (also in hb + s * ldh), w_s -= U_s h_s, H_s[:, j] = (h_s, |w_s|),
-// U_s[:, j+1] = w_s / |w_s|.  Slot s: U + s * ldu (column c at c * n),
-// W + s * n, H + s * (kin + 1) * kin (column-major, leading dimension
-// kin + 1); partial: arnoldi_partial_elems(n, P, kin); kin <= 64
+// step j of P near-field inner solves after w_s = A V_s[:, j] (one classical
+// Gram-Schmidt pass): V_s[:, j + 1] from w_s, H_s[:, j] and the norm of V_s[:, j].
+// The columns are m_c times the basis vectors, m_0 = 1, m_c left at H_s[kin, c - 1]
+// for 1 <= c < kin.  Slot s: V = U + s * ldu (column c at c * n), W + s * n, H +
+// s * (kin + 1) * kin (column-major, leading dimension kin + 1), complete after
+// step kin - 1; hb: kin + 2 values per slot (ldh); partial:
+// arnoldi_partial_elems(n, P, kin); kin <= 64
 template <class T>
 void launch_arnoldi_cgs(int64_t n, int P, int j, int kin, T *U, size_t ldu, T *W, zd *hb, int ldh,
                         zd *H, zd *partial, hipStream_t st);
