@@ -33,6 +33,7 @@ void quad_edge_nodes(const QuadMesh &m, int s, int *n1, int *n2);
 // constants of the kernels (materials and 1-D Gauss-Legendre rules)
 struct QuadDev {
   zd k1, k2, ie1, ie2, e1, e2, ceps, iwe, iwm;
+  zd riwe, nriwm, niwe;  // 1 / iwe, -1 / iwm, -iwe
   double x4[4], w4[4], x5[5], w5[5], x6[6], w6[6], x15[15], w15[15];
 };
 

@@ -56,15 +56,16 @@ struct QBuf {
 };
 
 
-__device__ inline void qgreen(zd k, double R, zd &G, zd &DG) {
+__device__ inline void qgreen(zd k, double R, double rinv, zd &G, zd &DG) {
   // Diver_Green (src/lib_sie_quad_calculation_mod.f90:553-564)
-  const double ph = -k.x * R, mag = exp(k.y * R);
+  const double ph = -k.x * R, mag = k.y != 0.0 ? exp(k.y * R) : 1.0;
   double sn, cs;
   sincos(ph, &sn, &cs);
   const zd E = {mag * cs, mag * sn};  // exp(-i k R)
   const zd ikr = {-k.y * R, k.x * R};
-  G = E * (1.0 / (4 * QPI * R));
-  DG = -((zd{1.0 + ikr.x, ikr.y} * E) * (1.0 / (4 * QPI * (R * R))));
+  const double g = rinv * (1.0 / (4 * QPI));
+  G = E * g;
+  DG = -((zd{1.0 + ikr.x, ikr.y} * E) * (g * rinv));
 }
 
 // shape functions and derivatives (R_shape, N_differential, f_edge_new)
@@ -177,56 +178,72 @@ __device__ inline void obs_fn(const Geo &g, int pI, double k, double e, double N
   for (int d = 0; d < 3; ++d) Na[d] = f * v[d];
 }
 
-// ff_ABC_II_Edge accumulated with weight w into S[5][10]
-// (src/lib_sie_quad_singularity.f90:581-618)
-__device__ inline void acc_ff(const QuadDev &D, const double Na[3], const double R[3],
-                              const Geo &q, double kq, double eq, double w, zd S[5][10]) {
-  const double nR = sqrt(dot3(R, R));
-  const double rn[3] = {R[0] / nR, R[1] / nR, R[2] / nR};
+// ff_ABC_II_Edge accumulated with weight w (src/lib_sie_quad_singularity.f90:
+// 581-618) into S = (A, DE, DH), A = KA, DE = KBE / iwe + iwm KCE, DH = -KBH /
+// iwm - iwe KCH.  Source function n is F(n) times au (n < 5) or av, its n x curl
+// factor fr(n), so a point gives one coefficient per direction and kind for
+// all ten; ju, jv: JJ (n x au), JJ (n x av) of the source point.  Summing the
+// five integrals of each function over its own cross products kept 200
+// doubles of sums per thread and three times the arithmetic.  The kernels stay
+// bound by the FP64 vector ALU at one or two waves per SIMD: dense fill of 20 x
+// 20 elements, regular pairs 8.0 -> 3.9 ms, self terms 6.2 -> 2.6, edge-adjacent
+// pairs 8.9 -> 6.5, corner pairs 0.65 -> 0.30; near pairs of 60 x 60 elements 26
+// -> 13.2 ms.  The regular kernels gain from two waves per SIMD (2.45 -> 1.95
+// ms a launch) though that spills 56 bytes; the self and edge-adjacent ones
+// spill a kilobyte there and double their time.
+template <class FF, class FR>
+__device__ __forceinline__ void acc_point(const QuadDev &D, const double Na[3], const double R[3],
+                                          const double *ju, const double *jv, const FF &F,
+                                          const FR &fr, double w, zd S[3][10]) {
+  const double R2 = dot3(R, R), nR = sqrt(R2), rinv = 1.0 / nR;
+  const double rn[3] = {R[0] * rinv, R[1] * rinv, R[2] * rinv};
   zd Ga, GSa, Gm, GSm;
-  qgreen(D.k1, nR, Ga, GSa);
-  qgreen(D.k2, nR, Gm, GSm);
-  const zd gA = GSa + GSm, gBE = D.ie1 * GSa + D.ie2 * GSm, gC = Ga + Gm;
-  const zd gCH = D.e1 * Ga + D.e2 * Gm;
-  const double Nrn = dot3(Na, rn);
+  qgreen(D.k1, nR, rinv, Ga, GSa);
+  qgreen(D.k2, nR, rinv, Gm, GSm);
+  const zd gA = GSa + GSm;
+  const double wr = dot3(Na, rn) * w;
+  const zd bE = D.riwe * (D.ie1 * GSa + D.ie2 * GSm) * wr, bH = D.nriwm * gA * wr;
+  const zd cE = D.iwm * (Ga + Gm), cH = D.niwe * (D.e1 * Ga + D.e2 * Gm);
 #pragma unroll
-  for (int n = 0; n < 10; ++n) {
-    const double f = fedge(n, kq, eq);
-    const double *v = n < 5 ? q.au : q.av;
-    const double Nq[3] = {f * v[0], f * v[1], f * v[2]};
-    double aa[3], t[3];
-    cross3(q.nq, Nq, aa);
-    cross3(aa, rn, t);
-    const double nrot = fedge_rot(n, kq, eq) / q.JJ;
-    const double f1 = dot3(Na, t) * q.JJ;
-    const double f2 = Nrn * nrot * q.JJ;
-    const double f3 = dot3(Na, aa) * q.JJ;
-    S[0][n] = S[0][n] + gA * (f1 * w);
-    S[1][n] = S[1][n] + gBE * (f2 * w);
-    S[2][n] = S[2][n] + gA * (f2 * w);
-    S[3][n] = S[3][n] + gC * (f3 * w);
-    S[4][n] = S[4][n] + gCH * (f3 * w);
+  for (int dir = 0; dir < 2; ++dir) {
+    const double *jj = dir ? jv : ju;
+    double t[3];
+    cross3(jj, rn, t);
+    const double f3 = dot3(Na, jj) * w;
+    const zd a = gA * (dot3(Na, t) * w), e = cE * f3, h = cH * f3;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      const int n = 5 * dir + q;
+      const double fn = F(n), rot = fr(n);
+      S[0][n] = S[0][n] + a * fn;
+      S[1][n] = S[1][n] + e * fn + bE * rot;
+      S[2][n] = S[2][n] + h * fn + bH * rot;
+    }
   }
 }
-
-// (KA, KBE, KBH, KCE, KCH) -> (A, DE, DH)
-__device__ inline void combine(const QuadDev &D, zd S[5][10], zd out[3][10]) {
-#pragma unroll
-  for (int n = 0; n < 10; ++n) {
-    out[0][n] = S[0][n];
-    out[1][n] = S[1][n] / D.iwe - (-(D.iwm * S[3][n]));
-    out[2][n] = S[2][n] / (-D.iwm) - D.iwe * S[4][n];
+__device__ inline void acc_ff(const QuadDev &D, const double Na[3], const double R[3],
+                              const Geo &q, double kq, double eq, double w, zd S[3][10]) {
+  double ju[3], jv[3];
+  cross3(q.nq, q.au, ju);
+  cross3(q.nq, q.av, jv);
+  for (int d = 0; d < 3; ++d) {
+    ju[d] *= q.JJ;
+    jv[d] *= q.JJ;
   }
+  acc_point(D, Na, R, ju, jv, [&](int n) { return fedge(n, kq, eq); },
+            [&](int n) { return fedge_rot(n, kq, eq); }, w, S);
+}
+__device__ inline void zero30(zd S[3][10]) {
+  for (int k = 0; k < 3; ++k)
+    for (int n = 0; n < 10; ++n) S[k][n] = zd{0, 0};
 }
 
 // regular pair: NG x NG Gauss on both elements (Element_integration 'Normal'
 // and Integration_KABCD_Edge_new, :479-522)
 template <int NG>
 __device__ void regular_pair(const QuadDev &D, const double *x, const double *w, const double *Ea,
-                             const double *Eq, int pI, zd out[3][10]) {
-  zd S[5][10];
-  for (int k = 0; k < 5; ++k)
-    for (int n = 0; n < 10; ++n) S[k][n] = zd{0, 0};
+                             const double *Eq, int pI, zd S[3][10]) {
+  zero30(S);
   for (int j = 0; j < NG; ++j)
     for (int i = 0; i < NG; ++i) {
       Geo ga;
@@ -245,17 +262,16 @@ __device__ void regular_pair(const QuadDev &D, const double *x, const double *w,
           acc_ff(D, Na, R, gq, x[a], x[b], (w[a] * w[b]) * TRF, S);
         }
     }
-  combine(D, S, out);
 }
 
 // Source-element data of the regular NG x NG rule at point (a, b), shared by
 // every pair of a workgroup that integrates over the same element: position,
-// rule weight and, per edge function n, JJ (n x N_n) and the n x curl factor
-// fedge_rot (JJ times nrot of acc_ff).
+// rule weight, JJ (n x au), JJ (n x av) and, per edge function n, its value and
+// its n x curl factor.
 struct QSrc {
   double R[3], w;
-  double aJ[10][3];
-  double fr[10];
+  double j[2][3];
+  double F[10], fr[10];
 };
 template <int NG>
 __device__ inline void qsrc_point(const QuadDev &D, const double *Eq, int a, int b, QSrc &o) {
@@ -265,14 +281,14 @@ __device__ inline void qsrc_point(const QuadDev &D, const double *Eq, int a, int
   geo(k, e, Eq, g);
   rloc(k, e, Eq, o.R);
   o.w = wt[a] * wt[b];
-#pragma unroll
+  cross3(g.nq, g.au, o.j[0]);
+  cross3(g.nq, g.av, o.j[1]);
+  for (int d = 0; d < 3; ++d) {
+    o.j[0][d] *= g.JJ;
+    o.j[1][d] *= g.JJ;
+  }
   for (int n = 0; n < 10; ++n) {
-    const double f = fedge(n, k, e);
-    const double *v = n < 5 ? g.au : g.av;
-    const double Nq[3] = {f * v[0], f * v[1], f * v[2]};
-    double aa[3];
-    cross3(g.nq, Nq, aa);
-    for (int d = 0; d < 3; ++d) o.aJ[n][d] = aa[d] * g.JJ;
+    o.F[n] = fedge(n, k, e);
     o.fr[n] = fedge_rot(n, k, e);
   }
 }
@@ -282,7 +298,7 @@ __device__ inline void qsrc_point(const QuadDev &D, const double *Eq, int a, int
 // loop order of regular_pair), accumulated into S
 template <int NG>
 __device__ void outer_point_tab(const QuadDev &D, const double *Ea, const QSrc *src, int pI,
-                                int i, int j, zd S[5][10]) {
+                                int i, int j, zd S[3][10]) {
   const double *x = NG == 6 ? D.x6 : D.x4, *wt = NG == 6 ? D.w6 : D.w4;
   Geo ga;
   geo(x[i], x[j], Ea, ga);
@@ -293,37 +309,17 @@ __device__ void outer_point_tab(const QuadDev &D, const double *Ea, const QSrc *
   for (int p = 0; p < NG * NG; ++p) {
     const QSrc &P = src[p];
     const double R[3] = {Ra[0] - P.R[0], Ra[1] - P.R[1], Ra[2] - P.R[2]};
-    const double nR = sqrt(dot3(R, R));
-    const double rn[3] = {R[0] / nR, R[1] / nR, R[2] / nR};
-    zd Ga, GSa, Gm, GSm;
-    qgreen(D.k1, nR, Ga, GSa);
-    qgreen(D.k2, nR, Gm, GSm);
-    const zd gA = GSa + GSm, gBE = D.ie1 * GSa + D.ie2 * GSm, gC = Ga + Gm;
-    const zd gCH = D.e1 * Ga + D.e2 * Gm;
-    const double Nrn = dot3(Na, rn), w = P.w * TRF;
-#pragma unroll
-    for (int n = 0; n < 10; ++n) {
-      double t[3];
-      cross3(P.aJ[n], rn, t);
-      const double f1 = dot3(Na, t), f2 = Nrn * P.fr[n], f3 = dot3(Na, P.aJ[n]);
-      S[0][n] = S[0][n] + gA * (f1 * w);
-      S[1][n] = S[1][n] + gBE * (f2 * w);
-      S[2][n] = S[2][n] + gA * (f2 * w);
-      S[3][n] = S[3][n] + gC * (f3 * w);
-      S[4][n] = S[4][n] + gCH * (f3 * w);
-    }
+    acc_point(D, Na, R, P.j[0], P.j[1], [&](int n) { return P.F[n]; },
+              [&](int n) { return P.fr[n]; }, P.w * TRF, S);
   }
 }
 
 // regular_pair<4> with the source element's 16 points read from src
 __device__ void regular_pair_tab(const QuadDev &D, const double *Ea, const QSrc *src, int pI,
-                                 zd out[3][10]) {
-  zd S[5][10];
-  for (int k = 0; k < 5; ++k)
-    for (int n = 0; n < 10; ++n) S[k][n] = zd{0, 0};
-  for (int j = 0; j < 4; ++j)
-    for (int i = 0; i < 4; ++i) outer_point_tab<4>(D, Ea, src, pI, i, j, S);
-  combine(D, S, out);
+                                 zd S[3][10]) {
+  zero30(S);
+#pragma unroll 1
+  for (int ij = 0; ij < 16; ++ij) outer_point_tab<4>(D, Ea, src, pI, ij & 3, ij >> 2, S);
 }
 
 __device__ inline int pair_class(const QuadTopo &T, int s, int t, int *side) {
@@ -348,7 +344,7 @@ __device__ inline void store30(zd out[3][10], zd *dst) {
 // dense fill, rows [s0, s0 + rows): workgroup = (element t, 64 rows), the
 // regular pairs (no shared node) on the element's source table; self,
 // edge- and corner-adjacent pairs come from the list kernels
-__global__ void __launch_bounds__(64) k_quad_regular_grid(QuadDev D, QuadTopo T, int s0, int rows,
+__global__ void __launch_bounds__(64, 2) k_quad_regular_grid(QuadDev D, QuadTopo T, int s0, int rows,
                                                           int nrb, zd *sums) {
   __shared__ QSrc src[16];
   const int t = blockIdx.x / nrb, rb = blockIdx.x - t * nrb;
@@ -417,14 +413,11 @@ __global__ void __launch_bounds__(64) k_quad_corner(QuadDev D, QuadTopo T, const
     qsrc_point<6>(D, T.el + (size_t)t * 24, threadIdx.x / 6, threadIdx.x % 6, src[threadIdx.x]);
   __syncthreads();
   const int ii = T.edge_p[5 * s] - 1, pI = T.edge_p[5 * s + 1];
-  zd S[5][10];
-  for (int k = 0; k < 5; ++k)
-    for (int n = 0; n < 10; ++n) S[k][n] = zd{0, 0};
+  zd S[3][10];
+  zero30(S);
   if (threadIdx.x < 36)
     outer_point_tab<6>(D, T.el + (size_t)ii * 24, src, pI, threadIdx.x % 6, threadIdx.x / 6, S);
-  zd r[3][10];
-  combine(D, S, r);
-  block_reduce30(r, out + (size_t)blockIdx.x * 30);
+  block_reduce30(S, out + (size_t)blockIdx.x * 30);
 }
 
 // self term at one outer point: Integration_KABCD_Taylor_ST_4FEdge (:299-380),
@@ -432,7 +425,7 @@ __global__ void __launch_bounds__(64) k_quad_corner(QuadDev D, QuadTopo T, const
 // 6-10) at unit value; the term is linear in the test function's value, so
 // function pI's is fedge(pI - 1, mu, nu) times the result of its direction
 __device__ void taylor_point(const QuadDev &D, int dir, double mu, double nu, const double *El,
-                             zd out[3][10]) {
+                             zd S[3][10]) {
   double dk[8], de[8], Eu[3] = {0, 0, 0}, Ev[3] = {0, 0, 0}, Ra[3];
   shape_diff(mu, nu, dk, de);
   for (int d = 0; d < 3; ++d) {
@@ -448,9 +441,11 @@ __device__ void taylor_point(const QuadDev &D, int dir, double mu, double nu, co
   const double pb[5] = {atan((1 - nu) / (1 - mu)), QPI - atan((1 - nu) / (1 + mu)),
                         QPI + atan((1 + nu) / (1 + mu)), 2 * QPI - atan((1 + nu) / (1 - mu)),
                         2 * QPI + atan((1 - nu) / (1 - mu))};
-  zd S[5][10];
-  for (int k = 0; k < 5; ++k)
-    for (int n = 0; n < 10; ++n) S[k][n] = zd{0, 0};
+  zero30(S);
+  double ju[3], jv[3];
+  cross3(gp.nq, gp.au, ju);
+  cross3(gp.nq, gp.av, jv);
+  const zd cE = D.riwe * D.ceps;
   for (int m = 0; m < 4; ++m) {
     const double a = (pb[m + 1] - pb[m]) / 2, cc = (pb[m + 1] + pb[m]) / 2;
     for (int i = 0; i < 15; ++i) {
@@ -460,25 +455,15 @@ __device__ void taylor_point(const QuadDev &D, int dir, double mu, double nu, co
       double A[3];
       for (int d = 0; d < 3; ++d) A[d] = -Eu[d] * cp - Ev[d] * sp;
       const double Aamp = sqrt(dot3(A, A));
-      double rho2;
-      if (m == 0) rho2 = (1 - nu) / sin(QPI - phi);
-      else if (m == 1) rho2 = fabs((1 + mu) / cos(QPI - phi));
-      else if (m == 2) rho2 = fabs((1 + nu) / cos(1.5 * QPI - phi));
-      else rho2 = fabs((1 - mu) / cos(phi));
-      // ff_phi_AB_Edge (:621-637): the 1/rho parts of KA and KB
-      double bb[3];
+      const double rho2 = m == 0   ? (1 - nu) / sp
+                          : m == 1 ? fabs((1 + mu) / cp)
+                          : m == 2 ? fabs((1 + nu) / sp)
+                                   : fabs((1 - mu) / cp);
+      // ff_phi_AB_Edge (:621-637): the 1/rho parts of KA and KB, taken out at
+      // every rho and added back as their integral
+      double bb[3], t[3];
       for (int d = 0; d < 3; ++d) bb[d] = -A[d] / (Aamp * Aamp * Aamp) / (4 * QPI);
-      double fA[10], fB[10];
-      for (int n = 0; n < 10; ++n) {
-        const double f = fedge(n, mu, nu);
-        const double *v = n < 5 ? gp.au : gp.av;
-        const double Nq[3] = {f * v[0], f * v[1], f * v[2]};
-        double aa[3], t[3];
-        cross3(gp.nq, Nq, aa);
-        cross3(aa, bb, t);
-        fA[n] = dot3(Na, t) * gp.JJ;
-        fB[n] = dot3(Na, bb) * gp.JJ * (fedge_rot(n, mu, nu) / gp.JJ);
-      }
+      double T0 = log(fabs(rho2) * Aamp) * D.w15[i] * a;
       for (int j = 0; j < 5; ++j) {
         const double rho = rho2 / 2 * (1 + D.x5[j]);
         const double mq = mu + rho * cp, nq = nu + rho * sp;
@@ -489,21 +474,23 @@ __device__ void taylor_point(const QuadDev &D, int dir, double mu, double nu, co
         for (int d = 0; d < 3; ++d) R[d] = Ra[d] - Rq[d];
         const double TRF = 0.5 * rho2 * D.w15[i] * D.w5[j] * a;
         acc_ff(D, Na, R, gq, mq, nq, rho * TRF, S);
-        for (int n = 0; n < 10; ++n) {
-          S[0][n].x -= 2 * fA[n] / rho * TRF;
-          S[1][n] = S[1][n] - D.ceps * (fB[n] / rho * TRF);
-          S[2][n].x -= 2 * fB[n] / rho * TRF;
-        }
+        T0 -= TRF / rho;
       }
-      const double T0 = log(fabs(rho2) * Aamp) * D.w15[i] * a;
+      cross3(ju, bb, t);
+      const double fu = 2 * T0 * dot3(Na, t) * gp.JJ;
+      cross3(jv, bb, t);
+      const double fv = 2 * T0 * dot3(Na, t) * gp.JJ;
+      const double fb = T0 * dot3(Na, bb);
+      const zd bE = cE * fb, bH = D.nriwm * (2 * fb);
+#pragma unroll
       for (int n = 0; n < 10; ++n) {
-        S[0][n].x += 2 * fA[n] * T0;
-        S[1][n] = S[1][n] + D.ceps * (fB[n] * T0);
-        S[2][n].x += 2 * fB[n] * T0;
+        const double rot = fedge_rot(n, mu, nu);
+        S[0][n].x += (n < 5 ? fu : fv) * fedge(n, mu, nu);
+        S[1][n] = S[1][n] + bE * rot;
+        S[2][n] = S[2][n] + bH * rot;
       }
     }
   }
-  combine(D, S, out);
 }
 
 // self terms of all ten test functions of element els[blockIdx.x] against
@@ -666,9 +653,8 @@ __global__ void __launch_bounds__(128) k_quad_edge_adj(QuadDev D, QuadTopo T, co
     double pab[2];
     ea_psi(ll, mm, nn, th, pab);
     const double pam = (pab[1] - pab[0]) / 2, pbm = (pab[1] + pab[0]) / 2;
-    zd S[5][10];
-    for (int k = 0; k < 5; ++k)
-      for (int n = 0; n < 10; ++n) S[k][n] = zd{0, 0};
+    zd r[3][10];
+    zero30(r);
     for (int i3 = 0; i3 < 5; ++i3) {
       const double ps = pam * x[i3] + pbm;
       double mab[2];
@@ -694,12 +680,10 @@ __global__ void __launch_bounds__(128) k_quad_edge_adj(QuadDev D, QuadTopo T, co
           rloc(muq, nuq, Eq, Rq);
           for (int d = 0; d < 3; ++d) R[d] = Ra[d] - Rq[d];
           const double TRF = lam * w[i1] * ga.JJ * (X * X) * cps;
-          acc_ff(D, Na, R, gq, muq, nuq, (tam * w[i4]) * (pam * w[i3]) * (mam * w[i2]) * TRF, S);
+          acc_ff(D, Na, R, gq, muq, nuq, (tam * w[i4]) * (pam * w[i3]) * (mam * w[i2]) * TRF, r);
         }
       }
     }
-    zd r[3][10];
-    combine(D, S, r);
     // back to the unrotated source functions
     for (int n = 1; n <= 10; ++n) {
       int iq, sq_;
@@ -1059,7 +1043,7 @@ __device__ inline int upper_box(const int64_t *off, int b0, int b1, int64_t g) {
   return lo;
 }
 
-__global__ void __launch_bounds__(64) k_qn_regular(QuadDev D, QuadTopo T, int b0, int b1,
+__global__ void __launch_bounds__(64, 2) k_qn_regular(QuadDev D, QuadTopo T, int b0, int b1,
                                                    const int64_t *toff, const int64_t *pbase,
                                                    const int *tb_off, const int *tb_list,
                                                    const int *box_first, const int *box_count,
@@ -1177,7 +1161,7 @@ __global__ void __launch_bounds__(256) k_quad_field(QuadDev D, QuadTopo T, const
         const double R[3] = {Ra[0] - Rq[0], Ra[1] - Rq[1], Ra[2] - Rq[2]};
         const double nR = sqrt(dot3(R, R));
         zd G, DG;
-        qgreen(D.k1, nR, G, DG);
+        qgreen(D.k1, nR, 1.0 / nR, G, DG);
         const zd gg[3] = {DG * (R[0] / nR), DG * (R[1] / nR), DG * (R[2] / nR)};
         const double ff = g.JJ * D.w5[i] * D.w5[j];
         for (int n = 0; n < 10; ++n) {
@@ -1392,6 +1376,9 @@ void quad_constants(const spk_params &p, QuadDev *D, zd *eta_a, zd *eta12) {
   D->ceps = Z(1.0 + 1.0 / er2);
   D->iwe = Z(C(0.0, 1.0) * omega * kEps0);
   D->iwm = Z(C(0.0, 1.0) * omega * kMy0);
+  D->riwe = zd{1.0, 0.0} / D->iwe;
+  D->nriwm = zd{-1.0, 0.0} / D->iwm;
+  D->niwe = -D->iwe;
   gauss_legendre(4, D->x4, D->w4);
   gauss_legendre(5, D->x5, D->w5);
   gauss_legendre(6, D->x6, D->w6);
