@@ -40,15 +40,14 @@ HBM_PEAK_GBS = 8000.0
 # default workload (100 x 100 cells, 10 lambda, ICTF, complex128), each counter
 # scaled by what it reads for a plain 1 GiB device copy (FETCH x 2.0,
 # WRITE x 1.0); profiles/matvec_traffic_rough10x10_ictf.txt and
-# profiles/near_spmv_bf16_rough10x10_ictf.txt, profiles/near_spmv_fp8_rough10x10_ictf.txt
-MEASURED_TRAFFIC = {("near_spmv", 100, 10.0, "fp64"): 1.8555e9,
-                    ("aggregation", 100, 10.0, "fp64"): 1.4732e9,
-                    ("disaggregation", 100, 10.0, "fp64"): 1.6627e9,
-                    ("near_spmv", 100, 10.0, "c64"): 0.9289e9,
-                    ("aggregation", 100, 10.0, "c64"): 0.7573e9,
-                    ("disaggregation", 100, 10.0, "c64"): 0.8181e9,
-                    ("near_spmv_bf16", 100, 10.0, "bf16"): 0.4716e9,
-                    ("near_spmv_fp8", 100, 10.0, "fp8"): 0.2462e9}
+# profiles/near_spmv_fp8_rough10x10_ictf.txt
+MEASURED_TRAFFIC = {("near_spmv", 100, 10.0, "fp64"): 1.4146e9,
+                    ("aggregation", 100, 10.0, "fp64"): 0.7925e9,
+                    ("disaggregation", 100, 10.0, "fp64"): 0.9551e9,
+                    ("near_spmv", 100, 10.0, "c64"): 0.7166e9,
+                    ("aggregation", 100, 10.0, "c64"): 0.4008e9,
+                    ("disaggregation", 100, 10.0, "c64"): 0.4676e9,
+                    ("near_spmv_fp8", 100, 10.0, "fp8"): 0.2004e9}
 
 
 def _sync():

@@ -301,8 +301,8 @@ NearArgs near_args(const spk_handle *h) {
 
 // The block's coefficients for the triangle kernel, or false where it does not
 // apply: formulations with normal components or with each medium's own K,
-// other rules than the three-point one, and surfaces of more than some
-// thousand wavelengths (side D), beyond sincos_near's arguments.
+// other rules than the three-point one, and octree sides D beyond
+// sincos_near's arguments (some million wavelengths).
 bool make_tri_form(const NearArgs &a, double D, TriForm *q) {
   if (a.ngp != 3) return false;
   for (int i = 0; i < 3; ++i)
