@@ -470,11 +470,11 @@ int spk_profile_matvec_c64(spk_handle *h, int reps, double *ms, double *bytes);
 /* No counterpart in the reference: timing of the near-field preconditioner's
  * SpMV (bf16 blocks, complex64 vectors; SPK_PRECOND_NEAR_FIELD on an
  * SPK_MIXED handle) with HIP events on the handle's stream: *ms = mean over
- * reps launches, *bytes = its algorithmic HBM bytes (16 B per 2x2 block,
+ * reps launches, *bytes = its algorithmic HBM bytes (4 B per kept component,
  * x read and y written at 8 B per complex). */
 int spk_profile_near_bf(spk_handle *h, int reps, double *ms, double *bytes);
 /* No counterpart in the reference: the same timing for the single-vector
- * preconditioner's fp8 copy (OCP E4M3FN, 8 B per 2x2 block plus 16 B of
+ * preconditioner's fp8 copy (OCP E4M3FN, 2 B per kept component plus 16 B of
  * per-row component scales per edge). */
 int spk_profile_near_f8(spk_handle *h, int reps, double *ms, double *bytes);
 

@@ -44,6 +44,13 @@ def test_products_of_the_kept_components(form, s_opt, eps):
     for tr in (False, True):
         s.set_transposed(tr)
         Z = A.T if tr else A
+        if tr:  # the four components again, in the transposed blocks' order
+            it, jt, vt = s.near_csr()
+            vt = vt.reshape(-1, 4)
+            for i in range(2):
+                for j in range(2):
+                    d = sp.csr_matrix((vt[:, 2 * i + j], jt, it), shape=(n, n)) - Z.tocsr()[i * n:(i + 1) * n, j * n:(j + 1) * n]
+                    assert abs(d).max() <= 1e-15 * np.abs(v[:, 2 * j + i]).max()
         Y = np.stack([Z @ x.astype(np.complex128) for x in X])
         assert half_err(s.matvec_parts(X[0].astype(np.complex128))[0], Y[0], n) < 1e-12, tr
         for fmt, tol in (("c64", 2e-6), ("bf16", 5e-3), ("fp8", 6e-2)):
