@@ -8,11 +8,10 @@
 // index s mapped to consecutive lanes everywhere (coalesced [..][S] rows).
 // Near SpMV: one workgroup per (leaf box, row chunk) over the box's dense
 // block matrix, x gathered once into LDS.
-#include <algorithm>
-
 #include <hipcub/hipcub.hpp>
 
 #include "spk_device.h"
+#include "spk_scat.h"
 #include "spk_fp8.h"
 
 namespace spk {
@@ -3206,11 +3205,8 @@ void launch_scattered(const ScatArgs &a, double reach, const FnRec *fn, const zd
   if (a.npts <= 0) return;
   const int64_t ns = 6 * (int64_t)a.N;
   const int tiles = nblk(a.npts, 64);
-  // chunks of whole groups of 64 sources: enough for three waves on every SIMD
-  // (3072 workgroups), as long as their sums fit the workspace
-  int64_t nch = std::max<int64_t>(1, std::min<int64_t>(3072 / tiles, kScatPartials / a.npts));
-  int64_t per = ((ns + nch - 1) / nch + 63) / 64 * 64;
-  nch = (ns + per - 1) / per;
+  int64_t nch;
+  const int64_t per = scat_chunk(ns, a.npts, kScatPartials, &nch);
   const bool lossy = a.k1.y != 0.0, near = fabs(a.k1.x) * reach < 1e8;
   auto *f = near ? (lossy ? k_scattered<true, true> : k_scattered<true, false>)
                  : (lossy ? k_scattered<false, true> : k_scattered<false, false>);

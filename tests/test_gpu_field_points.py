@@ -1,6 +1,6 @@
-"""The scattered field over its launch shapes (one point, a tile's edges, enough
-points for a single chunk of sources), media and distances (arguments beyond
-the short reduction of sine and cosine), against the oracle.
+"""The scattered field over its launch shapes (one point, a tile's edges, chunks
+of 8, 16 and 64 sources, enough points for a single chunk), media and distances
+(arguments beyond the short reduction of sine and cosine), against the oracle.
 
 Tolerance: a sum of about 10^4 terms in FP64, 1e-12; at a distance of a
 kilometre k R is 1e10 and its rounding alone 1e-6.
@@ -17,7 +17,8 @@ LAM = 633e-9
 
 @pytest.mark.parametrize("npts,dist,eps1,tol", [
     (1, 3 * LAM, 1.0, 1e-12), (63, 2 * LAM, 1.0, 1e-12), (64, 2 * LAM, 1.3 - 0.05j, 1e-12),
-    (65, 1e3 * LAM, 1.0, 1e-11), (7, 1e3, 1.0, 1e-5), (131073, 2 * LAM, 1.0, 1e-12),
+    (65, 1e3 * LAM, 1.0, 1e-11), (900, 2 * LAM, 1.3 - 0.05j, 1e-12), (7, 1e3, 1.0, 1e-5),
+    (131073, 2 * LAM, 1.0, 1e-12),
 ])
 def test_scattered_field(npts, dist, eps1, tol):
     pp, tt = meshes.rough_surface(9, 7, 0.9, 0.7, 0.1, 0.5, 3, LAM)
