@@ -529,11 +529,12 @@ __device__ inline void finish_D(const NearArgs &A, zd *D) {
 }
 
 // block g in the layout of NearRel
-__device__ inline void put_block(const NearRel &rel, int64_t g, const zd *D, zd *blocks) {
-  if (rel.nc == 3) {
+template <int NC>
+__device__ inline void put_block(zd ic, int64_t g, const zd *D, zd *blocks) {
+  if constexpr (NC == 3) {
     blocks[3 * g] = D[0];
     blocks[3 * g + 1] = D[1];
-    blocks[3 * g + 2] = D[3] * rel.ic;
+    blocks[3 * g + 2] = D[3] * ic;
   } else {
     for (int k = 0; k < 4; ++k) blocks[4 * g + k] = D[k];
   }
@@ -641,8 +642,11 @@ __global__ void __launch_bounds__(128) k_near_singular(NearArgs A, int ntask, co
   for (int k = 0; k < 4; ++k) zz[4 * (int64_t)t + k] = z[k];
 }
 
-template <bool NEED_N>
-__global__ void __launch_bounds__(256) k_near_regular(NearArgs A, NearRel rel, int64_t nnz,
+// NC components (NearRel; ic: 1 / c) as a template: the choice at run time kept
+// six more scalar registers spilled through the loop, 1.60 -> 1.63 ms at 4,720
+// edges of MCTF2
+template <bool NEED_N, int NC>
+__global__ void __launch_bounds__(256) k_near_regular(NearArgs A, zd ic, int64_t nnz,
                                                       const uint8_t *cls, const int *base_a,
                                                       const zd *zz, zd *blocks) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -667,7 +671,7 @@ __global__ void __launch_bounds__(256) k_near_regular(NearArgs A, NearRel rel, i
     accumulate_D(A, D, z);
   }
   finish_D(A, D);
-  put_block(rel, g, D, blocks);
+  put_block<NC>(ic, g, D, blocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -993,7 +997,10 @@ __global__ void __launch_bounds__(256, 2) k_near_tri(NearArgs A, TriForm Q, Near
         D[1] = D[1] + Q.c[2] * K;
         D[2] = D[2] + Q.c[3] * Ka;
         D[3] = D[3] + Q.c[4] * T1 + Q.c[5] * T2;
-        put_block(rel, g, D, blocks);
+        if (rel.nc == 3)
+          put_block<3>(rel.ic, g, D, blocks);
+        else
+          put_block<4>(rel.ic, g, D, blocks);
       }
       __syncthreads();
     }
@@ -1070,12 +1077,11 @@ void launch_near_regular(const NearArgs &a, const NearRel &rel, int64_t nnz, con
                          const int *base_a, const zd *zz, zd *blocks, hipStream_t st) {
   if (nnz <= 0) return;
   const bool need_n = (a.form == SPK_JMCFIE || a.form == SPK_CNF || a.form == SPK_MNMF);
-  if (need_n)
-    hipLaunchKernelGGL(k_near_regular<true>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, rel, nnz,
-                       cls, base_a, zz, blocks);
-  else
-    hipLaunchKernelGGL(k_near_regular<false>, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, rel, nnz,
-                       cls, base_a, zz, blocks);
+  auto *f = need_n          ? k_near_regular<true, 4>  // they keep four components
+            : rel.nc == 3 ? k_near_regular<false, 3>
+                          : k_near_regular<false, 4>;
+  hipLaunchKernelGGL(f, dim3(nblk(nnz, 256)), dim3(256), 0, st, a, rel.ic, nnz, cls, base_a, zz,
+                     blocks);
 }
 
 // The triangle kernel takes the formulations without normal components and
