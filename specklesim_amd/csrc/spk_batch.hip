@@ -578,7 +578,7 @@ __device__ __forceinline__ void kb_disagg_mx_part(int N, PatLay lay, int R, cons
                                                   const int *box_count, const int *perm,
                                                   const zf *rt, const zf *W, zf sc1, zf sc2, zf *yp,
                                                   float4 *wl) {
-  constexpr int PM = HALF ? 2 : 1;
+  constexpr int PM = HALF ? 2 : 1, UN = HALF ? 1 : 2;
   const int b = tile_box[blockIdx.x], p0 = tile_p0[blockIdx.x];
   const int cnt = min(128, box_first[b] + box_count[b] - p0);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -588,7 +588,8 @@ __device__ __forceinline__ void kb_disagg_mx_part(int N, PatLay lay, int R, cons
   const int k = blockIdx.y >> 1, L = lay.L[k];
   const zf *F = rt + (size_t)(p0 + min(ew + m, cnt - 1)) * lay.stride() + lay.row(k, 0);
   const zf *Wb = W + ((size_t)b * 8 + k * 4) * lay.SW * R;
-  const int sblk = ((L + 63) / 64) * kMxSC;
+  constexpr int Q = HALF ? 32 : 16;  // entries that a half is a multiple of
+  const int sblk = ((L + 2 * Q - 1) / (2 * Q)) * Q;
   const int s_lo = (blockIdx.y & 1) * sblk, s_hi = min(L, s_lo + sblk);
   mxf4 er = {0.f, 0.f, 0.f, 0.f}, ei = er, hr = er, hi = er;
   // both pattern rows at entries s + 4g .. s + 4g + 3 (pairs clamped, L is even)
@@ -619,6 +620,7 @@ __device__ __forceinline__ void kb_disagg_mx_part(int N, PatLay lay, int R, cons
     }
     __syncthreads();
     if (!active) continue;
+#pragma unroll UN
     for (int sg = 0; sg < kMxSC && s0 + sg < s_hi; sg += 16) {
       float4 nx[4];
       load(s0 + sg + 16, nx);
@@ -1197,8 +1199,11 @@ __global__ void __launch_bounds__(256) kb_agg_mx64(PatLay lay, int R, const int 
 
 // disaggregation: workgroup = (up to 128 edges of a box; blockIdx.y = half of
 // one medium's entries), wave = 16 edges; k-step = 4 entries (lane group g
-// takes entry s + 4g + j in step j); W staged in LDS 16 entries at a time as
-// [P/M][entry][e/h][r]; HALF as in kb_disagg_mx
+// takes entry s + 4g + j in step j); W staged in LDS as [P/M][entry][e/h][r],
+// kMx64SC entries of a HALF medium's P and M or 2 kMx64SC of the other's W, a
+// barrier pair for 32 products of a lane either way (with half of that a whole
+// row took 268 us for 219 at 4,720 edges and two media with losses, 685 for 573
+// at 19,040); HALF as in kb_disagg_mx
 constexpr int kMx64SC = 16;
 template <bool HALF>
 __device__ __forceinline__ void kb_disagg_mx64_part(int N, PatLay lay, int R, const int *tile_box,
@@ -1206,7 +1211,7 @@ __device__ __forceinline__ void kb_disagg_mx64_part(int N, PatLay lay, int R, co
                                                     const int *box_count, const int *perm,
                                                     const zd *rt, const zd *W, zd sc1, zd sc2,
                                                     zd *yp, double4 *wl) {
-  constexpr int PM = HALF ? 2 : 1;
+  constexpr int NG = HALF ? 1 : 2, SC = NG * kMx64SC;  // groups of 16 entries a staging
   const int b = tile_box[blockIdx.x], p0 = tile_p0[blockIdx.x];
   const int cnt = min(128, box_first[b] + box_count[b] - p0);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1217,7 +1222,7 @@ __device__ __forceinline__ void kb_disagg_mx64_part(int N, PatLay lay, int R, co
   const double2 *F = reinterpret_cast<const double2 *>(
       rt + (size_t)(p0 + min(ew + m, cnt - 1)) * lay.stride() + lay.row(k, 0));
   const zd *Wb = W + ((size_t)b * 8 + k * 4) * lay.SW * R;
-  const int sblk = ((L + 31) / 32) * kMx64SC;
+  const int sblk = ((L + 2 * SC - 1) / (2 * SC)) * SC;
   const int s_lo = (blockIdx.y & 1) * sblk, s_hi = min(L, s_lo + sblk);
   mxd4 er = {0.0, 0.0, 0.0, 0.0}, ei = er, hr = er, hi = er;
   // both pattern rows at entries s + 4g .. s + 4g + 3 (clamped)
@@ -1231,70 +1236,73 @@ __device__ __forceinline__ void kb_disagg_mx64_part(int N, PatLay lay, int R, co
   };
   double2 cur[8];
   if (active && s_lo < s_hi) load(s_lo, cur);
-  for (int s0 = s_lo; s0 < s_hi; s0 += kMx64SC) {
+  for (int s0 = s_lo; s0 < s_hi; s0 += SC) {
     __syncthreads();
     {
       // W[it][s0 + i][r] -> wl as complex [((pm * SC + i) * 2 + half) * 16 + r][jj], it = 2half + jj
       zd *wc = reinterpret_cast<zd *>(wl);
 #pragma unroll
-      for (int u = 0; u < 2 * PM; ++u) {
+      for (int u = 0; u < 4; ++u) {
         const int t = threadIdx.x + 512 * u;
-        const int r = t & 15, i = (t >> 4) & (kMx64SC - 1), it = (t >> 8) & 3, pm = t >> 10;
+        const int r = t & 15, i = (t >> 4) & (SC - 1), q = t / (16 * SC), it = q & 3, pm = q >> 2;
         const int s = s0 + i;
         const bool ok = r < R && s < s_hi;
         const zd v = Wb[((size_t)it * lay.SW + pm * L + min(s, L - 1)) * R + min(r, R - 1)];
         const int half = it >> 1, jj = it & 1;
-        wc[(((pm * kMx64SC + i) * 2 + half) * 16 + r) * 2 + jj] = ok ? v : zd{0.0, 0.0};
+        wc[(((pm * SC + i) * 2 + half) * 16 + r) * 2 + jj] = ok ? v : zd{0.0, 0.0};
       }
     }
     __syncthreads();
     if (!active) continue;
-    double2 nx[8];
-    load(s0 + kMx64SC, nx);
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = 4 * g + j;
-      const double4 we = wl[(i * 2 + 0) * 16 + m];  // (e,a), (e,b)
-      const double4 wh = wl[(i * 2 + 1) * 16 + m];  // (h,a), (h,b)
-      const double ar = cur[j].x, ai = cur[j].y, br = cur[4 + j].x, bi = cur[4 + j].y;
-      er = SPK_MFMA64(ar, we.x, er);
-      ei = SPK_MFMA64(ar, we.y, ei);
-      hr = SPK_MFMA64(ar, wh.x, hr);
-      hi = SPK_MFMA64(ar, wh.y, hi);
-      if constexpr (HALF) {
-        const double4 me = wl[((kMx64SC + i) * 2 + 0) * 16 + m];
-        const double4 mh = wl[((kMx64SC + i) * 2 + 1) * 16 + m];
-        er = SPK_MFMA64(ai, me.x, er);
-        ei = SPK_MFMA64(ai, me.y, ei);
-        hr = SPK_MFMA64(ai, mh.x, hr);
-        hi = SPK_MFMA64(ai, mh.y, hi);
-        er = SPK_MFMA64(br, we.z, er);
-        ei = SPK_MFMA64(br, we.w, ei);
-        hr = SPK_MFMA64(br, wh.z, hr);
-        hi = SPK_MFMA64(br, wh.w, hi);
-        er = SPK_MFMA64(bi, me.z, er);
-        ei = SPK_MFMA64(bi, me.w, ei);
-        hr = SPK_MFMA64(bi, mh.z, hr);
-        hi = SPK_MFMA64(bi, mh.w, hi);
-      } else {
-        er = SPK_MFMA64(-ai, we.y, er);
-        ei = SPK_MFMA64(ai, we.x, ei);
-        hr = SPK_MFMA64(-ai, wh.y, hr);
-        hi = SPK_MFMA64(ai, wh.x, hi);
-        er = SPK_MFMA64(br, we.z, er);
-        ei = SPK_MFMA64(br, we.w, ei);
-        hr = SPK_MFMA64(br, wh.z, hr);
-        hi = SPK_MFMA64(br, wh.w, hi);
-        er = SPK_MFMA64(-bi, we.w, er);
-        ei = SPK_MFMA64(bi, we.z, ei);
-        hr = SPK_MFMA64(-bi, wh.w, hr);
-        hi = SPK_MFMA64(bi, wh.z, hi);
+    for (int q = 0; q < NG; ++q) {
+      double2 nx[8];
+      load(s0 + 16 * q + 16, nx);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 16 * q + 4 * g + j;
+        const double4 we = wl[(i * 2 + 0) * 16 + m];  // (e,a), (e,b)
+        const double4 wh = wl[(i * 2 + 1) * 16 + m];  // (h,a), (h,b)
+        const double ar = cur[j].x, ai = cur[j].y, br = cur[4 + j].x, bi = cur[4 + j].y;
+        er = SPK_MFMA64(ar, we.x, er);
+        ei = SPK_MFMA64(ar, we.y, ei);
+        hr = SPK_MFMA64(ar, wh.x, hr);
+        hi = SPK_MFMA64(ar, wh.y, hi);
+        if constexpr (HALF) {
+          const double4 me = wl[((SC + i) * 2 + 0) * 16 + m];
+          const double4 mh = wl[((SC + i) * 2 + 1) * 16 + m];
+          er = SPK_MFMA64(ai, me.x, er);
+          ei = SPK_MFMA64(ai, me.y, ei);
+          hr = SPK_MFMA64(ai, mh.x, hr);
+          hi = SPK_MFMA64(ai, mh.y, hi);
+          er = SPK_MFMA64(br, we.z, er);
+          ei = SPK_MFMA64(br, we.w, ei);
+          hr = SPK_MFMA64(br, wh.z, hr);
+          hi = SPK_MFMA64(br, wh.w, hi);
+          er = SPK_MFMA64(bi, me.z, er);
+          ei = SPK_MFMA64(bi, me.w, ei);
+          hr = SPK_MFMA64(bi, mh.z, hr);
+          hi = SPK_MFMA64(bi, mh.w, hi);
+        } else {
+          er = SPK_MFMA64(-ai, we.y, er);
+          ei = SPK_MFMA64(ai, we.x, ei);
+          hr = SPK_MFMA64(-ai, wh.y, hr);
+          hi = SPK_MFMA64(ai, wh.x, hi);
+          er = SPK_MFMA64(br, we.z, er);
+          ei = SPK_MFMA64(br, we.w, ei);
+          hr = SPK_MFMA64(br, wh.z, hr);
+          hi = SPK_MFMA64(br, wh.w, hi);
+          er = SPK_MFMA64(-bi, we.w, er);
+          ei = SPK_MFMA64(bi, we.z, ei);
+          hr = SPK_MFMA64(-bi, wh.w, hr);
+          hi = SPK_MFMA64(bi, wh.z, hi);
+        }
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) cur[u] = nx[u];
+      for (int u = 0; u < 8; ++u) cur[u] = nx[u];
+    }
   }
   const int n = m;
   if (!active || n >= R) return;
@@ -1315,7 +1323,7 @@ __global__ void __launch_bounds__(512) kb_disagg_mx64(int N, PatLay lay, int R, 
                                                       const int *box_count, const int *perm,
                                                       const zd *rt, const zd *W, zd sc1, zd sc2,
                                                       zd *yp) {
-  __shared__ double4 wl[(MODE ? 2 : 1) * kMx64SC * 2 * 16];
+  __shared__ double4 wl[2 * kMx64SC * 2 * 16];
   if (MODE == 1 || (MODE == 2 && lay.half[blockIdx.y >> 1]))
     kb_disagg_mx64_part<true>(N, lay, R, tile_box, tile_p0, box_first, box_count, perm, rt, W, sc1,
                               sc2, yp, wl);
