@@ -1996,10 +1996,13 @@ void launch_batch_orth(int64_t n, int P, int maxk, const int *ks, const T *const
 // by the launch that needs it, so no launch only scales a vector.
 //   dot:  partial[s][c][g] = sum over the rows of chunk g of conj(V_s[:, c]) w_s
 //   upd:  h_c = sum_g partial / (m_c m_j), V_s[:, j + 1] = (w / m_j - sum h_c u_c) / q_j
-//         with q_j = |h|, which keeps the column near 1 whatever the operator's
-//         scale, pn[s][g] = |V_s[:, j + 1]|^2 over chunk g;
+//         with q_j = |h| (1 where h is zero), pn[s][g] = |V_s[:, j + 1]|^2 over
+//         chunk g;
 //         H[:, j] = h, H[j, j - 1] = q_(j-1) m_j, and m_j at H[kin, j - 1]
 //   tail: H[kin, kin - 1] after the last step
+// A column's length is |w_perp| / |h|: free of the operator's scale, near 1 where w
+// has a share of both, large where h is small (1e8 in complex64 where it is
+// rounding alone), which costs a floating format no digits.
 // All sums in a fixed order, in complex128.  Slot s: V = U + s * ldu (column c
 // at c * n), w: W + s * n, hb + s * ldh: (m_c, q_(c-1)) of column c,
 // H + s * (kin + 1) * kin (column-major, leading dimension kin + 1).

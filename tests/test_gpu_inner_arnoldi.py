@@ -1,7 +1,9 @@
 """The inner Arnoldi steps of the near-field preconditioned solves against
 flexible GMRES written out in numpy with the same operator and near blocks:
 inner lengths at the edges of the update's column groups, one vector and a
-batch (whose row chunks differ), FP64 handles.  The inner solve is the same
+batch (whose row chunks differ), on FP64 handles with the exact blocks and on
+mixed ones, whose columns are complex64 and whose product is the fp8 or bf16 one
+(in numpy too, one call of it per inner step).  The inner solve is the same
 mathematics in another order, so the outer iteration counts may differ by one
 where an estimate meets the tolerance; a wrong coefficient or scale in a
 column costs many.  Zero inner residuals (a right-hand side of zeros) end at
@@ -70,6 +72,43 @@ def test_outer_iterations_match_numpy(case, kin, tol):
                                      use_initial_guess=False, near_field=True, inner_iterations=kin)
     for r in range(2):
         assert abs(infos[r]["iters"] - want[r]) <= 1, (kin, r, infos[r], want[r])
+
+
+@pytest.fixture(scope="module")
+def mixed(case):
+    pp, tt = meshes.rough_surface(16, 16, 2.0, 2.0, 0.1, 0.5, 6, LAM)
+    return SieTriMlfmm(LAM, 2.25, formulation="ICTF", normal_convention=2,
+                       precision="mixed").precalculation_tri(pp, tt)
+
+
+# 4 to 8 vectors take complex64 blocks, 9 and more the matrix-core products
+@pytest.mark.parametrize("fmt,R,kin,tol", [
+    ("fp8", 1, 1, 0.1), ("fp8", 1, 9, 1e-3), ("fp8", 1, 64, 1e-6), ("bf16", 1, 33, 1e-5),
+    ("fp8", 3, 8, 1e-3), ("c64", 5, 9, 1e-3), ("c64", 5, 64, 1e-6), ("fp8", 10, 2, 0.03),
+    ("fp8", 10, 33, 1e-6), ("bf16", 10, 33, 1e-6),
+])
+def test_low_precision_inner_steps_match_numpy(mixed, monkeypatch, fmt, R, kin, tol):
+    s = mixed
+    monkeypatch.setenv("SPK_NEAR_F8", "0" if fmt == "bf16" else "1")
+    monkeypatch.setenv("SPK_RELAX", "0")
+
+    def near(z):
+        X = np.tile(z.astype(np.complex64), (R if R > 3 else 1, 1))
+        return s.near_product_lowp(X, fmt, batched=R > 3)[0].astype(np.complex128)
+
+    B = [s.get_vector_b_tri(*plane_wave(0.05 * r, 0.0, 2, "TM")) for r in range(R)]
+    pick = sorted({0, R - 1})
+    want = {r: _gmres(s.calculate_vector_b_tri, lambda v: _gmres(near, lambda z: z, v, kin)[0],
+                      B[r], 90, tol)[1] for r in pick}
+    bs = [DeviceBuffer(b.nbytes).upload(b) for b in B]
+    xs = [DeviceBuffer(32 * s.N) for _ in B]
+    kw = dict(tolerance=tol, use_initial_guess=False, near_field=True, inner_iterations=kin)
+    infos = (s.gmres_run_batch_device([d.ptr for d in bs], [d.ptr for d in xs], **kw) if R > 1
+             else [s.gmres_run_device(bs[0].ptr, xs[0].ptr, **kw)])
+    for r in pick:
+        x = xs[r].download()
+        assert np.linalg.norm(B[r] - s.calculate_vector_b_tri(x)) <= 1.01 * tol * np.linalg.norm(B[r])
+        assert abs(infos[r]["iters"] - want[r]) <= 1, (r, infos[r]["iters"], want[r])
 
 
 def test_zero_right_hand_side_in_a_batch(case):

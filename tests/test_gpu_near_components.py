@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 import scipy.sparse as sp
 
-from specklesim_amd import SieTriMlfmm, meshes
+from specklesim_amd import SieTriMlfmm, meshes, plane_wave
 
 pytestmark = pytest.mark.gpu
 LAM = 633e-9
@@ -93,3 +93,37 @@ def test_rows_per_wave(cells):
         yb = s.near_product_lowp(X, fmt, batched=True)[0].astype(np.complex128)
         assert half_err(y, ref, s.N) < tol, fmt
         assert half_err(yb, y, s.N) < max(2e-6, 5e-3 * (fmt == "fp8")), fmt
+
+
+@pytest.mark.parametrize("form", ["ICTF", "PMCHWT", "MCTF", "MCTF2"])
+def test_block_jacobi_of_the_kept_components(form):
+    """The four leaf boxes of this patch have one parent, so the block-Jacobi
+    inverse is the near field's: flexible GMRES with it takes the outer steps
+    that numpy takes with the near blocks solved, forward and transposed (one
+    more or less where an estimate meets the tolerance)."""
+    pp, tt = meshes.rough_surface(16, 16, 2.0, 2.0, 0.1, 0.5, 6, LAM)
+    s = SieTriMlfmm(LAM, 2.25, formulation=form, normal_convention=2).precalculation_tri(pp, tt)
+    n = s.N
+    ia, ja, v = s.near_csr()
+    v = v.reshape(-1, 4)
+    A = sp.bmat([[sp.csr_matrix((v[:, 2 * i + j], ja, ia), shape=(n, n)) for j in range(2)]
+                 for i in range(2)], format="csr").toarray()
+    b = s.get_vector_b_tri(*plane_wave(0.2, 0.0, 2, "TM"))
+    for tr in (False, True):
+        s.set_transposed(tr)
+        inv = np.linalg.inv(A.T if tr else A)
+        V, Z, W = [b / np.linalg.norm(b)], [], []
+        for j in range(40):
+            Z.append(inv @ V[j])
+            W.append(s.calculate_vector_b_tri(Z[j]))
+            c = np.linalg.lstsq(np.column_stack(W), b, rcond=None)[0]
+            if np.linalg.norm(b - np.column_stack(W) @ c) <= 1e-6 * np.linalg.norm(b):
+                break
+            q = np.linalg.qr(np.column_stack(V))[0]
+            w = W[j] - q @ (q.conj().T @ W[j])
+            V.append(w / np.linalg.norm(w))
+        x, inf = s.gmres_run(b, tolerance=1e-6, use_initial_guess=False, near_field="block_lu",
+                             max_iterations=40)
+        r = np.linalg.norm(b - s.calculate_vector_b_tri(x)) / np.linalg.norm(b)
+        assert abs(inf["iters"] - j - 1) <= 1 and r <= 1.01e-6, (tr, inf, j + 1, r)
+    s.set_transposed(False)
