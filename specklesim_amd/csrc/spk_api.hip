@@ -1806,9 +1806,10 @@ static double scat_reach(const spk_handle *h, int npts, const double *r) {
   return 4.0 * m;  // 2 sqrt(3) largest coordinate
 }
 
-// One field evaluation through device staging: the points dr[3*npts] are
-// copied in, one workgroup per point writes every component of dE, dH
-// [3*npts], which are copied out.
+// One field evaluation through device staging: the points are copied into
+// dr[3*npts], every component of dE, dH [3*npts] is written (triangles: by
+// k_scattered's chunks of sources and their sum, quadrilaterals: by a workgroup
+// per point) and copied out.
 static int scattered_staged(spk_handle *h, int npts, const double *r, const zd *d_x, double *E,
                             double *H, double *dr, zd *dE, zd *dH) {
   const ScatArgs a = scat_args(h, npts);

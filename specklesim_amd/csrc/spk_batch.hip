@@ -796,13 +796,14 @@ __global__ void __launch_bounds__(256) kb_near(int N, int R, const int *row_box,
 // so each complex product is four real ones into four accumulators:
 //   e_re += Z0r xer - Z0i xei + Z1r xhr - Z1i xhi,  e_im += Z0r xei + Z0i xer + ...
 //   h_re, h_im the same with Z2, Z3.
-// A lane loads the whole 2x2 block of its (row, column), 32 bytes; the
+// A lane loads the whole 2x2 block of its (row, column), 32 bytes or, with
+// three components (NearRel: Z2 is Z1), 24; the
 // columns' (xe, xh) of the 16 right-hand sides are staged in LDS, 128
 // columns at a time, and a wave loads its next 16 columns' blocks before it
 // multiplies the current ones.  Rows and columns past the end are clamped on
 // load (their x is zero in LDS, their results are not written).  The four
 // waves' sums are added in wave order through LDS.
-// BF: the blocks are the bf16 copy (one 16-byte load per block, widened to
+// BF: the blocks are the bf16 copy (one load of NC words per block, widened to
 // fp32 in registers).
 constexpr int kMxCols = 128;
 template <bool BF, int NC>
@@ -1338,7 +1339,8 @@ __global__ void __launch_bounds__(512) kb_disagg_mx64(int N, PatLay lay, int R, 
 // A[m][4g .. 4g+3] and B[4g .. 4g+3][n = m], D[4g + i][n] in element i, as
 // probed on the device).  One product covers 4 columns: k = 4 * column +
 // component, A = the bf16 block of (row, column) as stored: (Z0r, Z0i, Z1r,
-// Z1i) for the e rows and (Z2r, Z2i, Z3r, Z3i) for the h rows; B = x in bf16
+// Z1i) for the e rows and (Z2r, Z2i, Z3r, Z3i) for the h rows (with three
+// components, NearRel, the middle one serves both); B = x in bf16
 // arranged per (column, right-hand side) as (xer, -xei, xhr, -xhi) for the
 // real parts and (xei, xer, xhi, xhr) for the imaginary parts.  Products
 // accumulate in fp32.  Workgroup = (box, 16 rows), the 4 waves take every
@@ -1756,10 +1758,7 @@ __global__ void __launch_bounds__(256) kb_near_mxf8g(int N, int R, const int *gr
   }
 }
 
-// the preconditioner's product for 9..16 right-hand sides on the fp8 copy
-// (blocks, scale as k_near_spmv_f8 reads them); workgroups = row tiles of
-// 16 rows.  Two tiles per workgroup (x staged once for 32 rows, 156 VGPRs)
-// measured the same, 105 us at 16 vectors on the 10 x 10 lambda patch.
+// x of a batch for the fp8 products:
 // XB[(m * 2 + cur) * 16 + r] = x_r[m + cur N] in bf16 (re in the low half, im
 // in the high half), rounded to nearest even as bf16_pair rounds, zero for r >=
 // R; the second half scaled where NearRel asks for it.  Workgroup = 64

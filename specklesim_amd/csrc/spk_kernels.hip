@@ -757,11 +757,10 @@ __device__ inline double fma_sc(double a, double b, double c) {
   asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
   return d;
 }
-// sin and cos of |x| < 1e8: one quarter turn subtracted in two parts (exact to
-// 1e-25 there), Taylor
-// series to r^17 and r^16 on |r| <= pi/4 (truncation 1e-19 and 2e-18).  The
-// library's sincos carries the reduction of any argument, whose registers
-// spill in the fill kernels.
+// sin and cos of |x| < 1e8: quarter turns subtracted in two parts (what is left of
+// pi / 2 is 1e-25 there), Taylor series to r^17 and r^16 on |r| <= pi/4 (truncation
+// 1e-19 and 2e-18).  The library's sincos carries the reduction of any argument,
+// whose registers spill in the fill kernels.
 __device__ inline void sincos_near(double x, double *sn, double *cs) {
   const double n = rint(x * 0.63661977236758134308);
   double r = fma(-n, 1.5707963267948965580, x);
@@ -1221,7 +1220,7 @@ void launch_blu_scatter(int ngroups, int nmax, int N, const int *p0, const int *
 // triangles (offset from the leaf centre, weighted function value) go to LDS
 // once, then each thread takes every 128th sample: where both media keep half
 // of the samples (PatLay) those, else all S.  NEAR: sincos_near (arguments
-// below 1e5).  Bound by the FP64 ALU (12 exponentials a sample): 0.28 ms at
+// below 1e8).  Bound by the FP64 ALU (12 exponentials a sample): 0.28 ms at
 // 29,800 edges and 362 samples; with a thread per sample that repeated the
 // geometry and the library's sincos 0.90 ms.
 template <bool NEAR>
