@@ -44,7 +44,18 @@ def _far_err(g, X, far, y, batched):
     (8, 1.2 - 0.1j, 2.25 - 0.2j), (3, 1.0, 2.25),
 ])
 def test_products_on_half_and_whole_rows(mesh, K, eps1, eps2):
-    pp, tt = mesh
+    _check(*mesh, K, eps1, eps2)
+
+
+@pytest.mark.parametrize("K,eps1,eps2", [(12, 1.0, 2.25), (9, 1.0, 2.25 - 0.2j),
+                                         (8, 1.2 - 0.1j, 2.25 - 0.2j)])
+def test_boxes_of_more_edges_than_a_stage(K, eps1, eps2):
+    """147 to 176 edges a box: two stages of the single-vector aggregation's x
+    and two tiles of the matrix-core disaggregation."""
+    _check(*meshes.rough_surface(30, 30, 3.0, 3.0, 0.1, 0.5, 9, LAM), K, eps1, eps2)
+
+
+def _check(pp, tt, K, eps1, eps2):
     kw = dict(eps_r1=eps1, formulation="ICTF", normal_convention=2)
     o = O.Oracle(pp, tt, LAM, eps2, K=K, **kw)
     o.tree()

@@ -28,6 +28,8 @@ def _fin(pp, tt):
 def _mesh(kind):
     if kind == "sphere":
         return meshes.icosphere(2, 0.5 * LAM)
+    if kind == "wide":  # 1157 columns in one box's rows: two chunks
+        return meshes.rough_surface(21, 19, 2.1, 1.9, 0.1, 0.5, 6, LAM)
     pp, tt = meshes.rough_surface(15, 14, 1.5, 1.4, 0.1, 0.5, 6, LAM)
     return _fin(pp, tt) if kind == "fin" else (pp, tt)
 
@@ -41,6 +43,8 @@ def _mesh(kind):
     ("MCTF", "patch", 100, 4.0, 3),
     ("PMCHWT-S", "sphere", 4000, 2.25 - 0.3j, 3),
     ("PMCHWT-S", "patch", 50, 2.25, 3),
+    ("ICTF", "wide", 4000, 2.25, 3),
+    ("PMCHWT-S", "wide", 4000, 2.25 - 0.3j, 3),
     ("ICTF", "fin", 100, 2.25, 3),
     ("ICTF", "patch", 250, 2.25, 7),
     ("MCTF2", "patch", 250, 2.25, 3),
@@ -50,6 +54,7 @@ def test_near_blocks_equal_single_blocks(form, kind, s_opt, eps, ng):
     pp, tt = _mesh(kind)
     g = SieTriMlfmm(LAM, eps, formulation=form, ng=ng, tree_s_opt=s_opt).precalculation_tri(pp, tt)
     ia, ja, v = g.near_csr()
+    assert kind != "wide" or np.diff(ia).max() > 1024
     rows = np.repeat(np.arange(g.N), np.diff(ia))
     pick = np.random.default_rng(1).permutation(len(ja))[:6000]
     # every column of the first and the last row too
